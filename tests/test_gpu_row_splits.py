@@ -1,0 +1,76 @@
+"""Row splits and component folds at the sizes where they change: rows at and
+around the lane / 16-lane / chunk limits in the 64-source pull, and component
+minima over a giant component, pairs and isolated vertices."""
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+G = pytest.importorskip("graptor_amd")
+
+
+@pytest.fixture(scope="module", autouse=True)
+def device():
+    G.lib()
+    yield
+
+
+# rows at the limits of the lane (32), 16-lane (2048) and chunk (8192) splits
+HUBS = (1, 31, 32, 33, 64, 65, 2047, 2048, 2049, 8191, 8192, 8193, 16400)
+
+
+def hub_graph(n):
+    """Vertex i < len(HUBS) has edges to HUBS[i] later vertices; the others hang off them."""
+    src, dst = [], []
+    for i, d in enumerate(HUBS):
+        src.append(np.full(d, i, np.uint32))
+        dst.append((len(HUBS) + (np.arange(d) * 7 + i) % (n - len(HUBS))).astype(np.uint32))
+    return O.build_csr(n, np.concatenate(src), np.concatenate(dst))
+
+
+@pytest.mark.parametrize("reorder", [False, True])
+@pytest.mark.parametrize("k", [1, 15, 16, 17, 63, 64])
+def test_msbfs_pull_row_lengths(k, reorder):
+    n = 25013
+    index, nbrs = hub_graph(n)
+    src = (np.arange(k, dtype=np.uint32) * 389) % n
+    with G.Graph.from_csr(index, nbrs) as g:
+        if reorder:
+            g.reorder()
+        ref = O.msbfs_levels(index, nbrs, src)
+        for d in (G.DIR_PULL, G.DIR_AUTO):
+            lv, _ = g.msbfs(src, direction=d)
+            assert np.array_equal(lv, ref), d
+
+
+@pytest.mark.parametrize("reorder", [False, True])
+@pytest.mark.parametrize("n", [1, 2, 63, 257, 2049, 70001])
+def test_component_minima(n, reorder):
+    # a chain over the odd vertices (one giant component that starts at 1),
+    # pairs among the multiples of 8, the other even vertices alone
+    v = np.arange(n, dtype=np.uint32)
+    odd = v[v % 2 == 1]
+    pair = v[(v % 16 == 0) & (v + 8 < n)]
+    src = np.concatenate((odd[:-1], pair)) if len(odd) else pair
+    dst = np.concatenate((odd[1:], pair + 8)) if len(odd) else pair + 8
+    index, nbrs = O.build_csr(n, src.astype(np.uint32), dst.astype(np.uint32))
+    with G.Graph.from_csr(index, nbrs) as g:
+        if reorder:
+            g.reorder()
+        lab, _ = g.ccv()
+    assert np.array_equal(lab, O.cc_labels(index, nbrs))
+
+
+def test_component_minima_two_giants():
+    # two interleaved giants: every wave meets both labels
+    n = 300007
+    v = np.arange(n - 2, dtype=np.uint32)
+    index, nbrs = O.build_csr(n, v, v + 2)
+    with G.Graph.from_csr(index, nbrs) as g:
+        p = g.prop()
+        p.upload((np.arange(n) % 2).astype(np.uint32))
+        out = np.empty(n, np.uint32)
+        G._check(G.lib().gpr_cc_recode(p.h, out.ctypes.data))
+        p.destroy()
+    assert np.array_equal(out, (np.arange(n) % 2).astype(np.uint32))
