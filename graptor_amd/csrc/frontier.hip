@@ -149,6 +149,15 @@ __global__ void k_list_edges(const uint32_t *__restrict__ list, uint32_t k,
     if (threadIdx.x == 0 && s) atomicAdd(&ctr_stripe(ctr)->nacte, (unsigned long long)s);
 }
 
+int list_edges(gpr_graph *g, const uint32_t *list, uint32_t k, uint64_t *nacte) {
+    GPR_TRY(reset_counters(g));
+    if (k) hipLaunchKernelGGL(k_list_edges, dim3(grid_for(k, 256, 1024)), dim3(256), 0, g->stream, list, k, g->deg, g->ctr);
+    GPR_HIP(hipGetLastError());
+    GPR_TRY(read_counters(g));
+    *nacte = g->hctr->nacte;
+    return GPR_OK;
+}
+
 int fill_words(gpr_graph *g, uint64_t *p, size_t words, uint64_t v) {
     hipLaunchKernelGGL(k_fill_u64, dim3(grid_for(words, 256, 4096)), dim3(256), 0, g->stream, p, words, v);
     GPR_HIP(hipGetLastError());
@@ -275,13 +284,9 @@ extern "C" int gpr_frontier_set_neighbours(gpr_frontier *f, uint32_t v) {
     const uint32_t k = (uint32_t)(ix[1] - ix[0]);
     GPR_TRY(frontier_ensure_list(f));
     if (k) GPR_HIP(hipMemcpyAsync(f->list, g->nbrs + ix[0], sizeof(uint32_t) * k, hipMemcpyDeviceToDevice, g->stream));
-    GPR_TRY(reset_counters(g));
-    if (k) hipLaunchKernelGGL(k_list_edges, dim3(grid_for(k, 256, 1024)), dim3(256), 0, g->stream, f->list, k, g->deg, g->ctr);
-    GPR_HIP(hipGetLastError());
-    GPR_TRY(read_counters(g));
+    GPR_TRY(list_edges(g, f->list, k, &f->nacte));
     f->kind = k ? GPR_FRONTIER_LIST : GPR_FRONTIER_EMPTY;
     f->nactv = k;
-    f->nacte = g->hctr->nacte;
     return GPR_OK;
 }
 
@@ -301,13 +306,9 @@ extern "C" int gpr_frontier_set_list(gpr_frontier *f, const uint32_t *vs, uint32
     GPR_TRY(frontier_ensure_list(f));
     if (k) GPR_HIP(hipMemcpyAsync(f->list, vs, sizeof(uint32_t) * k, hipMemcpyHostToDevice, g->stream));
     GPR_TRY(map_ids(g, f->list, k, true));
-    GPR_TRY(reset_counters(g));
-    if (k) hipLaunchKernelGGL(k_list_edges, dim3(grid_for(k, 256, 1024)), dim3(256), 0, g->stream, f->list, k, g->deg, g->ctr);
-    GPR_HIP(hipGetLastError());
-    GPR_TRY(read_counters(g));
+    GPR_TRY(list_edges(g, f->list, k, &f->nacte));
     f->kind = GPR_FRONTIER_LIST;
     f->nactv = k;
-    f->nacte = g->hctr->nacte;
     return GPR_OK;
 }
 

@@ -323,6 +323,7 @@ int frontier_ensure_bits(gpr_frontier *f);
 int frontier_to_bits(gpr_frontier *f);            // convert LIST/ALL -> BITMAP
 int frontier_to_list(gpr_frontier *f);            // convert BITMAP/ALL -> LIST
 int fill_words(gpr_graph *g, uint64_t *p, size_t words, uint64_t v);
+int list_edges(gpr_graph *g, const uint32_t *list, uint32_t k, uint64_t *nacte);   // out-degree sum; synchronises
 int clear_dedup_of_list(gpr_graph *g, const uint32_t *list, uint64_t max_count);
 int ids_download(gpr_graph *g, const gpr_prop *p, uint32_t *host);   // ID-valued property, original IDs
 struct PolicyCtx;

@@ -9,9 +9,14 @@
 //                  consecutive frontier edges as in the single-source push;
 //   pull (dense):  every v not yet seen by all sources ORs cur[u] over its
 //                  in-edges, stopping once every missing bit has arrived;
+//                  a workgroup takes a pull bucket (<= STREAM_ITEMS rows +
+//                  edges) or a chunk of a long row, so no wave waits for
+//                  one that walks the hubs' rows alone;
 // followed by a dense finalize: new = nxt & ~seen, seen |= new, cur = new,
-// levels[j][v] = level+1 for every bit j of new, and the next active list
-// (wave-aggregated append) with its out-degree sum.  Direction follows the
+// level[v][j] = level+1 for every bit j of new, and the next active list
+// (through LDS queues) with its out-degree sum.  The levels are kept by
+// vertex, one row of k words each, and turned into the caller's one row a
+// source, in original IDs, at the end.  Direction follows the
 // reference's rule on the aggregate frontier (nactv + nacte <= m/20 pushes,
 // api.h:150-153).  Each lane's result equals a single-source BFSLVLv run
 // (bench/BFSLVLv.C:110-254) from that source.
@@ -37,15 +42,15 @@ __global__ void k_ms_init(uint32_t n, uint32_t k, uint32_t *levels, uint64_t *se
     }
 }
 
-__global__ void k_ms_sources(const uint32_t *__restrict__ src, uint32_t k, uint32_t n, uint32_t *levels, uint64_t *seen,
-                             uint64_t *cur) {
-    if (threadIdx.x == 0 && blockIdx.x == 0)
-        for (uint32_t j = 0; j < k; ++j) {
-            const uint32_t s = src[j];
-            seen[s] |= 1ull << j;
-            cur[s] |= 1ull << j;
-            levels[(uint64_t)j * n + s] = 0;
-        }
+// lane j: source j (k <= 64); two sources may be the same vertex
+__global__ void __launch_bounds__(64)
+k_ms_sources(const uint32_t *__restrict__ src, uint32_t k, uint32_t *levels, uint64_t *seen, uint64_t *cur) {
+    const uint32_t j = threadIdx.x;
+    if (j >= k) return;
+    const uint32_t s = src[j];
+    atomicOr((unsigned long long *)&seen[s], 1ull << j);
+    atomicOr((unsigned long long *)&cur[s], 1ull << j);
+    levels[(uint64_t)s * k + j] = 0;
 }
 
 // push over the active list (degree prefix in pos/btot as for the
@@ -106,91 +111,153 @@ k_ms_push(const uint32_t *__restrict__ flist, uint32_t kf, const uint64_t *__res
     }
 }
 
-// pull: wave per 64 destinations, lane-serial rows up to 32 in-edges, the
-// wave together on heavier rows; stop once every missing source arrived
-__global__ void __launch_bounds__(MS_THREADS)
-k_ms_pull(uint32_t n, const uint64_t *__restrict__ cindex, const uint32_t *__restrict__ cnbrs,
-          const uint64_t *__restrict__ cur, const uint64_t *__restrict__ seen, uint64_t full, uint64_t *nxt) {
-    const uint32_t ngroups = (n + 63) / 64;
-    const uint32_t wid = (blockIdx.x * MS_THREADS + threadIdx.x) / 64, nw = gridDim.x * (MS_THREADS / 64);
-    const unsigned ln = lane();
-    for (uint32_t grp = wid; grp < ngroups; grp += nw) {
-        const uint32_t d = grp * 64 + ln;
-        const bool valid = d < n;
-        const uint64_t sd = valid ? seen[d] : full;
-        const uint64_t miss = full & ~sd;
-        uint64_t acc = 0;
-        uint64_t beg = 0, end = 0;
-        if (miss) {
-            beg = cindex[d];
-            end = cindex[d + 1];
-        }
-        const bool heavy = miss && end - beg > 32;
-        if (miss && !heavy)
-            for (uint64_t e = beg; e < end; ++e) {
-                acc |= cur[cnbrs[e]];
-                if ((acc & miss) == miss) break;
-            }
-        uint64_t hm = __ballot(heavy);
-        while (hm) {
-            const int L = __ffsll((long long)hm) - 1;
-            hm &= hm - 1;
-            const uint64_t b = __shfl(beg, L, 64), en = __shfl(end, L, 64), ms = __shfl(miss, L, 64);
-            uint64_t a = 0;
-            for (uint64_t base = b; base < en; base += 64) {
-                const uint64_t e = base + ln;
-                uint64_t v = e < en ? cur[cnbrs[e]] : 0ull;
+// Pull, one workgroup per pull bucket or per chunk of a long row (both from
+// the graph's CSC partition).  Bound by the gathers of cur[] (8 B at random;
+// they stay in the L2 up to about 500K vertices).  In a bucket: rows up to
+// MS_LIGHT in-edges one lane each, MS_PU gathers in flight; longer ones go to
+// an LDS queue and are taken by 16 lanes each, 16 * MS_PU edges a step.
+// Every row stops once its missing bits have arrived; slots past a row's end
+// gather its first neighbour again, which changes no OR.  A long row's
+// chunks OR into nxt[row] and stop as well when the row is complete there.
+// The split it replaces (a wave per 64 rows, the wave walking their longer
+// rows in turn) left the 64 largest hubs to one wave: 6.2 ms a dense level
+// on a relabelled 500K-vertex, 15M-edge RMAT graph, 0.06 ms like this.
+constexpr int MS_PU = 4;
+constexpr uint32_t MS_LIGHT = 32;
+constexpr int MS_SUB = 16;   // lanes of a queued row
+constexpr uint32_t MS_QCAP = (STREAM_ITEMS + LONG_DEG) / (MS_LIGHT + 1) + 1;
+
+template <int STRIDE>
+__device__ __forceinline__ uint64_t ms_gather(const uint32_t *__restrict__ cnbrs, const uint64_t *__restrict__ cur,
+                                              uint64_t e, uint64_t first, uint64_t end) {
+    uint32_t s[MS_PU];
 #pragma unroll
-                for (int o = 32; o > 0; o >>= 1) v |= __shfl_xor(v, o, 64);
-                a |= v;
-                if ((a & ms) == ms) break;
-            }
-            if ((int)ln == L) acc = a;
+    for (int u = 0; u < MS_PU; ++u) s[u] = cnbrs[e + u * STRIDE < end ? e + u * STRIDE : first];
+    uint64_t v = 0;
+#pragma unroll
+    for (int u = 0; u < MS_PU; ++u) v |= cur[s[u]];
+    return v;
+}
+
+__global__ void __launch_bounds__(MS_THREADS)
+k_ms_pull(uint32_t nbuckets, const uint32_t *__restrict__ bucket, const uint64_t *__restrict__ cindex,
+          const uint32_t *__restrict__ cnbrs, const uint32_t *__restrict__ long_rows,
+          const uint32_t *__restrict__ long_base, uint32_t nlong, const uint64_t *__restrict__ cur,
+          const uint64_t *__restrict__ seen, uint64_t full, uint64_t *nxt) {
+    __shared__ uint32_t q[MS_QCAP];
+    __shared__ uint32_t qn;
+    if (blockIdx.x >= nbuckets) {
+        // one chunk of a long row
+        const uint32_t c = blockIdx.x - nbuckets;
+        uint32_t lo = 0, hi = nlong;   // the row whose chunks c is among
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (long_base[mid] <= c) lo = mid + 1; else hi = mid;
         }
-        if (valid && (acc & miss)) nxt[d] = acc & miss;
+        const uint32_t row = long_rows[lo - 1];
+        const uint64_t ms = full & ~seen[row];
+        if (!ms) return;
+        const uint64_t cb = cindex[row] + (uint64_t)(c - long_base[lo - 1]) * LONG_CHUNK;
+        const uint64_t re = cindex[row + 1], ce = cb + LONG_CHUNK < re ? cb + LONG_CHUNK : re;
+        uint64_t a = 0;
+        for (uint64_t base = cb + (threadIdx.x & ~63u) * MS_PU; base < ce; base += MS_THREADS * MS_PU) {
+            uint64_t v = ms_gather<64>(cnbrs, cur, base + lane(), cb, ce);
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) v |= __shfl_xor(v, o, 64);
+            a |= v;
+            const uint64_t have = __hip_atomic_load(&nxt[row], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (((a | have) & ms) == ms) break;
+        }
+        if (lane() == 0 && (a & ms)) atomicOr((unsigned long long *)&nxt[row], (unsigned long long)(a & ms));
+        return;
+    }
+    if (threadIdx.x == 0) qn = 0;
+    __syncthreads();
+    const uint32_t r0 = bucket[blockIdx.x], r1 = bucket[blockIdx.x + 1];
+    for (uint32_t r = r0 + threadIdx.x; r < r1; r += MS_THREADS) {
+        const uint64_t ms = full & ~seen[r];
+        if (!ms) continue;
+        const uint64_t beg = cindex[r], end = cindex[r + 1];
+        if (end - beg > LONG_DEG) continue;   // by its chunks
+        if (end - beg > MS_LIGHT) {
+            q[atomicAdd(&qn, 1u)] = r;
+            continue;
+        }
+        uint64_t a = 0;
+        for (uint64_t e = beg; e < end && (a & ms) != ms; e += MS_PU) a |= ms_gather<1>(cnbrs, cur, e, beg, end);
+        if (a & ms) nxt[r] = a & ms;
+    }
+    __syncthreads();
+    const uint32_t cnt = qn, sl = threadIdx.x % MS_SUB;
+    for (uint32_t i = threadIdx.x / MS_SUB; i < cnt; i += MS_THREADS / MS_SUB) {
+        const uint32_t r = q[i];
+        const uint64_t ms = full & ~seen[r];
+        const uint64_t beg = cindex[r], end = cindex[r + 1];
+        uint64_t a = 0;
+        for (uint64_t base = beg; base < end && (a & ms) != ms; base += MS_SUB * MS_PU) {
+            uint64_t v = ms_gather<MS_SUB>(cnbrs, cur, base + sl, beg, end);
+#pragma unroll
+            for (int o = MS_SUB / 2; o > 0; o >>= 1) v |= __shfl_xor(v, o, MS_SUB);
+            a |= v;
+        }
+        if (sl == 0 && (a & ms)) nxt[r] = a & ms;
     }
 }
 
-// finalize a level: levels of the new bits, seen/cur update, next active
-// list with its out-degree sum
+// Finalize a level: levels of the new bits, seen/cur update, next active
+// list with its out-degree sum.  Bound by the streams (32 B a vertex) and
+// the levels written: a vertex's row is one store of the wave, lane j for
+// source j, so each row is written in whole cache lines (one lane per vertex
+// with a store per bit: 66 us a dense level at 500K vertices and 64 sources,
+// with an atomic a wave on the list position; 28 us like this).
+constexpr uint32_t MS_LQ = 512;   // LDS queue entries per wave
 __global__ void __launch_bounds__(MS_THREADS)
-k_ms_finalize(uint32_t n, uint32_t level, uint32_t *levels, uint64_t *seen, uint64_t *cur, uint64_t *nxt,
+k_ms_finalize(uint32_t n, uint32_t k, uint32_t level, uint32_t *levels, uint64_t *seen, uint64_t *cur, uint64_t *nxt,
               const uint32_t *__restrict__ deg, uint32_t *list, DevCounters *ctr) {
     __shared__ uint64_t red[MS_THREADS / 64];
+    __shared__ uint32_t s_q[MS_THREADS / 64 * MS_LQ];
+    __shared__ uint32_t s_c[MS_THREADS / 64], s_base;
     uint64_t my_e = 0;
     const uint32_t ngroups = (n + 63) / 64;
     const uint32_t wid = (blockIdx.x * MS_THREADS + threadIdx.x) / 64, nw = gridDim.x * (MS_THREADS / 64);
-    const unsigned ln = lane();
+    const unsigned ln = lane(), w = threadIdx.x / 64;
+    WaveQueue wq{s_q + w * MS_LQ, MS_LQ, 0};
     for (uint32_t grp = wid; grp < ngroups; grp += nw) {
         const uint32_t v = grp * 64 + ln;
         uint64_t nb = 0;
         if (v < n) {
             const uint64_t x = nxt[v];
-            cur[v] = 0;
             if (x) {
-                nb = x & ~seen[v];
+                const uint64_t sv = seen[v];
+                nb = x & ~sv;
                 nxt[v] = 0;
                 if (nb) {
-                    seen[v] |= nb;
-                    cur[v] = nb;
-                    uint64_t t = nb;
-                    while (t) {
-                        const int j = __ffsll((long long)t) - 1;
-                        t &= t - 1;
-                        levels[(uint64_t)j * n + v] = level + 1;
-                    }
+                    seen[v] = sv | nb;
                     my_e += deg[v];
                 }
             }
+            cur[v] = nb;
         }
-        const uint64_t w = __ballot(nb != 0);
-        if (w) {
-            uint32_t base = 0;
-            if (ln == 0) base = atomicAdd(&ctr->listpos, (unsigned)__popcll(w));
-            base = __shfl(base, 0, 64);
-            if (nb) list[base + mbcnt(w)] = v;
+        const uint64_t word = __ballot(nb != 0);
+        for (uint64_t t = word; t; t &= t - 1) {
+            const int L = __ffsll((long long)t) - 1;
+            const uint64_t b = __shfl(nb, L, 64);
+            if ((b >> ln) & 1ull) levels[(uint64_t)(grp * 64 + L) * k + ln] = level + 1;
         }
+        wq.push(nb != 0, word, v, list, &ctr->listpos);
     }
+    // the waves' remaining queues in one append per workgroup
+    if (ln == 0) s_c[w] = wq.cnt;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t t = 0;
+        for (int j = 0; j < MS_THREADS / 64; ++j) t += s_c[j];
+        s_base = t ? atomicAdd(&ctr->listpos, t) : 0u;
+    }
+    __syncthreads();
+    uint32_t off = s_base;
+    for (unsigned j = 0; j < w; ++j) off += s_c[j];
+    for (uint32_t j = ln; j < wq.cnt; j += 64) list[off + j] = wq.q[j];
     const uint64_t te = block_sum(my_e, red);
     if (threadIdx.x == 0 && te) atomicAdd(&ctr_stripe(ctr)->nacte, (unsigned long long)te);
 }
@@ -206,13 +273,26 @@ k_ms_edges(uint32_t n, const uint64_t *__restrict__ seen, const uint32_t *__rest
     if (threadIdx.x == 0 && s) atomicAdd(&ctr_stripe(ctr)->edges, (unsigned long long)s);
 }
 
-__global__ void k_ms_scatter(const uint32_t *__restrict__ src, const uint32_t *__restrict__ order, uint32_t n,
-                             uint32_t k, uint32_t *dst) {
-    const uint64_t total = (uint64_t)k * n;
-    for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < total; i += (uint64_t)gridDim.x * blockDim.x) {
-        const uint64_t j = i / n, v = i % n;
-        dst[j * n + order[v]] = src[i];
+// Sources [j0, j0 + js) of the levels as one row of n a source, in original
+// IDs: a workgroup turns the rows of MS_OUT_V vertices through LDS, so reads
+// are runs of js words and writes runs of MS_OUT_V, whatever the vertex
+// order (reading a row a source and scattering it took 216 us at 500K
+// vertices and 64 sources, this 93 us).
+constexpr uint32_t MS_OUT_V = 64, MS_OUT_J = 16;
+__global__ void __launch_bounds__(256)
+k_ms_out(const uint32_t *__restrict__ levels, const uint32_t *__restrict__ perm, uint32_t n, uint32_t k, uint32_t j0,
+         uint32_t js, uint32_t *dst) {
+    __shared__ uint32_t t[MS_OUT_V][MS_OUT_J + 1];
+    const uint32_t o0 = blockIdx.x * MS_OUT_V;
+    for (uint32_t i = threadIdx.x / MS_OUT_J, j = threadIdx.x % MS_OUT_J; i < MS_OUT_V; i += 256 / MS_OUT_J) {
+        const uint32_t o = o0 + i;
+        if (o < n && j < js) t[i][j] = levels[(uint64_t)(perm ? perm[o] : o) * k + j0 + j];
     }
+    __syncthreads();
+    const uint32_t o = o0 + threadIdx.x % MS_OUT_V;
+    if (o < n)
+        for (uint32_t j = threadIdx.x / MS_OUT_V; j < js; j += 256 / MS_OUT_V)
+            dst[(uint64_t)j * n + o] = t[threadIdx.x % MS_OUT_V][j];
 }
 
 int scan_frontier_degrees(gpr_graph *g, const uint32_t *list, uint32_t k);
@@ -259,20 +339,10 @@ extern "C" int gpr_msbfs(gpr_graph *g, const uint32_t *sources, int k, const gpr
         (void)hipEventRecord(g->rev0, g->stream);
         hipLaunchKernelGGL(k_ms_init, dim3(grid_for((uint64_t)k * n, 256, 16384)), dim3(256), 0, g->stream, n, (uint32_t)k,
                            lev, seen, cur, nxt);
-        hipLaunchKernelGGL(k_ms_sources, dim3(1), dim3(64), 0, g->stream, src, (uint32_t)k, n, lev, seen, cur);
-        if ((r = reset_counters(g))) break;
+        hipLaunchKernelGGL(k_ms_sources, dim3(1), dim3(64), 0, g->stream, src, (uint32_t)k, lev, seen, cur);
         // out-degree sum of the sources
         uint64_t nacte = 0;
-        {
-            std::vector<uint64_t> ix(2);
-            for (uint32_t v : uniq) {
-                uint32_t vi = v;
-                if ((r = to_internal_id(g, v, &vi))) break;
-                if (hipMemcpy(ix.data(), g->index + vi, 16, hipMemcpyDeviceToHost) != hipSuccess) { r = GPR_E_HIP; break; }
-                nacte += ix[1] - ix[0];
-            }
-            if (r) break;
-        }
+        if ((r = list_edges(g, list[0], (uint32_t)uniq.size(), &nacte))) break;
         uint32_t nactv = (uint32_t)uniq.size();
         const uint64_t full = k == 64 ? ~0ull : ((1ull << k) - 1);
         int cl = 0;
@@ -287,12 +357,13 @@ extern "C" int gpr_msbfs(gpr_graph *g, const uint32_t *sources, int k, const gpr
                                        list[cl], nactv, g->scan, g->scan_blk, nacte, g->index, g->nbrs, cur, seen, nxt);
                 inf.push_iters++;
             } else {
-                hipLaunchKernelGGL(k_ms_pull, dim3(grid_for((n + 63) / 64, MS_THREADS / 64, 2048)), dim3(MS_THREADS), 0,
-                                   g->stream, n, g->cindex, g->cnbrs, cur, seen, full, nxt);
+                hipLaunchKernelGGL(k_ms_pull, dim3(g->nbuckets + g->nlong_chunks), dim3(MS_THREADS), 0, g->stream,
+                                   g->nbuckets, g->bucket, g->cindex, g->cnbrs, g->long_rows, g->long_base, g->nlong,
+                                   cur, seen, full, nxt);
             }
             if ((r = reset_counters(g))) break;
             hipLaunchKernelGGL(k_ms_finalize, dim3(grid_for((n + 63) / 64, MS_THREADS / 64, 2048)), dim3(MS_THREADS), 0,
-                               g->stream, n, level, lev, seen, cur, nxt, g->deg, list[cl ^ 1], g->ctr);
+                               g->stream, n, (uint32_t)k, level, lev, seen, cur, nxt, g->deg, list[cl ^ 1], g->ctr);
             if (hipGetLastError() != hipSuccess) { r = GPR_E_HIP; break; }
             if ((r = read_counters(g))) break;
             nactv = g->hctr->listpos;
@@ -312,15 +383,16 @@ extern "C" int gpr_msbfs(gpr_graph *g, const uint32_t *sources, int k, const gpr
         if ((r = read_counters(g))) break;
         inf.edges = g->hctr->edges;
         if (levels) {
-            const uint32_t *outp = lev;
+            // MS_OUT_J sources at a time through one staging buffer
             uint32_t *tmp = nullptr;
-            if (g->order) {
-                if ((r = dev_alloc((void **)&tmp, 4ull * k * n, "msbfs levels"))) break;
-                hipLaunchKernelGGL(k_ms_scatter, dim3(grid_for((uint64_t)k * n, 256, 16384)), dim3(256), 0, g->stream, lev,
-                                   g->order, n, (uint32_t)k, tmp);
-                outp = tmp;
+            if ((r = dev_alloc((void **)&tmp, 4ull * std::min<uint32_t>(k, MS_OUT_J) * n, "msbfs levels"))) break;
+            hipError_t e = hipSuccess;
+            for (uint32_t j0 = 0; j0 < (uint32_t)k && e == hipSuccess; j0 += MS_OUT_J) {
+                const uint32_t js = std::min<uint32_t>(MS_OUT_J, k - j0);
+                hipLaunchKernelGGL(k_ms_out, dim3(grid_for(n, MS_OUT_V)), dim3(256), 0, g->stream, lev, g->perm, n,
+                                   (uint32_t)k, j0, js, tmp);
+                e = hipMemcpyAsync(levels + (uint64_t)j0 * n, tmp, 4ull * js * n, hipMemcpyDeviceToHost, g->stream);
             }
-            hipError_t e = hipMemcpyAsync(levels, outp, 4ull * k * n, hipMemcpyDeviceToHost, g->stream);
             if (e == hipSuccess) e = hipStreamSynchronize(g->stream);
             dev_free(tmp);
             if (e != hipSuccess) { r = GPR_E_HIP; break; }
