@@ -124,25 +124,31 @@ struct PrScalars {
 // at or above `from`: the sources outside the cache-resident prefix of a
 // degree-ordered graph, whose gathers would each cost a cache line (all
 // sources when from = 0).  Cold edges are grouped into tiles of consecutive
-// sources (<= COLD_TILE_V sources, <= COLD_TILE_E edges) and bins of
+// sources (<= tile_v <= COLD_TILE_V sources, <= COLD_TILE_E edges) and bins of
 // COLD_BIN destinations; the edges of one source into one bin form a pair,
 // which carries one value.  The write kernel reads each tile's pairs in
 // (bin, source) order and writes each pair's value to its slot in the
 // bin-major value array, where a bin's pairs are contiguous (its runs, one
 // per tile); the accumulation kernel streams each bin's entries (one per
-// edge, grouped by pair) into LDS.  Bins with more than COLD_CHUNK_E entries
-// are split into chunks whose integer partials a third kernel adds up.
+// edge, grouped by pair) into LDS.  Bins with more entries than one chunk
+// (by the graph's size, at most COLD_CHUNK_E) are split into chunks whose
+// integer partials a third kernel adds up.
 constexpr uint32_t COLD_BIN = 16384;
 constexpr uint32_t COLD_TILE_V = 32768;
 constexpr uint64_t COLD_TILE_E = 1ull << 24;
-constexpr uint64_t COLD_WCHUNK = 131072;   // pairs per write chunk
-constexpr uint64_t COLD_CHUNK_E = 1u << 20;
+constexpr uint32_t COLD_TILE_V_MIN = 1024;
+constexpr uint64_t COLD_WCHUNK = 131072;   // pairs per write chunk, at most
+constexpr uint64_t COLD_WCHUNK_MIN = 4096;
+constexpr uint64_t COLD_CHUNK_E = 1u << 20;   // entries per accumulation chunk, at most
+constexpr uint64_t COLD_CHUNK_E_MIN = 32768;
 constexpr uint64_t COLD_PAD_E = 65536;          // zero tail of the destination array (and of the pair bases / 64)
 constexpr uint32_t COLD_DIRECT = 0xffffffffu;   // chunk slot of a bin in one chunk
 constexpr uint32_t COLD_GROUP = 16;             // chunk partials summed per first-level combine group
 struct ColdLayout {
     uint32_t from = 0;              // first cold source
     uint32_t ntiles = 0, nbins = 0;
+    uint32_t tile_v = 0;            // sources a tile spans at most
+    uint32_t max_chunks = 1;        // accumulation chunks of one bin, at most
     uint64_t ncold = 0;             // cold edges (entries)
     uint64_t npairs = 0;            // distinct (source, bin) pairs over the cold edges
     uint32_t *tile_lo = nullptr;    // ntiles+1 source boundaries

@@ -62,6 +62,7 @@
 #include "device.hpp"
 #include "pr_codec.hpp"
 
+#include <algorithm>
 #include <cstring>
 #include <rocprim/rocprim.hpp>
 
@@ -216,11 +217,12 @@ void cold_free(gpr_graph *g) {
 }
 
 // Tiles over [from, n): each starts at a source with edges and grows while
-// it spans < COLD_TILE_V sources and its edges stay <= COLD_TILE_E (a
+// it spans < tile_v sources and its edges stay <= COLD_TILE_E (a
 // single source with more edges gets a tile of its own).  lo[t+1] is the
 // start of the next tile (or the end); sources without edges between two
 // tiles belong to neither.
-static void make_tiles(const std::vector<uint64_t> &idx, uint32_t from, uint32_t n, std::vector<uint32_t> &lo) {
+static void make_tiles(const std::vector<uint64_t> &idx, uint32_t from, uint32_t n, uint32_t tile_v,
+                       std::vector<uint32_t> &lo) {
     lo.clear();
     uint32_t u = from;
     while (u < n) {
@@ -228,7 +230,7 @@ static void make_tiles(const std::vector<uint64_t> &idx, uint32_t from, uint32_t
         if (u >= n) break;
         const uint32_t t0 = u;
         uint64_t e = 0;
-        while (u < n && u - t0 < COLD_TILE_V) {
+        while (u < n && u - t0 < tile_v) {
             const uint64_t d = idx[u + 1 - from] - idx[u - from];
             if (e > 0 && e + d > COLD_TILE_E) break;
             e += d;
@@ -284,8 +286,23 @@ int cold_prepare(gpr_graph *g, uint32_t from) {
     // no cold edges, or more than 32-bit entry positions address: the pull
     // handles every edge
     if (ncold == 0 || ncold >= 0xffffffffull) return GPR_OK;
+    // Tiles and chunks by the graph's size, so that both stages have a
+    // workgroup for every CU: an accumulation chunk of 2^20 entries takes
+    // 190 us whatever the graph, and a graph of 60000 vertices had five of
+    // them and two write chunks.  One chunk a CU: smaller ones pay more for
+    // clearing and writing out their bin's sums (30 us at 31M edges with
+    // four a CU) than they gain in balance; below COLD_CHUNK_E_MIN entries
+    // and COLD_WCHUNK_MIN pairs that cost is all there is.  Per iteration
+    // (FP32, RMAT, edge factor 16): 240 -> 52 us at scale 16, 266 -> 112 at
+    // 20, 278 -> 225 at 22, 751 -> 699 at 24; from scale 25 on the limits
+    // are the largest sizes.
+    const uint64_t cus = (uint64_t)num_cus();
+    uint32_t tile_v = COLD_TILE_V_MIN;
+    while (tile_v < COLD_TILE_V && 2 * tile_v * cus < n - from) tile_v *= 2;
+    const uint64_t chunk_e = std::min(COLD_CHUNK_E, std::max(COLD_CHUNK_E_MIN, ncold / cus));
+    L->tile_v = tile_v;
     std::vector<uint32_t> lo;
-    make_tiles(idx, from, n, lo);
+    make_tiles(idx, from, n, tile_v, lo);
     // the sources outside every tile's span [lo[t], lo[t] + w_t): their
     // ranks are updated by a kernel of their own when the PageRank tail is
     // fused into the write stage
@@ -294,7 +311,7 @@ int cold_prepare(gpr_graph *g, uint32_t from) {
         uint32_t at = from;
         for (size_t t = 0; t + 1 < lo.size(); ++t) {
             if (lo[t] > at) { gap_lo.push_back(at); gap_len.push_back(lo[t] - at); }
-            at = lo[t] + std::min<uint32_t>(lo[t + 1] - lo[t], COLD_TILE_V);
+            at = lo[t] + std::min<uint32_t>(lo[t + 1] - lo[t], tile_v);
         }
         if (n > at) { gap_lo.push_back(at); gap_len.push_back(n - at); }
     }
@@ -309,7 +326,7 @@ int cold_prepare(gpr_graph *g, uint32_t from) {
     int r = GPR_OK;
     std::vector<uint32_t> ecnt, pcnt, edel, pdel, ord, roff, tcell;
     std::vector<uint32_t> wch, ach, multi, groups;   // plans, 4 words per item
-    uint32_t nslots = 0, nslots2 = 0;
+    uint32_t nslots = 0, nslots2 = 0, max_chunks = 1;
     uint64_t npairs = 0;
     const unsigned pg = grid_for(ncold, CK_EDGES, 65536);
     const unsigned eg = grid_for(ncold, 256, 65536);
@@ -394,11 +411,13 @@ int cold_prepare(gpr_graph *g, uint32_t from) {
         ecnt.shrink_to_fit();
         for (uint32_t b = 0; b < nbins; ++b) {
             const uint64_t e0 = ebstart[b], e1 = ebstart[b + 1];
-            const uint32_t k = e1 > e0 ? (uint32_t)((e1 - e0 + COLD_CHUNK_E - 1) / COLD_CHUNK_E) : 1u;
+            // k pieces of the same number of 64-entry blocks
+            const uint64_t b0 = e0 & ~63ull, nblk = (e1 - b0 + 63) / 64, pblk = chunk_e / 64;
+            const uint32_t k = e1 > e0 ? (uint32_t)((nblk + pblk - 1) / pblk) : 1u;
             for (uint32_t i = 0; i < k; ++i) {
                 ach.push_back(b);
-                ach.push_back((uint32_t)std::min<uint64_t>(e1, e0 + (uint64_t)i * COLD_CHUNK_E));
-                ach.push_back((uint32_t)std::min<uint64_t>(e1, e0 + (uint64_t)(i + 1) * COLD_CHUNK_E));
+                ach.push_back(i ? (uint32_t)(b0 + 64 * (nblk * i / k)) : (uint32_t)e0);
+                ach.push_back(i + 1 < k ? (uint32_t)(b0 + 64 * (nblk * (i + 1) / k)) : (uint32_t)e1);
                 ach.push_back(k == 1 ? COLD_DIRECT : nslots + i);
             }
             if (k > 1) {
@@ -412,10 +431,18 @@ int cold_prepare(gpr_graph *g, uint32_t from) {
                     groups.push_back(nslots + g0);
                     groups.push_back(std::min<uint32_t>(COLD_GROUP, k - g0));
                     groups.push_back(nslots2++);
-                    groups.push_back(0);
+                    groups.push_back(b);
                 }
                 nslots += k;
+                max_chunks = std::max(max_chunks, k);
             }
+        }
+        // the largest chunks first: the smaller ones fill the last wave
+        {
+            struct Chunk { uint32_t w[4]; };
+            Chunk *c = (Chunk *)ach.data();
+            std::stable_sort(c, c + ach.size() / 4,
+                             [](const Chunk &x, const Chunk &y) { return x.w[2] - x.w[1] > y.w[2] - y.w[1]; });
         }
         // ---- pair plan: bin-major pair slots, write chunks per tile
         {
@@ -438,13 +465,14 @@ int cold_prepare(gpr_graph *g, uint32_t from) {
                 }
             }
             tcell[ntiles] = (uint32_t)roff.size();
+            const uint64_t wpairs = std::min(COLD_WCHUNK, std::max(COLD_WCHUNK_MIN, npairs / cus));
             for (uint32_t t = 0; t < ntiles; ++t) {
                 const uint64_t t0 = pos;
                 for (uint32_t b = 0; b < nbins; ++b) pos += pcnt[(size_t)t * nbins + b];
-                for (uint64_t q = t0; q < pos; q += COLD_WCHUNK) {
+                for (uint64_t q = t0; q < pos; q += wpairs) {
                     wch.push_back(t);
                     wch.push_back((uint32_t)q);
-                    wch.push_back((uint32_t)std::min<uint64_t>(pos, q + COLD_WCHUNK));
+                    wch.push_back((uint32_t)std::min<uint64_t>(pos, q + wpairs));
                     wch.push_back(q == t0 ? 1u : 0u);
                 }
             }
@@ -547,6 +575,7 @@ int cold_prepare(gpr_graph *g, uint32_t from) {
     L->nbins = nbins;
     L->ncold = ncold;
     L->npairs = npairs;
+    L->max_chunks = max_chunks;
     return GPR_OK;
 }
 
@@ -677,16 +706,16 @@ k_cold_write(const uint32_t *__restrict__ wchunk, uint32_t nwchunks, const uint3
              const uint32_t *__restrict__ roff, uint32_t stage_max,
              const typename Codec<FMT>::store_t *__restrict__ contrib, typename Codec<FMT>::store_t *__restrict__ vals,
              const uint32_t *__restrict__ deg, double *__restrict__ mass, const PrScalars *__restrict__ prs,
-             PrTail tail) {
+             PrTail tail, uint32_t tile_v) {
     using S = typename Codec<FMT>::store_t;
     __shared__ S win[COLD_TILE_V];
     __shared__ uint32_t dls[CW_DELTA_LDS];
     __shared__ double red[CW_THREADS / 64];
     const uint32_t c = xcd_chunk(blockIdx.x, nwchunks);
     const uint32_t t = wchunk[4 * c], p0 = wchunk[4 * c + 1], p1 = wchunk[4 * c + 2], first = wchunk[4 * c + 3];
-    // a tile's sources span < COLD_TILE_V IDs; tile_lo[t+1] may lie further
-    // on when sources without edges follow the tile
-    const uint32_t lo = tile_lo[t], w = min(tile_lo[t + 1] - lo, COLD_TILE_V);
+    // a tile's sources span <= tile_v IDs; tile_lo[t+1] may lie further on
+    // when sources without edges follow the tile
+    const uint32_t lo = tile_lo[t], w = min(tile_lo[t + 1] - lo, tile_v);
     // the tile's first chunk: the mass of its edges, sum of |contribution|
     // x out-degree over its sources (a value is added once per edge)
     PrTail tl = tail;
@@ -794,7 +823,8 @@ k_cold_accum(const uint32_t *__restrict__ achunk, uint32_t n, const uint16_t *cd
     __shared__ float fred[CA_THREADS / 64];
     const uint32_t b = achunk[4 * blockIdx.x], p0 = achunk[4 * blockIdx.x + 1], p1 = achunk[4 * blockIdx.x + 2];
     const uint32_t slot = achunk[4 * blockIdx.x + 3];
-    for (uint32_t i = threadIdx.x; i < COLD_BIN; i += CA_THREADS) acc[i] = 0ull;
+    const uint32_t d0 = b * COLD_BIN, nd = min(COLD_BIN, n - d0);
+    for (uint32_t i = threadIdx.x; i < nd; i += CA_THREADS) acc[i] = 0ull;
     __syncthreads();
     const double unit = prs->cold_unit;
     const float dscale = FMT == GPR_CONTRIB_F16 ? 1.0f / prs->enc_scale : 1.0f;
@@ -911,11 +941,10 @@ k_cold_accum(const uint32_t *__restrict__ achunk, uint32_t n, const uint16_t *cd
         process(base + step, key2, vv2);
     }
     __syncthreads();
-    const uint32_t d0 = b * COLD_BIN, nd = min(COLD_BIN, n - d0);
     if (slot != COLD_DIRECT) {
         // one of several chunks of this bin: integer partials for the combine
         long long *pp = partials + (size_t)slot * COLD_BIN;
-        for (uint32_t i = threadIdx.x; i < COLD_BIN; i += CA_THREADS) pp[i] = (long long)acc[i];
+        for (uint32_t i = threadIdx.x; i < nd; i += CA_THREADS) pp[i] = (long long)acc[i];
         if (threadIdx.x == 0) {
             part[b] = 0.0;
             part_max[b] = 0.0f;
@@ -930,17 +959,19 @@ k_cold_accum(const uint32_t *__restrict__ achunk, uint32_t n, const uint16_t *cd
 }
 
 constexpr int CC_THREADS = 1024;
-constexpr uint32_t CC_PER_BIN = COLD_BIN / CC_THREADS;
+// workgroups per bin of the two combine kernels
+static uint32_t combine_per_bin(uint32_t n) { return (std::min(n, COLD_BIN) + CC_THREADS - 1) / CC_THREADS; }
 
 // Bins in several chunks, first level: one workgroup per (group of <=
 // COLD_GROUP chunk partials, CC_THREADS destinations) adds the group's
 // partials, all loads in flight together, into the group's slot.
 __global__ void __launch_bounds__(CC_THREADS)
-k_cold_combine_groups(const uint32_t *__restrict__ groups, const long long *__restrict__ partials,
-                      long long *__restrict__ partials2) {
-    const uint32_t gi = blockIdx.x / CC_PER_BIN, sub = blockIdx.x % CC_PER_BIN;
-    const uint32_t first = groups[4 * gi], cnt = groups[4 * gi + 1], slot2 = groups[4 * gi + 2];
+k_cold_combine_groups(const uint32_t *__restrict__ groups, uint32_t n, uint32_t per_bin,
+                      const long long *__restrict__ partials, long long *__restrict__ partials2) {
+    const uint32_t gi = blockIdx.x / per_bin, sub = blockIdx.x % per_bin;
+    const uint32_t first = groups[4 * gi], cnt = groups[4 * gi + 1], slot2 = groups[4 * gi + 2], b = groups[4 * gi + 3];
     const uint32_t i = sub * CC_THREADS + threadIdx.x;
+    if (i >= min(COLD_BIN, n - b * COLD_BIN)) return;
     long long t[COLD_GROUP];
 #pragma unroll
     for (uint32_t c = 0; c < COLD_GROUP; ++c) t[c] = c < cnt ? partials[(size_t)(first + c) * COLD_BIN + i] : 0ll;
@@ -951,17 +982,18 @@ k_cold_combine_groups(const uint32_t *__restrict__ groups, const long long *__re
 }
 
 // Second level: one workgroup per CC_THREADS destinations of a bin adds its
-// groups' sums and stores y; its y sum and y/deg maximum go to slot
+// groups' sums (its chunks' sums when no bin has more than COLD_GROUP
+// chunks, direct) and stores y; its y sum and y/deg maximum go to slot
 // nbins + blockIdx.x.  Integer sums: exact in any grouping.
 __global__ void __launch_bounds__(CC_THREADS)
-k_cold_combine(const uint32_t *__restrict__ multi, uint32_t nbins, uint32_t n, const long long *__restrict__ partials2,
-               const uint32_t *__restrict__ deg, float *__restrict__ y, int add, double *__restrict__ part,
-               float *__restrict__ part_max, const PrScalars *__restrict__ prs, int f16) {
+k_cold_combine(const uint32_t *__restrict__ multi, uint32_t nbins, uint32_t n, uint32_t per_bin, int direct,
+               const long long *__restrict__ parts, const uint32_t *__restrict__ deg, float *__restrict__ y, int add,
+               double *__restrict__ part, float *__restrict__ part_max, const PrScalars *__restrict__ prs, int f16) {
     __shared__ double dred[CC_THREADS / 64];
     __shared__ float fred[CC_THREADS / 64];
-    const uint32_t mb = blockIdx.x / CC_PER_BIN, sub = blockIdx.x % CC_PER_BIN;
-    const uint32_t b = multi[4 * mb], first = multi[4 * mb + 3];
-    const uint32_t k = (multi[4 * mb + 2] + COLD_GROUP - 1) / COLD_GROUP;
+    const uint32_t mb = blockIdx.x / per_bin, sub = blockIdx.x % per_bin;
+    const uint32_t b = multi[4 * mb], first = direct ? multi[4 * mb + 1] : multi[4 * mb + 3];
+    const uint32_t k = direct ? multi[4 * mb + 2] : (multi[4 * mb + 2] + COLD_GROUP - 1) / COLD_GROUP;
     const uint32_t i = sub * CC_THREADS + threadIdx.x;
     const uint32_t d0 = b * COLD_BIN, nd = min(COLD_BIN, n - d0);
     double my_sum = 0.0;
@@ -972,11 +1004,11 @@ k_cold_combine(const uint32_t *__restrict__ multi, uint32_t nbins, uint32_t n, c
         for (; c + 8 <= k; c += 8) {
             long long t[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) t[j] = partials2[(size_t)(first + c + j) * COLD_BIN + i];
+            for (int j = 0; j < 8; ++j) t[j] = parts[(size_t)(first + c + j) * COLD_BIN + i];
 #pragma unroll
             for (int j = 0; j < 8; ++j) s += t[j];
         }
-        for (; c < k; ++c) s += partials2[(size_t)(first + c) * COLD_BIN + i];
+        for (; c < k; ++c) s += parts[(size_t)(first + c) * COLD_BIN + i];
         cold_store(y, d0 + i, s, prs->cold_unit, add, my_sum, my_max, deg, f16 != 0);
     }
     block_emit<CC_THREADS>(my_sum, my_max, part, part_max, nbins + blockIdx.x, dred, fred);
@@ -1019,7 +1051,7 @@ int cold_launch_write(gpr_graph *g, int fmt, const void *contrib, const float *y
     hipLaunchKernelGGL((k_cold_write<F, U>), dim3(L->nwchunks), dim3(CW_THREADS), 0, g->stream, L->wchunk,      \
                        L->nwchunks, L->tile_lo, L->tcell, L->wsrc, L->wbase, L->roff, stage_max,                \
                        (const typename Codec<F>::store_t *)contrib, (typename Codec<F>::store_t *)L->vals, g->deg,  \
-                       L->mass, g->prs, tail)
+                       L->mass, g->prs, tail, L->tile_v)
 #define CW(F)                                                                                                   \
     if (upd) CW_(F, true); else CW_(F, false)
     switch (fmt) {
@@ -1051,15 +1083,19 @@ int cold_launch_accum(gpr_graph *g, int fmt, float *y, int add, double *part, fl
     case GPR_CONTRIB_SCFP16: CA(GPR_CONTRIB_SCFP16); break;
     }
 #undef CA
+    const uint32_t per_bin = combine_per_bin(g->n);
     if (L->nmulti) {
-        hipLaunchKernelGGL(k_cold_combine_groups, dim3(L->ngroups * CC_PER_BIN), dim3(CC_THREADS), 0, g->stream,
-                           L->groups, (const long long *)L->partials, L->partials2);
-        hipLaunchKernelGGL(k_cold_combine, dim3(L->nmulti * CC_PER_BIN), dim3(CC_THREADS), 0, g->stream, L->multi,
-                           L->nbins, g->n, (const long long *)L->partials2, g->deg, y, add, part, part_max, g->prs,
-                           fmt == GPR_CONTRIB_F16 ? 1 : 0);
+        const bool direct = L->max_chunks <= COLD_GROUP;
+        if (!direct)
+            hipLaunchKernelGGL(k_cold_combine_groups, dim3(L->ngroups * per_bin), dim3(CC_THREADS), 0, g->stream,
+                               L->groups, g->n, per_bin, (const long long *)L->partials, L->partials2);
+        hipLaunchKernelGGL(k_cold_combine, dim3(L->nmulti * per_bin), dim3(CC_THREADS), 0, g->stream, L->multi,
+                           L->nbins, g->n, per_bin, direct ? 1 : 0,
+                           (const long long *)(direct ? L->partials : L->partials2), g->deg, y, add, part, part_max,
+                           g->prs, fmt == GPR_CONTRIB_F16 ? 1 : 0);
     }
     GPR_HIP(hipGetLastError());
-    *nparts = L->nbins + L->nmulti * CC_PER_BIN;
+    *nparts = L->nbins + L->nmulti * per_bin;
     return GPR_OK;
 }
 

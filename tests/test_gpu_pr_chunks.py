@@ -1,0 +1,57 @@
+"""PageRank's binned edgemap where its tiles and chunks change with the graph:
+sizes around one bin (16384), one tile (1024), bins in one chunk, in up to a
+group of 16 and in several groups, directed and relabelled graphs.
+
+Bars as in test_gpu_pr_split: relative L1 against FP64 of 1e-6 for FP32 (each
+rank is rounded to 24 bits a few times an iteration, and errors contract by
+the damping) and 1e-3 for 16-bit contributions on power-law graphs; repeated
+runs are bit-identical.
+"""
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+G = pytest.importorskip("graptor_amd")
+
+
+@pytest.fixture(scope="module", autouse=True)
+def device():
+    G.lib()
+    yield
+
+
+def rel_l1(a, b):
+    return float(np.abs(a.astype(np.float64) - b).sum() / np.abs(b).sum())
+
+
+def skewed(n, m, seed):
+    """m directed edges whose ends follow a power law over n vertices."""
+    rng = np.random.default_rng(seed)
+    return tuple((n * rng.random(m) ** 3).astype(np.uint32) for _ in range(2))
+
+
+# vertices, edges drawn: one bin or tile more or less, few and many chunks
+SIZES = [(1023, 4000), (1025, 60000), (16383, 40000), (16385, 300000), (40001, 1500000), (70003, 6000000),
+         (600011, 3000000)]
+
+
+@pytest.mark.parametrize("n,m", SIZES)
+@pytest.mark.parametrize("directed", [False, True])
+def test_ranks_across_layout_sizes(n, m, directed):
+    src, dst = skewed(n, m, n)
+    index, nbrs = O.build_csr(n, src, dst, symmetrize=not directed)
+    if directed:
+        ci, cn = O.build_csr(n, dst, src, symmetrize=False)
+        x64, _, _ = O.pr_fp64(ci, cn, 12, 0.0, outdeg=np.diff(index).astype(np.uint32))
+    else:
+        x64, _, _ = O.pr_fp64(index, nbrs, 12, 0.0)
+    with G.Graph.from_csr(index, nbrs, symmetric=not directed) as g:
+        if not directed:
+            g.reorder()
+        for fmt, bar in (("fp32", 1e-6), ("fp16", 1e-3)):
+            x, _ = g.pr_vary([(fmt, 0.0)], max_iter=12)
+            assert rel_l1(x, x64) <= bar, (fmt, rel_l1(x, x64))
+            x2, _ = g.pr_vary([(fmt, 0.0)], max_iter=12)
+            assert np.array_equal(x, x2), fmt
