@@ -340,6 +340,19 @@ struct CCv {
     }
 };
 
+// y[d] += contrib[s] over every edge: A::edgemap(GA, A::relax(A::pr_sum(...)))
+// without its statistics, whose time stamp would wait for the stream
+template <class CT>
+void pr_sum_step(const Graph &GA, A::vertexprop<float> &y, A::vertexprop<CT> &contrib, int fmt, float dampen = 0.85f) {
+    gpr_emap_desc d = {};
+    d.relax = GPR_RELAX_PR_SUM;
+    d.prop = y.get();
+    d.contrib = contrib.get();
+    d.contrib_fmt = fmt;
+    d.damping = dampen;
+    check(gpr_edgemap(GA.get(), &d, nullptr, nullptr, nullptr), "pr edgemap");
+}
+
 // ---- PRv / PR_vary --------------------------------------------------------------
 struct PRv {
     Graph GA;
@@ -383,10 +396,7 @@ struct PRv {
                 }
                 pending = false;
             }
-            if (rc != GPR_OK) {
-                auto lazy = A::edgemap(GA, A::relax(A::pr_sum(y_mem, contrib, fmt, dampen)));
-                lazy.materialize();
-            }
+            if (rc != GPR_OK) pr_sum_step(GA, y_mem, contrib, fmt, dampen);
             // the vertex_scan / vertex_map tail of PRv.C:214-269, fused
             // (deferred into the next iteration when that one is fused)
             if (fuse_tail && iter + 1 < o.max_iter)
@@ -477,8 +487,7 @@ struct APRv {
                 check(apr_contrib(GA.get(), fmt, delta_mem.get(), contrib.get(), factor,
                                   kind == 2 ? F.get() : nullptr),
                       "apr contributions");
-                auto lazy = A::edgemap(GA, A::relax(A::pr_sum(z_mem, contrib, fmt)));
-                lazy.materialize();
+                pr_sum_step(GA, z_mem, contrib, fmt);
                 st.direction = GPR_DIR_PULL;
             } else {
                 check(apr_push(GA.get(), fmt, F.get(), delta_mem.get(), factor, z_mem.get()), "apr push");

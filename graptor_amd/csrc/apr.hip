@@ -28,6 +28,7 @@
 // rounds separately.
 #include "internal.hpp"
 #include "device.hpp"
+#include "grid_sync.hpp"
 #include "pr_codec.hpp"
 #include "apr.hpp"
 
@@ -149,10 +150,11 @@ template <bool FIRST>
 __global__ void __launch_bounds__(AT_THREADS)
 k_apr_tail(uint32_t n, const float *__restrict__ y, float factor, float dampen, float cst, float ninv, float eps2,
            float *__restrict__ x, float *__restrict__ delta, const uint32_t *__restrict__ deg,
-           uint64_t *__restrict__ bits, double *__restrict__ part, uint64_t *__restrict__ cpart) {
+           uint64_t *__restrict__ bits, double *part, uint64_t *cpart, unsigned int *ticket, HostScalars *h) {
 #pragma clang fp contract(off)
     __shared__ double r1[AT_WAVES], r2[AT_WAVES];
     __shared__ uint64_t r3[AT_WAVES], r4[AT_WAVES];
+    __shared__ int s_last;
     const uint32_t words = (uint32_t)(((uint64_t)n + 63) / 64);
     const uint32_t wv = threadIdx.x / 64;
     const uint32_t nwv = gridDim.x * AT_WAVES;
@@ -211,47 +213,31 @@ k_apr_tail(uint32_t n, const float *__restrict__ y, float factor, float dampen, 
             c += r3[i];
             d += r4[i];
         }
-        part[2 * blockIdx.x] = a;
-        part[2 * blockIdx.x + 1] = b;
-        cpart[2 * blockIdx.x] = c;
-        cpart[2 * blockIdx.x + 1] = d;
+        st_part(&part[2 * blockIdx.x], a);
+        st_part(&part[2 * blockIdx.x + 1], b);
+        st_part(&cpart[2 * blockIdx.x], c);
+        st_part(&cpart[2 * blockIdx.x + 1], d);
     }
-}
-
-// Totals of the tail's partials in a fixed order: out = {L1, sum |x|,
-// nactv, nacte} (the last two as integers in the same 8-byte slots).
-__global__ void __launch_bounds__(256)
-k_apr_reduce(const double *__restrict__ part, const uint64_t *__restrict__ cpart, uint32_t count,
-             AprTotals *out) {
-    __shared__ double r1[256], r2[256];
-    __shared__ uint64_t r3[256], r4[256];
-    double a = 0.0, b = 0.0;
-    uint64_t c = 0, d = 0;
-    for (uint32_t i = threadIdx.x; i < count; i += 256) {
-        a += part[2 * i];
-        b += part[2 * i + 1];
-        c += cpart[2 * i];
-        d += cpart[2 * i + 1];
+    // the last workgroup adds the partials in a fixed order, into the host's
+    // line
+    if (!last_workgroup(ticket, &s_last)) return;
+    sl1 = sx = 0.0;
+    cv = ce = 0;
+    for (uint32_t i = threadIdx.x; i < gridDim.x; i += AT_THREADS) {
+        sl1 += ld_part(&part[2 * i]);
+        sx += ld_part(&part[2 * i + 1]);
+        cv += ld_part(&cpart[2 * i]);
+        ce += ld_part(&cpart[2 * i + 1]);
     }
-    r1[threadIdx.x] = a;
-    r2[threadIdx.x] = b;
-    r3[threadIdx.x] = c;
-    r4[threadIdx.x] = d;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (threadIdx.x < (unsigned)o) {
-            r1[threadIdx.x] += r1[threadIdx.x + o];
-            r2[threadIdx.x] += r2[threadIdx.x + o];
-            r3[threadIdx.x] += r3[threadIdx.x + o];
-            r4[threadIdx.x] += r4[threadIdx.x + o];
-        }
-        __syncthreads();
-    }
+    sl1 = block_sum(sl1, r1);
+    sx = block_sum(sx, r2);
+    cv = block_sum(cv, r3);
+    ce = block_sum(ce, r4);
     if (threadIdx.x == 0) {
-        out->l1 = r1[0];
-        out->sum_x = r2[0];
-        out->nactv = r3[0];
-        out->nacte = r4[0];
+        h->l1 = sl1;
+        h->sum_abs = sx;
+        h->nactv = cv;
+        h->nacte = ce;
     }
 }
 
@@ -342,10 +328,9 @@ int apr_tail(gpr_graph *g, bool first, const gpr_prop *yp, float factor, float e
     const uint32_t n = g->n;
     GPR_TRY(frontier_ensure_bits(out));
     const unsigned grid = grid_for(nwords(n), AT_WAVES, AT_MAX_BLOCKS);
-    GPR_TRY(ensure_partials(g, 4 * (size_t)grid + 8));
+    GPR_TRY(ensure_partials(g, 4 * (size_t)grid));
     double *part = g->partial;
     uint64_t *cpart = (uint64_t *)(g->partial + 2 * (size_t)grid);
-    AprTotals *dtot = (AprTotals *)(g->partial + 4 * (size_t)grid);
     const float dampen = 0.85f;
     const float ninv = 1.0f / (float)n;
     const float cst = (1.0f - dampen) * ninv;
@@ -353,15 +338,17 @@ int apr_tail(gpr_graph *g, bool first, const gpr_prop *yp, float factor, float e
         ProfScope ps(g, "apr_tail");
         if (first)
             hipLaunchKernelGGL(k_apr_tail<true>, dim3(grid), dim3(AT_THREADS), 0, g->stream, n, y, factor, dampen,
-                               cst, ninv, eps2, x, delta, g->deg, out->bits, part, cpart);
+                               cst, ninv, eps2, x, delta, g->deg, out->bits, part, cpart, g->ticket, g->hsc_dev);
         else
             hipLaunchKernelGGL(k_apr_tail<false>, dim3(grid), dim3(AT_THREADS), 0, g->stream, n, y, factor, dampen,
-                               cst, ninv, eps2, x, delta, g->deg, out->bits, part, cpart);
-        hipLaunchKernelGGL(k_apr_reduce, dim3(1), dim3(256), 0, g->stream, part, cpart, grid, dtot);
+                               cst, ninv, eps2, x, delta, g->deg, out->bits, part, cpart, g->ticket, g->hsc_dev);
     }
     GPR_HIP(hipGetLastError());
-    GPR_HIP(hipMemcpyAsync(tot, dtot, sizeof(AprTotals), hipMemcpyDeviceToHost, g->stream));
     GPR_HIP(hipStreamSynchronize(g->stream));
+    tot->l1 = g->hsc->l1;
+    tot->sum_x = g->hsc->sum_abs;
+    tot->nactv = g->hsc->nactv;
+    tot->nacte = g->hsc->nacte;
     out->nactv = (uint32_t)tot->nactv;
     out->nacte = tot->nacte;
     out->kind = tot->nactv ? GPR_FRONTIER_BITMAP : GPR_FRONTIER_EMPTY;

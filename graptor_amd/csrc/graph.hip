@@ -6,6 +6,7 @@
 // findHighestDegreeVertex :2446-2451; api::vertexprop api/vertexprop.h:28-143.
 #include "internal.hpp"
 #include "device.hpp"
+#include "grid_sync.hpp"
 
 #include <stdio.h>
 #include <string.h>
@@ -95,11 +96,16 @@ static int finish_graph(gpr_graph *g, const uint64_t *host_index, const uint64_t
     g->max_deg = n ? (uint32_t)(host_index[g->hdv + 1] - host_index[g->hdv]) : 0;
     GPR_TRY(dev_alloc((void **)&g->ctr, COUNTER_BYTES, "counters"));
     GPR_HIP(hipMemset(g->ctr, 0, COUNTER_BYTES));
+    GPR_TRY(dev_alloc((void **)&g->ticket, sizeof(unsigned int) * LW_WORDS, "last-workgroup counters"));
+    GPR_HIP(hipMemset(g->ticket, 0, sizeof(unsigned int) * LW_WORDS));
     // the counter read-back target: fine-grained (coherent) pinned host
     // memory that a one-wave kernel writes the sums into, so that a step's
     // counts come back with the stream's completion and no copy
-    GPR_HIP(hipHostMalloc((void **)&g->hctr, sizeof(DevCounters), hipHostMallocMapped | hipHostMallocCoherent));
+    GPR_HIP(hipHostMalloc((void **)&g->hctr, sizeof(DevCounters) + sizeof(HostScalars), hipHostMallocMapped | hipHostMallocCoherent));
     GPR_HIP(hipHostGetDevicePointer((void **)&g->hctr_dev, g->hctr, 0));
+    g->hsc = (HostScalars *)(g->hctr + 1);
+    g->hsc_dev = (HostScalars *)(g->hctr_dev + 1);
+    *g->hsc = HostScalars{};
     GPR_TRY(dev_alloc((void **)&g->dedup, sizeof(uint64_t) * nwords(n), "dedup bitmap"));
     GPR_HIP(hipMemset(g->dedup, 0, sizeof(uint64_t) * nwords(n)));
     GPR_TRY(dev_alloc((void **)&g->scan, sizeof(uint64_t) * ((size_t)n + 1), "frontier prefix"));
@@ -130,6 +136,7 @@ static void graph_free(gpr_graph *g) {
     dev_free(g->long_base);
     dev_free(g->long_partial);
     dev_free(g->ctr);
+    dev_free(g->ticket);
     if (g->hctr) hipHostFree(g->hctr);
     dev_free(g->dedup);
     dev_free(g->scan);

@@ -31,6 +31,47 @@ __device__ __forceinline__ unsigned long long bcast64(unsigned long long v) {
     return ((unsigned long long)hi << 32) | lo;
 }
 
+// Whether this workgroup is the last of its launch to get here, in every
+// thread (all call it).  Thread 0's earlier stores are acknowledged before
+// it counts itself, so what every workgroup's thread 0 stored with
+// agent-scope stores can be read by the last one with agent-scope loads: a
+// reduction of per-workgroup partials then needs no launch of its own (a
+// launch in a stream costs about 6 us, most of a small graph's iteration).
+// Atomics on one address go one after another, about 12 ns each (50 us for
+// 4096 workgroups of a kernel that takes 10), so above LW_GROUPS workgroups
+// each counts on one of LW_GROUPS lines and the last of a line on the top
+// one.  All counters are zero again when the launch ends.
+constexpr unsigned LW_GROUPS = 64;
+constexpr unsigned LW_LINE = 32;                                   // u32 per 128-byte line
+constexpr size_t LW_WORDS = (LW_GROUPS + 1) * (size_t)LW_LINE;     // top, then the groups
+__device__ __forceinline__ bool count_zeroed(unsigned int *c, unsigned int all) {
+    if (__hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != all - 1) return false;
+    __hip_atomic_store(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return true;
+}
+__device__ __forceinline__ bool last_workgroup(unsigned int *ticket, int *s_last) {
+    if (threadIdx.x == 0) {
+        __builtin_amdgcn_s_waitcnt(WAIT_VM0);
+        bool l = true;
+        unsigned int tops = gridDim.x;
+        if (gridDim.x > LW_GROUPS) {
+            const unsigned grp = blockIdx.x % LW_GROUPS;
+            tops = LW_GROUPS;
+            l = count_zeroed(ticket + (1 + grp) * LW_LINE,
+                             gridDim.x / LW_GROUPS + (grp < gridDim.x % LW_GROUPS ? 1u : 0u));
+        }
+        *s_last = l && count_zeroed(ticket, tops);
+    }
+    __syncthreads();
+    return *s_last != 0;
+}
+template <class T> __device__ __forceinline__ void st_part(T *p, T v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T> __device__ __forceinline__ T ld_part(const T *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Grid barrier in two levels.  Block b arrives on the counter of group
 // b % ngroups (at most GS_GROUP blocks each); the last block of a group to
 // arrive at level `lvl` counts the group on `arrive`, and level `lvl` ends

@@ -89,8 +89,6 @@ struct alignas(128) DevCounters {
     unsigned long long edges;   // host mirror: edges examined
     unsigned int nactv;         // host mirror: vertices of the frontier produced
     unsigned int listpos;       // append position of the list being produced
-    unsigned int pad0;
-    unsigned int ticket2;       // last-workgroup ticket of the FP64 reductions (reset by that workgroup)
     unsigned int decision;      // host mirror: the policy's choice for the next step
     unsigned int pad;
 };
@@ -104,6 +102,15 @@ constexpr size_t COUNTER_BYTES = sizeof(DevCounters) + CTR_STRIPES * sizeof(CtrS
 __device__ __forceinline__ CtrStripe *ctr_stripe(DevCounters *c) {
     return reinterpret_cast<CtrStripe *>(c + 1) + (blockIdx.x % CTR_STRIPES);
 }
+
+// Totals of the last PageRank or delta PageRank tail, written by the device
+// into the pinned line after the counters' mirror: the host reads them after
+// the stream's completion, without a copy.
+struct alignas(128) HostScalars {
+    double delta, sum_x;            // PageRank: L1 residual, sum of the ranks
+    double l1, sum_abs;             // delta PageRank: sum |delta|, sum |x|
+    unsigned long long nactv, nacte;
+};
 
 // Scalars of the PageRank iteration, kept on the device so that an
 // iteration needs no host round trip.
@@ -211,6 +218,9 @@ struct gpr_graph {
     gpr::DevCounters *ctr = nullptr;     // device
     gpr::DevCounters *hctr = nullptr;    // host mirror: fine-grained pinned memory the device writes
     gpr::DevCounters *hctr_dev = nullptr;  // its device address
+    unsigned int *ticket = nullptr;      // last_workgroup's counters, zero between launches
+    gpr::HostScalars *hsc = nullptr;     // the line after hctr: scalars of the last vertex-map tail
+    gpr::HostScalars *hsc_dev = nullptr;
     uint64_t *dedup = nullptr;           // n/64 words, all zero between steps
     uint64_t *scan = nullptr;            // frontier degree prefix (n+1)
     uint64_t *scan_blk = nullptr;        // per-scan-block totals
@@ -218,7 +228,7 @@ struct gpr_graph {
     size_t partial_cap = 0;
     float *partial_f = nullptr;          // per-workgroup partial maxima
     double *long_partial = nullptr;      // per long chunk
-    double *dsum_slices = nullptr;       // 64 slice sums of deterministic_sum
+    double *dsum_slices = nullptr;       // slice sums and maxima of k_pr_reduce
     gpr::PrScalars *prs = nullptr;       // device
     // trace of the last run
     std::vector<gpr_iter_stats> trace;
@@ -273,6 +283,7 @@ struct gpr_frontier {
     uint64_t nacte = 0;
     uint32_t *list = nullptr;   // capacity n
     uint64_t *bits = nullptr;   // (n+63)/64 words
+    bool counted = false;       // BITMAP: nactv and nacte are those of the bits (a caller's list may repeat IDs)
 };
 
 namespace gpr {
@@ -320,8 +331,8 @@ int scan_frontier_degrees(gpr_graph *g, const uint32_t *list, uint32_t k);
 // with the previous iteration's tail fused in (x' written, cold_tail_fusable)
 int cold_launch_write(gpr_graph *g, int fmt, const void *contrib, const float *y, float *x, float damping);
 bool cold_tail_fusable(const gpr_graph *g);
-// y (+)= the binned sums; *nparts receives the number of y partial slots
-int cold_launch_accum(gpr_graph *g, int fmt, float *y, int add, double *part, float *part_max, uint32_t *nparts);
+// y (+)= the binned sums; sets the iteration's scalars from the sum of y
+int cold_launch_accum(gpr_graph *g, int fmt, float *y, int add, double *part, float *part_max, float damping);
 
 // Host entry points shared between translation units.
 int frontier_ensure_list(gpr_frontier *f);
@@ -342,8 +353,6 @@ int graph_setup(gpr_graph *g);                    // deg, buckets, long rows
 // ID mapping between original (ABI) and internal (relabelled) vertex IDs.
 int map_ids(gpr_graph *g, uint32_t *d_ids, uint32_t k, bool to_internal);
 int to_internal_id(gpr_graph *g, uint32_t orig, uint32_t *internal);
-int deterministic_sum(gpr_graph *g, const double *parts, uint32_t count,
-                      double *dst);               // device-side, async
 int batch_noalloc_setup(int dev);                 // scratch address of gpr_batch_cc_noalloc (batch.hip)
 // push/pull switch (edgemap.hip): pct <= 0 is default_threshold (m/20),
 // pct > 0 frac_threshold(pct)

@@ -6,18 +6,20 @@
 // (customfp.h:20-211, variants :449-648), dense pull over the CSC
 // (dsl/emap/GraptorCSCDataParCached.h:60-302 / GraphCSx_csc.h:50-140).
 //
-// Per iteration, four launches on the handle's stream, no host round trip:
+// Per iteration, on the handle's stream, with no host round trip (pull; the
+// binned sums of pr_cold.hip are the default):
 //   k_pr_pull    buckets of <= STREAM_ITEMS rows+edges: neighbour IDs are read
 //                coalesced, contributions gathered into LDS, then each row is
 //                summed from LDS (lane per short row, wave per row above 64
 //                edges).  Rows above LONG_DEG are cut into LONG_CHUNK-edge
 //                chunks, one workgroup each, summed by k_pr_long.
-//   k_pr_reduce  deterministic FP64 sum of the workgroup partials of y and
-//                the maximum of y/deg; the last workgroup derives w, 1/s and
-//                the FP16 encode scale.
+//                The last workgroup to finish sums the workgroup partials of
+//                y and the maximum of y/deg in a fixed order (FP64) and
+//                derives w, 1/s and the FP16 encode scale (pr_fold.hpp);
+//                k_pr_reduce does where there are many partials.
 //   k_pr_update  x' = (y + w) / s, |x - x'| partials, x = x', contrib =
-//                d*x'/deg encoded in the contribution format.
-//   k_pr_reduce  (again) sums the residual partials into delta.
+//                d*x'/deg encoded in the contribution format; the last
+//                workgroup sums the residual partials into delta.
 // FP32 contributions are accumulated in FP64 registers as PRv does (y_acc
 // is double over FP32 storage, PRv.C:127); 16-bit contributions are
 // accumulated in FP32.
@@ -25,6 +27,7 @@
 #include "device.hpp"
 #include "pr_codec.hpp"
 #include "grid_sync.hpp"
+#include "pr_fold.hpp"
 
 #include <math.h>
 
@@ -55,8 +58,8 @@ k_pr_pull(uint32_t nbuckets, const uint32_t *__restrict__ bucket, const uint64_t
           const uint32_t *__restrict__ cnbrs, const uint32_t *__restrict__ deg,
           const typename Codec<FMT>::store_t *__restrict__ contrib, float *__restrict__ y,
           const uint32_t *__restrict__ long_rows, const uint32_t *__restrict__ long_base, uint32_t nlong,
-          double *__restrict__ long_partial, double *__restrict__ part, float *__restrict__ part_max,
-          const PrScalars *__restrict__ prs, uint32_t cold_from) {
+          double *__restrict__ long_partial, double *part, float *part_max, const PrScalars *prs,
+          uint32_t cold_from, PrFold fold) {
     using C = Codec<FMT>;
     using acc_t = typename C::acc_t;
     __shared__ float vals[PR_LDS_EDGES];
@@ -65,6 +68,7 @@ k_pr_pull(uint32_t nbuckets, const uint32_t *__restrict__ bucket, const uint64_t
     __shared__ uint32_t nmed;
     __shared__ double dred[PR_THREADS / 64];
     __shared__ float fred[PR_THREADS / 64];
+    __shared__ int s_last;
     const float dscale = FMT == GPR_CONTRIB_F16 ? 1.0f / prs->enc_scale : 1.0f;
     const uint32_t b = blockIdx.x;
     if (b >= nbuckets) {
@@ -98,10 +102,10 @@ k_pr_pull(uint32_t nbuckets, const uint32_t *__restrict__ bucket, const uint64_t
         double tot = block_sum((double)acc, dred);
         if (threadIdx.x == 0) {
             long_partial[c] = tot;
-            part[b] = 0.0;
-            part_max[b] = 0.0f;
+            st_part(&part[b], 0.0);
+            st_part(&part_max[b], 0.0f);
         }
-        return;
+        return;   // with long rows the fold is k_pr_long's
     }
     // ---- a bucket of rows
     const uint32_t r0 = bucket[b], r1 = bucket[b + 1];
@@ -189,124 +193,94 @@ k_pr_pull(uint32_t nbuckets, const uint32_t *__restrict__ bucket, const uint64_t
     if (threadIdx.x == 0) {
         float mx = fred[0];
         for (int i = 1; i < PR_THREADS / 64; ++i) mx = fmaxf(mx, fred[i]);
-        part[b] = ts;
-        part_max[b] = mx;
+        st_part(&part[b], ts);
+        st_part(&part_max[b], mx);
     }
+    pr_fold_sum<PR_THREADS, FMT == GPR_CONTRIB_F16>(fold, part, part_max, dred, &s_last);
 }
 
 // One thread per long row: fold its chunk partials in chunk order.
-__global__ void k_pr_long(uint32_t nlong, const uint32_t *__restrict__ long_rows, const uint32_t *__restrict__ long_base,
-                          const double *__restrict__ long_partial, const uint32_t *__restrict__ deg, float *y,
-                          double *part, float *part_max, uint32_t slot0, const PrScalars *__restrict__ prs, int f16) {
-    const float dscale = f16 ? 1.0f / prs->enc_scale : 1.0f;
+template <bool F16>
+__global__ void __launch_bounds__(PR_THREADS)
+k_pr_long(uint32_t nlong, const uint32_t *__restrict__ long_rows, const uint32_t *__restrict__ long_base,
+          const double *__restrict__ long_partial, const uint32_t *__restrict__ deg, float *y,
+          double *part, float *part_max, uint32_t slot0, const PrScalars *prs, PrFold fold) {
+    __shared__ double dred[PR_THREADS / 64];
+    __shared__ int s_last;
+    const float dscale = F16 ? 1.0f / prs->enc_scale : 1.0f;
     for (uint32_t li = blockIdx.x * blockDim.x + threadIdx.x; li < nlong; li += gridDim.x * blockDim.x) {
         double s = 0.0;
         for (uint32_t c = long_base[li]; c < long_base[li + 1]; ++c) s += long_partial[c];
         const uint32_t row = long_rows[li];
         const float yv = (float)s * dscale;
         y[row] = yv;
-        part[slot0 + li] = (double)yv;
+        st_part(&part[slot0 + li], (double)yv);
         const uint32_t dg = deg[row];
-        part_max[slot0 + li] = dg ? yv / (float)dg : 0.0f;
+        st_part(&part_max[slot0 + li], dg ? yv / (float)dg : 0.0f);
     }
+    // every thread wrote partials: all of the workgroup's are acknowledged
+    // before its thread 0 counts it
+    __builtin_amdgcn_s_waitcnt(WAIT_VM0);
+    __syncthreads();
+    pr_fold_sum<PR_THREADS, F16>(fold, part, part_max, dred, &s_last);
 }
 
-// Deterministic reduction of `count` partial sums (and maxima).  mode 0:
-// after the pull -- set sum_y, w, inv_s and the encode scale.  mode 1: after
-// the update -- set delta and sum_x from the two partial arrays.  mode 2:
-// maximum only.  mode 3: the cold-edge mass -- set the fixed-point unit.
+// Deterministic reduction of `count` partial sums and maxima by many
+// workgroups, for pulls of more than PR_FOLD_MAX partials: the last
+// workgroup sets the scalars (set_sum) or leaves the slices' maxima to
+// k_pr_set_scale.
 constexpr int RED_THREADS = 256;
 constexpr int RED_BLOCKS = 64;
-// Workgroups of a reduction: one for a few thousand partials (a launch of
-// 64 and the last-workgroup fold cost more than the sums), RED_BLOCKS above
-// that; the sums stay deterministic for a given count
-static unsigned red_grid(uint32_t count) { return count <= 16384u ? 1u : (unsigned)RED_BLOCKS; }
+// partials a pull's own last workgroup folds (64 loads a thread)
+constexpr uint32_t PR_FOLD_MAX = 16384;
 __global__ void __launch_bounds__(RED_THREADS)
-k_pr_reduce(const double *__restrict__ part, const float *__restrict__ part_max, const double *__restrict__ part2,
-            uint32_t count, double *slices, unsigned int *ticket, PrScalars *prs, int mode, uint32_t n,
-            float damping, int f16) {
-    __shared__ double r1[RED_THREADS], r2[RED_THREADS];
+k_pr_reduce(const double *__restrict__ part, const float *__restrict__ part_max, uint32_t count, double *slices,
+            unsigned int *ticket, PrScalars *prs, int set_sum, uint32_t n, float damping, int f16) {
+    __shared__ double r1[RED_THREADS];
     __shared__ float r3[RED_THREADS];
-    __shared__ bool last;
+    __shared__ int s_last;
     const uint32_t per = (count + gridDim.x - 1) / gridDim.x;
     const uint32_t lo = blockIdx.x * per, hi = min(count, lo + per);
-    double s1 = 0.0, s2 = 0.0;
+    double s1 = 0.0;
     float mx = 0.0f;
     for (uint32_t i = lo + threadIdx.x; i < hi; i += RED_THREADS) {
         s1 += part[i];
-        if (mode == 0 || mode == 2) mx = fmaxf(mx, part_max[i]);
-        if (mode == 1) s2 += part2[i];
+        mx = fmaxf(mx, part_max[i]);
     }
     r1[threadIdx.x] = s1;
-    r2[threadIdx.x] = s2;
     r3[threadIdx.x] = mx;
     __syncthreads();
     for (int o = RED_THREADS / 2; o > 0; o >>= 1) {
         if (threadIdx.x < (unsigned)o) {
             r1[threadIdx.x] += r1[threadIdx.x + o];
-            r2[threadIdx.x] += r2[threadIdx.x + o];
             r3[threadIdx.x] = fmaxf(r3[threadIdx.x], r3[threadIdx.x + o]);
         }
         __syncthreads();
     }
-    // slices: agent-scope stores, acknowledged (s_waitcnt vmcnt(0)) before
-    // the ticket; the last workgroup reads them with agent-scope loads (no
-    // fence, which would write back the XCD's L2)
     if (threadIdx.x == 0) {
-        __hip_atomic_store(&slices[3 * blockIdx.x], r1[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(&slices[3 * blockIdx.x + 1], r2[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(&slices[3 * blockIdx.x + 2], (double)r3[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __builtin_amdgcn_s_waitcnt(WAIT_VM0);
-        last = atomicAdd(ticket, 1u) == gridDim.x - 1;
+        st_part(&slices[2 * blockIdx.x], r1[0]);
+        st_part(&slices[2 * blockIdx.x + 1], (double)r3[0]);
     }
-    __syncthreads();
-    if (!last || threadIdx.x != 0) return;
-    double a = 0.0, c = 0.0, m = 0.0;
+    if (!last_workgroup(ticket, &s_last) || threadIdx.x != 0 || !set_sum) return;
+    double a = 0.0, m = 0.0;
     for (unsigned i = 0; i < gridDim.x; ++i) {
-        a += __hip_atomic_load(&slices[3 * i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        c += __hip_atomic_load(&slices[3 * i + 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        m = fmax(m, __hip_atomic_load(&slices[3 * i + 2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        a += ld_part(&slices[2 * i]);
+        m = fmax(m, ld_part(&slices[2 * i + 1]));
     }
-    if (mode == 0) {
-        // PRv.C:214-240: w = (1 - s)/n; y += w; s = sum y; y *= 1/s.
-        // sum(y + w) = s + n*w is formed analytically in FP64.
-        const double w = (1.0 - a) / (double)n;
-        const double s2t = a + (double)n * w;
-        prs->sum_y = a;
-        prs->w = w;
-        prs->inv_s = 1.0 / s2t;
-        prs->max_ratio = (float)m;
-        if (f16) {
-            // largest next contribution <= d * (max y/deg + w) / s; keep it
-            // at or below 2^15 so the FP16 store cannot overflow (max 65504)
-            const double u = (double)damping * (m + w) / s2t;
-            int k = u > 0.0 ? (int)floor(log2(32768.0 / u)) : 0;
-            k = k > 100 ? 100 : k < -100 ? -100 : k;
-            prs->enc_scale = (float)ldexp(1.0, k);
-        } else {
-            prs->enc_scale = 1.0f;
-        }
-    } else if (mode == 1) {
-        prs->delta = a;
-        prs->sum_x = c;
-    } else if (mode == 3) {
-        // fixed-point unit of the cold sums: 2^E with M <= 2^61 units, M the
-        // total |contribution| over the cold edges
-        int e = 0;
-        if (a > 0.0 && a < 1e300) e = ilogb(a) + 1 - 61;
-        prs->cold_exp = e;
-        prs->cold_unit = ldexp(1.0, e);
-    }
-    // mode 2 (maximum only): the slices are read by k_pr_set_scale
-    *ticket = 0;
+    if (f16) pr_set_sum<true>(prs, a, m, n, damping);
+    else pr_set_sum<false>(prs, a, m, n, damping);
 }
 
+// Bound by its streams (20 B a vertex in FP32).  The last workgroup also
+// sums the residual and the ranks, into the device's scalars and the host's
+// line.
 template <int FMT>
 __global__ void __launch_bounds__(256)
 k_pr_update(uint32_t n, const float *__restrict__ y, float *__restrict__ x, typename Codec<FMT>::store_t *contrib,
-            const uint32_t *__restrict__ deg, float damping, const PrScalars *__restrict__ prs, double *part_delta,
-            double *part_sum) {
+            const uint32_t *__restrict__ deg, float damping, PrScalars *prs, double *part_delta, double *part_sum,
+            unsigned int *ticket, HostScalars *h) {
     __shared__ double r1[4], r2[4];
+    __shared__ int s_last;
     const double w = prs->w, inv_s = prs->inv_s;
     const float sc = FMT == GPR_CONTRIB_F16 ? prs->enc_scale : 1.0f;
     double dl = 0.0, sx = 0.0;
@@ -322,8 +296,22 @@ k_pr_update(uint32_t n, const float *__restrict__ y, float *__restrict__ x, type
     dl = block_sum(dl, r1);
     sx = block_sum(sx, r2);
     if (threadIdx.x == 0) {
-        part_delta[blockIdx.x] = dl;
-        part_sum[blockIdx.x] = sx;
+        st_part(&part_delta[blockIdx.x], dl);
+        st_part(&part_sum[blockIdx.x], sx);
+    }
+    if (!last_workgroup(ticket, &s_last)) return;
+    dl = sx = 0.0;
+    for (uint32_t i = threadIdx.x; i < gridDim.x; i += 256) {
+        dl += ld_part(&part_delta[i]);
+        sx += ld_part(&part_sum[i]);
+    }
+    dl = block_sum(dl, r1);
+    sx = block_sum(sx, r2);
+    if (threadIdx.x == 0) {
+        prs->delta = dl;
+        prs->sum_x = sx;
+        h->delta = dl;
+        h->sum_x = sx;
     }
 }
 
@@ -357,7 +345,7 @@ k_pr_xmax(uint32_t n, const float *__restrict__ x, double *part, float *part_max
 __global__ void k_pr_set_scale(PrScalars *prs, const double *slices, uint32_t nslices, float damping, int f16) {
     if (threadIdx.x != 0) return;
     double m = 0.0;
-    for (uint32_t i = 0; i < nslices; ++i) m = fmax(m, slices[3 * i + 2]);
+    for (uint32_t i = 0; i < nslices; ++i) m = fmax(m, slices[2 * i + 1]);
     if (f16) {
         const double u = (double)damping * m;
         int k = u > 0.0 ? (int)floor(log2(32768.0 / u)) : 0;
@@ -405,21 +393,25 @@ static int pr_edgemap_impl(gpr_graph *g, const gpr_emap_desc *desc, gpr_frontier
     float *y = (float *)desc->prop->d;
     const void *cb = desc->contrib->d;
     const float damping = desc->damping > 0.f ? desc->damping : 0.85f;
-    GPR_HIP(hipEventRecord(g->ev0, g->stream));
+    if (st) GPR_HIP(hipEventRecord(g->ev0, g->stream));
     if (split) {
         ProfScope ps(g, "pr_cold_write");
         GPR_TRY(cold_launch_write(g, fmt, cb, y, x_tail, damping));
-        hipLaunchKernelGGL(k_pr_reduce, dim3(red_grid(g->cold->nwchunks)), dim3(RED_THREADS), 0, g->stream, g->cold->mass,
-                           (const float *)nullptr, (const double *)nullptr, g->cold->nwchunks, g->dsum_slices,
-                           &g->ctr->ticket2, g->prs, 3, g->n, damping, 0);
     }
+    // the kernel that writes the last of y's partials also folds them into
+    // the scalars: the binned sums' last kernel; without them the pull, or
+    // the long rows' kernel after it
+    const uint32_t nparts = nblk + g->nlong;
+    PrFold fold = {g->ticket, g->prs, split || nparts > PR_FOLD_MAX ? 0 : nparts, g->n, damping};
+    PrFold pull_fold = fold;
+    if (g->nlong) pull_fold.count = 0;
     if (cold_from > 0) {
         // the pull over sources [0, cold_from); every source when not split
         ProfScope ps(g, "pr_pull");
 #define PR_PULL(F)                                                                                              \
     hipLaunchKernelGGL(k_pr_pull<F>, dim3(nblk), dim3(PR_THREADS), 0, g->stream, g->nbuckets, g->bucket,        \
                        g->cindex, g->cnbrs, g->deg, (const typename Codec<F>::store_t *)cb, y, g->long_rows,   \
-                       g->long_base, g->nlong, g->long_partial, g->partial, g->partial_f, g->prs, cold_from)
+                       g->long_base, g->nlong, g->long_partial, g->partial, g->partial_f, g->prs, cold_from, pull_fold)
         switch (fmt) {
         case GPR_CONTRIB_F32: PR_PULL(GPR_CONTRIB_F32); break;
         case GPR_CONTRIB_BF16: PR_PULL(GPR_CONTRIB_BF16); break;
@@ -432,25 +424,26 @@ static int pr_edgemap_impl(gpr_graph *g, const gpr_emap_desc *desc, gpr_frontier
     }
     if (cold_from > 0 && g->nlong) {
         ProfScope ps(g, "pr_long");
-        hipLaunchKernelGGL(k_pr_long, dim3(grid_for(g->nlong, 256, 1024)), dim3(256), 0, g->stream, g->nlong,
-                           g->long_rows, g->long_base, g->long_partial, g->deg, y, g->partial, g->partial_f, nblk,
-                           g->prs, fmt == GPR_CONTRIB_F16);
+#define PR_LONG(F16)                                                                                            \
+    hipLaunchKernelGGL(k_pr_long<F16>, dim3(grid_for(g->nlong, PR_THREADS, 1024)), dim3(PR_THREADS), 0, g->stream, \
+                       g->nlong, g->long_rows, g->long_base, g->long_partial, g->deg, y, g->partial, g->partial_f, \
+                       nblk, g->prs, fold)
+        if (fmt == GPR_CONTRIB_F16) PR_LONG(true); else PR_LONG(false);
+#undef PR_LONG
     }
-    uint32_t nparts = nblk + g->nlong;
     if (split) {
         // y (+)= the binned sums; their per-bin partials replace the pull's
         ProfScope ps(g, "pr_cold_accum");
-        GPR_TRY(cold_launch_accum(g, fmt, y, cold_from > 0 ? 1 : 0, g->partial, g->partial_f, &nparts));
-    }
-    {
+        GPR_TRY(cold_launch_accum(g, fmt, y, cold_from > 0 ? 1 : 0, g->partial, g->partial_f, damping));
+    } else if (!fold.count) {
         ProfScope ps(g, "pr_reduce");
-        hipLaunchKernelGGL(k_pr_reduce, dim3(red_grid(nparts)), dim3(RED_THREADS), 0, g->stream, g->partial, g->partial_f,
-                           (const double *)nullptr, nparts, g->dsum_slices, &g->ctr->ticket2, g->prs, 0, g->n,
-                           damping, fmt == GPR_CONTRIB_F16);
+        hipLaunchKernelGGL(k_pr_reduce, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, g->stream, g->partial, g->partial_f,
+                           nparts, g->dsum_slices, g->ticket, g->prs, 1, g->n, damping,
+                           fmt == GPR_CONTRIB_F16);
     }
     GPR_HIP(hipGetLastError());
-    GPR_HIP(hipEventRecord(g->ev1, g->stream));
     if (st) {
+        GPR_HIP(hipEventRecord(g->ev1, g->stream));
         gpr_iter_stats s = {};
         s.nactv_in = g->n;
         s.nacte_in = g->m;
@@ -510,7 +503,7 @@ extern "C" int gpr_pr_contrib(gpr_graph *g, const gpr_prop *x, gpr_prop *contrib
         hipLaunchKernelGGL(k_pr_xmax, dim3(grid), dim3(256), 0, g->stream, n, (const float *)x->d, g->partial,
                            g->partial_f);
         hipLaunchKernelGGL(k_pr_reduce, dim3(RED_BLOCKS), dim3(RED_THREADS), 0, g->stream, g->partial, g->partial_f,
-                           (const double *)nullptr, grid, g->dsum_slices, &g->ctr->ticket2, g->prs, 2, n, damping, 0);
+                           grid, g->dsum_slices, g->ticket, g->prs, 0, n, damping, 0);
         hipLaunchKernelGGL(k_pr_set_scale, dim3(1), dim3(64), 0, g->stream, g->prs, g->dsum_slices, RED_BLOCKS,
                            damping, 1);
     } else {
@@ -545,7 +538,8 @@ extern "C" int gpr_pr_finish(gpr_graph *g, gpr_prop *x, const gpr_prop *y, gpr_p
         ProfScope ps(g, "pr_update");
 #define PR_UPDATE(F)                                                                                           \
     hipLaunchKernelGGL(k_pr_update<F>, dim3(grid), dim3(256), 0, g->stream, n, (const float *)y->d, (float *)x->d, \
-                       (typename Codec<F>::store_t *)contrib->d, g->deg, damping, g->prs, pd, psum)
+                       (typename Codec<F>::store_t *)contrib->d, g->deg, damping, g->prs, pd, psum,               \
+                       g->ticket, g->hsc_dev)
         switch (fmt) {
         case GPR_CONTRIB_F32: PR_UPDATE(GPR_CONTRIB_F32); break;
         case GPR_CONTRIB_BF16: PR_UPDATE(GPR_CONTRIB_BF16); break;
@@ -555,22 +549,24 @@ extern "C" int gpr_pr_finish(gpr_graph *g, gpr_prop *x, const gpr_prop *y, gpr_p
         case GPR_CONTRIB_SCFP16: PR_UPDATE(GPR_CONTRIB_SCFP16); break;
         }
 #undef PR_UPDATE
-        hipLaunchKernelGGL(k_pr_reduce, dim3(red_grid(grid)), dim3(RED_THREADS), 0, g->stream, pd, g->partial_f, psum, grid,
-                           g->dsum_slices, &g->ctr->ticket2, g->prs, 1, n, damping, 0);
     }
     GPR_HIP(hipGetLastError());
     if (delta || sum_x) {
-        PrScalars h;
-        GPR_HIP(hipMemcpyAsync(&h, g->prs, sizeof(h), hipMemcpyDeviceToHost, g->stream));
         GPR_HIP(hipStreamSynchronize(g->stream));
-        if (delta) *delta = h.delta;
-        if (sum_x) *sum_x = h.sum_x;
+        if (delta) *delta = g->hsc->delta;
+        if (sum_x) *sum_x = g->hsc->sum_x;
     }
     return GPR_OK;
 }
 
 extern "C" int gpr_pr_scalars(gpr_graph *g, double *sum_y, double *delta, double *sum_x, float *enc_scale) {
     if (!g) return GPR_E_INVAL;
+    if (!sum_y && !enc_scale) {
+        GPR_HIP(hipStreamSynchronize(g->stream));
+        if (delta) *delta = g->hsc->delta;
+        if (sum_x) *sum_x = g->hsc->sum_x;
+        return GPR_OK;
+    }
     PrScalars h;
     GPR_HIP(hipMemcpyAsync(&h, g->prs, sizeof(h), hipMemcpyDeviceToHost, g->stream));
     GPR_HIP(hipStreamSynchronize(g->stream));

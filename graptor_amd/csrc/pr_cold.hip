@@ -61,6 +61,7 @@
 #include "internal.hpp"
 #include "device.hpp"
 #include "pr_codec.hpp"
+#include "pr_fold.hpp"
 
 #include <algorithm>
 #include <cstring>
@@ -705,8 +706,8 @@ k_cold_write(const uint32_t *__restrict__ wchunk, uint32_t nwchunks, const uint3
              const uint32_t *__restrict__ tcell, const uint16_t *__restrict__ wsrc, const uint32_t *wbase,
              const uint32_t *__restrict__ roff, uint32_t stage_max,
              const typename Codec<FMT>::store_t *__restrict__ contrib, typename Codec<FMT>::store_t *__restrict__ vals,
-             const uint32_t *__restrict__ deg, double *__restrict__ mass, const PrScalars *__restrict__ prs,
-             PrTail tail, uint32_t tile_v) {
+             const uint32_t *__restrict__ deg, double *mass, const PrScalars *prs, PrTail tail, uint32_t tile_v,
+             PrFold fold) {
     using S = typename Codec<FMT>::store_t;
     __shared__ S win[COLD_TILE_V];
     __shared__ uint32_t dls[CW_DELTA_LDS];
@@ -733,7 +734,20 @@ k_cold_write(const uint32_t *__restrict__ wchunk, uint32_t nwchunks, const uint3
     if (staged) cold_copy<FMT>(p0, p1, wsrc, wbase, (const uint32_t *)dls, o0, nc, win, vals);
     else cold_copy<FMT>(p0, p1, wsrc, wbase, roff + o0, o0, nc, win, vals);
     const double ms = block_sum(ms0, red);
-    if (threadIdx.x == 0) mass[c] = FMT == GPR_CONTRIB_F16 ? ms / (double)prs->enc_scale : ms;
+    if (threadIdx.x == 0) st_part(&mass[c], FMT == GPR_CONTRIB_F16 ? ms / (double)prs->enc_scale : ms);
+    // the last workgroup sets the fixed-point unit of the sums: 2^E with
+    // M <= 2^61 units, M the total |contribution| over the cold edges
+    __shared__ int s_last;
+    if (!last_workgroup(fold.ticket, &s_last)) return;
+    double s = 0.0;
+    for (uint32_t i = threadIdx.x; i < nwchunks; i += CW_THREADS) s += ld_part(&mass[i]);
+    const double a = block_sum(s, red);
+    if (threadIdx.x == 0) {
+        int e = 0;
+        if (a > 0.0 && a < 1e300) e = ilogb(a) + 1 - 61;
+        fold.prs->cold_exp = e;
+        fold.prs->cold_unit = ldexp(1.0, e);
+    }
 }
 
 constexpr int CA_THREADS = 1024;
@@ -783,8 +797,8 @@ __device__ __forceinline__ void block_emit(double my_sum, float my_max, double *
     if (threadIdx.x == 0) {
         float mx = fred[0];
         for (int i = 1; i < NT / 64; ++i) mx = fmaxf(mx, fred[i]);
-        part[slot] = ts;
-        part_max[slot] = mx;
+        st_part(&part[slot], ts);
+        st_part(&part_max[slot], mx);
     }
 }
 
@@ -815,10 +829,11 @@ __global__ void __launch_bounds__(CA_THREADS)
 k_cold_accum(const uint32_t *__restrict__ achunk, uint32_t n, const uint16_t *cdst, const uint32_t *bbase,
              const typename Codec<FMT>::store_t *vals, uint64_t npairs,
              const uint32_t *__restrict__ deg, float *__restrict__ y, long long *__restrict__ partials, int add,
-             double *__restrict__ part, float *__restrict__ part_max, const PrScalars *__restrict__ prs) {
+             double *part, float *part_max, const PrScalars *prs, PrFold fold) {
     using C = Codec<FMT>;
     using S = typename C::store_t;
     __shared__ unsigned long long acc[COLD_BIN];
+    __shared__ int s_last;
     __shared__ double dred[CA_THREADS / 64];
     __shared__ float fred[CA_THREADS / 64];
     const uint32_t b = achunk[4 * blockIdx.x], p0 = achunk[4 * blockIdx.x + 1], p1 = achunk[4 * blockIdx.x + 2];
@@ -946,16 +961,17 @@ k_cold_accum(const uint32_t *__restrict__ achunk, uint32_t n, const uint16_t *cd
         long long *pp = partials + (size_t)slot * COLD_BIN;
         for (uint32_t i = threadIdx.x; i < nd; i += CA_THREADS) pp[i] = (long long)acc[i];
         if (threadIdx.x == 0) {
-            part[b] = 0.0;
-            part_max[b] = 0.0f;
+            st_part(&part[b], 0.0);
+            st_part(&part_max[b], 0.0f);
         }
-        return;
+    } else {
+        double my_sum = 0.0;
+        float my_max = 0.0f;
+        for (uint32_t i = threadIdx.x; i < nd; i += CA_THREADS)
+            cold_store(y, d0 + i, (long long)acc[i], unit, add, my_sum, my_max, deg, FMT == GPR_CONTRIB_F16);
+        block_emit<CA_THREADS>(my_sum, my_max, part, part_max, b, dred, fred);
     }
-    double my_sum = 0.0;
-    float my_max = 0.0f;
-    for (uint32_t i = threadIdx.x; i < nd; i += CA_THREADS)
-        cold_store(y, d0 + i, (long long)acc[i], unit, add, my_sum, my_max, deg, FMT == GPR_CONTRIB_F16);
-    block_emit<CA_THREADS>(my_sum, my_max, part, part_max, b, dred, fred);
+    pr_fold_sum<CA_THREADS, FMT == GPR_CONTRIB_F16>(fold, part, part_max, dred, &s_last);
 }
 
 constexpr int CC_THREADS = 1024;
@@ -985,10 +1001,12 @@ k_cold_combine_groups(const uint32_t *__restrict__ groups, uint32_t n, uint32_t 
 // groups' sums (its chunks' sums when no bin has more than COLD_GROUP
 // chunks, direct) and stores y; its y sum and y/deg maximum go to slot
 // nbins + blockIdx.x.  Integer sums: exact in any grouping.
+template <bool F16>
 __global__ void __launch_bounds__(CC_THREADS)
 k_cold_combine(const uint32_t *__restrict__ multi, uint32_t nbins, uint32_t n, uint32_t per_bin, int direct,
                const long long *__restrict__ parts, const uint32_t *__restrict__ deg, float *__restrict__ y, int add,
-               double *__restrict__ part, float *__restrict__ part_max, const PrScalars *__restrict__ prs, int f16) {
+               double *part, float *part_max, const PrScalars *prs, PrFold fold) {
+    __shared__ int s_last;
     __shared__ double dred[CC_THREADS / 64];
     __shared__ float fred[CC_THREADS / 64];
     const uint32_t mb = blockIdx.x / per_bin, sub = blockIdx.x % per_bin;
@@ -1009,9 +1027,10 @@ k_cold_combine(const uint32_t *__restrict__ multi, uint32_t nbins, uint32_t n, u
             for (int j = 0; j < 8; ++j) s += t[j];
         }
         for (; c < k; ++c) s += parts[(size_t)(first + c) * COLD_BIN + i];
-        cold_store(y, d0 + i, s, prs->cold_unit, add, my_sum, my_max, deg, f16 != 0);
+        cold_store(y, d0 + i, s, prs->cold_unit, add, my_sum, my_max, deg, F16);
     }
     block_emit<CC_THREADS>(my_sum, my_max, part, part_max, nbins + blockIdx.x, dred, fred);
+    pr_fold_sum<CC_THREADS, F16>(fold, part, part_max, dred, &s_last);
 }
 
 // x' = (y + w) / s for the sources in no tile (no out-edges), whose
@@ -1044,6 +1063,7 @@ int cold_launch_write(gpr_graph *g, int fmt, const void *contrib, const float *y
     // no rank (x stays null in the kernel)
     const PrTail tail = {y, g->pr_skip_ranks ? nullptr : x, damping};
     const bool upd = x != nullptr;
+    const PrFold fold = {g->ticket, g->prs, 0, g->n, damping};
     if (upd && L->ngaps && !g->pr_skip_unlinked)
         hipLaunchKernelGGL(k_pr_update_gaps, dim3(grid_for(g->n, 256, 2048)), dim3(256), 0, g->stream, L->gaps,
                            L->ngaps, y, x, g->prs, g->symmetric ? 1 : 0);
@@ -1051,7 +1071,7 @@ int cold_launch_write(gpr_graph *g, int fmt, const void *contrib, const float *y
     hipLaunchKernelGGL((k_cold_write<F, U>), dim3(L->nwchunks), dim3(CW_THREADS), 0, g->stream, L->wchunk,      \
                        L->nwchunks, L->tile_lo, L->tcell, L->wsrc, L->wbase, L->roff, stage_max,                \
                        (const typename Codec<F>::store_t *)contrib, (typename Codec<F>::store_t *)L->vals, g->deg,  \
-                       L->mass, g->prs, tail, L->tile_v)
+                       L->mass, g->prs, tail, L->tile_v, fold)
 #define CW(F)                                                                                                   \
     if (upd) CW_(F, true); else CW_(F, false)
     switch (fmt) {
@@ -1068,12 +1088,17 @@ int cold_launch_write(gpr_graph *g, int fmt, const void *contrib, const float *y
     return GPR_OK;
 }
 
-int cold_launch_accum(gpr_graph *g, int fmt, float *y, int add, double *part, float *part_max, uint32_t *nparts) {
+int cold_launch_accum(gpr_graph *g, int fmt, float *y, int add, double *part, float *part_max, float damping) {
     ColdLayout *L = g->cold;
+    const uint32_t per_bin = combine_per_bin(g->n);
+    // the last of the kernels that write y sums the partials of all of them
+    const PrFold fold = {g->ticket, g->prs, L->nbins + L->nmulti * per_bin, g->n, damping};
+    PrFold accum_fold = fold;
+    if (L->nmulti) accum_fold.count = 0;
 #define CA(F)                                                                                                    \
     hipLaunchKernelGGL(k_cold_accum<F>, dim3(L->nachunks), dim3(CA_THREADS), 0, g->stream, L->achunk, g->n,       \
                        L->cdst, L->bbase, (const typename Codec<F>::store_t *)L->vals, L->npairs, g->deg, y,      \
-                       L->partials, add, part, part_max, g->prs)
+                       L->partials, add, part, part_max, g->prs, accum_fold)
     switch (fmt) {
     case GPR_CONTRIB_F32: CA(GPR_CONTRIB_F32); break;
     case GPR_CONTRIB_BF16: CA(GPR_CONTRIB_BF16); break;
@@ -1083,19 +1108,19 @@ int cold_launch_accum(gpr_graph *g, int fmt, float *y, int add, double *part, fl
     case GPR_CONTRIB_SCFP16: CA(GPR_CONTRIB_SCFP16); break;
     }
 #undef CA
-    const uint32_t per_bin = combine_per_bin(g->n);
     if (L->nmulti) {
         const bool direct = L->max_chunks <= COLD_GROUP;
         if (!direct)
             hipLaunchKernelGGL(k_cold_combine_groups, dim3(L->ngroups * per_bin), dim3(CC_THREADS), 0, g->stream,
                                L->groups, g->n, per_bin, (const long long *)L->partials, L->partials2);
-        hipLaunchKernelGGL(k_cold_combine, dim3(L->nmulti * per_bin), dim3(CC_THREADS), 0, g->stream, L->multi,
-                           L->nbins, g->n, per_bin, direct ? 1 : 0,
-                           (const long long *)(direct ? L->partials : L->partials2), g->deg, y, add, part, part_max,
-                           g->prs, fmt == GPR_CONTRIB_F16 ? 1 : 0);
+        const long long *parts = direct ? L->partials : L->partials2;
+#define CC(F16)                                                                                                  \
+    hipLaunchKernelGGL(k_cold_combine<F16>, dim3(L->nmulti * per_bin), dim3(CC_THREADS), 0, g->stream, L->multi,  \
+                       L->nbins, g->n, per_bin, direct ? 1 : 0, parts, g->deg, y, add, part, part_max, g->prs, fold)
+        if (fmt == GPR_CONTRIB_F16) CC(true); else CC(false);
+#undef CC
     }
     GPR_HIP(hipGetLastError());
-    *nparts = L->nbins + L->nmulti * per_bin;
     return GPR_OK;
 }
 

@@ -122,54 +122,6 @@ int ensure_partials(gpr_graph *g, size_t count) {
     return GPR_OK;
 }
 
-// Deterministic FP64 sum of `count` partials: every workgroup folds a fixed
-// slice in a fixed order, the last workgroup (by ticket) folds the slice
-// sums in index order.  The result does not depend on scheduling.
-constexpr int DSUM_THREADS = 256;
-constexpr int DSUM_BLOCKS = 64;
-__global__ void __launch_bounds__(DSUM_THREADS)
-k_deterministic_sum(const double *__restrict__ parts, uint32_t count, double *slices,
-                    unsigned int *ticket, double *dst) {
-    __shared__ double red[DSUM_THREADS];
-    __shared__ bool last;
-    uint32_t per = (count + gridDim.x - 1) / gridDim.x;
-    uint32_t lo = blockIdx.x * per, hi = min(count, lo + per);
-    double s = 0.0;
-    for (uint32_t i = lo + threadIdx.x; i < hi; i += blockDim.x) s += parts[i];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int o = blockDim.x / 2; o > 0; o >>= 1) {
-        if (threadIdx.x < (unsigned)o) red[threadIdx.x] += red[threadIdx.x + o];
-        __syncthreads();
-    }
-    // the slice as an agent-scope store, acknowledged before the ticket; the
-    // last workgroup reads the slices with agent-scope loads (no fence)
-    if (threadIdx.x == 0) {
-        __hip_atomic_store(&slices[blockIdx.x], red[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __builtin_amdgcn_s_waitcnt(WAIT_VM0);
-        unsigned t = atomicAdd(ticket, 1u);
-        last = (t == gridDim.x - 1);
-    }
-    __syncthreads();
-    if (!last) return;
-    if (threadIdx.x == 0) {
-        double tot = 0.0;
-        for (unsigned i = 0; i < gridDim.x; ++i)
-            tot += __hip_atomic_load(&slices[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        *dst = tot;
-        *ticket = 0;
-    }
-}
-
-int deterministic_sum(gpr_graph *g, const double *parts, uint32_t count, double *dst) {
-    // slices live after the partials: reserve DSUM_BLOCKS doubles at the end
-    double *slices = g->dsum_slices;
-    hipLaunchKernelGGL(k_deterministic_sum, dim3(DSUM_BLOCKS), dim3(DSUM_THREADS), 0, g->stream,
-                       parts, count, slices, &g->ctr->ticket2, dst);
-    GPR_HIP(hipGetLastError());
-    return GPR_OK;
-}
-
 Tunables &tun() {
     static Tunables t;
     return t;
