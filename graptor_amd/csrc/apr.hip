@@ -352,6 +352,7 @@ int apr_tail(gpr_graph *g, bool first, const gpr_prop *yp, float factor, float e
     out->nactv = (uint32_t)tot->nactv;
     out->nacte = tot->nacte;
     out->kind = tot->nactv ? GPR_FRONTIER_BITMAP : GPR_FRONTIER_EMPTY;
+    out->counted = true;
     return GPR_OK;
 }
 

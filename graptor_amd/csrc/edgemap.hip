@@ -822,6 +822,7 @@ int edgemap_minrelax(gpr_graph *g, const gpr_emap_desc *desc, gpr_frontier *in, 
     if (list_or_bits && g->hctr->listpos > list_limit) okind = GPR_FRONTIER_BITMAP;   // the list is incomplete
     if (out) {
         out->kind = okind;
+        out->counted = true;
         out->nactv = okind == GPR_FRONTIER_LIST ? g->hctr->listpos : g->hctr->nactv;
         out->nacte = g->hctr->nacte;
         if (out->nactv == 0) out->kind = GPR_FRONTIER_EMPTY;
@@ -953,6 +954,7 @@ extern "C" int gpr_vertex_filter(gpr_graph *g, gpr_frontier *in, gpr_prop *p, ui
         GPR_HIP(hipGetLastError());
         GPR_TRY(read_counters(g));
         out->kind = GPR_FRONTIER_BITMAP;
+        out->counted = true;
         out->nactv = g->hctr->nactv;
         out->nacte = g->hctr->nacte;
     }

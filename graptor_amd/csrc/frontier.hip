@@ -58,11 +58,15 @@ __global__ void k_list_to_bits(const uint32_t *__restrict__ list, uint32_t k, ui
 }
 
 // Bitmap -> ascending vertex list (packDense, frontier.h:923-980), in two
-// phases: phase 0 counts the set bits of each workgroup's 256 words (and
-// their out-degree sum); after an exclusive scan of those counts, phase 1
-// writes each word's vertices at its wave-scanned offset.  The list comes
-// out globally ascending and the result is deterministic.
+// phases: phase 0 counts the set bits of each workgroup's 256 words (with
+// COUNT, for a bitmap whose counts are not known, their out-degree sum too);
+// after an exclusive scan of those counts, phase 1 writes each word's
+// vertices at its wave-scanned offset.  The list comes out globally
+// ascending and the result is deterministic.  A bitmap that the engine wrote
+// has its counts, and its conversion neither gathers degrees nor reads
+// anything back (25 us of a traversal step).
 constexpr int B2L_THREADS = 256;
+template <bool COUNT>
 __global__ void __launch_bounds__(B2L_THREADS)
 k_bits_to_list(const uint64_t *__restrict__ bits, size_t words, uint32_t *list,
                const uint32_t *__restrict__ deg, unsigned long long *blk_counts, int phase,
@@ -74,19 +78,21 @@ k_bits_to_list(const uint64_t *__restrict__ bits, size_t words, uint32_t *list,
     uint32_t c = __popcll(w);
     if (phase == 0) {
         // count per workgroup, and edge sum
-        uint64_t es = 0;
-        uint64_t t = w;
-        while (t) {
-            int b = __ffsll((long long)t) - 1;
-            t &= t - 1;
-            es += deg[i * 64 + b];
-        }
         uint32_t tot = block_sum(c, red);
-        uint64_t etot = block_sum(es, redl);
-        if (threadIdx.x == 0) {
-            blk_counts[blockIdx.x] = tot;
-            atomicAdd(&ctr_stripe(ctr)->nactv, tot);
-            atomicAdd(&ctr_stripe(ctr)->nacte, (unsigned long long)etot);
+        if (threadIdx.x == 0) blk_counts[blockIdx.x] = tot;
+        if constexpr (COUNT) {
+            uint64_t es = 0;
+            uint64_t t = w;
+            while (t) {
+                int b = __ffsll((long long)t) - 1;
+                t &= t - 1;
+                es += deg[i * 64 + b];
+            }
+            uint64_t etot = block_sum(es, redl);
+            if (threadIdx.x == 0) {
+                atomicAdd(&ctr_stripe(ctr)->nactv, tot);
+                atomicAdd(&ctr_stripe(ctr)->nacte, (unsigned long long)etot);
+            }
         }
         return;
     }
@@ -207,6 +213,7 @@ int frontier_to_bits(gpr_frontier *f) {
     GPR_TRY(frontier_ensure_bits(f));
     size_t words = nwords(g->n);
     ProfScope ps(g, "frontier_convert");
+    f->counted = f->kind == GPR_FRONTIER_ALL;
     if (f->kind == GPR_FRONTIER_ALL) {
         hipLaunchKernelGGL(k_fill_all_bits, dim3(grid_for(words, 256, 4096)), dim3(256), 0, g->stream, f->bits, g->n);
     } else {
@@ -224,7 +231,8 @@ void excl_scan_counts(gpr_graph *g, unsigned long long *counts, uint32_t count) 
     hipLaunchKernelGGL(k_excl_scan_u64, dim3(1), dim3(1024), 0, g->stream, counts, count);
 }
 
-// Bitmap/all -> ascending list.  Recomputes nactv and nacte.
+// Bitmap/all -> ascending list.  Computes nactv and nacte where they may
+// not be those of the bits.
 int frontier_to_list(gpr_frontier *f) {
     gpr_graph *g = f->g;
     if (f->kind == GPR_FRONTIER_LIST) return GPR_OK;
@@ -235,20 +243,25 @@ int frontier_to_list(gpr_frontier *f) {
     unsigned blocks = grid_for(words, B2L_THREADS);
     GPR_TRY(ensure_partials(g, blocks));
     unsigned long long *cnt = (unsigned long long *)g->partial;
-    GPR_TRY(reset_counters(g));
+    if (!f->counted) GPR_TRY(reset_counters(g));
     {
         ProfScope ps(g, "frontier_convert");
-        hipLaunchKernelGGL(k_bits_to_list, dim3(blocks), dim3(B2L_THREADS), 0, g->stream, f->bits, words, f->list,
-                           g->deg, cnt, 0, g->ctr);
-        hipLaunchKernelGGL(k_excl_scan_u64, dim3(1), dim3(1024), 0, g->stream, cnt, blocks);
-        hipLaunchKernelGGL(k_bits_to_list, dim3(blocks), dim3(B2L_THREADS), 0, g->stream, f->bits, words, f->list,
-                           g->deg, cnt, 1, g->ctr);
+        if (f->counted)
+            hipLaunchKernelGGL(k_bits_to_list<false>, dim3(blocks), dim3(B2L_THREADS), 0, g->stream, f->bits, words,
+                               f->list, g->deg, cnt, 0, g->ctr);
+        else
+            hipLaunchKernelGGL(k_bits_to_list<true>, dim3(blocks), dim3(B2L_THREADS), 0, g->stream, f->bits, words,
+                               f->list, g->deg, cnt, 0, g->ctr);
+        excl_scan_counts(g, cnt, blocks);
+        hipLaunchKernelGGL(k_bits_to_list<false>, dim3(blocks), dim3(B2L_THREADS), 0, g->stream, f->bits, words,
+                           f->list, g->deg, cnt, 1, g->ctr);
     }
     GPR_HIP(hipGetLastError());
+    f->kind = GPR_FRONTIER_LIST;
+    if (f->counted) return GPR_OK;
     GPR_TRY(read_counters(g));
     f->nactv = g->hctr->nactv;
     f->nacte = g->hctr->nacte;
-    f->kind = GPR_FRONTIER_LIST;
     return GPR_OK;
 }
 
