@@ -145,6 +145,7 @@ static void graph_free(gpr_graph *g) {
     dev_free(g->partial_f);
     dev_free(g->dsum_slices);
     dev_free(g->prs);
+    dev_free(g->pr_contrib);
     dev_free(g->pol_params);
     cold_free(g);
     dev_free(g->fbuf);

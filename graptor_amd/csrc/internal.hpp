@@ -65,6 +65,7 @@ struct Tunables {
     double pull_blocks_per_cu = 8;            // pull grid = CUs * this
     double push_blocks_per_cu = 32;           // push grid cap = CUs * this
     double pr_split_bytes = 0;                // FP32 bytes of pulled sources (0: all binned; >= 4n: no split)
+    double pr_pull_edges = 1 << 23;           // graphs up to this many edges are pulled when pr_split_bytes is 0
     double fusion_spin_limit = 1 << 22;       // fused push: polls without progress before it gives up
     double fusion_blocks = 0;                 // fused push: cooperative grid size (0: one per CU)
     double pr_write_stage_cells = 4096;       // PR write: a tile's run offsets go to LDS up to this many cells
@@ -230,6 +231,7 @@ struct gpr_graph {
     double *long_partial = nullptr;      // per long chunk
     double *dsum_slices = nullptr;       // slice sums and maxima of k_pr_reduce
     gpr::PrScalars *prs = nullptr;       // device
+    void *pr_contrib = nullptr;          // contributions of a pulled fused iteration (built on first use)
     // trace of the last run
     std::vector<gpr_iter_stats> trace;
     gpr::Profile prof;

@@ -92,7 +92,7 @@ k_pr_pull(uint32_t nbuckets, const uint32_t *__restrict__ bucket, const uint64_t
 #pragma unroll
             for (int u = 0; u < PR_UNROLL; ++u) {
                 const uint64_t e = base + (uint64_t)u * PR_THREADS + threadIdx.x;
-                s[u] = e < ce ? __builtin_nontemporal_load(&cnbrs[e]) : 0xffffffffu;
+                s[u] = e < ce ? cnbrs[e] : 0xffffffffu;
             }
             float v[PR_UNROLL];
             gather_all<FMT>(contrib, s, cold_from, v);
@@ -123,7 +123,7 @@ k_pr_pull(uint32_t nbuckets, const uint32_t *__restrict__ bucket, const uint64_t
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
                 const uint32_t i = base + u * PR_THREADS + threadIdx.x;
-                ix[u] = i <= nrows ? __builtin_nontemporal_load(&cindex[r0 + i]) : 0;
+                ix[u] = i <= nrows ? cindex[r0 + i] : 0;
             }
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
@@ -131,6 +131,9 @@ k_pr_pull(uint32_t nbuckets, const uint32_t *__restrict__ bucket, const uint64_t
                 if (i <= nrows) rs[i] = (uint32_t)(ix[u] - e0);
             }
         }
+        // (plain loads: a small graph's neighbours stay in the L2s from one
+        // iteration to the next; non-temporal ones took 46 us instead of 39
+        // an iteration on 7.6M edges)
         // a bucket holds < PR_LDS_EDGES edges: one round of PR_UNROLL
         // independent neighbour loads and gathers per lane covers it
         for (uint32_t base = 0; base < ne; base += PR_THREADS * PR_UNROLL) {
@@ -138,7 +141,7 @@ k_pr_pull(uint32_t nbuckets, const uint32_t *__restrict__ bucket, const uint64_t
 #pragma unroll
             for (int u = 0; u < PR_UNROLL; ++u) {
                 const uint32_t i = base + u * PR_THREADS + threadIdx.x;
-                s[u] = i < ne ? __builtin_nontemporal_load(&cnbrs[e0 + i]) : 0xffffffffu;
+                s[u] = i < ne ? cnbrs[e0 + i] : 0xffffffffu;
             }
             float v[PR_UNROLL];
             gather_all<FMT>(contrib, s, cold_from, v);
@@ -274,7 +277,10 @@ k_pr_reduce(const double *__restrict__ part, const float *__restrict__ part_max,
 // Bound by its streams (20 B a vertex in FP32).  The last workgroup also
 // sums the residual and the ranks, into the device's scalars and the host's
 // line.
-template <int FMT>
+//
+// FUSED (gpr_pr_iterate_fused where the edgemap pulls): no residual, and x
+// unwritten when null.
+template <int FMT, bool FUSED>
 __global__ void __launch_bounds__(256)
 k_pr_update(uint32_t n, const float *__restrict__ y, float *__restrict__ x, typename Codec<FMT>::store_t *contrib,
             const uint32_t *__restrict__ deg, float damping, PrScalars *prs, double *part_delta, double *part_sum,
@@ -286,13 +292,16 @@ k_pr_update(uint32_t n, const float *__restrict__ y, float *__restrict__ x, type
     double dl = 0.0, sx = 0.0;
     for (uint32_t v = blockIdx.x * 256 + threadIdx.x; v < n; v += gridDim.x * 256) {
         const float xn = (float)(((double)y[v] + w) * inv_s);
-        dl += (double)fabsf(x[v] - xn);
-        sx += (double)xn;
-        x[v] = xn;
+        if constexpr (!FUSED) {
+            dl += (double)fabsf(x[v] - xn);
+            sx += (double)xn;
+        }
+        if (!FUSED || x) x[v] = xn;
         const uint32_t dg = deg[v];
         const float cv = dg ? damping * xn / (float)dg : 0.0f;
         contrib[v] = Codec<FMT>::enc(cv * sc);
     }
+    if constexpr (FUSED) return;
     dl = block_sum(dl, r1);
     sx = block_sum(sx, r2);
     if (threadIdx.x == 0) {
@@ -370,6 +379,19 @@ static uint32_t split_point(gpr_graph *g) {
     return h >= (double)g->n ? g->n : (uint32_t)h;
 }
 
+// Whether the automatic split (pr_split_bytes 0) pulls every edge instead of
+// binning it.  Binned sums take up to four launches an iteration,
+// with every bin cleared and written out, and pay it back by streaming; a pull is two launches, and its
+// gathers run at 200 G/s and more while the contributions stay in an XCD's
+// 4 MB L2.  PRv per iteration, pull against bins (FP32): RMAT with 0.1M
+// edges 12 / 25 us, 1.8M 19 / 35, 7.6M 39 / 53, 15M 73 / 71, 31M 129 / 91;
+// uniform random with 8M edges on 1M vertices 64 / 70.  So up to
+// pr_pull_edges (2^23) edges, on at most 2^20 vertices.  A new graph is
+// spared the layout's construction as well.
+static bool pulls_all(const gpr_graph *g) {
+    return tun().pr_split_bytes < 4.0 && (double)g->m <= tun().pr_pull_edges && g->n <= (1u << 20);
+}
+
 // x_tail != nullptr: the previous iteration's tail is fused into the write
 // stage (the caller has checked cold_tail_fusable after cold_prepare)
 static int pr_edgemap_impl(gpr_graph *g, const gpr_emap_desc *desc, gpr_frontier *in, gpr_iter_stats *st,
@@ -380,7 +402,7 @@ static int pr_edgemap_impl(gpr_graph *g, const gpr_emap_desc *desc, gpr_frontier
     GPR_REQUIRE(fmt >= GPR_CONTRIB_F32 && fmt <= GPR_CONTRIB_SCFP16, "PR edgemap: unknown contribution format %d", fmt);
     GPR_REQUIRE(desc->contrib && desc->contrib->elem == fmt_bytes(fmt),
                 "PR edgemap: contribution property has the wrong element size for format %d", fmt);
-    uint32_t cold_from = split_point(g);
+    uint32_t cold_from = pulls_all(g) ? g->n : split_point(g);
     if (cold_from < g->n) {
         GPR_TRY(cold_prepare(g, cold_from));
         if (g->cold->ntiles == 0) cold_from = g->n;   // no cold edges
@@ -458,6 +480,32 @@ static int pr_edgemap_impl(gpr_graph *g, const gpr_emap_desc *desc, gpr_frontier
     return GPR_OK;
 }
 
+// x' and its contributions from y; the residual too unless fused.
+static int launch_update(gpr_graph *g, int fmt, bool fused, const float *y, float *x, void *contrib, float damping) {
+    const uint32_t n = g->n;
+    const unsigned grid = update_grid(n);
+    GPR_TRY(ensure_partials(g, 2 * (size_t)grid + 64));
+    ProfScope ps(g, "pr_update");
+#define PR_UPDATE_(F, U)                                                                                       \
+    hipLaunchKernelGGL((k_pr_update<F, U>), dim3(grid), dim3(256), 0, g->stream, n, y, x,                       \
+                       (typename Codec<F>::store_t *)contrib, g->deg, damping, g->prs, g->partial,             \
+                       g->partial + grid, g->ticket, g->hsc_dev)
+#define PR_UPDATE(F)                                                                                           \
+    if (fused) PR_UPDATE_(F, true); else PR_UPDATE_(F, false)
+    switch (fmt) {
+    case GPR_CONTRIB_F32: PR_UPDATE(GPR_CONTRIB_F32); break;
+    case GPR_CONTRIB_BF16: PR_UPDATE(GPR_CONTRIB_BF16); break;
+    case GPR_CONTRIB_F16: PR_UPDATE(GPR_CONTRIB_F16); break;
+    case GPR_CONTRIB_CFP16: PR_UPDATE(GPR_CONTRIB_CFP16); break;
+    case GPR_CONTRIB_BF16T: PR_UPDATE(GPR_CONTRIB_BF16T); break;
+    case GPR_CONTRIB_SCFP16: PR_UPDATE(GPR_CONTRIB_SCFP16); break;
+    }
+#undef PR_UPDATE
+#undef PR_UPDATE_
+    GPR_HIP(hipGetLastError());
+    return GPR_OK;
+}
+
 int pr_edgemap(gpr_graph *g, const gpr_emap_desc *desc, gpr_frontier *in, gpr_iter_stats *st) {
     return pr_edgemap_impl(g, desc, in, st, nullptr);
 }
@@ -471,19 +519,28 @@ extern "C" int gpr_pr_iterate_fused(gpr_graph *g, gpr_prop *x, gpr_prop *y, int 
     if (!g || !x || !y || x->dtype != GPR_F32 || y->dtype != GPR_F32 || x->g != g || y->g != g) return GPR_E_INVAL;
     GPR_REQUIRE(fmt >= GPR_CONTRIB_F32 && fmt <= GPR_CONTRIB_SCFP16, "pr_iterate_fused: unknown format %d", fmt);
     GPR_REQUIRE(split_point(g) == 0, "pr_iterate_fused: needs every edge binned (pr_split_bytes 0)");
-    GPR_TRY(cold_prepare(g, 0));
-    GPR_REQUIRE(cold_tail_fusable(g), "pr_iterate_fused: the graph has no binned edges");
+    const bool pull = pulls_all(g);
+    if (!pull) GPR_TRY(cold_prepare(g, 0));
+    GPR_REQUIRE(pull ? g->m > 0 : cold_tail_fusable(g), "pr_iterate_fused: the graph has no binned edges");
     gpr_emap_desc d = {};
     d.relax = GPR_RELAX_PR_SUM;
     d.prop = y;
     d.contrib_fmt = fmt;
     d.damping = damping;
-    // the contribution property is never read: the write stage computes
-    // the contributions; a stand-in of the right element size passes the
-    // checks
+    // the contribution property is never read by the write stage, which
+    // computes the contributions: a stand-in of the right element size
+    // passes the checks.  A pull reads them from the handle's scratch.
     gpr_prop stand_in = *y;
     stand_in.elem = (uint32_t)fmt_bytes(fmt);
     d.contrib = &stand_in;
+    if (pull) {
+        if (!g->pr_contrib)
+            GPR_TRY(dev_alloc((void **)&g->pr_contrib, sizeof(float) * (size_t)g->n, "pagerank contributions"));
+        stand_in.d = g->pr_contrib;
+        GPR_TRY(launch_update(g, fmt, true, (const float *)y->d, flags & GPR_PR_SKIP_RANKS ? nullptr : (float *)x->d,
+                              g->pr_contrib, damping > 0.f ? damping : 0.85f));
+        return pr_edgemap_impl(g, &d, nullptr, st, nullptr);
+    }
     g->pr_skip_unlinked = (flags & (GPR_PR_SKIP_UNLINKED | GPR_PR_SKIP_RANKS)) != 0;
     g->pr_skip_ranks = (flags & GPR_PR_SKIP_RANKS) != 0;
     const int r = pr_edgemap_impl(g, &d, nullptr, st, (float *)x->d);
@@ -530,27 +587,7 @@ extern "C" int gpr_pr_finish(gpr_graph *g, gpr_prop *x, const gpr_prop *y, gpr_p
     if (!g || !x || !y || !contrib || x->dtype != GPR_F32 || y->dtype != GPR_F32) return GPR_E_INVAL;
     GPR_REQUIRE(fmt >= GPR_CONTRIB_F32 && fmt <= GPR_CONTRIB_SCFP16 && contrib->elem == fmt_bytes(fmt),
                 "pr_finish: bad contribution format %d / property", fmt);
-    const uint32_t n = g->n;
-    const unsigned grid = update_grid(n);
-    GPR_TRY(ensure_partials(g, 2 * (size_t)grid + 64));
-    double *pd = g->partial, *psum = g->partial + grid;
-    {
-        ProfScope ps(g, "pr_update");
-#define PR_UPDATE(F)                                                                                           \
-    hipLaunchKernelGGL(k_pr_update<F>, dim3(grid), dim3(256), 0, g->stream, n, (const float *)y->d, (float *)x->d, \
-                       (typename Codec<F>::store_t *)contrib->d, g->deg, damping, g->prs, pd, psum,               \
-                       g->ticket, g->hsc_dev)
-        switch (fmt) {
-        case GPR_CONTRIB_F32: PR_UPDATE(GPR_CONTRIB_F32); break;
-        case GPR_CONTRIB_BF16: PR_UPDATE(GPR_CONTRIB_BF16); break;
-        case GPR_CONTRIB_F16: PR_UPDATE(GPR_CONTRIB_F16); break;
-        case GPR_CONTRIB_CFP16: PR_UPDATE(GPR_CONTRIB_CFP16); break;
-        case GPR_CONTRIB_BF16T: PR_UPDATE(GPR_CONTRIB_BF16T); break;
-        case GPR_CONTRIB_SCFP16: PR_UPDATE(GPR_CONTRIB_SCFP16); break;
-        }
-#undef PR_UPDATE
-    }
-    GPR_HIP(hipGetLastError());
+    GPR_TRY(launch_update(g, fmt, false, (const float *)y->d, (float *)x->d, contrib->d, damping));
     if (delta || sum_x) {
         GPR_HIP(hipStreamSynchronize(g->stream));
         if (delta) *delta = g->hsc->delta;

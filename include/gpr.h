@@ -276,12 +276,12 @@ int gpr_pr_scalars(gpr_graph *g, double *sum_y, double *delta, double *sum_x,
  * runs the maps of :214-269 after the edgemap of :202-212).  Equal to
  * gpr_pr_finish(g, x, y, contrib, fmt, damping, NULL, NULL) followed by
  * the GPR_RELAX_PR_SUM edgemap into y, except that the contributions are
- * computed in the edgemap's write stage and never stored (a contribution
+ * computed on the way and never stored for the caller (a contribution
  * property is left as it was) and no residual is computed (the device's
  * delta and sum_x keep their values); x and y come out bit-identical to
  * that sequence's.  For fixed iteration counts (no convergence test
- * between iterations).  Needs every edge in the binned layout (tunable
- * pr_split_bytes 0) and a graph with edges: GPR_E_INVAL otherwise.  st
+ * between iterations).  Needs tunable pr_split_bytes 0 (every edge binned,
+ * or a small graph pulled) and a graph with edges: GPR_E_INVAL otherwise.  st
  * (optional) receives the step's stats.  flags GPR_PR_SKIP_UNLINKED: the
  * ranks of sources without out-edges are not written (their contributions
  * are 0 and no edge reads them): x is then complete only after a later
@@ -485,8 +485,12 @@ int gpr_trace_get(const gpr_graph *g, gpr_iter_stats *out, int cap, int *k);
  *   pr_split_bytes      PageRank: FP32 bytes of source contributions the
  *                       pull gathers (the sources [0, bytes/4)); edges from
  *                       the other sources are summed by streaming through a
- *                       binned layout.  0 bins every edge; >= 4n pulls every
+ *                       binned layout.  0 bins every edge (a small graph,
+ *                       pr_pull_edges, is pulled instead); >= 4n pulls every
  *                       edge.  Default 0
+ *   pr_pull_edges       PageRank with pr_split_bytes 0: graphs of at most
+ *                       this many edges and 2^20 vertices are pulled
+ *                       (default 2^23; 0: never)
  *   pull_serial_max     pull rows up to this in-degree run lane-serially
  *   pull_blocks_per_cu  pull grid size per compute unit
  *   push_blocks_per_cu  push grid cap per compute unit

@@ -1,6 +1,7 @@
 """PageRank's binned edgemap where its tiles and chunks change with the graph:
 sizes around one bin (16384), one tile (1024), bins in one chunk, in up to a
-group of 16 and in several groups, directed and relabelled graphs.
+group of 16 and in several groups, directed and relabelled graphs; and where
+the rule for small graphs (pr_pull_edges) pulls instead.
 
 Bars as in test_gpu_pr_split: relative L1 against FP64 of 1e-6 for FP32 (each
 rank is rounded to 24 bits a few times an iteration, and errors contract by
@@ -19,7 +20,9 @@ G = pytest.importorskip("graptor_amd")
 @pytest.fixture(scope="module", autouse=True)
 def device():
     G.lib()
+    old = G.tune_get("pr_pull_edges")
     yield
+    G.tune_set("pr_pull_edges", old)
 
 
 def rel_l1(a, b):
@@ -39,7 +42,9 @@ SIZES = [(1023, 4000), (1025, 60000), (16383, 40000), (16385, 300000), (40001, 1
 
 @pytest.mark.parametrize("n,m", SIZES)
 @pytest.mark.parametrize("directed", [False, True])
-def test_ranks_across_layout_sizes(n, m, directed):
+@pytest.mark.parametrize("pull", [0, 1 << 23])
+def test_ranks_across_layout_sizes(n, m, directed, pull):
+    G.tune_set("pr_pull_edges", pull)   # 0: every edge binned
     src, dst = skewed(n, m, n)
     index, nbrs = O.build_csr(n, src, dst, symmetrize=not directed)
     if directed:
@@ -55,3 +60,18 @@ def test_ranks_across_layout_sizes(n, m, directed):
             assert rel_l1(x, x64) <= bar, (fmt, rel_l1(x, x64))
             x2, _ = g.pr_vary([(fmt, 0.0)], max_iter=12)
             assert np.array_equal(x, x2), fmt
+
+
+@pytest.mark.parametrize("fmt", ["fp32", "bf16", "fp16", "cfp16", "scfp16"])
+@pytest.mark.parametrize("pull", [0, 1 << 23])
+def test_fused_iterations_equal_unfused(fmt, pull):
+    """A fixed iteration count (tails fused into the next iteration) and a
+    convergence test that never stops the run give the same ranks."""
+    G.tune_set("pr_pull_edges", pull)
+    n = 30011
+    src, dst = skewed(n, 400000, 3)
+    index, nbrs = O.build_csr(n, src, dst)
+    with G.Graph.from_csr(index, nbrs).reorder() as g:
+        xf, _ = g.pr_vary([(fmt, 0.0)], max_iter=9)
+        xu, _ = g.pr_vary([(fmt, 1e-300)], max_iter=9)
+    assert np.array_equal(xf.view(np.uint32), xu.view(np.uint32))
