@@ -22,6 +22,7 @@
 #include "../../include/gpr/api.hpp"
 #include "apr.hpp"
 #include "kcore.hpp"
+#include "whole.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -605,8 +606,13 @@ extern "C" int gpr_bfslvl(gpr_graph *g, uint32_t start, const gpr_run_opts *opts
     gpr_graph_info(g, &n, nullptr, nullptr);
     if (start >= n) return guarded([&] { check(GPR_E_INVAL, "bfslvl: start vertex out of range"); });
     return guarded([&] {
-        BFSLVLv app(g, o);
         gpr_run_info local = {};
+        if (whole_run(g, o, false)) {
+            check(whole_bfs(g, start, o.threshold_pct, levels, &local), "bfslvl");
+            if (info) *info = local;
+            return;
+        }
+        BFSLVLv app(g, o);
         if (o.trace) trace_clear(g);
         stream_time_ms(g, true);
         app.run(start, &local);
@@ -639,8 +645,13 @@ extern "C" int gpr_ccv(gpr_graph *g, const gpr_run_opts *opts, uint32_t *labels,
     if (!g) return GPR_E_INVAL;
     gpr_run_opts o = defaults(opts);
     return guarded([&] {
-        CCv app(g, o);
         gpr_run_info local = {};
+        if (whole_run(g, o, true)) {
+            check(whole_cc(g, labels, &local), "ccv");
+            if (info) *info = local;
+            return;
+        }
+        CCv app(g, o);
         if (o.trace) trace_clear(g);
         stream_time_ms(g, true);
         app.run(&local);

@@ -7,6 +7,7 @@
 #include "internal.hpp"
 #include "device.hpp"
 #include "grid_sync.hpp"
+#include "label_fold.hpp"
 
 #include <stdio.h>
 #include <string.h>
@@ -152,6 +153,10 @@ static void graph_free(gpr_graph *g) {
     dev_free(g->fctl);
     dev_free(g->kbuf);
     dev_free(g->kctl);
+    dev_free(g->wbuf);
+    dev_free(g->wctl);
+    if (g->wstage) hipHostFree(g->wstage);
+    if (g->whost) hipHostFree(g->whost);
     if (g->ev0) hipEventDestroy(g->ev0);
     if (g->ev1) hipEventDestroy(g->ev1);
     if (g->rev0) hipEventDestroy(g->rev0);
@@ -294,81 +299,28 @@ static int permute_positions(gpr_graph *g, const void *src, void *dst, size_t el
     return GPR_OK;
 }
 
-// Per component, the smallest original ID of its vertices, at the
-// component's root (the vertex that carries its own ID as its label;
-// minorig starts at ~0).  Bound by the two streams it reads, 8 B a vertex.
-// A giant component sends most vertices to one address: a read before each
-// atomic does not help, because every wave in flight reads ~0 before the
-// first atomic lands, and those atomics then queue on the address (6.1 ms
-// at 33.6M vertices, RMAT; 0.26 ms at 50021).  So a thread keeps one label
-// and its minimum in registers over RM_ITEMS vertices a step, the smaller
-// label of two it meets (a label is the smallest internal ID of its
-// component, so a giant's is small); the other goes to memory at once.
-// A wave then folds the lanes that hold its smallest label, a workgroup the
-// waves that hold its smallest, and one atomic a workgroup is left for a
-// giant: 0.11 ms and 5 us on the same graphs.  A root's own ID needs no
-// fold (one vertex a component).
-constexpr int RM_THREADS = 256, RM_ITEMS = 8;
-__device__ __forceinline__ void recode_lower(uint32_t *minorig, uint32_t l, uint32_t o) {
-    if (o < __hip_atomic_load(&minorig[l], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(&minorig[l], o);
-}
-__global__ void __launch_bounds__(RM_THREADS)
+// Per component, the smallest original ID, at the component's root (minorig
+// starts at ~0; label_fold.hpp).  Bound by the two streams it reads, 8 B a
+// vertex.
+__global__ void __launch_bounds__(LF_THREADS)
 k_recode_min(const uint32_t *__restrict__ label, const uint32_t *__restrict__ order, uint32_t n, uint32_t *minorig) {
-    __shared__ uint32_t s_l[RM_THREADS / 64], s_o[RM_THREADS / 64];
-    uint32_t kl = 0xffffffffu, ko = 0xffffffffu;   // the label kept, and its minimum
-    const uint64_t step = (uint64_t)gridDim.x * RM_THREADS * RM_ITEMS;
-    for (uint64_t base = (uint64_t)blockIdx.x * RM_THREADS * RM_ITEMS; base < n; base += step) {
-        uint32_t l[RM_ITEMS], o[RM_ITEMS];
+    LabelFold f;
+    const uint64_t step = (uint64_t)gridDim.x * LF_THREADS * LF_ITEMS;
+    for (uint64_t base = (uint64_t)blockIdx.x * LF_THREADS * LF_ITEMS; base < n; base += step) {
+        uint32_t l[LF_ITEMS], o[LF_ITEMS];
 #pragma unroll
-        for (int u = 0; u < RM_ITEMS; ++u) {
-            const uint64_t i = base + u * RM_THREADS + threadIdx.x;
+        for (int u = 0; u < LF_ITEMS; ++u) {
+            const uint64_t i = base + u * LF_THREADS + threadIdx.x;
             l[u] = i < n ? label[i] : 0xffffffffu;
             o[u] = i < n ? (order ? order[i] : (uint32_t)i) : 0xffffffffu;
         }
 #pragma unroll
-        for (int u = 0; u < RM_ITEMS; ++u) {
-            const uint64_t i = base + u * RM_THREADS + threadIdx.x;
-            if (i >= n) continue;
-            if (l[u] == i) {
-                recode_lower(minorig, l[u], o[u]);
-            } else if (l[u] == kl) {
-                ko = o[u] < ko ? o[u] : ko;
-            } else if (l[u] < kl) {
-                if (kl != 0xffffffffu) recode_lower(minorig, kl, ko);
-                kl = l[u];
-                ko = o[u];
-            } else {
-                recode_lower(minorig, l[u], o[u]);
-            }
+        for (int u = 0; u < LF_ITEMS; ++u) {
+            const uint64_t i = base + u * LF_THREADS + threadIdx.x;
+            if (i < n) f.add(minorig, i, l[u], o[u]);
         }
     }
-    const uint32_t wl = wave_min(kl);
-    const uint32_t wo = wave_min(kl == wl ? ko : 0xffffffffu);
-    if (kl != wl && kl != 0xffffffffu) recode_lower(minorig, kl, ko);
-    const unsigned w = threadIdx.x / 64;
-    if (lane() == 0) {
-        s_l[w] = wl;
-        s_o[w] = wo;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t bl = s_l[0], bo = s_o[0];
-        for (unsigned j = 1; j < RM_THREADS / 64; ++j) {
-            const uint32_t jl = s_l[j], jo = s_o[j];
-            if (jl == bl) {
-                bo = jo < bo ? jo : bo;
-            } else {
-                const bool lower = jl < bl;
-                const uint32_t fl = lower ? bl : jl, fo = lower ? bo : jo;
-                if (fl != 0xffffffffu) recode_lower(minorig, fl, fo);
-                if (lower) {
-                    bl = jl;
-                    bo = jo;
-                }
-            }
-        }
-        if (bl != 0xffffffffu) recode_lower(minorig, bl, bo);
-    }
+    f.finish(minorig);
 }
 __global__ void k_recode_out(const uint32_t *__restrict__ label, const uint32_t *__restrict__ order, uint32_t n,
                              const uint32_t *__restrict__ minorig, uint32_t *out) {
@@ -609,7 +561,7 @@ extern "C" int gpr_cc_recode(const gpr_prop *p, uint32_t *labels) {
     uint32_t *out = minorig + n;
     const unsigned grid = grid_for(n, 256, 8192);
     hipLaunchKernelGGL(k_fill_u32, dim3(grid), dim3(256), 0, g->stream, minorig, n, 0xffffffffu);
-    hipLaunchKernelGGL(k_recode_min, dim3(grid_for(n, RM_THREADS * RM_ITEMS, 1024)), dim3(RM_THREADS), 0, g->stream,
+    hipLaunchKernelGGL(k_recode_min, dim3(grid_for(n, LF_THREADS * LF_ITEMS, 1024)), dim3(LF_THREADS), 0, g->stream,
                        (const uint32_t *)p->d, g->order, n, minorig);
     hipLaunchKernelGGL(k_recode_out, dim3(grid), dim3(256), 0, g->stream, (const uint32_t *)p->d, g->order, n, minorig, out);
     GPR_HIP(hipGetLastError());

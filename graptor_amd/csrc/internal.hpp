@@ -66,6 +66,7 @@ struct Tunables {
     double push_blocks_per_cu = 32;           // push grid cap = CUs * this
     double pr_split_bytes = 0;                // FP32 bytes of pulled sources (0: all binned; >= 4n: no split)
     double pr_pull_edges = 1 << 23;           // graphs up to this many edges are pulled when pr_split_bytes is 0
+    double whole_edges = 1 << 24;             // default BFS and CC of graphs up to this many edges run whole on the device
     double fusion_spin_limit = 1 << 22;       // fused push: polls without progress before it gives up
     double fusion_blocks = 0;                 // fused push: cooperative grid size (0: one per CU)
     double pr_write_stage_cells = 4096;       // PR write: a tile's run offsets go to LDS up to this many cells
@@ -269,6 +270,12 @@ struct gpr_graph {
     void *kbuf = nullptr;              // k-core peeling: candidate and frontier lists (built on first use)
     size_t kbuf_bytes = 0;
     void *kctl = nullptr;              // k-core peeling: control block
+    void *wbuf = nullptr;              // whole runs (whole.hip): values, lists, results (built on first use)
+    void *wctl = nullptr;              // whole runs: control block
+    uint32_t *wstage = nullptr;        // whole runs: pinned results of small graphs, and the device's address
+    uint32_t *wstage_dev = nullptr;
+    void *whost = nullptr;             // whole runs: pinned progress line, and the device's address
+    void *whost_dev = nullptr;
 };
 
 struct gpr_prop {

@@ -143,6 +143,14 @@ void trace_clear(gpr_graph *g) { g->trace.clear(); }
 
 // Device time of an application run: events on the handle's stream at the
 // start and end of run() (the reference times run() only, driver.C:245-255).
+// stream_time_mark: the end alone, for a caller that queues more behind it;
+// stream_time_read_ms: the time, once the stream has passed the mark.
+void stream_time_mark(gpr_graph *g) { hipEventRecord(g->rev1, g->stream); }
+double stream_time_read_ms(gpr_graph *g) {
+    float ms = 0.f;
+    hipEventElapsedTime(&ms, g->rev0, g->rev1);
+    return ms;
+}
 double stream_time_ms(gpr_graph *g, bool start) {
     if (!g->rev0) {
         hipEventCreate(&g->rev0);
@@ -152,11 +160,9 @@ double stream_time_ms(gpr_graph *g, bool start) {
         hipEventRecord(g->rev0, g->stream);
         return 0.0;
     }
-    hipEventRecord(g->rev1, g->stream);
+    stream_time_mark(g);
     hipEventSynchronize(g->rev1);
-    float ms = 0.f;
-    hipEventElapsedTime(&ms, g->rev0, g->rev1);
-    return ms;
+    return stream_time_read_ms(g);
 }
 
 void prof_flush(gpr_graph *g) {
@@ -210,6 +216,7 @@ static double *tunable(const char *name) {
     if (!strcmp(name, "push_blocks_per_cu")) return &t.push_blocks_per_cu;
     if (!strcmp(name, "pr_split_bytes")) return &t.pr_split_bytes;
     if (!strcmp(name, "pr_pull_edges")) return &t.pr_pull_edges;
+    if (!strcmp(name, "whole_edges")) return &t.whole_edges;
     if (!strcmp(name, "fusion_spin_limit")) return &t.fusion_spin_limit;
     if (!strcmp(name, "fusion_blocks")) return &t.fusion_blocks;
     if (!strcmp(name, "pr_write_stage_cells")) return &t.pr_write_stage_cells;

@@ -1,0 +1,610 @@
+// whole.hip -- BFSLVLv and CCv of small graphs as whole runs on the device.
+//
+// A host-driven step costs 25-45 us (its launches, the counts read back),
+// whatever the frontier: on a graph of a few million edges that is nearly all
+// of a run.  Here the host launches a run and waits once.
+//
+// BFS (k_wb_level): a launch a level, every level a push, queued ahead of the
+// device without waiting for counts: a level reads the list lengths that the
+// one before left, block 0 tells the host through pinned memory how far
+// it is and when the frontier was empty, and the host keeps WB_AHEAD launches
+// queued until then (the launches past the end find empty lists and return).
+// No barrier inside a launch, so no launch needs all its blocks resident.
+// Rows up to WB_LIGHT edges are one lane's work, longer ones are listed as
+// WB_SLICE-edge slices, a wave each.  A vertex is discovered by atomicMin on
+// the levels, which start at n+1: the one that finds n+1 lists it, so no
+// bitmap is needed.  A plain load looks first; levels only fall, so what it
+// sees at or below the new level proves that there is nothing to do, however
+// stale.  Discovered rows are staged per wave in LDS; a workgroup reserves
+// list space once, or when a stage fills.  Block 0 counts what the host-driven
+// loop reports: its steps, the steps that its threshold rule would push, and
+// the frontiers' edges.
+//
+// CC (k_uf_*): union-find, larger roots hooked under smaller ones, with path
+// halving (the scheme of Jaiganesh and Burtscher, "A high-performance
+// connected components implementation for GPUs", HPDC 2018).  A vertex starts
+// under its first neighbour if that is smaller.  Where no hub joins most of
+// the graph that way, two rounds over the first neighbours lower roots by a
+// plain atomicMin and flatten the trees; a join lost there is found again.
+// Then every edge is joined, over the CSC's pull buckets and long-row chunks,
+// and a last pass flattens.  The root of a component is its smallest internal
+// ID, the label that CCv converges to.  Parents only fall and each is an
+// ancestor, so a stale read costs time only; a join is a compare-and-swap on
+// a root, and a failed one looks for the roots again, which are smaller.
+#include "internal.hpp"
+#include "device.hpp"
+#include "label_fold.hpp"
+#include "whole.hpp"
+
+#include <algorithm>
+#include <cstring>
+
+namespace gpr {
+
+double stream_time_ms(gpr_graph *g, bool start);
+void stream_time_mark(gpr_graph *g);
+double stream_time_read_ms(gpr_graph *g);
+
+constexpr int WB_THREADS = 256;
+constexpr int WB_WAVES = WB_THREADS / 64;
+constexpr uint32_t WB_LIGHT = 32;    // rows up to this length: a lane each
+constexpr uint32_t WB_SLICE = 256;   // longer rows: a wave per slice of this many edges
+constexpr int WB_U = 4;              // edges per lane in flight
+constexpr uint32_t WB_STAGE = 512;   // staged list entries per wave
+static_assert(WB_SLICE == 64 * WB_U, "a slice is one pass of the wave");
+// A listed row is its first edge and its length, read with the vertex's
+// degree when it is discovered: the next level then starts at the neighbours,
+// one dependent load sooner.
+constexpr int WB_START_BITS = 26;    // first edge (< 2^26 edges); the length (<= WB_LIGHT) above it
+static_assert(WB_LIGHT < 1u << (32 - WB_START_BITS), "a light row in 32 bits");
+
+// Counts of the lists, rotating over three slots: level L reads slot L%3,
+// adds to (L+1)%3 and clears (L+2)%3, last read by level L-1.  Vertices and
+// edges discovered are striped: one line would take an atomic from every
+// workgroup of a wide level.
+constexpr unsigned WB_STRIPES = 16;
+struct alignas(128) WbStripe {
+    unsigned long long nact[3], nedge[3];   // vertices discovered, and their out-edges
+};
+struct alignas(128) WbCtl {
+    unsigned int nlight[3], nheavy[3];      // list lengths
+    unsigned long long edges;               // of the frontiers so far
+    unsigned int pushes;                    // steps the threshold rule would push
+    WbStripe stripe[WB_STRIPES];
+};
+
+struct WbLists {
+    uint32_t *light[2];
+    uint64_t *heavy[2];                   // slices: (first edge << 32) | edges
+};
+
+// What one wave discovered and has not listed yet (light rows), and its
+// counts of the level.
+struct WbFound {
+    uint32_t *buf;   // WB_STAGE entries of LDS
+    uint32_t n = 0;  // wave-uniform
+    uint32_t act = 0;             // per lane
+    unsigned long long edge = 0;  // per lane
+};
+
+// The slice of a row's edges from its k-th on.
+__device__ __forceinline__ uint64_t wb_slice(uint32_t first, uint32_t len, uint32_t k) {
+    return ((uint64_t)(first + k) << 32) | (len - k < WB_SLICE ? len - k : WB_SLICE);
+}
+
+__device__ __forceinline__ void wb_store(uint32_t *list, uint32_t at, const WbFound &f) {
+    for (uint32_t i = lane(); i < f.n; i += 64) list[at + i] = f.buf[i];
+}
+
+// Discover up to WB_U destinations per lane at level nl.  Wave-uniform.
+__device__ __forceinline__ void wb_relax(const bool (&act)[WB_U], const uint32_t (&d)[WB_U], uint32_t nl,
+                                         uint32_t *level, const uint64_t *__restrict__ index,
+                                         const uint32_t *__restrict__ deg, const WbLists &L, int nb, WbCtl *ctl,
+                                         int nx, WbFound &f) {
+    bool need[WB_U];
+    bool any = false;
+#pragma unroll
+    for (int j = 0; j < WB_U; ++j)
+        need[j] = act[j] && __hip_atomic_load(&level[d[j]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) > nl;
+#pragma unroll
+    for (int j = 0; j < WB_U; ++j) any |= need[j];
+    if (!__ballot(any)) return;
+    uint32_t old[WB_U], dg[WB_U], first[WB_U];
+#pragma unroll
+    for (int j = 0; j < WB_U; ++j) {
+        old[j] = need[j] ? atomicMin(&level[d[j]], nl) : 0u;
+        dg[j] = need[j] ? deg[d[j]] : 0u;
+        first[j] = need[j] ? (uint32_t)index[d[j]] : 0u;
+    }
+    uint32_t ch = 0;
+#pragma unroll
+    for (int j = 0; j < WB_U; ++j) {
+        const bool found = need[j] && old[j] > nl;
+        if (found) {
+            ++f.act;
+            f.edge += dg[j];
+        }
+        dg[j] = found ? dg[j] : 0u;
+        const bool light = dg[j] > 0 && dg[j] <= WB_LIGHT;
+        const uint64_t word = __ballot(light);
+        if (word) {
+            if (f.n + 64 > WB_STAGE) {
+                __builtin_amdgcn_wave_barrier();
+                uint32_t b = 0;
+                if (lane() == 0) b = atomicAdd(&ctl->nlight[nx], f.n);
+                wb_store(L.light[nb], __builtin_amdgcn_readfirstlane(b), f);
+                __builtin_amdgcn_wave_barrier();
+                f.n = 0;
+            }
+            if (light) f.buf[f.n + mbcnt(word)] = first[j] | dg[j] << WB_START_BITS;
+            f.n += (uint32_t)__popcll(word);
+        }
+        if (dg[j] > WB_LIGHT) ch += (dg[j] + WB_SLICE - 1) / WB_SLICE;
+    }
+    if (!__ballot(ch)) return;
+    const uint32_t ih = wave_incl_scan(ch), th = __shfl(ih, 63, 64);
+    uint32_t b = 0;
+    if (lane() == 0) b = atomicAdd(&ctl->nheavy[nx], th);
+    b = __builtin_amdgcn_readfirstlane(b) + (ih - ch);
+#pragma unroll
+    for (int j = 0; j < WB_U; ++j)
+        if (dg[j] > WB_LIGHT)
+            for (uint32_t k = 0; k < dg[j]; k += WB_SLICE) L.heavy[nb][b++] = wb_slice(first[j], dg[j], k);
+}
+
+// The threshold rule (threshold_sparse): integer nactv + nacte <= limit, or
+// with frac its float and double roundings against rhs.
+struct WbRule {
+    unsigned long long limit;
+    double rhs;
+    int frac;
+};
+
+// What block 0 tells the host (pinned memory).
+constexpr unsigned WB_EVERY = 4;
+struct alignas(128) WbHost {
+    unsigned int level;             // levels begun, every WB_EVERY of them
+    unsigned int done;              // 1: the frontier was empty; the fields below are final
+    unsigned int steps, pushes;
+    unsigned long long edges;
+};
+
+// Levels n+1 but for the start's 0, the start's row as the first frontier,
+// the counts.
+__global__ void __launch_bounds__(WB_THREADS)
+k_wb_init(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__restrict__ deg,
+          const uint32_t *__restrict__ perm, uint32_t start, uint32_t *level, WbLists L, WbCtl *ctl) {
+    const uint32_t s = perm ? perm[start] : start;
+    for (uint32_t v = blockIdx.x * WB_THREADS + threadIdx.x; v < n; v += gridDim.x * WB_THREADS)
+        level[v] = v == s ? 0u : n + 1;
+    if (blockIdx.x != 0) return;
+    const uint32_t ds = deg[s], es = (uint32_t)index[s];
+    const uint32_t sl = ds > WB_LIGHT ? (ds + WB_SLICE - 1) / WB_SLICE : 0u;
+    for (uint32_t k = threadIdx.x; k < sl; k += WB_THREADS) L.heavy[0][k] = wb_slice(es, ds, k * WB_SLICE);
+    unsigned int *w = (unsigned int *)ctl;
+    for (unsigned i = threadIdx.x; i < sizeof(WbCtl) / 4; i += WB_THREADS) w[i] = 0;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        if (ds && !sl) L.light[0][0] = es | ds << WB_START_BITS;
+        ctl->nlight[0] = ds && !sl;
+        ctl->nheavy[0] = sl;
+        ctl->stripe[0].nact[0] = 1;
+        ctl->stripe[0].nedge[0] = ds;
+    }
+}
+
+__global__ void __launch_bounds__(WB_THREADS)
+k_wb_level(uint32_t n, uint32_t lvl, const uint64_t *__restrict__ index, const uint32_t *__restrict__ nbrs,
+           const uint32_t *__restrict__ deg, uint32_t *level, WbLists L, WbCtl *ctl, WbRule rule, WbHost *h) {
+    __shared__ uint32_t s_stage[WB_WAVES * WB_STAGE];
+    __shared__ uint32_t s_n[WB_WAVES], s_act[WB_WAVES], s_base[WB_WAVES];
+    __shared__ unsigned long long s_edge[WB_WAVES];
+    const unsigned ln = lane(), wv = threadIdx.x / 64;
+    const uint32_t W = gridDim.x * WB_WAVES;
+    // wave rank interleaved over the blocks: a small level lands on many CUs
+    const uint32_t w = wv * gridDim.x + blockIdx.x;
+    const int c = lvl % 3, nx = (lvl + 1) % 3, stale = (lvl + 2) % 3, cb = lvl & 1, nb = cb ^ 1;
+    // the wave's first rows are loaded beside the lengths that say whether
+    // they are there (a list holds n rows)
+    uint32_t row = L.light[cb][min(w * 64 + ln, n - 1)];
+    const uint32_t nL = ctl->nlight[c], nH = ctl->nheavy[c];
+    if (blockIdx.x == 0) {
+        unsigned long long na = 0, ne = 0;
+        if (threadIdx.x < WB_STRIPES) {
+            WbStripe &st = ctl->stripe[threadIdx.x];
+            na = st.nact[c];
+            ne = st.nedge[c];
+            st.nact[stale] = 0;
+            st.nedge[stale] = 0;
+        }
+        if (threadIdx.x < 64) {
+            na = wave_sum(na);
+            ne = wave_sum(ne);
+        }
+        if (threadIdx.x == 0) {
+            ctl->nlight[stale] = 0;
+            ctl->nheavy[stale] = 0;
+            if (na) {
+                ctl->edges += ne;
+                ctl->pushes += rule.frac ? (double)(float)(na + ne) <= rule.rhs : na + ne <= rule.limit;
+            } else if (!h->done) {
+                h->steps = lvl;
+                h->pushes = ctl->pushes;
+                h->edges = ctl->edges;
+                __hip_atomic_store(&h->done, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+            }
+            if ((lvl + 1) % WB_EVERY == 0)
+                __hip_atomic_store(&h->level, lvl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
+    WbFound f{&s_stage[wv * WB_STAGE]};
+    for (uint32_t base = w * 64; base < nL; base += W * 64) {
+        if (base != w * 64) row = L.light[cb][min(base + ln, n - 1)];
+        uint32_t e = 0, e1 = 0;
+        if (base + ln < nL) {
+            e = row & ((1u << WB_START_BITS) - 1);
+            e1 = e + (row >> WB_START_BITS);
+        }
+        while (__ballot(e < e1)) {
+            bool act[WB_U];
+            uint32_t d[WB_U];
+#pragma unroll
+            for (int j = 0; j < WB_U; ++j) {
+                act[j] = e + j < e1;
+                d[j] = act[j] ? nbrs[e + j] : 0u;
+            }
+            e = e + WB_U < e1 ? e + WB_U : e1;
+            wb_relax(act, d, lvl + 1, level, index, deg, L, nb, ctl, nx, f);
+        }
+    }
+    for (uint32_t j = W - 1 - w; j < nH; j += W) {
+        const uint64_t ent = L.heavy[cb][j];
+        const uint32_t e0 = (uint32_t)(ent >> 32), len = (uint32_t)ent;
+        bool act[WB_U];
+        uint32_t d[WB_U];
+#pragma unroll
+        for (int k = 0; k < WB_U; ++k) {
+            act[k] = ln + 64 * k < len;
+            d[k] = act[k] ? nbrs[e0 + ln + 64 * k] : 0u;
+        }
+        wb_relax(act, d, lvl + 1, level, index, deg, L, nb, ctl, nx, f);
+    }
+    // the block's stages and counts, with one reservation
+    const uint32_t ta = wave_sum(f.act);
+    const unsigned long long te = wave_sum(f.edge);
+    if (ln == 0) {
+        s_n[wv] = f.n;
+        s_act[wv] = ta;
+        s_edge[wv] = te;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t tn = 0, a = 0;
+        unsigned long long e = 0;
+        for (int i = 0; i < WB_WAVES; ++i) {
+            s_base[i] = tn;
+            tn += s_n[i];
+            a += s_act[i];
+            e += s_edge[i];
+        }
+        if (a) {
+            WbStripe &st = ctl->stripe[blockIdx.x % WB_STRIPES];
+            const uint32_t b = tn ? atomicAdd(&ctl->nlight[nx], tn) : 0u;
+            atomicAdd(&st.nact[nx], (unsigned long long)a);
+            atomicAdd(&st.nedge[nx], e);
+            for (int i = 0; i < WB_WAVES; ++i) s_base[i] += b;
+        }
+    }
+    __syncthreads();
+    wb_store(L.light[nb], s_base[wv], f);
+}
+
+// Results in original IDs, in order (they may go to host memory).
+__global__ void __launch_bounds__(WB_THREADS)
+k_wb_out(uint32_t n, const uint32_t *__restrict__ level, const uint32_t *__restrict__ perm, uint32_t *out) {
+    for (uint32_t o = blockIdx.x * WB_THREADS + threadIdx.x; o < n; o += gridDim.x * WB_THREADS)
+        out[o] = level[perm ? perm[o] : o];
+}
+
+// ---- union-find CC ------------------------------------------------------------
+constexpr int UF_THREADS = 256;
+constexpr uint32_t UF_LIGHT = 32;
+constexpr int UF_SUB = 16;
+constexpr uint32_t UF_QCAP = (STREAM_ITEMS + LONG_DEG) / (UF_LIGHT + 1) + 1;
+
+template <int SCOPE> __device__ __forceinline__ uint32_t uf_get(const uint32_t *parent, uint32_t v) {
+    return __hip_atomic_load(&parent[v], __ATOMIC_RELAXED, SCOPE);
+}
+// The root above v, halving the path on the way.
+template <int SCOPE> __device__ __forceinline__ uint32_t uf_root(uint32_t *parent, uint32_t v) {
+    uint32_t p = uf_get<SCOPE>(parent, v);
+    while (p != v) {
+        const uint32_t q = uf_get<SCOPE>(parent, p);
+        if (q == p) return p;
+        __hip_atomic_store(&parent[v], q, __ATOMIC_RELAXED, SCOPE);
+        v = p;
+        p = q;
+    }
+    return v;
+}
+// Join the components of a and b.  The first look goes through the caches,
+// which hold nearly every answer on a flattened forest; only after a failed
+// swap does it read past them (reads of one hot root from every edge would
+// queue).
+__device__ __forceinline__ void uf_join(uint32_t *parent, uint32_t a, uint32_t b) {
+    a = uf_root<__HIP_MEMORY_SCOPE_WORKGROUP>(parent, a);
+    b = uf_root<__HIP_MEMORY_SCOPE_WORKGROUP>(parent, b);
+    while (a != b) {
+        const uint32_t hi = a > b ? a : b, lo = a > b ? b : a;
+        const uint32_t old = atomicCAS(&parent[hi], hi, lo);
+        if (old == hi) return;
+        a = uf_root<__HIP_MEMORY_SCOPE_AGENT>(parent, old);   // hi was hooked already, under old < hi
+        b = uf_root<__HIP_MEMORY_SCOPE_AGENT>(parent, lo);
+    }
+}
+
+__global__ void __launch_bounds__(UF_THREADS)
+k_uf_init(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__restrict__ nbrs, uint32_t *parent,
+          uint32_t *minorig) {
+    for (uint32_t v = blockIdx.x * UF_THREADS + threadIdx.x; v < n; v += gridDim.x * UF_THREADS) {
+        const uint64_t b = index[v];
+        uint32_t p = v;
+        if (b < index[v + 1]) p = min(v, nbrs[b]);
+        parent[v] = p;
+        if (minorig) minorig[v] = 0xffffffffu;
+    }
+}
+
+// One round over the first UF_FIRST_NBRS neighbours: the larger of two roots
+// goes under the smaller by atomicMin, without a second try.  A root that was
+// hooked in between may lose that hook to a smaller one; k_uf_link sees every
+// edge again.  On a random graph of 500K vertices and 3M edges joining every
+// edge at once took 1.5-2.5 ms, most swaps failing on roots that had just
+// been hooked; after two rounds the whole run takes 0.3-0.4 ms.
+constexpr uint64_t UF_FIRST_NBRS = 4;
+constexpr int UF_ROUNDS = 2;
+__global__ void __launch_bounds__(UF_THREADS)
+k_uf_round(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__restrict__ nbrs, uint32_t *parent) {
+    constexpr int WG = __HIP_MEMORY_SCOPE_WORKGROUP;
+    for (uint32_t v = blockIdx.x * UF_THREADS + threadIdx.x; v < n; v += gridDim.x * UF_THREADS) {
+        const uint64_t b = index[v], e = min(index[v + 1], b + UF_FIRST_NBRS);
+        const uint32_t a = uf_get<WG>(parent, v);
+        for (uint64_t j = b; j < e; ++j) {
+            const uint32_t c = uf_get<WG>(parent, nbrs[j]);
+            const uint32_t hi = a > c ? a : c, lo = a > c ? c : a;
+            if (hi != lo && uf_get<WG>(parent, hi) > lo) atomicMin(&parent[hi], lo);
+        }
+    }
+}
+
+// Every edge once, from its larger endpoint; the split of rows as in the
+// 64-source pull: lanes, 16-lane groups, chunks of long rows.
+__global__ void __launch_bounds__(UF_THREADS)
+k_uf_link(uint32_t nbuckets, const uint32_t *__restrict__ bucket, const uint64_t *__restrict__ index,
+          const uint32_t *__restrict__ nbrs, const uint32_t *__restrict__ long_rows,
+          const uint32_t *__restrict__ long_base, uint32_t nlong, uint32_t *parent) {
+    __shared__ uint32_t q[UF_QCAP];
+    __shared__ uint32_t qn;
+    if (blockIdx.x >= nbuckets) {
+        const uint32_t c = blockIdx.x - nbuckets;
+        uint32_t lo = 0, hi = nlong;   // the row whose chunks c is among
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (long_base[mid] <= c) lo = mid + 1; else hi = mid;
+        }
+        const uint32_t row = long_rows[lo - 1];
+        const uint64_t cb = index[row] + (uint64_t)(c - long_base[lo - 1]) * LONG_CHUNK;
+        const uint64_t re = index[row + 1], ce = cb + LONG_CHUNK < re ? cb + LONG_CHUNK : re;
+        for (uint64_t e = cb + threadIdx.x; e < ce; e += UF_THREADS) {
+            const uint32_t u = nbrs[e];
+            if (u < row) uf_join(parent, row, u);
+        }
+        return;
+    }
+    if (threadIdx.x == 0) qn = 0;
+    __syncthreads();
+    const uint32_t r0 = bucket[blockIdx.x], r1 = bucket[blockIdx.x + 1];
+    for (uint32_t r = r0 + threadIdx.x; r < r1; r += UF_THREADS) {
+        const uint64_t beg = index[r], end = index[r + 1];
+        if (end - beg > LONG_DEG) continue;   // by its chunks
+        if (end - beg > UF_LIGHT) {
+            q[atomicAdd(&qn, 1u)] = r;
+            continue;
+        }
+        for (uint64_t e = beg; e < end; ++e) {
+            const uint32_t u = nbrs[e];
+            if (u < r) uf_join(parent, r, u);
+        }
+    }
+    __syncthreads();
+    const uint32_t cnt = qn;
+    for (uint32_t i = threadIdx.x / UF_SUB; i < cnt; i += UF_THREADS / UF_SUB) {
+        const uint32_t r = q[i];
+        const uint64_t end = index[r + 1];
+        for (uint64_t e = index[r] + threadIdx.x % UF_SUB; e < end; e += UF_SUB) {
+            const uint32_t u = nbrs[e];
+            if (u < r) uf_join(parent, r, u);
+        }
+    }
+}
+
+// Every vertex under its root; with minorig, the components' smallest
+// original IDs at the roots too, with out the roots as results.  A launch of
+// its own, so no root is hooked meanwhile; a parent rewritten is an ancestor.
+__global__ void __launch_bounds__(LF_THREADS)
+k_uf_flatten(uint32_t n, uint32_t *parent, const uint32_t *__restrict__ order, uint32_t *minorig, uint32_t *out) {
+    constexpr int WG = __HIP_MEMORY_SCOPE_WORKGROUP;
+    LabelFold f;
+    for (uint64_t i = blockIdx.x * (uint64_t)LF_THREADS + threadIdx.x; i < n; i += (uint64_t)gridDim.x * LF_THREADS) {
+        const uint32_t r = uf_root<WG>(parent, (uint32_t)i);
+        __hip_atomic_store(&parent[i], r, __ATOMIC_RELAXED, WG);
+        if (minorig) f.add(minorig, i, r, order[i]);
+        if (out) out[i] = r;
+    }
+    if (minorig) f.finish(minorig);
+}
+
+__global__ void __launch_bounds__(UF_THREADS)
+k_uf_out(uint32_t n, const uint32_t *__restrict__ parent, const uint32_t *__restrict__ perm,
+         const uint32_t *__restrict__ minorig, uint32_t *out) {
+    for (uint32_t o = blockIdx.x * UF_THREADS + threadIdx.x; o < n; o += gridDim.x * UF_THREADS)
+        out[o] = minorig[parent[perm[o]]];
+}
+
+// ---- host side ------------------------------------------------------------------
+constexpr uint32_t WHOLE_STAGE_V = 1u << 18;   // results up to this many vertices go straight to pinned memory
+
+// The line at whole_edges (2^24): a whole BFS against the host-driven one,
+// results downloaded, in us: RMAT 0.1M edges 99 / 190, 1.8M 135 / 236, 7.6M
+// 253 / 260, 15M 289 / 361, 31M 458 / 387 (a dense level is cheaper pulled);
+// meshes and random graphs, of more levels, gain everywhere (8M edges 1300 /
+// 3200 and 593 / 735).  Whole CC gains to twice that: RMAT 0.1M 47 / 230, 7.6M
+// 131 / 317, 31M 257 / 457, 128M 1055 / 764; random 18M 1150 / 1840.
+bool whole_run(const gpr_graph *g, const gpr_run_opts &o, bool cc) {
+    const double limit = std::min(tun().whole_edges * (cc ? 2.0 : 1.0), (double)(1u << WB_START_BITS));
+    if ((double)g->m > limit || (double)g->n > limit || g->n == 0) return false;
+    if (o.direction != GPR_DIR_AUTO || o.out_kind != 0 || o.trace || o.deferred_update || g->prof.on) return false;
+    return cc ? o.fusion == 0 && g->symmetric && !(o.threshold_pct > 0.f) : o.fusion <= 0;
+}
+
+struct WholeBuf {
+    uint64_t heavy_cap;
+    size_t light[2], heavy[2], out, bytes;   // byte offsets; values at 0
+};
+static WholeBuf whole_layout(const gpr_graph *g) {
+    WholeBuf b;
+    const uint64_t long_rows = std::min<uint64_t>(g->n, g->m / (WB_LIGHT + 1));
+    b.heavy_cap = g->m / WB_SLICE + long_rows + 64;
+    auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
+    const size_t v = up(4ull * g->n);
+    b.light[0] = v;
+    b.light[1] = 2 * v;
+    b.heavy[0] = 3 * v;
+    b.heavy[1] = b.heavy[0] + up(8 * b.heavy_cap);
+    b.out = b.heavy[1] + up(8 * b.heavy_cap);
+    b.bytes = b.out + v;
+    return b;
+}
+static int whole_ensure(gpr_graph *g, const WholeBuf &b) {
+    if (!g->wbuf) GPR_TRY(dev_alloc(&g->wbuf, b.bytes, "whole-run buffers"));
+    if (!g->wctl) GPR_TRY(dev_alloc(&g->wctl, sizeof(WbCtl), "whole-run control"));
+    if (!g->whost) {
+        GPR_HIP(hipHostMalloc(&g->whost, sizeof(WbHost), hipHostMallocMapped | hipHostMallocCoherent));
+        GPR_HIP(hipHostGetDevicePointer(&g->whost_dev, g->whost, 0));
+    }
+    if (!g->wstage && g->n <= WHOLE_STAGE_V) {
+        GPR_HIP(hipHostMalloc((void **)&g->wstage, 4ull * g->n, hipHostMallocMapped | hipHostMallocCoherent));
+        GPR_HIP(hipHostGetDevicePointer((void **)&g->wstage_dev, g->wstage, 0));
+    }
+    return GPR_OK;
+}
+// Waits for the stream; the n results at dev (the staging memory or the
+// device) into host, when asked for.
+static int whole_results(gpr_graph *g, const uint32_t *dev, uint32_t *host) {
+    const bool staged = dev == g->wstage_dev;
+    if (host && !staged) GPR_HIP(hipMemcpyAsync(host, dev, 4ull * g->n, hipMemcpyDeviceToHost, g->stream));
+    GPR_HIP(hipStreamSynchronize(g->stream));
+    if (host && staged) std::memcpy(host, g->wstage, 4ull * g->n);
+    return GPR_OK;
+}
+
+// Launches queued beyond the last level reported: the host needs about 4 us a
+// launch and a small level takes 8; those past the end cost about 3 us each.
+// Reporting every level instead of every fourth (a write to the host that
+// the launch waits for) took 460 us instead of 434 on 47 levels.
+constexpr unsigned WB_AHEAD = 6;
+// Blocks of a level's launch: one per WB_BLOCK_EDGES edges of the graph.
+constexpr uint64_t WB_BLOCK_EDGES = 4096;
+
+int whole_bfs(gpr_graph *g, uint32_t start, float threshold_pct, uint32_t *levels, gpr_run_info *info) {
+    const WholeBuf b = whole_layout(g);
+    GPR_TRY(whole_ensure(g, b));
+    char *base = (char *)g->wbuf;
+    const uint32_t n = g->n;
+    uint32_t *level = (uint32_t *)base;
+    const uint32_t *perm = g->order ? g->perm : nullptr;
+    WbLists L = {{(uint32_t *)(base + b.light[0]), (uint32_t *)(base + b.light[1])},
+                 {(uint64_t *)(base + b.heavy[0]), (uint64_t *)(base + b.heavy[1])}};
+    WbCtl *ctl = (WbCtl *)g->wctl;
+    WbRule rule = {g->m / 20, 0.0, 0};
+    if (threshold_pct > 0.f) {
+        rule.frac = 1;
+        rule.rhs = (double)(float)g->m / (100.0 / (double)threshold_pct);
+    }
+    const unsigned grid = (unsigned)std::min<uint64_t>(1024, std::max<uint64_t>(32, g->m / WB_BLOCK_EDGES));
+    volatile WbHost *h = (volatile WbHost *)g->whost;
+    h->level = 0;
+    h->done = 0;
+    stream_time_ms(g, true);
+    hipLaunchKernelGGL(k_wb_init, dim3(grid_for(n, WB_THREADS, 1024)), dim3(WB_THREADS), 0, g->stream, n, g->index,
+                       g->deg, perm, start, level, L, ctl);
+    unsigned launched = 0, polls = 0;
+    while (!__atomic_load_n(&((WbHost *)g->whost)->done, __ATOMIC_ACQUIRE)) {
+        if (launched - h->level < WB_AHEAD) {
+            hipLaunchKernelGGL(k_wb_level, dim3(grid), dim3(WB_THREADS), 0, g->stream, n, launched, g->index, g->nbrs,
+                               g->deg, level, L, ctl, rule, (WbHost *)g->whost_dev);
+            ++launched;
+            GPR_HIP(hipGetLastError());
+        } else if (++polls % 4096 == 0) {
+            // a stream that failed would never report a level
+            const hipError_t e = hipStreamQuery(g->stream);
+            if (e != hipSuccess && e != hipErrorNotReady) GPR_HIP(e);
+        }
+    }
+    stream_time_mark(g);
+    uint32_t *out = g->wstage ? g->wstage_dev : (uint32_t *)(base + b.out);
+    if (levels)
+        hipLaunchKernelGGL(k_wb_out, dim3(grid_for(n, WB_THREADS, 1024)), dim3(WB_THREADS), 0, g->stream, n, level,
+                           perm, out);
+    GPR_HIP(hipGetLastError());
+    GPR_TRY(whole_results(g, out, levels));
+    info->ms = stream_time_read_ms(g);
+    info->iters = (int)h->steps;
+    info->push_iters = (int)h->pushes;
+    info->edges = h->edges;
+    return GPR_OK;
+}
+
+int whole_cc(gpr_graph *g, uint32_t *labels, gpr_run_info *info) {
+    const WholeBuf b = whole_layout(g);
+    GPR_TRY(whole_ensure(g, b));
+    char *base = (char *)g->wbuf;
+    const uint32_t n = g->n;
+    uint32_t *parent = (uint32_t *)base;
+    // the recode (labels asked for, vertices relabelled): minima by original ID
+    uint32_t *minorig = labels && g->order ? (uint32_t *)(base + b.light[0]) : nullptr;
+    uint32_t *out = !labels ? nullptr : g->wstage ? g->wstage_dev : (uint32_t *)(base + b.out);
+    const unsigned grid = grid_for(n, UF_THREADS, 4096);
+    stream_time_ms(g, true);
+    hipLaunchKernelGGL(k_uf_init, dim3(grid), dim3(UF_THREADS), 0, g->stream, n, g->index, g->nbrs, parent, minorig);
+    // a hub next to 1/32 of the vertices, with the smallest ID (relabelled by
+    // degree), already holds most of its component: the rounds would cost
+    // their launches (10-14 us) and save nothing
+    const bool hub = g->order && (uint64_t)g->max_deg * 32 >= n;
+    const dim3 fgrid(grid_for(n, LF_THREADS, 1024));
+    for (int k = 0; !hub && k < UF_ROUNDS; ++k) {
+        if (k == 0)
+            hipLaunchKernelGGL(k_uf_flatten, fgrid, dim3(LF_THREADS), 0, g->stream, n, parent, (const uint32_t *)nullptr,
+                               (uint32_t *)nullptr, (uint32_t *)nullptr);
+        hipLaunchKernelGGL(k_uf_round, dim3(grid), dim3(UF_THREADS), 0, g->stream, n, g->index, g->nbrs, parent);
+        hipLaunchKernelGGL(k_uf_flatten, fgrid, dim3(LF_THREADS), 0, g->stream, n, parent, (const uint32_t *)nullptr,
+                           (uint32_t *)nullptr, (uint32_t *)nullptr);
+    }
+    hipLaunchKernelGGL(k_uf_link, dim3(g->nbuckets + g->nlong_chunks), dim3(UF_THREADS), 0, g->stream, g->nbuckets,
+                       g->bucket, g->index, g->nbrs, g->long_rows, g->long_base, g->nlong, parent);
+    hipLaunchKernelGGL(k_uf_flatten, fgrid, dim3(LF_THREADS), 0, g->stream, n, parent, g->order, minorig,
+                       minorig ? nullptr : out);
+    if (minorig)
+        hipLaunchKernelGGL(k_uf_out, dim3(grid), dim3(UF_THREADS), 0, g->stream, n, parent, g->perm, minorig, out);
+    GPR_HIP(hipGetLastError());
+    stream_time_mark(g);
+    GPR_TRY(whole_results(g, out, labels));
+    info->ms = stream_time_read_ms(g);
+    // one step, over every edge
+    info->iters = 1;
+    info->push_iters = 1;
+    info->edges = g->m;
+    return GPR_OK;
+}
+
+} // namespace gpr

@@ -491,6 +491,13 @@ int gpr_trace_get(const gpr_graph *g, gpr_iter_stats *out, int cap, int *k);
  *   pr_pull_edges       PageRank with pr_split_bytes 0: graphs of at most
  *                       this many edges and 2^20 vertices are pulled
  *                       (default 2^23; 0: never)
+ *   whole_edges         BFSLVLv and CCv with default options (automatic
+ *                       direction and output, the benchmark's own fusion
+ *                       setting, no trace): graphs of at most this many edges
+ *                       (CC: twice, symmetric) run without the host between
+ *                       their steps (default 2^24; 0: never).  Levels, labels
+ *                       and BFS's counts are the same; such a CC run is one
+ *                       step in gpr_run_info
  *   pull_serial_max     pull rows up to this in-degree run lane-serially
  *   pull_blocks_per_cu  pull grid size per compute unit
  *   push_blocks_per_cu  push grid cap per compute unit
