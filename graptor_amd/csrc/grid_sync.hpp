@@ -117,4 +117,23 @@ __device__ __forceinline__ bool grid_barrier(unsigned long long *arrive, unsigne
     return *s_ok != 0;
 }
 
+// K words that every block reads after a barrier, by one lane of the block
+// each and handed on through LDS (s: K words): a read by every wave of a
+// 256-block grid of 1024 threads is 4096 requests for one line, about 10 us.
+// All threads call it.
+template <int K>
+__device__ __forceinline__ void block_read(const unsigned long long *const (&p)[K], unsigned long long *s,
+                                           unsigned long long (&v)[K]) {
+    __syncthreads();   // the last values are read
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int k = 0; k < K; ++k) v[k] = ld_agent(p[k]);
+#pragma unroll
+        for (int k = 0; k < K; ++k) s[k] = v[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] = s[k];
+}
+
 } // namespace gpr

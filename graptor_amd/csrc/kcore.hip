@@ -36,11 +36,14 @@
 // decrement that finds the count at or below K (a race with another
 // decrement at the floor) is undone with atomicAdd before the round's
 // barrier, so after every barrier each count is exact.
+// Bound by its rounds' chains of dependent accesses and barriers (RMAT-20: 670
+// rounds of 7 us and 2.3 us for the barrier; 20 us together with one lane per
+// row, every hub counter looked at each round and 256 blocks).
 // Frontier lists as in the fused push: rows up to KC_LIGHT_MAX edges one
-// lane per vertex, longer rows one wave per KC_SLICE-edge slice.  Light
-// appends are staged per wave in LDS and reserved in the shared list once
-// per KC_STAGE entries, heavy slices are reserved per wave step.  List
-// counts rotate over three slots per round and level minima over two slots
+// lane per vertex (KC_SUB lanes in small rounds), longer rows one wave per
+// KC_SLICE-edge slice.  Light appends are staged per wave in LDS and reserved
+// in the shared list once per KC_STAGE entries, heavy slices are reserved per
+// wave step.  List counts rotate over three slots per round and level minima over two slots
 // per level, each cleared one phase after its last read and at least one
 // barrier before its next write.
 // Memory ordering and the barrier: grid_sync.hpp.  Termination: every block
@@ -66,8 +69,12 @@ constexpr int KC_STAGE = 512;           // light appends staged per wave in LDS
 constexpr int KC_PU = 4;                // candidate chunks per wave step in passes A and B
 constexpr uint32_t KC_HUBS = 24576;      // count-downs of vertices below this ID add up in LDS
 static_assert(KC_HUBS % KC_THREADS == 0, "whole passes over the hub counters");
+constexpr uint32_t KC_FEW_HUBS = KC_THREADS;   // the same in a small round (256 to 4096 measure alike)
+constexpr uint32_t KC_HUB_ROWS = KC_HUBS / KC_THREADS;   // one hub counter per thread in each
 constexpr unsigned KC_MAX_WAVES = GS_GROUP * GS_MAX_GROUPS * KC_WAVES;
 static_assert(KC_SLICE == 64 * KC_U, "a slice is one pass of the wave");
+constexpr unsigned KC_SUB = 8;          // lanes of a light row in a small round
+static_assert(KC_SUB * KC_U == KC_LIGHT_MAX, "a light row is one step of its lanes");
 // phase kinds timed by block 0: the candidate pass, its barrier, round
 // work, round barriers
 constexpr int KC_PROF = 4;
@@ -100,6 +107,18 @@ __device__ __forceinline__ uint32_t ld32(const uint32_t *p) {
 }
 __device__ __forceinline__ uint64_t ld64(const uint64_t *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The smaller of two words, read once per block (block_read).
+__device__ __forceinline__ uint32_t block_read_min(const unsigned int &a, const unsigned int &b,
+                                                   unsigned long long *s) {
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const uint32_t x = ld32(&a), y = ld32(&b);
+        s[0] = x < y ? x : y;
+    }
+    __syncthreads();
+    return (uint32_t)s[0];
 }
 
 __device__ __forceinline__ uint32_t kc_slices(uint32_t dg) {
@@ -154,16 +173,18 @@ __device__ __forceinline__ void kc_flush_block(KcStage &st, uint32_t *list, unsi
 }
 
 // Append the vertices v[j] with put[j] to the frontier lists of buffer cb:
-// light rows through the stage, heavy rows' slices directly.  Wave-uniform:
-// every lane calls it.
+// light rows through the stage, heavy rows' slices directly.  dg[j]: the
+// degree, where the caller has it (else KC_NODEG).  Wave-uniform: every lane
+// calls it.
+constexpr uint32_t KC_NODEG = 0xffffffffu;
 __device__ __forceinline__ void kc_append(const bool (&put)[KC_U], const uint32_t (&v)[KC_U],
-                                          const uint32_t *__restrict__ deg, const KcLists &L, int cb,
-                                          unsigned long long *nlight, unsigned long long *nheavy, KcStage &st) {
-    uint32_t dg[KC_U];
+                                          uint32_t (&dg)[KC_U], const uint32_t *__restrict__ deg, const KcLists &L,
+                                          int cb, unsigned long long *nlight, unsigned long long *nheavy,
+                                          KcStage &st) {
     uint32_t cl = 0, ch = 0;
 #pragma unroll
     for (int j = 0; j < KC_U; ++j) {
-        dg[j] = put[j] ? deg[v[j]] : 0u;
+        if (put[j] && dg[j] == KC_NODEG) dg[j] = deg[v[j]];
         if (put[j]) {
             const uint32_t s = kc_slices(dg[j]);
             cl += s == 0;
@@ -204,20 +225,32 @@ __device__ __forceinline__ void kc_append(const bool (&put)[KC_U], const uint32_
 __device__ __forceinline__ void kc_count_down(const bool (&act)[KC_U], const uint32_t (&d)[KC_U], uint32_t K,
                                               uint32_t *core, const uint32_t *__restrict__ deg, const KcLists &L,
                                               int nb, unsigned long long *nlight, unsigned long long *nheavy,
-                                              KcStage &st, uint32_t *hub, uint32_t &dmin) {
+                                              KcStage &st, uint32_t *hub, uint32_t *hub_row, uint32_t hubs,
+                                              uint32_t &dmin) {
     bool need[KC_U];
+    uint32_t dg[KC_U];
+    // a count seen at K+1 is about to be listed: its degree comes beside the
+    // atomic instead of after it
 #pragma unroll
-    for (int j = 0; j < KC_U; ++j) need[j] = act[j] && core[d[j]] > K;
+    for (int j = 0; j < KC_U; ++j) {
+        const uint32_t c = act[j] ? core[d[j]] : 0u;
+        need[j] = act[j] && c > K;
+        dg[j] = c == K + 1 ? d[j] : KC_NODEG;
+    }
     // hubs: counted in this block's LDS, applied once per round (kc_hub_flush)
 #pragma unroll
     for (int j = 0; j < KC_U; ++j)
-        if (need[j] && d[j] < KC_HUBS) {
+        if (need[j] && d[j] < hubs) {
             atomicAdd(&hub[d[j]], 1u);
+            hub_row[d[j] / KC_THREADS] = 1;
             need[j] = false;
         }
     uint32_t old[KC_U];
 #pragma unroll
-    for (int j = 0; j < KC_U; ++j) old[j] = need[j] ? atomicSub(&core[d[j]], 1u) : 0u;
+    for (int j = 0; j < KC_U; ++j) {
+        if (need[j] && dg[j] != KC_NODEG) dg[j] = deg[d[j]];
+        old[j] = need[j] ? atomicSub(&core[d[j]], 1u) : 0u;
+    }
     bool put[KC_U];
 #pragma unroll
     for (int j = 0; j < KC_U; ++j) {
@@ -225,37 +258,56 @@ __device__ __forceinline__ void kc_count_down(const bool (&act)[KC_U], const uin
         put[j] = need[j] && old[j] == K + 1;
         if (need[j] && old[j] > K + 1 && old[j] - 1 < dmin) dmin = old[j] - 1;
     }
-    kc_append(put, d, deg, L, nb, nlight, nheavy, st);
+    kc_append(put, d, dg, deg, L, nb, nlight, nheavy, st);
 }
 
 // Apply this block's hub count-downs of the round: subtract each sum delta
-// at once.  The count falls to max(K, c - delta) as delta single steps would:
+// at once.  Only the rows of counters that the round touched are looked at
+// (hub_row): most rounds are small, and looking at all 24 took every block
+// 4 us a round.  The count falls to max(K, c - delta) as delta single steps would:
 // a subtraction that starts at or below K is undone, one that crosses K is
 // topped back up to K, and that crossing one (there is exactly one per hub
 // and level) appends the hub.  Block-uniform: every thread calls it.
-__device__ __forceinline__ void kc_hub_flush(uint32_t *hub, uint32_t n, uint32_t K, uint32_t *core,
+__device__ __forceinline__ void kc_hub_flush(uint32_t *hub, uint32_t *hub_row, uint32_t n, uint32_t K, uint32_t *core,
                                              const uint32_t *__restrict__ deg, const KcLists &L, int nb,
                                              unsigned long long *nlight, unsigned long long *nheavy, KcStage &st,
                                              uint32_t &dmin) {
     __syncthreads();
-    for (uint32_t base = 0; base < KC_HUBS; base += KC_THREADS) {
-        const uint32_t j = base + threadIdx.x;
-        const uint32_t dl = hub[j];
-        bool put[KC_U] = {false, false, false, false};
-        uint32_t v[KC_U] = {j, j, j, j};
-        if (dl) {
-            hub[j] = 0;
-            const uint32_t old = atomicSub(&core[j], dl);
-            if (old <= K) {
-                atomicAdd(&core[j], dl);
-            } else if (old - dl <= K) {
-                if (old - dl < K) atomicAdd(&core[j], K - (old - dl));
-                put[0] = true;
-            } else if (old - dl < dmin) {
-                dmin = old - dl;
+    // the touched rows as a wave-uniform mask; cleared for the next round
+    // once every wave has it
+    uint64_t rows = __ballot(lane() < KC_HUB_ROWS && hub_row[lane()]);
+    if (!rows) return;
+    __syncthreads();
+    if (threadIdx.x < KC_HUB_ROWS) hub_row[threadIdx.x] = 0;
+    while (rows) {
+        // KC_U rows at a time: their subtractions are in flight together
+        bool put[KC_U];
+        uint32_t v[KC_U], dl[KC_U], old[KC_U], dg[KC_U];
+#pragma unroll
+        for (int u = 0; u < KC_U; ++u) {
+            const bool on = rows != 0;
+            v[u] = on ? (uint32_t)(__ffsll((long long)rows) - 1) * KC_THREADS + threadIdx.x : 0u;
+            rows &= rows - 1;   // 0 stays 0
+            dl[u] = on ? hub[v[u]] : 0u;
+            if (dl[u]) hub[v[u]] = 0;
+        }
+#pragma unroll
+        for (int u = 0; u < KC_U; ++u) old[u] = dl[u] ? atomicSub(&core[v[u]], dl[u]) : 0u;
+#pragma unroll
+        for (int u = 0; u < KC_U; ++u) {
+            put[u] = false;
+            dg[u] = KC_NODEG;
+            if (!dl[u]) continue;
+            if (old[u] <= K) {
+                atomicAdd(&core[v[u]], dl[u]);
+            } else if (old[u] - dl[u] <= K) {
+                if (old[u] - dl[u] < K) atomicAdd(&core[v[u]], K - (old[u] - dl[u]));
+                put[u] = true;
+            } else if (old[u] - dl[u] < dmin) {
+                dmin = old[u] - dl[u];
             }
         }
-        kc_append(put, v, deg, L, nb, nlight, nheavy, st);
+        kc_append(put, v, dg, deg, L, nb, nlight, nheavy, st);
     }
 }
 
@@ -265,7 +317,9 @@ k_kcore(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__restri
     __shared__ int s_ok;
     __shared__ uint32_t s_stage[KC_WAVES * KC_STAGE];
     __shared__ uint32_t s_hub[KC_HUBS];
+    __shared__ uint32_t s_row[64];   // KC_HUB_ROWS flags, a wave's width for the ballot
     for (uint32_t j = threadIdx.x; j < KC_HUBS; j += KC_THREADS) s_hub[j] = 0;
+    if (threadIdx.x < 64) s_row[threadIdx.x] = 0;
     __syncthreads();
     const unsigned ln = lane();
     const unsigned long long W = (unsigned long long)gridDim.x * KC_WAVES;
@@ -296,6 +350,7 @@ k_kcore(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__restri
     unsigned long long my_edges = 0;
     __shared__ uint32_t s_dmin, s_dflushed, s_smin;
     __shared__ uint32_t s_wcnt[KC_WAVES];
+    __shared__ unsigned long long s_rd[2];
     __shared__ unsigned long long s_wbase[KC_WAVES];
     // block 0's phase times live in LDS (registers are the scarce resource)
     __shared__ unsigned long long s_prof[KC_PROF + 1];
@@ -357,7 +412,8 @@ k_kcore(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__restri
                     keep[u] = in[u] && c[u] > K;
                     if (keep[u] && c[u] < smin) smin = c[u];
                 }
-                kc_append(put, v, deg, L, cb, &ctl->nlight[c3], &ctl->nheavy[c3], st);
+                uint32_t dg[KC_U] = {KC_NODEG, KC_NODEG, KC_NODEG, KC_NODEG};
+                kc_append(put, v, dg, deg, L, cb, &ctl->nlight[c3], &ctl->nheavy[c3], st);
                 // every read of these KC_PU chunks precedes the writes, which
                 // land at or below the chunks' own positions
 #pragma unroll
@@ -380,11 +436,14 @@ k_kcore(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__restri
         mark(0);
         if (!grid_barrier(&ctl->arrive, &ctl->error, ctl->group, ph++, spin_limit, &s_ok)) break;
         mark(1);
+        unsigned long long nq[2];   // the frontier's list lengths
         {
             const int c3 = r % 3;
-            if (ld_agent(&ctl->nlight[c3]) == 0 && ld_agent(&ctl->nheavy[c3]) == 0) {
+            const unsigned long long *const p[2] = {&ctl->nlight[c3], &ctl->nheavy[c3]};
+            block_read(p, s_rd, nq);
+            if (nq[0] == 0 && nq[1] == 0) {
                 // no vertex at K: no round runs, the kept counts are exact
-                const uint32_t ks = __hip_atomic_load(&ctl->kmin_s[s3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const uint32_t ks = (uint32_t)block_read_min(ctl->kmin_s[s3], ctl->kmin_s[s3], s_rd);
                 if (ks == ~0u) break;              // every vertex peeled
                 K = ks;
                 continue;
@@ -395,8 +454,7 @@ k_kcore(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__restri
         for (;;) {
             const int c3 = r % 3, cb = r & 1;
             const int n3 = (r + 1) % 3, nb = (r + 1) & 1;
-            const unsigned long long nL = ld_agent(&ctl->nlight[c3]);
-            const unsigned long long nH = ld_agent(&ctl->nheavy[c3]);
+            const unsigned long long nL = nq[0], nH = nq[1];
             if (nL == 0 && nH == 0) break;
             if (leader) {
                 // slot (r+2)%3 was last read in round r-1
@@ -404,8 +462,36 @@ k_kcore(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__restri
                 __hip_atomic_store(&ctl->nlight[o3], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 __hip_atomic_store(&ctl->nheavy[o3], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
-            // light rows: one lane per vertex, KC_U edges in flight
-            for (unsigned long long base = wid * 64; base < nL; base += W * 64) {
+            // light rows of a round that leaves most lanes idle otherwise:
+            // KC_SUB lanes per vertex, so that a row is one step (a lane per
+            // vertex takes up to eight, each a chain of a neighbour, a count
+            // and an atomic)
+            const bool few = nL * KC_SUB <= W * 64;
+            // a small round spreads its count-downs thinly over the blocks:
+            // summing them in LDS saves atomics only on the first hubs, and
+            // costs a look at every row of counters touched
+            const uint32_t hubs = few && nH <= W ? KC_FEW_HUBS : KC_HUBS;
+            if (few && wid * (64 / KC_SUB) < nL) {
+                const unsigned long long i = wid * (64 / KC_SUB) + ln / KC_SUB;
+                uint64_t rb = 0, re = 0;
+                if (i < nL) {
+                    const uint32_t v = ld32(&L.light[cb][i]);
+                    rb = index[v];
+                    re = index[v + 1];
+                    if (ln % KC_SUB == 0) my_edges += re - rb;
+                }
+                bool act[KC_U];
+                uint32_t d[KC_U];
+#pragma unroll
+                for (int j = 0; j < KC_U; ++j) {
+                    const uint64_t e = rb + ln % KC_SUB + KC_SUB * j;
+                    act[j] = e < re;
+                    d[j] = act[j] ? nbrs[e] : 0u;
+                }
+                kc_count_down(act, d, K, core, deg, L, nb, &ctl->nlight[n3], &ctl->nheavy[n3], st, s_hub, s_row, hubs, dmin);
+            }
+            // else one lane per vertex, KC_U edges in flight
+            for (unsigned long long base = wid * 64; !few && base < nL; base += W * 64) {
                 const unsigned long long i = base + ln;
                 uint64_t e = 0, e1 = 0;
                 if (i < nL) {
@@ -423,7 +509,7 @@ k_kcore(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__restri
                         d[j] = act[j] ? nbrs[e + j] : 0u;
                     }
                     e = e + KC_U < e1 ? e + KC_U : e1;
-                    kc_count_down(act, d, K, core, deg, L, nb, &ctl->nlight[n3], &ctl->nheavy[n3], st, s_hub, dmin);
+                    kc_count_down(act, d, K, core, deg, L, nb, &ctl->nlight[n3], &ctl->nheavy[n3], st, s_hub, s_row, hubs, dmin);
                 }
             }
             // heavy rows: one wave per slice
@@ -442,9 +528,9 @@ k_kcore(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__restri
                     act[u] = e < ee;
                     d[u] = act[u] ? nbrs[e] : 0u;
                 }
-                kc_count_down(act, d, K, core, deg, L, nb, &ctl->nlight[n3], &ctl->nheavy[n3], st, s_hub, dmin);
+                kc_count_down(act, d, K, core, deg, L, nb, &ctl->nlight[n3], &ctl->nheavy[n3], st, s_hub, s_row, hubs, dmin);
             }
-            kc_hub_flush(s_hub, n, K, core, deg, L, nb, &ctl->nlight[n3], &ctl->nheavy[n3], st, dmin);
+            kc_hub_flush(s_hub, s_row, n, K, core, deg, L, nb, &ctl->nlight[n3], &ctl->nheavy[n3], st, dmin);
             kc_flush_block(st, L.light[nb], &ctl->nlight[n3], s_wcnt, s_wbase);
             // the block's smallest count decremented to above K, sent on when
             // it improved (one global atomic per block and round at most)
@@ -464,6 +550,8 @@ k_kcore(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__restri
                 break;
             }
             mark(3);
+            const unsigned long long *const p[2] = {&ctl->nlight[n3], &ctl->nheavy[n3]};
+            block_read(p, s_rd, nq);
         }
         if (!ok) break;
         ++levels;
@@ -472,9 +560,7 @@ k_kcore(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__restri
             __hip_atomic_store(&ctl->levels, levels, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(&ctl->rounds, r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        const uint32_t ks = __hip_atomic_load(&ctl->kmin_s[s3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const uint32_t kd = __hip_atomic_load(&ctl->kmin_d[s3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const uint32_t kn = ks < kd ? ks : kd;
+        const uint32_t kn = block_read_min(ctl->kmin_s[s3], ctl->kmin_d[s3], s_rd);
         if (kn == ~0u) break;                      // nothing left above K
         K = kn;
     }
@@ -518,7 +604,12 @@ static KcBuf kc_layout(const gpr_graph *g) {
     return b;
 }
 
-static int kc_blocks(unsigned *nblocks) {
+// Blocks of the cooperative grid: by the graph's edges, from 16 to one per CU.
+// A barrier of 256 blocks takes 4-7 us, of 32 2.3, and a small graph's rounds
+// are little more than their barriers (RMAT, 32 / 64 / 128 / 256 blocks: scale
+// 16 3.2 / 3.4 / 3.7 / 4.0 ms, 20 11.6 / 10.1 / 10.3 / 11.3, 24 57 / 38 / 33 /
+// 34, before the small rounds' shorter hub window).
+static int kc_blocks(const gpr_graph *g, unsigned *nblocks) {
     static int per_cu = 0;
     if (!per_cu) GPR_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)k_kcore, KC_THREADS, 0));
     if (per_cu < 1) {
@@ -528,7 +619,9 @@ static int kc_blocks(unsigned *nblocks) {
     const double want = tun().fusion_blocks;
     unsigned cap = (unsigned)(per_cu * num_cus());
     if (cap > GS_GROUP * GS_MAX_GROUPS) cap = GS_GROUP * GS_MAX_GROUPS;
-    const unsigned nb = want >= 1 ? (unsigned)want : (unsigned)num_cus();
+    const uint64_t by_size = g->m < (1ull << 18) ? 16 : g->m < (1ull << 22) ? 32 : g->m < (1ull << 25) ? 64
+                             : g->m < (1ull << 30) ? 128 : (uint64_t)num_cus();
+    const unsigned nb = want >= 1 ? (unsigned)want : (unsigned)std::min<uint64_t>(by_size, num_cus());
     *nblocks = nb < cap ? nb : cap;
     return GPR_OK;
 }
@@ -560,7 +653,7 @@ int kcore_peel(gpr_graph *g, gpr_prop *core, KcStats *st) {
     const double sl = tun().fusion_spin_limit;
     unsigned spin = sl < 0 ? 0u : sl > 2147483647.0 ? 2147483647u : (unsigned)sl;
     unsigned nblocks = 0;
-    GPR_TRY(kc_blocks(&nblocks));
+    GPR_TRY(kc_blocks(g, &nblocks));
     {
         ProfScope ps(g, "kcore");
         uint32_t nn = g->n;

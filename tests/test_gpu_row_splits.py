@@ -74,3 +74,25 @@ def test_component_minima_two_giants():
         G._check(G.lib().gpr_cc_recode(p.h, out.ctypes.data))
         p.destroy()
     assert np.array_equal(out, (np.arange(n) % 2).astype(np.uint32))
+
+
+@pytest.mark.parametrize("n", [700, 5003, 60013])
+@pytest.mark.parametrize("d", [2, 8, 30, 32, 34, 256, 258])
+def test_kcore_regular_rows(n, d):
+    """A ring where every vertex has d neighbours, and a pendant path: rows at
+    the lane and slice limits in rounds of few and of many vertices (one round
+    peels the whole ring)."""
+    v = np.arange(n, dtype=np.uint32)
+    src = [np.repeat(v, d // 2)]
+    dst = [((src[0] + np.tile(np.arange(1, d // 2 + 1), n)) % n).astype(np.uint32)]
+    tail = np.arange(n, n + 40, dtype=np.uint32)
+    src.append(np.concatenate((np.zeros(1, np.uint32), tail[:-1])))
+    dst.append(tail)
+    index, nbrs = O.build_csr(n + 40, np.concatenate(src), np.concatenate(dst))
+    for reorder in (False, True):
+        with G.Graph.from_csr(index, nbrs) as g:
+            if reorder:
+                g.reorder()
+            core, kmax, info = g.kcore()
+        assert kmax == d and (core[:n] == d).all() and (core[n:] == 1).all()
+        assert info.edges == len(nbrs)
