@@ -19,6 +19,7 @@
 // replays without host work.
 #include "internal.hpp"
 #include "device.hpp"
+#include "grid_sync.hpp"
 
 #include <algorithm>
 #include <atomic>
@@ -51,6 +52,9 @@ struct gpr_batch {
 namespace gpr {
 
 constexpr int BCC_THREADS = 1024;
+constexpr int BCC_U = 2;              // 64-edge blocks of a wave in flight
+constexpr uint32_t BCC_HEAVY = 64;    // runs of 64 vertices left to all waves, at most
+constexpr uint32_t BCC_HEAVY_E = 4096;    // which have more edges than this
 constexpr uint32_t BCC_LDS_V = 65536;
 
 template <class P> struct Parents;
@@ -65,6 +69,12 @@ template <> struct Parents<uint16_t> {
         // only used during initialisation and the final pass (one writer)
         uint16_t *h = reinterpret_cast<uint16_t *>(w);
         h[x] = (uint16_t)p;
+    }
+    // x, no root, under q, an ancestor: a 16-bit store, which a hook of the
+    // word's other half (a compare-and-swap of the word) sees or fails on
+    __device__ void halve(uint32_t x, uint32_t q) const {
+        __hip_atomic_store(reinterpret_cast<uint16_t *>(w) + x, (uint16_t)q, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     // hook root r under q if r is still a root; true on success
     __device__ bool hook(uint32_t r, uint32_t q) const {
@@ -86,6 +96,9 @@ template <> struct Parents<uint32_t> {
         return __hip_atomic_load(&w[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __device__ void set(uint32_t x, uint32_t p) const { w[x] = p; }
+    __device__ void halve(uint32_t x, uint32_t q) const {
+        __hip_atomic_store(&w[x], q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     __device__ bool hook(uint32_t r, uint32_t q) const {
         uint32_t exp = r;
         return __hip_atomic_compare_exchange_strong(&w[r], &exp, q, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
@@ -93,12 +106,16 @@ template <> struct Parents<uint32_t> {
     }
 };
 
+// The root above x, halving the path on the way.
 template <class PT>
 __device__ __forceinline__ uint32_t uf_find(const PT &P, uint32_t x) {
     uint32_t p = P.get(x);
     while (p != x) {
+        const uint32_t q = P.get(p);
+        if (q == p) return p;
+        P.halve(x, q);
         x = p;
-        p = P.get(x);
+        p = q;
     }
     return x;
 }
@@ -119,43 +136,98 @@ __device__ __forceinline__ void uf_link(const PT &P, uint32_t u, uint32_t v) {
     }
 }
 
+// What a workgroup's waves share of the graph they work on.
+struct BccShare {
+    uint32_t next;                // the next run of 64 vertices to take
+    uint32_t nheavy;              // (counts past BCC_HEAVY, too)
+    uint32_t heavy[BCC_HEAVY];    // first vertices of those left to all waves
+};
+
+// Links the edges of the 64 vertices from v0 on: each undirected edge once, by
+// its smaller endpoint.  The 64 rows' edges are consecutive and are walked
+// 64 * BCC_U at a step, coalesced and in flight together, whatever the rows'
+// lengths; an edge's row is found among the 64 row starts in the lanes.  Wave
+// `part` of `parts` takes every parts-th step.  With parts == 1, a walk of more
+// than BCC_HEAVY_E edges is refused (false) if `defer`.
+//
 // Edge offsets are clamped to [0, m] and edges that leave the graph are
 // skipped, so a malformed batch in caller memory (gpr_batch_cc_noalloc,
 // which cannot check it on the host) yields wrong labels, never an access
 // outside the arrays.
 template <class PT>
-__device__ void solve_graph(const PT &P, uint32_t base, uint32_t nv, const uint64_t *__restrict__ index,
-                            const uint32_t *__restrict__ nbrs, uint64_t m, uint32_t *labels) {
+__device__ bool link_rows(const PT &P, uint32_t base, uint32_t nv, uint32_t v0, uint32_t part, uint32_t parts,
+                          bool defer, const uint64_t *__restrict__ index, const uint32_t *__restrict__ nbrs,
+                          uint64_t m) {
+    const unsigned ln = lane();
+    const uint32_t rows = nv - v0 < 64 ? nv - v0 : 64;
+    const uint64_t b = min(index[base + v0 + (ln < rows ? ln : rows)], m);
+    const uint64_t b0 = bcast64(b);
+    const uint64_t e0 = min(index[base + v0 + rows], m);
+    const uint32_t len = e0 > b0 ? (uint32_t)min(e0 - b0, (uint64_t)0xfff00000u) : 0u;
+    if (defer && len > BCC_HEAVY_E) return false;
+    // row starts from b0 on, in order (a malformed batch's may not be: a
+    // wrong row, no other access)
+    const uint32_t st = b > b0 ? (uint32_t)min(b - b0, (uint64_t)0xffffffffu) : 0u;
+    const uint32_t *nb = nbrs + b0;
+    for (uint32_t i0 = part * (64 * BCC_U); i0 < len; i0 += parts * (64 * BCC_U)) {
+        uint32_t x[BCC_U], v[BCC_U];
+#pragma unroll
+        for (int k = 0; k < BCC_U; ++k) {
+            const uint32_t i = i0 + k * 64 + ln;
+            x[k] = i < len ? nb[i] - base : 0xffffffffu;
+            v[k] = 0;
+        }
+        // the last row that starts at or before the edge
+#pragma unroll
+        for (int h = 32; h > 0; h >>= 1)
+#pragma unroll
+            for (int k = 0; k < BCC_U; ++k) {
+                const uint32_t t = v[k] + h;   // <= 63
+                if (__shfl(st, t, 64) <= i0 + k * 64 + ln && t < rows) v[k] = t;
+            }
+#pragma unroll
+        for (int k = 0; k < BCC_U; ++k)
+            if (x[k] > v0 + v[k] && x[k] < nv) uf_link(P, v0 + v[k], x[k]);
+    }
+    return true;
+}
+
+// Bound by the chains of LDS reads and by the largest graph: one workgroup a CU
+// (the parents take its LDS) leaves 16 waves to cover the chains, and a queue
+// of few graphs ends with its largest.  Edges are rarely even over the vertices
+// (the first 64 of a power-law graph hold as many as a wave's whole share), so
+// waves take 64 vertices at a time as they come free, and those with more than
+// BCC_HEAVY_E edges wait until all waves walk them together (1024: 2.56 ms
+// instead of 2.20).  2048 graphs (31M vertices, 317M edges) of up to 65536
+// vertices took 4.98 ms with every 1024th vertex to a lane, an edge at a time,
+// 4.25 with the 64-vertex runs dealt out in turn, 2.14 like this; 300 graphs of
+// up to 50000 3.28, 2.58 and 0.98.
+template <class PT>
+__device__ void solve_graph(const PT &P, BccShare &S, uint32_t base, uint32_t nv,
+                            const uint64_t *__restrict__ index, const uint32_t *__restrict__ nbrs, uint64_t m,
+                            uint32_t *labels) {
+    if (threadIdx.x == 0) S.next = S.nheavy = 0;
     for (uint32_t v = threadIdx.x; v < nv; v += BCC_THREADS) P.set(v, v);
     __syncthreads();
-    const unsigned ln = lane();
-    // vertex per lane; rows above 32 edges are walked by the whole wave.
-    // Each undirected edge is linked once, from its smaller endpoint.
-    for (uint32_t v0 = (threadIdx.x & ~63u); v0 < nv; v0 += BCC_THREADS) {
-        const uint32_t v = v0 + ln;
-        uint64_t b = 0, e = 0;
-        if (v < nv) {
-            b = min(index[base + v], m);
-            e = min(max(index[base + v + 1], b), m);
-        }
-        const bool heavy = e - b > 32;
-        if (!heavy)
-            for (uint64_t i = b; i < e; ++i) {
-                const uint32_t u = nbrs[i] - base;
-                if (u > v && u < nv) uf_link(P, v, u);
-            }
-        uint64_t hm = __ballot(heavy);
-        while (hm) {
-            const int L = __ffsll((long long)hm) - 1;
-            hm &= hm - 1;
-            const uint64_t hb = __shfl(b, L, 64), he = __shfl(e, L, 64);
-            const uint32_t hv = v0 + L;
-            for (uint64_t i = hb + ln; i < he; i += 64) {
-                const uint32_t u = nbrs[i] - base;
-                if (u > hv && u < nv) uf_link(P, hv, u);
-            }
-        }
+    // No branch in here is on the lane.  After one, the compiler can know of
+    // the other lanes that they do not fetch, give them the fetch's default
+    // instead of lane 0's value, and loop on it: lanes add 1 or 0 instead, and
+    // store a run all together.
+    const uint32_t one = lane() == 0 ? 1u : 0u;
+    const uint32_t runs = nv / 64 + (nv % 64 != 0);
+    while (true) {
+        const uint32_t run = __builtin_amdgcn_readfirstlane(atomicAdd(&S.next, one));
+        if (run >= runs) break;
+        if (link_rows(P, base, nv, run * 64, 0, 1, true, index, nbrs, m)) continue;
+        const uint32_t at = __builtin_amdgcn_readfirstlane(atomicAdd(&S.nheavy, one));
+        if (at >= BCC_HEAVY) link_rows(P, base, nv, run * 64, 0, 1, false, index, nbrs, m);
+        else S.heavy[at] = run * 64;
     }
+    __syncthreads();
+    const uint32_t nh = min(S.nheavy, BCC_HEAVY);
+    for (uint32_t k = 0; k < nh; ++k)
+        link_rows(P, base, nv, __builtin_amdgcn_readfirstlane(S.heavy[k]),
+                  __builtin_amdgcn_readfirstlane(threadIdx.x / 64), BCC_THREADS / 64, false, index, nbrs, m);
     __syncthreads();
     for (uint32_t v = threadIdx.x; v < nv; v += BCC_THREADS) labels[base + v] = base + uf_find(P, v);
     __syncthreads();
@@ -172,6 +244,7 @@ k_batch_cc(uint32_t count, uint32_t n, const uint32_t *__restrict__ work, const 
            uint32_t *gparent, unsigned int *queue) {
     __shared__ uint32_t words[BCC_LDS_V / 2];
     __shared__ uint32_t s_item;
+    __shared__ BccShare share;
     const uint64_t m = index[n];
     while (true) {
         if (threadIdx.x == 0) s_item = atomicAdd(queue, 1u);
@@ -185,11 +258,11 @@ k_batch_cc(uint32_t count, uint32_t n, const uint32_t *__restrict__ work, const 
         const uint32_t nv = end - base;
         if (nv <= BCC_LDS_V) {
             Parents<uint16_t> P{words};
-            solve_graph(P, base, nv, index, nbrs, m, labels);
+            solve_graph(P, share, base, nv, index, nbrs, m, labels);
         } else {
             // graphs are vertex-disjoint, so each owns its slice of gparent
             Parents<uint32_t> P{gparent + base};
-            solve_graph(P, base, nv, index, nbrs, m, labels);
+            solve_graph(P, share, base, nv, index, nbrs, m, labels);
         }
     }
 }

@@ -96,3 +96,33 @@ def test_kcore_regular_rows(n, d):
             core, kmax, info = g.kcore()
         assert kmax == d and (core[:n] == d).all() and (core[n:] == 1).all()
         assert info.edges == len(nbrs)
+
+
+def ring(n, reach, gap=0):
+    """Vertex i joined to the next `reach` ones around a ring; 0 is a cut-off vertex if gap."""
+    i = np.repeat(np.arange(gap, n), reach)
+    j = gap + (i - gap + np.tile(np.arange(1, reach + 1), n - gap)) % (n - gap)
+    return i.astype(np.uint32), j.astype(np.uint32)
+
+
+def test_batch_cc_row_runs():
+    """Graphs around the 64-vertex runs, the runs left to all waves (more of
+    them than are kept, and single rows of a whole run's edges) and the size
+    whose parents fit on chip."""
+    parts = [(n, ring(n, 1, 1)) for n in (3, 63, 64, 65, 127, 128, 129)]
+    for n in (64, 4096, 4097, 4098, 65536, 65537):   # stars: rows of 63 .. 65536 edges
+        hub = n - 1 if n % 2 else 0
+        leaf = np.delete(np.arange(n, dtype=np.uint32), hub)
+        parts.append((n, (np.full(n - 1, hub, np.uint32), leaf)))
+    parts.append((5000, ring(5000, 40, 1)))          # 79 runs of 5120 edges
+    parts.append((2, (np.zeros(0, np.uint32), np.zeros(0, np.uint32))))
+    voff, src, dst, n = [0], [], [], 0
+    for k, (a, b) in parts:
+        src.append(n + a)
+        dst.append(n + b)
+        n += k
+        voff.append(n)
+    index, nbrs = O.build_csr(n, np.concatenate(src).astype(np.uint32), np.concatenate(dst).astype(np.uint32))
+    with G.Batch.from_csr(index, nbrs, np.array(voff, np.uint32)) as b:
+        lab, _ = b.cc()
+    assert np.array_equal(lab, O.cc_labels(index, nbrs))
