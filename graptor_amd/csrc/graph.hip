@@ -163,6 +163,7 @@ static void graph_free(gpr_graph *g) {
     if (g->rev1) hipEventDestroy(g->rev1);
     for (void *p : g->pool_list) dev_free(p);
     for (void *p : g->pool_bits) dev_free(p);
+    g->pool->close();
     if (g->stream) hipStreamDestroy(g->stream);
     delete g;
 }
@@ -172,6 +173,7 @@ static int new_graph(uint32_t n, uint64_t m, int symmetric, gpr_graph **out) {
     g->n = n;
     g->m = m;
     g->symmetric = symmetric ? 1 : 0;
+    g->pool->bound(n);
     hipError_t e = hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking);
     if (e != hipSuccess) {
         set_error("hipStreamCreate: %s", hipGetErrorString(e));
@@ -501,12 +503,14 @@ extern "C" int gpr_prop_create(gpr_graph *g, int dtype, gpr_prop **out) {
     p->g = g;
     p->dtype = dtype;
     p->elem = elem;
-    int r = dev_alloc(&p->d, elem * std::max<uint32_t>(g->n, 1), "vertex property");
+    p->pool = g->pool;
+    int r = p->pool->take(&p->d, elem * std::max<uint32_t>(g->n, 1), "vertex property");
     if (r) {
         delete p;
         return r;
     }
-    GPR_HIP(hipMemsetAsync(p->d, 0, elem * std::max<uint32_t>(g->n, 1), g->stream));
+    p->bytes = elem * std::max<uint32_t>(g->n, 1);
+    GPR_HIP(hipMemsetAsync(p->d, 0, p->bytes, g->stream));
     *out = p;
     return GPR_OK;
 }
@@ -599,8 +603,8 @@ extern "C" int gpr_graph_original_id(gpr_graph *g, uint32_t internal, uint32_t *
 
 extern "C" int gpr_prop_destroy(gpr_prop *p) {
     if (!p) return GPR_E_INVAL;
-    if (p->g && p->g->stream) hipStreamSynchronize(p->g->stream);
-    dev_free(p->d);
+    if (p->pool->open()) hipStreamSynchronize(p->g->stream);    // else the graph is gone, its work done
+    p->pool->give(p->d, p->bytes);
     delete p;
     return GPR_OK;
 }

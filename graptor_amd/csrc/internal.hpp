@@ -14,9 +14,12 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <algorithm>
+#include <map>
+#include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
-#include <map>
 
 #include "../../include/gpr.h"
 
@@ -58,6 +61,37 @@ void set_error(const char *fmt, ...);
 
 int dev_alloc(void **p, size_t bytes, const char *what);
 void dev_free(void *p);
+
+// Device blocks of one graph's runs (properties, 64-source BFS levels), kept
+// for its next run: a run makes and drops the same sizes every time, and
+// hipFree waits for the whole device (0.1 - 0.3 ms each for tens of MB;
+// hipMalloc 0.02 - 0.1).  A block is given back by size; the oldest go when
+// more than `cap` bytes or POOL_BLOCKS blocks are held, all of them when the
+// graph goes, and when an allocation of any graph fails.  The graph's stream
+// orders a block's next use behind its last one.
+constexpr size_t POOL_BLOCKS = 32;
+constexpr size_t POOL_BYTES = 256u << 20;    // held by a graph at most, or
+constexpr size_t POOL_VERTEX_BYTES = 64;     // this a vertex where it is more
+struct BufPool {
+    BufPool();
+    ~BufPool();
+    int take(void **p, size_t bytes, const char *what);
+    void give(void *p, size_t bytes);
+    bool trim();      // frees all that it holds; false if that was nothing
+    void close();     // the graph goes: trims, and keeps nothing from now on
+    bool open() {
+        std::lock_guard<std::mutex> lk(mu);
+        return !closed;
+    }
+    void bound(uint32_t n) { cap = std::max(POOL_BYTES, POOL_VERTEX_BYTES * n); }
+
+  private:
+    struct Block { size_t bytes; void *p; };
+    std::mutex mu;
+    std::vector<Block> blocks;    // oldest first
+    size_t held = 0, cap = POOL_BYTES;
+    bool closed = false;
+};
 
 // ---- runtime tunables (set by the autotuner through gpr_tune_set) --------
 struct Tunables {
@@ -240,6 +274,7 @@ struct gpr_graph {
     hipEvent_t rev0 = nullptr, rev1 = nullptr;  // per application run
     // recycled frontier buffers (avoid hipMalloc per iteration)
     std::vector<void *> pool_list, pool_bits;
+    std::shared_ptr<gpr::BufPool> pool = std::make_shared<gpr::BufPool>();    // its properties hold it too
     // learned policy state of the current run
     float *pol_params = nullptr;    // device copy of the network (null: none)
     float pol_margin = 0.f;         // gate margin loaded with the network
@@ -280,8 +315,10 @@ struct gpr_graph {
 
 struct gpr_prop {
     gpr_graph *g = nullptr;
+    std::shared_ptr<gpr::BufPool> pool;
     int dtype = GPR_U32;
     size_t elem = 4;
+    size_t bytes = 0;
     void *d = nullptr;
 };
 

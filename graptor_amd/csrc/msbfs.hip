@@ -315,14 +315,21 @@ extern "C" int gpr_msbfs(gpr_graph *g, const uint32_t *sources, int k, const gpr
     uint64_t *seen = nullptr, *cur = nullptr, *nxt = nullptr;
     int r = GPR_OK;
     gpr_run_info inf = {};
+    struct { void *p; size_t bytes; } used[8];
+    int nused = 0;
+    auto take = [&](void **p, size_t bytes, const char *what) {
+        const int e = g->pool->take(p, bytes, what);
+        if (e == GPR_OK) used[nused++] = {*p, bytes};
+        return e;
+    };
     do {
-        if ((r = dev_alloc((void **)&lev, 4ull * k * n, "msbfs levels"))) break;
-        if ((r = dev_alloc((void **)&seen, 8ull * n, "msbfs seen"))) break;
-        if ((r = dev_alloc((void **)&cur, 8ull * n, "msbfs frontier"))) break;
-        if ((r = dev_alloc((void **)&nxt, 8ull * n, "msbfs next"))) break;
-        if ((r = dev_alloc((void **)&list[0], 4ull * n, "msbfs list"))) break;
-        if ((r = dev_alloc((void **)&list[1], 4ull * n, "msbfs list"))) break;
-        if ((r = dev_alloc((void **)&src, 4ull * k, "msbfs sources"))) break;
+        if ((r = take((void **)&lev, 4ull * k * n, "msbfs levels"))) break;
+        if ((r = take((void **)&seen, 8ull * n, "msbfs seen"))) break;
+        if ((r = take((void **)&cur, 8ull * n, "msbfs frontier"))) break;
+        if ((r = take((void **)&nxt, 8ull * n, "msbfs next"))) break;
+        if ((r = take((void **)&list[0], 4ull * n, "msbfs list"))) break;
+        if ((r = take((void **)&list[1], 4ull * n, "msbfs list"))) break;
+        if ((r = take((void **)&src, 4ull * k, "msbfs sources"))) break;
         std::vector<uint32_t> s(sources, sources + k);
         std::vector<uint32_t> uniq(s);
         std::sort(uniq.begin(), uniq.end());
@@ -385,7 +392,7 @@ extern "C" int gpr_msbfs(gpr_graph *g, const uint32_t *sources, int k, const gpr
         if (levels) {
             // MS_OUT_J sources at a time through one staging buffer
             uint32_t *tmp = nullptr;
-            if ((r = dev_alloc((void **)&tmp, 4ull * std::min<uint32_t>(k, MS_OUT_J) * n, "msbfs levels"))) break;
+            if ((r = take((void **)&tmp, 4ull * std::min<uint32_t>(k, MS_OUT_J) * n, "msbfs levels"))) break;
             hipError_t e = hipSuccess;
             for (uint32_t j0 = 0; j0 < (uint32_t)k && e == hipSuccess; j0 += MS_OUT_J) {
                 const uint32_t js = std::min<uint32_t>(MS_OUT_J, k - j0);
@@ -394,18 +401,11 @@ extern "C" int gpr_msbfs(gpr_graph *g, const uint32_t *sources, int k, const gpr
                 e = hipMemcpyAsync(levels + (uint64_t)j0 * n, tmp, 4ull * js * n, hipMemcpyDeviceToHost, g->stream);
             }
             if (e == hipSuccess) e = hipStreamSynchronize(g->stream);
-            dev_free(tmp);
             if (e != hipSuccess) { r = GPR_E_HIP; break; }
         }
     } while (0);
     if (r == GPR_E_HIP) set_error("msbfs: HIP error %s", hipGetErrorString(hipGetLastError()));
-    dev_free(lev);
-    dev_free(seen);
-    dev_free(cur);
-    dev_free(nxt);
-    dev_free(list[0]);
-    dev_free(list[1]);
-    dev_free(src);
+    while (nused) g->pool->give(used[nused - 1].p, used[nused - 1].bytes), --nused;
     if (r == GPR_OK && info) *info = inf;
     return r;
 }

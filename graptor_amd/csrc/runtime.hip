@@ -19,10 +19,87 @@ void set_error(const char *fmt, ...) {
     va_end(ap);
 }
 
+// Every graph's pool; never destroyed, as the last pool may go after it.
+struct PoolList {
+    std::mutex mu;
+    std::vector<BufPool *> pools;
+};
+static PoolList &pool_list() {
+    static PoolList *l = new PoolList();
+    return *l;
+}
+static bool trim_pools() {
+    PoolList &l = pool_list();
+    std::lock_guard<std::mutex> lk(l.mu);
+    bool any = false;
+    for (BufPool *p : l.pools) any = p->trim() || any;
+    return any;
+}
+
+BufPool::BufPool() {
+    blocks.reserve(POOL_BLOCKS + 1);
+    PoolList &l = pool_list();
+    std::lock_guard<std::mutex> lk(l.mu);
+    l.pools.push_back(this);
+}
+BufPool::~BufPool() {
+    PoolList &l = pool_list();
+    {
+        std::lock_guard<std::mutex> lk(l.mu);
+        l.pools.erase(std::find(l.pools.begin(), l.pools.end(), this));
+    }
+    trim();
+}
+int BufPool::take(void **p, size_t bytes, const char *what) {
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        for (size_t i = blocks.size(); i-- > 0;)
+            if (blocks[i].bytes == bytes) {
+                *p = blocks[i].p;
+                held -= bytes;
+                blocks.erase(blocks.begin() + i);
+                return GPR_OK;
+            }
+    }
+    return dev_alloc(p, bytes, what);
+}
+void BufPool::give(void *p, size_t bytes) {
+    if (!p) return;
+    std::lock_guard<std::mutex> lk(mu);
+    if (closed || bytes > cap) {
+        dev_free(p);
+        return;
+    }
+    while (!blocks.empty() && (held + bytes > cap || blocks.size() >= POOL_BLOCKS)) {
+        held -= blocks.front().bytes;
+        dev_free(blocks.front().p);
+        blocks.erase(blocks.begin());
+    }
+    blocks.push_back({bytes, p});
+    held += bytes;
+}
+bool BufPool::trim() {
+    std::lock_guard<std::mutex> lk(mu);
+    const bool any = !blocks.empty();
+    for (const Block &b : blocks) dev_free(b.p);
+    blocks.clear();
+    held = 0;
+    return any;
+}
+void BufPool::close() {
+    trim();
+    std::lock_guard<std::mutex> lk(mu);
+    closed = true;
+}
+
 int dev_alloc(void **p, size_t bytes, const char *what) {
     *p = nullptr;
     if (bytes == 0) bytes = 256;
     hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && trim_pools()) {
+        (void)hipGetLastError();
+        e = hipMalloc(p, bytes);
+    }
     if (e != hipSuccess) {
         set_error("hipMalloc(%zu) for %s failed: %s", bytes, what, hipGetErrorString(e));
         *p = nullptr;
