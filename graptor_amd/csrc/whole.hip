@@ -430,7 +430,8 @@ k_uf_link(uint32_t nbuckets, const uint32_t *__restrict__ bucket, const uint64_t
 
 // Every vertex under its root; with minorig, the components' smallest
 // original IDs at the roots too, with out the roots as results.  A launch of
-// its own, so no root is hooked meanwhile; a parent rewritten is an ancestor.
+// its own, so no root is hooked meanwhile.  A few parents may still be inner
+// ancestors afterwards: halving stores of other threads that come late.
 __global__ void __launch_bounds__(LF_THREADS)
 k_uf_flatten(uint32_t n, uint32_t *parent, const uint32_t *__restrict__ order, uint32_t *minorig, uint32_t *out) {
     constexpr int WG = __HIP_MEMORY_SCOPE_WORKGROUP;
@@ -444,11 +445,20 @@ k_uf_flatten(uint32_t n, uint32_t *parent, const uint32_t *__restrict__ order, u
     if (minorig) f.finish(minorig);
 }
 
+// The root above v in a forest at rest: nearly always its parent.
+__device__ __forceinline__ uint32_t uf_top(const uint32_t *__restrict__ parent, uint32_t v) {
+    uint32_t p = parent[v];
+    while (p != v) {
+        v = p;
+        p = parent[v];
+    }
+    return v;
+}
 __global__ void __launch_bounds__(UF_THREADS)
 k_uf_out(uint32_t n, const uint32_t *__restrict__ parent, const uint32_t *__restrict__ perm,
          const uint32_t *__restrict__ minorig, uint32_t *out) {
     for (uint32_t o = blockIdx.x * UF_THREADS + threadIdx.x; o < n; o += gridDim.x * UF_THREADS)
-        out[o] = minorig[parent[perm[o]]];
+        out[o] = minorig[uf_top(parent, perm[o])];
 }
 
 // ---- host side ------------------------------------------------------------------

@@ -113,3 +113,15 @@ def test_whole_cc(name, reorder):
             assert info.edges == len(nbrs)
         none, _ = g.ccv(download=False)
         assert none is None
+
+
+@pytest.mark.parametrize("n", [30011, 300007])
+def test_whole_cc_long_paths_relabelled(n):
+    """Long paths into deep trees: late path-halving stores leave parents that are not yet roots."""
+    k = np.arange(3 * n, dtype=np.uint64)
+    index, nbrs = O.build_csr(n, (k * 7919 % n).astype(np.uint32), (k * k * 31 % n).astype(np.uint32))
+    want = O.cc_labels(index, nbrs)
+    with G.Graph.from_csr(index, nbrs) as g:
+        g.reorder()
+        for _ in range(10):
+            assert np.array_equal(g.ccv()[0], want)
