@@ -30,6 +30,10 @@
 
 #include <rocprim/rocprim.hpp>
 
+namespace gpr {
+struct BatchDest { uint32_t *labels; };
+} // namespace gpr
+
 struct gpr_batch {
     uint32_t count = 0;
     uint32_t n = 0;
@@ -42,6 +46,9 @@ struct gpr_batch {
     uint32_t *gparent = nullptr;   // scratch for graphs above LDS capacity
     uint32_t max_nv = 0;
     unsigned int *queue = nullptr;
+    gpr::BatchDest *dest = nullptr;        // device
+    uint32_t **hdest = nullptr;            // pinned: where this run's labels go
+    uint32_t **hdest_dev = nullptr;
     hipStream_t stream = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -233,15 +240,19 @@ __device__ void solve_graph(const PT &P, BccShare &S, uint32_t base, uint32_t nv
     __syncthreads();
 }
 
-__global__ void k_batch_reset(unsigned int *queue) {
-    if (threadIdx.x == 0) *queue = 0;
+__global__ void k_batch_reset(unsigned int *queue, BatchDest *dest, uint32_t *const volatile *host_dest) {
+    if (threadIdx.x == 0) {
+        *queue = 0;
+        if (dest) dest->labels = *host_dest;
+    }
 }
 
 // work: queue order of the graphs (null: index order)
 __global__ void __launch_bounds__(BCC_THREADS)
 k_batch_cc(uint32_t count, uint32_t n, const uint32_t *__restrict__ work, const uint32_t *__restrict__ voff,
            const uint64_t *__restrict__ index, const uint32_t *__restrict__ nbrs, uint32_t *labels,
-           uint32_t *gparent, unsigned int *queue) {
+           uint32_t *gparent, unsigned int *queue, const BatchDest *dest) {
+    if (dest) labels = dest->labels;
     __shared__ uint32_t words[BCC_LDS_V / 2];
     __shared__ uint32_t s_item;
     __shared__ BccShare share;
@@ -334,6 +345,8 @@ static void batch_free(gpr_batch *b) {
     dev_free(b->labels);
     dev_free(b->gparent);
     dev_free(b->queue);
+    dev_free(b->dest);
+    if (b->hdest) (void)hipHostFree(b->hdest);
     if (b->e0) (void)hipEventDestroy(b->e0);
     if (b->e1) (void)hipEventDestroy(b->e1);
     if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -358,6 +371,9 @@ static int batch_finish(gpr_batch *b) {
     // global parents only for graphs above the LDS capacity
     GPR_TRY(dev_alloc((void **)&b->gparent, b->max_nv > BCC_LDS_V ? 4ull * b->n : 64, "batch parents"));
     GPR_TRY(dev_alloc((void **)&b->queue, 64, "batch queue"));
+    GPR_TRY(dev_alloc((void **)&b->dest, sizeof(BatchDest), "batch destination"));
+    GPR_HIP(hipHostMalloc((void **)&b->hdest, sizeof(uint32_t *), hipHostMallocMapped | hipHostMallocCoherent));
+    GPR_HIP(hipHostGetDevicePointer((void **)&b->hdest_dev, b->hdest, 0));
     GPR_HIP(hipMemset(b->queue, 0, 64));
     GPR_HIP(hipEventCreate(&b->e0));
     GPR_HIP(hipEventCreate(&b->e1));
@@ -443,9 +459,10 @@ extern "C" int gpr_batch_cc_noalloc(const uint64_t *d_index, const uint32_t *d_n
     const int cus = noalloc_dev[dev].cus.load(std::memory_order_relaxed);
     hipStream_t st = (hipStream_t)stream;
     const unsigned grid = (unsigned)std::max(1, std::min<int>(cus, (int)std::min<uint32_t>(count, 1u << 30)));
-    hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, st, (unsigned int *)sp);
+    hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, st, (unsigned int *)sp,
+                       (BatchDest *)nullptr, (uint32_t *const volatile *)nullptr);
     hipLaunchKernelGGL(k_batch_cc, dim3(grid), dim3(BCC_THREADS), 0, st, count, n, (const uint32_t *)nullptr, d_voff,
-                       d_index, d_nbrs, d_labels, sp + NOALLOC_PARENTS, (unsigned int *)sp);
+                       d_index, d_nbrs, d_labels, sp + NOALLOC_PARENTS, (unsigned int *)sp, (const BatchDest *)nullptr);
     GPR_HIP(hipGetLastError());
     return GPR_OK;
 }
@@ -603,9 +620,10 @@ extern "C" int gpr_batch_cc(gpr_batch *b, uint32_t *labels, gpr_run_info *info) 
         GPR_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
         const unsigned grid = (unsigned)std::max(1, std::min<int>(cus, (int)b->count));
         GPR_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-        hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, b->stream, b->queue);
+        hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, b->stream, b->queue, b->dest,
+                           (uint32_t *const volatile *)b->hdest_dev);
         hipLaunchKernelGGL(k_batch_cc, dim3(grid), dim3(BCC_THREADS), 0, b->stream, b->count, b->n, b->work, b->voff,
-                           b->index, b->nbrs, b->labels, b->gparent, b->queue);
+                           b->index, b->nbrs, b->labels, b->gparent, b->queue, (const BatchDest *)b->dest);
         hipError_t ce = hipStreamEndCapture(b->stream, &b->graph);
         if (ce != hipSuccess) {
             set_error("graph capture: %s", hipGetErrorString(ce));
@@ -613,13 +631,17 @@ extern "C" int gpr_batch_cc(gpr_batch *b, uint32_t *labels, gpr_run_info *info) 
         }
         GPR_HIP(hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
     }
+    // labels of a finished graph go over the link while others are worked on:
+    // 2048 graphs of up to 65536 vertices (123 MB of labels) 4.37 -> 3.03 ms
+    uint32_t *const target = (uint32_t *)host_target(labels, 4ull * b->n);
+    *b->hdest = target ? target : b->labels;
     GPR_HIP(hipEventRecord(b->e0, b->stream));
     GPR_HIP(hipGraphLaunch(b->exec, b->stream));
     GPR_HIP(hipEventRecord(b->e1, b->stream));
     GPR_HIP(hipEventSynchronize(b->e1));
     float ms = 0.f;
     GPR_HIP(hipEventElapsedTime(&ms, b->e0, b->e1));
-    if (labels && b->n) GPR_HIP(hipMemcpy(labels, b->labels, 4ull * b->n, hipMemcpyDeviceToHost));
+    if (labels && b->n && !target) GPR_HIP(hipMemcpy(labels, b->labels, 4ull * b->n, hipMemcpyDeviceToHost));
     if (info) {
         gpr_run_info r = {};
         r.iters = 1;

@@ -62,6 +62,10 @@ void set_error(const char *fmt, ...);
 int dev_alloc(void **p, size_t bytes, const char *what);
 void dev_free(void *p);
 
+// Where the device can write a caller's result of `bytes` bytes: the device
+// address of pinned host memory that holds all of it, else nullptr.
+void *host_target(void *host, size_t bytes);
+
 // Device blocks of one graph's runs (properties, 64-source BFS levels), kept
 // for its next run: a run makes and drops the same sizes every time, and
 // hipFree waits for the whole device (0.1 - 0.3 ms each for tens of MB;

@@ -19,6 +19,20 @@ void set_error(const char *fmt, ...) {
     va_end(ap);
 }
 
+void *host_target(void *host, size_t bytes) {
+    hipPointerAttribute_t a = {};
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (!host || !bytes) return nullptr;
+    if (hipPointerGetAttributes(&a, host) != hipSuccess || a.type != hipMemoryTypeHost || !a.devicePointer ||
+        hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)a.devicePointer) != hipSuccess) {
+        (void)hipGetLastError();    // pageable memory is an error to some of these
+        return nullptr;
+    }
+    const char *d = (const char *)a.devicePointer, *b = (const char *)base;
+    return d >= b && bytes <= size && (size_t)(d - b) <= size - bytes ? a.devicePointer : nullptr;
+}
+
 // Every graph's pool; never destroyed, as the last pool may go after it.
 struct PoolList {
     std::mutex mu;

@@ -510,9 +510,9 @@ static int whole_ensure(gpr_graph *g, const WholeBuf &b) {
 }
 // Waits for the stream; the n results at dev (the staging memory or the
 // device) into host, when asked for.
-static int whole_results(gpr_graph *g, const uint32_t *dev, uint32_t *host) {
-    const bool staged = dev == g->wstage_dev;
-    if (host && !staged) GPR_HIP(hipMemcpyAsync(host, dev, 4ull * g->n, hipMemcpyDeviceToHost, g->stream));
+static int whole_results(gpr_graph *g, const uint32_t *dev, uint32_t *host, bool direct) {
+    const bool staged = !direct && dev == g->wstage_dev;
+    if (host && !staged && !direct) GPR_HIP(hipMemcpyAsync(host, dev, 4ull * g->n, hipMemcpyDeviceToHost, g->stream));
     GPR_HIP(hipStreamSynchronize(g->stream));
     if (host && staged) std::memcpy(host, g->wstage, 4ull * g->n);
     return GPR_OK;
@@ -562,12 +562,13 @@ int whole_bfs(gpr_graph *g, uint32_t start, float threshold_pct, uint32_t *level
         }
     }
     stream_time_mark(g);
-    uint32_t *out = g->wstage ? g->wstage_dev : (uint32_t *)(base + b.out);
+    uint32_t *const target = (uint32_t *)host_target(levels, 4ull * n);
+    uint32_t *out = target ? target : g->wstage ? g->wstage_dev : (uint32_t *)(base + b.out);
     if (levels)
         hipLaunchKernelGGL(k_wb_out, dim3(grid_for(n, WB_THREADS, 1024)), dim3(WB_THREADS), 0, g->stream, n, level,
                            perm, out);
     GPR_HIP(hipGetLastError());
-    GPR_TRY(whole_results(g, out, levels));
+    GPR_TRY(whole_results(g, out, levels, target));
     info->ms = stream_time_read_ms(g);
     info->iters = (int)h->steps;
     info->push_iters = (int)h->pushes;
@@ -583,7 +584,8 @@ int whole_cc(gpr_graph *g, uint32_t *labels, gpr_run_info *info) {
     uint32_t *parent = (uint32_t *)base;
     // the recode (labels asked for, vertices relabelled): minima by original ID
     uint32_t *minorig = labels && g->order ? (uint32_t *)(base + b.light[0]) : nullptr;
-    uint32_t *out = !labels ? nullptr : g->wstage ? g->wstage_dev : (uint32_t *)(base + b.out);
+    uint32_t *const target = (uint32_t *)host_target(labels, 4ull * n);
+    uint32_t *out = !labels ? nullptr : target ? target : g->wstage ? g->wstage_dev : (uint32_t *)(base + b.out);
     const unsigned grid = grid_for(n, UF_THREADS, 4096);
     stream_time_ms(g, true);
     hipLaunchKernelGGL(k_uf_init, dim3(grid), dim3(UF_THREADS), 0, g->stream, n, g->index, g->nbrs, parent, minorig);
@@ -608,7 +610,7 @@ int whole_cc(gpr_graph *g, uint32_t *labels, gpr_run_info *info) {
         hipLaunchKernelGGL(k_uf_out, dim3(grid), dim3(UF_THREADS), 0, g->stream, n, parent, g->perm, minorig, out);
     GPR_HIP(hipGetLastError());
     stream_time_mark(g);
-    GPR_TRY(whole_results(g, out, labels));
+    GPR_TRY(whole_results(g, out, labels, target));
     info->ms = stream_time_read_ms(g);
     // one step, over every edge
     info->iters = 1;

@@ -405,7 +405,8 @@ int gpr_batch_info(const gpr_batch *b, uint32_t *count, uint32_t *n,
 int gpr_batch_download(const gpr_batch *b, uint64_t *index, uint32_t *nbrs,
                        uint32_t *voff);
 /* labels[v] = minimum global vertex ID of v's component.  Runs as one
- * hipGraph launch (queue reset + persistent kernel). */
+ * hipGraph launch (queue reset + persistent kernel).  Labels in pinned host
+ * memory are written by that kernel (info->ms then holds their transfer). */
 int gpr_batch_cc(gpr_batch *b, uint32_t *labels, gpr_run_info *info);
 int gpr_batch_destroy(gpr_batch *b);
 /* gpr_batch_cc on a batch in caller-owned device memory, allocating nothing
