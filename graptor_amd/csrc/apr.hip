@@ -43,6 +43,7 @@ constexpr int AP_TILE = AP_THREADS * AP_ITEMS;
 constexpr int AP_LDS = AP_TILE + 1;
 constexpr int AT_THREADS = 256;
 constexpr int AT_WAVES = AT_THREADS / 64;
+constexpr int AT_U = 4;                // bitmap words (64 vertices each) of a wave in flight
 constexpr unsigned AT_MAX_BLOCKS = 2048;
 
 // The value the pull adds for source s: the stored contribution, decoded.
@@ -160,37 +161,49 @@ k_apr_tail(uint32_t n, const float *__restrict__ y, float factor, float dampen, 
     const uint32_t nwv = gridDim.x * AT_WAVES;
     double sl1 = 0.0, sx = 0.0;
     uint64_t ce = 0, cv = 0;
-    for (uint32_t w = blockIdx.x * AT_WAVES + wv; w < words; w += nwv) {
-        const uint32_t v = w * 64 + lane();
-        bool a = false;
-        if (v < n) {
-            const float z = y[v] * factor;
-            float xv = x[v], dl;
-            if (FIRST) {
-                // :484-505: delta = d*z + (1-d)/n; x += delta; delta -= 1/n
-                dl = dampen * z + cst;
-                xv = xv + dl;
-                x[v] = xv;
-                dl = dl - ninv;
-                a = fabsf(dl) > eps2 * xv;
-            } else {
-                // :535-557 / :590-612: delta = z*d; x += delta where active
-                dl = z * dampen;
-                a = fabsf(dl) > eps2 * xv;
-                if (a) {
+    for (uint64_t w0 = blockIdx.x * AT_WAVES + wv; w0 < words; w0 += (uint64_t)nwv * AT_U) {
+        float yv[AT_U], xs[AT_U];
+#pragma unroll
+        for (int u = 0; u < AT_U; ++u) {
+            const uint64_t i = (w0 + (uint64_t)u * nwv) * 64 + lane(), v = i < n ? i : 0;
+            yv[u] = y[v];
+            xs[u] = x[v];
+        }
+#pragma unroll
+        for (int u = 0; u < AT_U; ++u) {
+            const uint64_t w = w0 + (uint64_t)u * nwv;
+            if (w >= words) break;
+            const uint64_t v = w * 64 + lane();
+            bool a = false;
+            if (v < n) {
+                const float z = yv[u] * factor;
+                float xv = xs[u], dl;
+                if (FIRST) {
+                    // :484-505: delta = d*z + (1-d)/n; x += delta; delta -= 1/n
+                    dl = dampen * z + cst;
                     xv = xv + dl;
                     x[v] = xv;
+                    dl = dl - ninv;
+                    a = fabsf(dl) > eps2 * xv;
+                } else {
+                    // :535-557 / :590-612: delta = z*d; x += delta where active
+                    dl = z * dampen;
+                    a = fabsf(dl) > eps2 * xv;
+                    if (a) {
+                        xv = xv + dl;
+                        x[v] = xv;
+                    }
                 }
+                delta[v] = dl;
+                sl1 += (double)fabsf(dl);
+                sx += (double)fabsf(xv);
+                if (a) ce += deg[v];
             }
-            delta[v] = dl;
-            sl1 += (double)fabsf(dl);
-            sx += (double)fabsf(xv);
-            if (a) ce += deg[v];
-        }
-        const uint64_t b = __ballot(a);
-        if (lane() == 0) {
-            bits[w] = b;
-            cv += (uint64_t)__popcll(b);
+            const uint64_t b = __ballot(a);
+            if (lane() == 0) {
+                bits[w] = b;
+                cv += (uint64_t)__popcll(b);
+            }
         }
     }
     sl1 = wave_sum(sl1);
@@ -221,18 +234,10 @@ k_apr_tail(uint32_t n, const float *__restrict__ y, float factor, float dampen, 
     // the last workgroup adds the partials in a fixed order, into the host's
     // line
     if (!last_workgroup(ticket, &s_last)) return;
-    sl1 = sx = 0.0;
-    cv = ce = 0;
-    for (uint32_t i = threadIdx.x; i < gridDim.x; i += AT_THREADS) {
-        sl1 += ld_part(&part[2 * i]);
-        sx += ld_part(&part[2 * i + 1]);
-        cv += ld_part(&cpart[2 * i]);
-        ce += ld_part(&cpart[2 * i + 1]);
-    }
-    sl1 = block_sum(sl1, r1);
-    sx = block_sum(sx, r2);
-    cv = block_sum(cv, r3);
-    ce = block_sum(ce, r4);
+    sl1 = block_sum(part_sum<AT_THREADS, 2>(part, gridDim.x), r1);
+    sx = block_sum(part_sum<AT_THREADS, 2>(part + 1, gridDim.x), r2);
+    cv = block_sum(part_sum<AT_THREADS, 2>(cpart, gridDim.x), r3);
+    ce = block_sum(part_sum<AT_THREADS, 2>(cpart + 1, gridDim.x), r4);
     if (threadIdx.x == 0) {
         h->l1 = sl1;
         h->sum_abs = sx;

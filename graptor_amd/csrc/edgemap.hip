@@ -38,7 +38,8 @@ constexpr int SCAN_THREADS = SCAN_BLOCK / 4;
 
 __global__ void __launch_bounds__(SCAN_THREADS)
 k_scan_local(const uint32_t *__restrict__ list, uint32_t k, const uint32_t *__restrict__ deg,
-             uint64_t *__restrict__ pos, uint64_t *__restrict__ btot) {
+             uint64_t *__restrict__ pos, uint64_t *btot, unsigned int *ticket) {
+    static_assert(sizeof(uint64_t) == sizeof(unsigned long long), "the totals are scanned as such");
     __shared__ uint64_t wsum[SCAN_THREADS / 64];
     uint32_t base = blockIdx.x * SCAN_BLOCK + threadIdx.x * 4;
     uint64_t d[4];
@@ -62,39 +63,18 @@ k_scan_local(const uint32_t *__restrict__ list, uint32_t k, const uint32_t *__re
         if (i < k) pos[i] = run;
         run += d[j];
     }
-    if (threadIdx.x == SCAN_THREADS - 1) {
-        if (gridDim.x == 1) {
-            // one block: its exclusive offset 0 and the total, as the top
-            // scan would write them (which then need not run)
-            btot[0] = 0;
-            btot[1] = off + inc;
-        } else {
-            btot[blockIdx.x] = off + inc;
-        }
+    // the last workgroup scans the totals in place; total at [gridDim.x]
+    __shared__ int s_last;
+    unsigned long long *bt = (unsigned long long *)btot, total = 0;
+    for (unsigned j = 0; j < SCAN_THREADS / 64; ++j) total += wsum[j];
+    if (gridDim.x == 1) {
+        if (threadIdx.x == 0) bt[0] = 0;
+    } else {
+        if (threadIdx.x == 0) st_part(&bt[blockIdx.x], total);
+        if (!last_workgroup(ticket, &s_last)) return;
+        total = part_excl_scan<SCAN_THREADS>(bt, gridDim.x);
     }
-}
-
-// Exclusive scan of the block totals in place; total written to a[count].
-__global__ void __launch_bounds__(1024) k_scan_top(uint64_t *a, uint32_t count) {
-    __shared__ uint64_t carry;
-    __shared__ uint64_t wsum[16];
-    if (threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    for (uint32_t b = 0; b < count; b += blockDim.x) {
-        uint32_t i = b + threadIdx.x;
-        uint64_t v = i < count ? a[i] : 0;
-        uint64_t inc = wave_incl_scan(v);
-        unsigned w = threadIdx.x / 64;
-        if (lane() == 63) wsum[w] = inc;
-        __syncthreads();
-        uint64_t off = carry;
-        for (unsigned j = 0; j < w; ++j) off += wsum[j];
-        if (i < count) a[i] = off + inc - v;
-        __syncthreads();
-        if (threadIdx.x == blockDim.x - 1) carry = off + inc;
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) a[count] = carry;
+    if (threadIdx.x == 0) bt[gridDim.x] = total;
 }
 
 template <int RELAX> __device__ __forceinline__ uint32_t relax_val(uint32_t ps) {
@@ -547,9 +527,8 @@ k_vfilter_list(const uint32_t *__restrict__ in, uint32_t k, const uint32_t *__re
 // Degree prefix of a vertex list into g->scan / g->scan_blk (pos(i) =
 // scan[i] + scan_blk[i / SCAN_BLOCK]).
 int scan_frontier_degrees(gpr_graph *g, const uint32_t *list, uint32_t k) {
-    const uint32_t nb = (k + SCAN_BLOCK - 1) / SCAN_BLOCK;
-    if (nb) hipLaunchKernelGGL(k_scan_local, dim3(nb), dim3(SCAN_THREADS), 0, g->stream, list, k, g->deg, g->scan, g->scan_blk);
-    if (nb != 1) hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, g->stream, g->scan_blk, nb);
+    hipLaunchKernelGGL(k_scan_local, dim3(grid_for(k, SCAN_BLOCK)), dim3(SCAN_THREADS), 0, g->stream, list, k, g->deg,
+                       g->scan, g->scan_blk, g->ticket);
     GPR_HIP(hipGetLastError());
     return GPR_OK;
 }
@@ -755,12 +734,8 @@ int edgemap_minrelax(gpr_graph *g, const gpr_emap_desc *desc, gpr_frontier *in, 
     if (dir == GPR_DIR_PUSH) {
         const uint32_t k = in->nactv;
         const uint64_t E = in->nacte;
-        const uint32_t nb = (k + SCAN_BLOCK - 1) / SCAN_BLOCK;
         ProfScope ps(g, "push");
-        if (nb)
-            hipLaunchKernelGGL(k_scan_local, dim3(nb), dim3(SCAN_THREADS), 0, g->stream, in->list, k, g->deg,
-                               g->scan, g->scan_blk);
-        if (nb != 1) hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, g->stream, g->scan_blk, nb);
+        GPR_TRY(scan_frontier_degrees(g, in->list, k));
         // activations are deduplicated on the output bitmap, or for a list
         // output on the graph's dedup bitmap, which is cleared again from
         // the list afterwards; without an output nothing is activated, so

@@ -8,6 +8,7 @@
 // a list for push and a bitmap (one wave64 ballot per word) for pull.
 #include "internal.hpp"
 #include "device.hpp"
+#include "grid_sync.hpp"
 
 #include <algorithm>
 
@@ -59,9 +60,9 @@ __global__ void k_list_to_bits(const uint32_t *__restrict__ list, uint32_t k, ui
 
 // Bitmap -> ascending vertex list (packDense, frontier.h:923-980), in two
 // phases: phase 0 counts the set bits of each workgroup's 256 words (with
-// COUNT, for a bitmap whose counts are not known, their out-degree sum too);
-// after an exclusive scan of those counts, phase 1 writes each word's
-// vertices at its wave-scanned offset.  The list comes out globally
+// COUNT, for a bitmap whose counts are not known, their out-degree sum too),
+// and its last workgroup scans them; phase 1 writes each word's vertices at
+// its wave-scanned offset.  The list comes out globally
 // ascending and the result is deterministic.  A bitmap that the engine wrote
 // has its counts, and its conversion neither gathers degrees nor reads
 // anything back (25 us of a traversal step).
@@ -70,7 +71,7 @@ template <bool COUNT>
 __global__ void __launch_bounds__(B2L_THREADS)
 k_bits_to_list(const uint64_t *__restrict__ bits, size_t words, uint32_t *list,
                const uint32_t *__restrict__ deg, unsigned long long *blk_counts, int phase,
-               DevCounters *ctr) {
+               DevCounters *ctr, unsigned int *ticket) {
     __shared__ uint32_t red[B2L_THREADS / 64];
     __shared__ uint64_t redl[B2L_THREADS / 64];
     size_t i = blockIdx.x * (size_t)B2L_THREADS + threadIdx.x;
@@ -79,7 +80,7 @@ k_bits_to_list(const uint64_t *__restrict__ bits, size_t words, uint32_t *list,
     if (phase == 0) {
         // count per workgroup, and edge sum
         uint32_t tot = block_sum(c, red);
-        if (threadIdx.x == 0) blk_counts[blockIdx.x] = tot;
+        if (threadIdx.x == 0) st_part(&blk_counts[blockIdx.x], (unsigned long long)tot);
         if constexpr (COUNT) {
             uint64_t es = 0;
             uint64_t t = w;
@@ -94,6 +95,8 @@ k_bits_to_list(const uint64_t *__restrict__ bits, size_t words, uint32_t *list,
                 atomicAdd(&ctr_stripe(ctr)->nacte, (unsigned long long)etot);
             }
         }
+        __shared__ int s_last;
+        if (last_workgroup(ticket, &s_last)) part_excl_scan<B2L_THREADS>(blk_counts, gridDim.x);
         return;
     }
     // phase 1: blk_counts holds exclusive offsets
@@ -248,13 +251,12 @@ int frontier_to_list(gpr_frontier *f) {
         ProfScope ps(g, "frontier_convert");
         if (f->counted)
             hipLaunchKernelGGL(k_bits_to_list<false>, dim3(blocks), dim3(B2L_THREADS), 0, g->stream, f->bits, words,
-                               f->list, g->deg, cnt, 0, g->ctr);
+                               f->list, g->deg, cnt, 0, g->ctr, g->ticket);
         else
             hipLaunchKernelGGL(k_bits_to_list<true>, dim3(blocks), dim3(B2L_THREADS), 0, g->stream, f->bits, words,
-                               f->list, g->deg, cnt, 0, g->ctr);
-        excl_scan_counts(g, cnt, blocks);
+                               f->list, g->deg, cnt, 0, g->ctr, g->ticket);
         hipLaunchKernelGGL(k_bits_to_list<false>, dim3(blocks), dim3(B2L_THREADS), 0, g->stream, f->bits, words,
-                           f->list, g->deg, cnt, 1, g->ctr);
+                           f->list, g->deg, cnt, 1, g->ctr, g->ticket);
     }
     GPR_HIP(hipGetLastError());
     f->kind = GPR_FRONTIER_LIST;

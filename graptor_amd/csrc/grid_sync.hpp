@@ -72,6 +72,62 @@ template <class T> __device__ __forceinline__ T ld_part(const T *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Thread t's share of a sum of partials, p[S*i] for i = t, t + NT, ... below
+// count, in that order, PART_U loads in flight (each takes about 0.7 us;
+// with them and half the workgroups, k_pr_update takes 13.5 us at 1.5M
+// vertices instead of 16.3).
+constexpr int PART_U = 8;
+template <int NT, int S, class T> __device__ __forceinline__ T part_sum(const T *p, uint32_t count) {
+    T s = T(0);
+    for (uint32_t i = threadIdx.x; i < count; i += NT * PART_U) {
+        T v[PART_U];
+#pragma unroll
+        for (int u = 0; u < PART_U; ++u) v[u] = ld_part(&p[(size_t)S * (i + u * NT < count ? i + u * NT : i)]);
+#pragma unroll
+        for (int u = 0; u < PART_U; ++u)
+            if (i + u * NT < count) s += v[u];
+    }
+    return s;
+}
+
+// Exclusive prefix sum in place of count per-workgroup counts (st_part), by
+// the last workgroup; returns the total.  A scan in a launch of its own costs
+// 2 us and a gap of 4 - 8 in a traversal step.
+template <int NT>
+__device__ __forceinline__ unsigned long long part_excl_scan(unsigned long long *a, uint32_t count) {
+    __shared__ unsigned long long wsum[NT / 64];
+    const unsigned w = threadIdx.x / 64;
+    unsigned long long carry = 0;
+    for (uint64_t b = 0; b < count; b += NT * PART_U) {
+        const uint64_t i0 = b + threadIdx.x * PART_U;
+        unsigned long long v[PART_U], s = 0;
+#pragma unroll
+        for (int u = 0; u < PART_U; ++u) v[u] = ld_part(&a[i0 + u < count ? i0 + u : 0]);
+#pragma unroll
+        for (int u = 0; u < PART_U; ++u) {
+            if (i0 + u >= count) v[u] = 0;
+            s += v[u];
+        }
+        const unsigned long long inc = wave_incl_scan(s);
+        if (lane() == 63) wsum[w] = inc;
+        __syncthreads();      // every read of this step precedes its writes
+        unsigned long long off = carry, tot = 0;
+        for (unsigned j = 0; j < NT / 64; ++j) {
+            if (j < w) off += wsum[j];
+            tot += wsum[j];
+        }
+        unsigned long long run = off + inc - s;
+#pragma unroll
+        for (int u = 0; u < PART_U; ++u) {
+            if (i0 + u < count) a[i0 + u] = run;
+            run += v[u];
+        }
+        carry += tot;
+        __syncthreads();
+    }
+    return carry;
+}
+
 // Grid barrier in two levels.  Block b arrives on the counter of group
 // b % ngroups (at most GS_GROUP blocks each); the last block of a group to
 // arrive at level `lvl` counts the group on `arrive`, and level `lvl` ends

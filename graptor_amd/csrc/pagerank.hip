@@ -280,42 +280,52 @@ k_pr_reduce(const double *__restrict__ part, const float *__restrict__ part_max,
 //
 // FUSED (gpr_pr_iterate_fused where the edgemap pulls): no residual, and x
 // unwritten when null.
+constexpr int PR_UPDATE_U = 4;
 template <int FMT, bool FUSED>
 __global__ void __launch_bounds__(256)
 k_pr_update(uint32_t n, const float *__restrict__ y, float *__restrict__ x, typename Codec<FMT>::store_t *contrib,
-            const uint32_t *__restrict__ deg, float damping, PrScalars *prs, double *part_delta, double *part_sum,
+            const uint32_t *__restrict__ deg, float damping, PrScalars *prs, double *part_delta, double *part_sums,
             unsigned int *ticket, HostScalars *h) {
     __shared__ double r1[4], r2[4];
     __shared__ int s_last;
     const double w = prs->w, inv_s = prs->inv_s;
     const float sc = FMT == GPR_CONTRIB_F16 ? prs->enc_scale : 1.0f;
     double dl = 0.0, sx = 0.0;
-    for (uint32_t v = blockIdx.x * 256 + threadIdx.x; v < n; v += gridDim.x * 256) {
-        const float xn = (float)(((double)y[v] + w) * inv_s);
-        if constexpr (!FUSED) {
-            dl += (double)fabsf(x[v] - xn);
-            sx += (double)xn;
+    const uint64_t step = (uint64_t)gridDim.x * 256;
+    for (uint64_t v0 = blockIdx.x * 256 + threadIdx.x; v0 < n; v0 += step * PR_UPDATE_U) {
+        float yv[PR_UPDATE_U], xv[PR_UPDATE_U];
+        uint32_t dg[PR_UPDATE_U];
+#pragma unroll
+        for (int u = 0; u < PR_UPDATE_U; ++u) {
+            const uint64_t v = v0 + u * step < n ? v0 + u * step : v0;
+            yv[u] = y[v];
+            if constexpr (!FUSED) xv[u] = x[v];
+            dg[u] = deg[v];
         }
-        if (!FUSED || x) x[v] = xn;
-        const uint32_t dg = deg[v];
-        const float cv = dg ? damping * xn / (float)dg : 0.0f;
-        contrib[v] = Codec<FMT>::enc(cv * sc);
+#pragma unroll
+        for (int u = 0; u < PR_UPDATE_U; ++u) {
+            const uint64_t v = v0 + u * step;
+            if (v >= n) break;
+            const float xn = (float)(((double)yv[u] + w) * inv_s);
+            if constexpr (!FUSED) {
+                dl += (double)fabsf(xv[u] - xn);
+                sx += (double)xn;
+            }
+            if (!FUSED || x) x[v] = xn;
+            const float cv = dg[u] ? damping * xn / (float)dg[u] : 0.0f;
+            contrib[v] = Codec<FMT>::enc(cv * sc);
+        }
     }
     if constexpr (FUSED) return;
     dl = block_sum(dl, r1);
     sx = block_sum(sx, r2);
     if (threadIdx.x == 0) {
         st_part(&part_delta[blockIdx.x], dl);
-        st_part(&part_sum[blockIdx.x], sx);
+        st_part(&part_sums[blockIdx.x], sx);
     }
     if (!last_workgroup(ticket, &s_last)) return;
-    dl = sx = 0.0;
-    for (uint32_t i = threadIdx.x; i < gridDim.x; i += 256) {
-        dl += ld_part(&part_delta[i]);
-        sx += ld_part(&part_sum[i]);
-    }
-    dl = block_sum(dl, r1);
-    sx = block_sum(sx, r2);
+    dl = block_sum(part_sum<256, 1>(part_delta, gridDim.x), r1);
+    sx = block_sum(part_sum<256, 1>(part_sums, gridDim.x), r2);
     if (threadIdx.x == 0) {
         prs->delta = dl;
         prs->sum_x = sx;
@@ -368,7 +378,7 @@ __global__ void k_pr_set_scale(PrScalars *prs, const double *slices, uint32_t ns
 // ---- host side -----------------------------------------------------------------
 static size_t fmt_bytes(int fmt) { return fmt == GPR_CONTRIB_F32 ? 4 : 2; }
 
-static unsigned update_grid(uint32_t n) { return grid_for(n, 256, 4096); }
+static unsigned update_grid(uint32_t n) { return grid_for(n, 256, 2048); }
 
 // First cold source of the PageRank edgemap: sources at or above it are
 // summed through the binned layout (pr_cold.hip), those below by the pull.

@@ -739,9 +739,7 @@ k_cold_write(const uint32_t *__restrict__ wchunk, uint32_t nwchunks, const uint3
     // M <= 2^61 units, M the total |contribution| over the cold edges
     __shared__ int s_last;
     if (!last_workgroup(fold.ticket, &s_last)) return;
-    double s = 0.0;
-    for (uint32_t i = threadIdx.x; i < nwchunks; i += CW_THREADS) s += ld_part(&mass[i]);
-    const double a = block_sum(s, red);
+    const double a = block_sum(part_sum<CW_THREADS, 1>(mass, nwchunks), red);
     if (threadIdx.x == 0) {
         int e = 0;
         if (a > 0.0 && a < 1e300) e = ilogb(a) + 1 - 61;

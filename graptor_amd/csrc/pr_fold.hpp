@@ -46,12 +46,10 @@ template <int NT, bool F16>
 __device__ __forceinline__ void pr_fold_sum(const PrFold &f, const double *part, const float *part_max, double *dred,
                                             int *s_last) {
     if (!f.count || !last_workgroup(f.ticket, s_last)) return;
-    double s = 0.0;
+    const double s = part_sum<NT, 1>(part, f.count);
     float m = 0.0f;
-    for (uint32_t i = threadIdx.x; i < f.count; i += NT) {
-        s += ld_part(&part[i]);
-        if constexpr (F16) m = fmaxf(m, ld_part(&part_max[i]));
-    }
+    if constexpr (F16)
+        for (uint32_t i = threadIdx.x; i < f.count; i += NT) m = fmaxf(m, ld_part(&part_max[i]));
     const double a = block_sum(s, dred);
     double mx = 0.0;
     if constexpr (F16) {

@@ -126,3 +126,25 @@ def test_batch_cc_row_runs():
     with G.Batch.from_csr(index, nbrs, np.array(voff, np.uint32)) as b:
         lab, _ = b.cc()
     assert np.array_equal(lab, O.cc_labels(index, nbrs))
+
+
+@pytest.mark.parametrize("n", [1, 64, 1024, 1025, 16385, 655361, 2 * 1048576 + 1026])
+def test_bitmap_to_list_and_degree_prefix(n):
+    """Per-workgroup counts scanned by the last workgroup: one, several, a thread's share (8) of each thread and
+    more (1024 list entries and 16384 bits a workgroup)."""
+    leaf = np.arange(1, n, dtype=np.uint32)
+    index, nbrs = O.build_csr(n, np.zeros(n - 1, np.uint32), leaf) if n > 1 else (
+        np.zeros(2, np.uint64), np.zeros(0, np.uint32))
+    with G.Graph.from_csr(index, nbrs) as g:
+        for every in (1, 3, 1000):
+            want = np.arange(0, n, every, dtype=np.uint32)
+            f = G.Frontier(g)
+            f.set_list(want)
+            f.convert(G.FRONTIER_BITMAP)
+            f.convert(G.FRONTIER_LIST)
+            assert f.stats()[:2] == (len(want), int(np.diff(index)[want].sum()))
+            assert np.array_equal(f.download(), want)
+            f.destroy()
+        # from a leaf: the hub, then a list of all other leaves
+        lv, _ = g.bfslvl(n - 1, direction=G.DIR_PUSH)
+        assert np.array_equal(lv, O.bfs_levels(index, nbrs, n - 1))
