@@ -52,6 +52,12 @@ __device__ __forceinline__ void gather_all(const typename Codec<FMT>::store_t *_
     for (int u = 0; u < PR_UNROLL; ++u) v[u] = s[u] < cold_from ? Codec<FMT>::dec(raw[u]) : 0.0f;
 }
 
+// Long rows in up to PR_LONG_HERE chunks are folded by the pull's last
+// workgroup: a launch less, 5 of an iteration's 20 us on 60000 vertices and
+// 1.7M edges.  Above, a thread's chain of chunk loads (8 at a time, 0.7 us
+// each) and the rows a thread has would hold the whole chip up, and k_pr_long
+// spreads them over workgroups.
+constexpr uint32_t PR_LONG_HERE = 256;
 template <int FMT>
 __global__ void __launch_bounds__(PR_THREADS)
 k_pr_pull(uint32_t nbuckets, const uint32_t *__restrict__ bucket, const uint64_t *__restrict__ cindex,
@@ -59,7 +65,7 @@ k_pr_pull(uint32_t nbuckets, const uint32_t *__restrict__ bucket, const uint64_t
           const typename Codec<FMT>::store_t *__restrict__ contrib, float *__restrict__ y,
           const uint32_t *__restrict__ long_rows, const uint32_t *__restrict__ long_base, uint32_t nlong,
           double *__restrict__ long_partial, double *part, float *part_max, const PrScalars *prs,
-          uint32_t cold_from, PrFold fold) {
+          uint32_t cold_from, PrFold fold, int long_here) {
     using C = Codec<FMT>;
     using acc_t = typename C::acc_t;
     __shared__ float vals[PR_LDS_EDGES];
@@ -101,83 +107,65 @@ k_pr_pull(uint32_t nbuckets, const uint32_t *__restrict__ bucket, const uint64_t
         }
         double tot = block_sum((double)acc, dred);
         if (threadIdx.x == 0) {
-            long_partial[c] = tot;
+            st_part(&long_partial[c], tot);
             st_part(&part[b], 0.0);
             st_part(&part_max[b], 0.0f);
         }
-        return;   // with long rows the fold is k_pr_long's
-    }
-    // ---- a bucket of rows
-    const uint32_t r0 = bucket[b], r1 = bucket[b + 1];
-    double my_sum = 0.0;
-    float my_max = 0.0f;
-    if (r0 < r1) {
-        uint32_t r1x = r1;
-        if (cindex[r1] - cindex[r1 - 1] > LONG_DEG) r1x = r1 - 1;
-        const uint64_t e0 = cindex[r0];
-        const uint32_t nrows = r1x - r0;
-        const uint32_t ne = (uint32_t)(cindex[r1x] - e0);
-        if (threadIdx.x == 0) nmed = 0;
-        for (uint32_t base = 0; base <= nrows; base += PR_THREADS * 8) {
-            uint64_t ix[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const uint32_t i = base + u * PR_THREADS + threadIdx.x;
-                ix[u] = i <= nrows ? cindex[r0 + i] : 0;
+        if (!long_here) return;   // the fold is k_pr_long's
+    } else {
+        // ---- a bucket of rows
+        const uint32_t r0 = bucket[b], r1 = bucket[b + 1];
+        double my_sum = 0.0;
+        float my_max = 0.0f;
+        if (r0 < r1) {
+            uint32_t r1x = r1;
+            if (cindex[r1] - cindex[r1 - 1] > LONG_DEG) r1x = r1 - 1;
+            const uint64_t e0 = cindex[r0];
+            const uint32_t nrows = r1x - r0;
+            const uint32_t ne = (uint32_t)(cindex[r1x] - e0);
+            if (threadIdx.x == 0) nmed = 0;
+            for (uint32_t base = 0; base <= nrows; base += PR_THREADS * 8) {
+                uint64_t ix[8];
+    #pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const uint32_t i = base + u * PR_THREADS + threadIdx.x;
+                    ix[u] = i <= nrows ? cindex[r0 + i] : 0;
+                }
+    #pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const uint32_t i = base + u * PR_THREADS + threadIdx.x;
+                    if (i <= nrows) rs[i] = (uint32_t)(ix[u] - e0);
+                }
             }
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const uint32_t i = base + u * PR_THREADS + threadIdx.x;
-                if (i <= nrows) rs[i] = (uint32_t)(ix[u] - e0);
+            // (plain loads: a small graph's neighbours stay in the L2s from one
+            // iteration to the next; non-temporal ones took 46 us instead of 39
+            // an iteration on 7.6M edges)
+            // a bucket holds < PR_LDS_EDGES edges: one round of PR_UNROLL
+            // independent neighbour loads and gathers per lane covers it
+            for (uint32_t base = 0; base < ne; base += PR_THREADS * PR_UNROLL) {
+                uint32_t s[PR_UNROLL];
+    #pragma unroll
+                for (int u = 0; u < PR_UNROLL; ++u) {
+                    const uint32_t i = base + u * PR_THREADS + threadIdx.x;
+                    s[u] = i < ne ? cnbrs[e0 + i] : 0xffffffffu;
+                }
+                float v[PR_UNROLL];
+                gather_all<FMT>(contrib, s, cold_from, v);
+    #pragma unroll
+                for (int u = 0; u < PR_UNROLL; ++u) {
+                    const uint32_t i = base + u * PR_THREADS + threadIdx.x;
+                    if (i < ne) vals[i] = v[u];
+                }
             }
-        }
-        // (plain loads: a small graph's neighbours stay in the L2s from one
-        // iteration to the next; non-temporal ones took 46 us instead of 39
-        // an iteration on 7.6M edges)
-        // a bucket holds < PR_LDS_EDGES edges: one round of PR_UNROLL
-        // independent neighbour loads and gathers per lane covers it
-        for (uint32_t base = 0; base < ne; base += PR_THREADS * PR_UNROLL) {
-            uint32_t s[PR_UNROLL];
-#pragma unroll
-            for (int u = 0; u < PR_UNROLL; ++u) {
-                const uint32_t i = base + u * PR_THREADS + threadIdx.x;
-                s[u] = i < ne ? cnbrs[e0 + i] : 0xffffffffu;
-            }
-            float v[PR_UNROLL];
-            gather_all<FMT>(contrib, s, cold_from, v);
-#pragma unroll
-            for (int u = 0; u < PR_UNROLL; ++u) {
-                const uint32_t i = base + u * PR_THREADS + threadIdx.x;
-                if (i < ne) vals[i] = v[u];
-            }
-        }
-        __syncthreads();
-        for (uint32_t i = threadIdx.x; i < nrows; i += PR_THREADS) {
-            const uint32_t a = rs[i], z = rs[i + 1];
-            if (z - a > PR_MED) {
-                medq[atomicAdd(&nmed, 1u)] = i;
-                continue;
-            }
-            acc_t acc = 0;
-            for (uint32_t j = a; j < z; ++j) acc += (acc_t)vals[j];
-            const float yv = (float)acc * dscale;
-            y[r0 + i] = yv;
-            my_sum += (double)yv;
-            if (FMT == GPR_CONTRIB_F16) {
-                const uint32_t dg = deg[r0 + i];
-                if (dg) my_max = fmaxf(my_max, yv / (float)dg);
-            }
-        }
-        __syncthreads();
-        const uint32_t nm = nmed;
-        const unsigned w = threadIdx.x / 64, ln = lane();
-        for (uint32_t q = w; q < nm; q += PR_THREADS / 64) {
-            const uint32_t i = medq[q];
-            const uint32_t a = rs[i], z = rs[i + 1];
-            acc_t acc = 0;
-            for (uint32_t j = a + ln; j < z; j += 64) acc += (acc_t)vals[j];
-            acc = wave_sum(acc);
-            if (ln == 0) {
+            __syncthreads();
+            for (uint32_t i = threadIdx.x; i < nrows; i += PR_THREADS) {
+                const uint32_t a = rs[i], z = rs[i + 1];
+                if (z - a > PR_MED) {
+                    medq[atomicAdd(&nmed, 1u)] = i;
+                    continue;
+                }
+                acc_t acc = 0;
+                for (uint32_t j = a; j < z; ++j) acc += (acc_t)vals[j];
                 const float yv = (float)acc * dscale;
                 y[r0 + i] = yv;
                 my_sum += (double)yv;
@@ -186,20 +174,67 @@ k_pr_pull(uint32_t nbuckets, const uint32_t *__restrict__ bucket, const uint64_t
                     if (dg) my_max = fmaxf(my_max, yv / (float)dg);
                 }
             }
+            __syncthreads();
+            const uint32_t nm = nmed;
+            const unsigned w = threadIdx.x / 64, ln = lane();
+            for (uint32_t q = w; q < nm; q += PR_THREADS / 64) {
+                const uint32_t i = medq[q];
+                const uint32_t a = rs[i], z = rs[i + 1];
+                acc_t acc = 0;
+                for (uint32_t j = a + ln; j < z; j += 64) acc += (acc_t)vals[j];
+                acc = wave_sum(acc);
+                if (ln == 0) {
+                    const float yv = (float)acc * dscale;
+                    y[r0 + i] = yv;
+                    my_sum += (double)yv;
+                    if (FMT == GPR_CONTRIB_F16) {
+                        const uint32_t dg = deg[r0 + i];
+                        if (dg) my_max = fmaxf(my_max, yv / (float)dg);
+                    }
+                }
+            }
+        }
+        const double ts = block_sum(my_sum, dred);
+        my_max = wave_max(my_max);
+        __syncthreads();
+        if (lane() == 0) fred[threadIdx.x / 64] = my_max;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            float mx = fred[0];
+            for (int i = 1; i < PR_THREADS / 64; ++i) mx = fmaxf(mx, fred[i]);
+            st_part(&part[b], ts);
+            st_part(&part_max[b], mx);
         }
     }
-    const double ts = block_sum(my_sum, dred);
-    my_max = wave_max(my_max);
-    __syncthreads();
-    if (lane() == 0) fred[threadIdx.x / 64] = my_max;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float mx = fred[0];
-        for (int i = 1; i < PR_THREADS / 64; ++i) mx = fmaxf(mx, fred[i]);
-        st_part(&part[b], ts);
-        st_part(&part_max[b], mx);
+    constexpr bool F16 = FMT == GPR_CONTRIB_F16;
+    if (!long_here) {
+        pr_fold_sum<PR_THREADS, F16>(fold, part, part_max, dred, &s_last);
+        return;
     }
-    pr_fold_sum<PR_THREADS, FMT == GPR_CONTRIB_F16>(fold, part, part_max, dred, &s_last);
+    // the last workgroup folds the long rows too (k_pr_long)
+    if (!last_workgroup(fold.ticket, &s_last)) return;
+    double s = part_sum<PR_THREADS, 1>(part, gridDim.x);
+    float m = F16 ? part_max_of<PR_THREADS>(part_max, gridDim.x) : 0.0f;
+    for (uint32_t li = threadIdx.x; li < nlong; li += PR_THREADS) {
+        const uint32_t c1 = long_base[li + 1], row = long_rows[li];
+        double t = 0.0;
+        for (uint32_t c = long_base[li]; c < c1; c += PART_U) {
+            double v[PART_U];
+#pragma unroll
+            for (int u = 0; u < PART_U; ++u) v[u] = ld_part(&long_partial[c + u < c1 ? c + u : c]);
+#pragma unroll
+            for (int u = 0; u < PART_U; ++u)
+                if (c + u < c1) t += v[u];
+        }
+        const float yv = (float)t * dscale;
+        y[row] = yv;
+        s += (double)yv;
+        if (F16) {
+            const uint32_t dg = deg[row];
+            if (dg) m = fmaxf(m, yv / (float)dg);
+        }
+    }
+    pr_fold_shares<PR_THREADS, F16>(fold, s, m, dred);
 }
 
 // One thread per long row: fold its chunk partials in chunk order.
@@ -436,14 +471,16 @@ static int pr_edgemap_impl(gpr_graph *g, const gpr_emap_desc *desc, gpr_frontier
     const uint32_t nparts = nblk + g->nlong;
     PrFold fold = {g->ticket, g->prs, split || nparts > PR_FOLD_MAX ? 0 : nparts, g->n, damping};
     PrFold pull_fold = fold;
-    if (g->nlong) pull_fold.count = 0;
+    const int long_here = fold.count && g->nlong && g->nlong_chunks <= PR_LONG_HERE;
+    if (g->nlong && !long_here) pull_fold.count = 0;
     if (cold_from > 0) {
         // the pull over sources [0, cold_from); every source when not split
         ProfScope ps(g, "pr_pull");
 #define PR_PULL(F)                                                                                              \
     hipLaunchKernelGGL(k_pr_pull<F>, dim3(nblk), dim3(PR_THREADS), 0, g->stream, g->nbuckets, g->bucket,        \
                        g->cindex, g->cnbrs, g->deg, (const typename Codec<F>::store_t *)cb, y, g->long_rows,   \
-                       g->long_base, g->nlong, g->long_partial, g->partial, g->partial_f, g->prs, cold_from, pull_fold)
+                       g->long_base, g->nlong, g->long_partial, g->partial, g->partial_f, g->prs, cold_from, pull_fold,    \
+                       long_here)
         switch (fmt) {
         case GPR_CONTRIB_F32: PR_PULL(GPR_CONTRIB_F32); break;
         case GPR_CONTRIB_BF16: PR_PULL(GPR_CONTRIB_BF16); break;
@@ -454,7 +491,7 @@ static int pr_edgemap_impl(gpr_graph *g, const gpr_emap_desc *desc, gpr_frontier
         }
 #undef PR_PULL
     }
-    if (cold_from > 0 && g->nlong) {
+    if (cold_from > 0 && g->nlong && !long_here) {
         ProfScope ps(g, "pr_long");
 #define PR_LONG(F16)                                                                                            \
     hipLaunchKernelGGL(k_pr_long<F16>, dim3(grid_for(g->nlong, PR_THREADS, 1024)), dim3(PR_THREADS), 0, g->stream, \

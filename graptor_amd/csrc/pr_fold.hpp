@@ -40,16 +40,10 @@ __device__ __forceinline__ void pr_set_sum(PrScalars *prs, double a, double m, u
     }
 }
 
-// The end of a kernel whose workgroups wrote part[] and part_max[] (thread
-// 0, st_part): the last one sets the scalars.  dred: NT/64 doubles of LDS.
+// The scalars from this thread's shares s and m of the sum and the maximum, by
+// all threads of the last workgroup.
 template <int NT, bool F16>
-__device__ __forceinline__ void pr_fold_sum(const PrFold &f, const double *part, const float *part_max, double *dred,
-                                            int *s_last) {
-    if (!f.count || !last_workgroup(f.ticket, s_last)) return;
-    const double s = part_sum<NT, 1>(part, f.count);
-    float m = 0.0f;
-    if constexpr (F16)
-        for (uint32_t i = threadIdx.x; i < f.count; i += NT) m = fmaxf(m, ld_part(&part_max[i]));
+__device__ __forceinline__ void pr_fold_shares(const PrFold &f, double s, float m, double *dred) {
     const double a = block_sum(s, dred);
     double mx = 0.0;
     if constexpr (F16) {
@@ -60,6 +54,21 @@ __device__ __forceinline__ void pr_fold_sum(const PrFold &f, const double *part,
         for (int i = 0; i < NT / 64; ++i) mx = fmax(mx, dred[i]);
     }
     if (threadIdx.x == 0) pr_set_sum<F16>(f.prs, a, mx, f.n, f.damping);
+}
+template <int NT>
+__device__ __forceinline__ float part_max_of(const float *part_max, uint32_t count) {
+    float m = 0.0f;
+    for (uint32_t i = threadIdx.x; i < count; i += NT) m = fmaxf(m, ld_part(&part_max[i]));
+    return m;
+}
+
+// The end of a kernel whose workgroups wrote part[] and part_max[] (thread
+// 0, st_part): the last one sets the scalars.  dred: NT/64 doubles of LDS.
+template <int NT, bool F16>
+__device__ __forceinline__ void pr_fold_sum(const PrFold &f, const double *part, const float *part_max, double *dred,
+                                            int *s_last) {
+    if (!f.count || !last_workgroup(f.ticket, s_last)) return;
+    pr_fold_shares<NT, F16>(f, part_sum<NT, 1>(part, f.count), F16 ? part_max_of<NT>(part_max, f.count) : 0.0f, dred);
 }
 
 } // namespace gpr

@@ -75,3 +75,22 @@ def test_fused_iterations_equal_unfused(fmt, pull):
         xf, _ = g.pr_vary([(fmt, 0.0)], max_iter=9)
         xu, _ = g.pr_vary([(fmt, 1e-300)], max_iter=9)
     assert np.array_equal(xf.view(np.uint32), xu.view(np.uint32))
+
+
+@pytest.mark.parametrize("hubs,degree", [(1, 2049), (255, 2100), (256, 2100), (257, 2100), (1, 256 * 8192), (1, 257 * 8192)])
+def test_long_rows_folded_in_the_pull(hubs, degree):
+    """Rows in as many chunks (8192 edges) as the pull's last workgroup folds, and in more."""
+    n = max(4001, degree + hubs)
+    dst = np.repeat(np.arange(hubs, dtype=np.uint32), degree)
+    src = (hubs + (np.arange(hubs * degree, dtype=np.uint64) * 7 + dst) % (n - hubs)).astype(np.uint32)
+    back = np.arange(n, dtype=np.uint32)     # every vertex has a way on
+    src, dst = np.concatenate([src, back]), np.concatenate([dst, (back * 31 + 7) % n])
+    index, nbrs = O.build_csr(n, src, dst.astype(np.uint32), symmetrize=False)
+    ci, cn = O.build_csr(n, dst.astype(np.uint32), src, symmetrize=False)
+    x64, _, _ = O.pr_fp64(ci, cn, 8, 0.0, outdeg=np.diff(index).astype(np.uint32))
+    with G.Graph.from_csr(index, nbrs, symmetric=False) as g:
+        for fmt, bar in (("fp32", 1e-6), ("fp16", 1e-3)):
+            x, _ = g.pr_vary([(fmt, 0.0)], max_iter=8)
+            assert rel_l1(x, x64) <= bar, (fmt, rel_l1(x, x64))
+            x2, _ = g.pr_vary([(fmt, 0.0)], max_iter=8)
+            assert np.array_equal(x, x2), fmt
