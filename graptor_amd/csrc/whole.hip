@@ -10,8 +10,11 @@
 // it is and when the frontier was empty, and the host keeps WB_AHEAD launches
 // queued until then (the launches past the end find empty lists and return).
 // No barrier inside a launch, so no launch needs all its blocks resident.
-// Rows up to WB_LIGHT edges are one lane's work, longer ones are listed as
-// WB_SLICE-edge slices, a wave each.  A vertex is discovered by atomicMin on
+// Rows up to WB_LIGHT edges are one lane's work, or that of up to 8 lanes where
+// a level leaves lanes idle (a lane's row is a chain of 2.5 us steps of WB_U
+// edges: 93 us instead of 76 on RMAT with 4096 vertices, 214 instead of 166 on
+// a random graph of 50021); longer ones are listed as WB_SLICE-edge slices, a
+// wave each.  A vertex is discovered by atomicMin on
 // the levels, which start at n+1: the one that finds n+1 lists it, so no
 // bitmap is needed.  A plain load looks first; levels only fall, so what it
 // sees at or below the new level proves that there is nothing to do, however
@@ -195,7 +198,8 @@ k_wb_init(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__rest
 
 __global__ void __launch_bounds__(WB_THREADS)
 k_wb_level(uint32_t n, uint32_t lvl, const uint64_t *__restrict__ index, const uint32_t *__restrict__ nbrs,
-           const uint32_t *__restrict__ deg, uint32_t *level, WbLists L, WbCtl *ctl, WbRule rule, WbHost *h) {
+           const uint32_t *__restrict__ deg, uint32_t *level, WbLists L, WbCtl *ctl, WbRule rule, WbHost *h,
+           uint32_t sub_max) {
     __shared__ uint32_t s_stage[WB_WAVES * WB_STAGE];
     __shared__ uint32_t s_n[WB_WAVES], s_act[WB_WAVES], s_base[WB_WAVES];
     __shared__ unsigned long long s_edge[WB_WAVES];
@@ -237,23 +241,29 @@ k_wb_level(uint32_t n, uint32_t lvl, const uint64_t *__restrict__ index, const u
                 __hip_atomic_store(&h->level, lvl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
     }
+    // 2^lg lanes a row while there are lanes to spare (up to sub_max)
+    uint32_t lg = 0;
+    while ((1u << lg) < sub_max && ((uint64_t)nL << (lg + 1)) <= (uint64_t)W * 64) ++lg;
+    const uint32_t sub = 1u << lg, rows = 64 >> lg;
     WbFound f{&s_stage[wv * WB_STAGE]};
-    for (uint32_t base = w * 64; base < nL; base += W * 64) {
-        if (base != w * 64) row = L.light[cb][min(base + ln, n - 1)];
+    for (uint32_t base = w * rows; base < nL; base += W * rows) {
+        const uint32_t i = base + (ln >> lg);
+        if (lg || base != w * 64) row = L.light[cb][min(i, n - 1)];
         uint32_t e = 0, e1 = 0;
-        if (base + ln < nL) {
+        if (i < nL) {
             e = row & ((1u << WB_START_BITS) - 1);
             e1 = e + (row >> WB_START_BITS);
+            e += ln & (sub - 1);
         }
         while (__ballot(e < e1)) {
             bool act[WB_U];
             uint32_t d[WB_U];
 #pragma unroll
             for (int j = 0; j < WB_U; ++j) {
-                act[j] = e + j < e1;
-                d[j] = act[j] ? nbrs[e + j] : 0u;
+                act[j] = e + (j << lg) < e1;
+                d[j] = act[j] ? nbrs[e + (j << lg)] : 0u;
             }
-            e = e + WB_U < e1 ? e + WB_U : e1;
+            e += WB_U << lg;    // < 2^26 + 64: no wrap
             wb_relax(act, d, lvl + 1, level, index, deg, L, nb, ctl, nx, f);
         }
     }
@@ -523,8 +533,11 @@ static int whole_results(gpr_graph *g, const uint32_t *dev, uint32_t *host, bool
 // Reporting every level instead of every fourth (a write to the host that
 // the launch waits for) took 460 us instead of 434 on 47 levels.
 constexpr unsigned WB_AHEAD = 6;
-// Blocks of a level's launch: one per WB_BLOCK_EDGES edges of the graph.
+// Blocks of a level's launch: one per WB_BLOCK_EDGES edges of the graph.  With
+// 32 at least instead of 128, a random graph of 50021 vertices took 182 us, not
+// 166; one of 4096 (RMAT) 87, not 76.
 constexpr uint64_t WB_BLOCK_EDGES = 4096;
+constexpr uint64_t WB_MIN_BLOCKS = 128;
 
 int whole_bfs(gpr_graph *g, uint32_t start, float threshold_pct, uint32_t *levels, gpr_run_info *info) {
     const WholeBuf b = whole_layout(g);
@@ -541,7 +554,10 @@ int whole_bfs(gpr_graph *g, uint32_t start, float threshold_pct, uint32_t *level
         rule.frac = 1;
         rule.rhs = (double)(float)g->m / (100.0 / (double)threshold_pct);
     }
-    const unsigned grid = (unsigned)std::min<uint64_t>(1024, std::max<uint64_t>(32, g->m / WB_BLOCK_EDGES));
+    const unsigned grid = (unsigned)std::min<uint64_t>(1024, std::max<uint64_t>(WB_MIN_BLOCKS, g->m / WB_BLOCK_EDGES));
+    // lanes that an average row keeps busy for one step
+    uint32_t sub_max = 1;
+    while (sub_max * WB_U < WB_LIGHT && (uint64_t)sub_max * WB_U * n < g->m) sub_max *= 2;
     volatile WbHost *h = (volatile WbHost *)g->whost;
     h->level = 0;
     h->done = 0;
@@ -552,7 +568,7 @@ int whole_bfs(gpr_graph *g, uint32_t start, float threshold_pct, uint32_t *level
     while (!__atomic_load_n(&((WbHost *)g->whost)->done, __ATOMIC_ACQUIRE)) {
         if (launched - h->level < WB_AHEAD) {
             hipLaunchKernelGGL(k_wb_level, dim3(grid), dim3(WB_THREADS), 0, g->stream, n, launched, g->index, g->nbrs,
-                               g->deg, level, L, ctl, rule, (WbHost *)g->whost_dev);
+                               g->deg, level, L, ctl, rule, (WbHost *)g->whost_dev, sub_max);
             ++launched;
             GPR_HIP(hipGetLastError());
         } else if (++polls % 4096 == 0) {

@@ -125,3 +125,20 @@ def test_whole_cc_long_paths_relabelled(n):
         g.reorder()
         for _ in range(10):
             assert np.array_equal(g.ccv()[0], want)
+
+
+@pytest.mark.parametrize("reach", [1, 2, 3, 4, 8, 9, 15, 16, 17])
+@pytest.mark.parametrize("n", [70, 4099, 33000])
+def test_whole_bfs_lanes_per_row(n, reach):
+    """Rows of 2 to 34 edges, in levels that leave lanes for 1 to 8 a row: a ring with a hub's worth of short cuts
+    from the start."""
+    i = np.repeat(np.arange(n), reach)
+    j = (i + np.tile(np.arange(1, reach + 1), n)) % n
+    cut = np.arange(1, n, max(1, n // 3000))
+    index, nbrs = O.build_csr(n, np.concatenate([i, 0 * cut]).astype(np.uint32), np.concatenate([j, cut]).astype(np.uint32))
+    with G.Graph.from_csr(index, nbrs) as g:
+        for s in (0, n // 2):
+            lv, info = g.bfslvl(s)
+            assert np.array_equal(lv, O.bfs_levels(index, nbrs, s))
+            _, b = host_driven(lambda: g.bfslvl(s))
+            assert (info.iters, info.push_iters, info.edges) == (b.iters, b.push_iters, b.edges)
