@@ -533,9 +533,19 @@ int scan_frontier_degrees(gpr_graph *g, const uint32_t *list, uint32_t k) {
     return GPR_OK;
 }
 
+// Waves of PULL_GROUPS 64-vertex groups each, as far as that leaves every
+// CU 8 workgroups (its 32 waves) and the tunable allows: a workgroup ends in
+// three block sums and counter atomics, which cost more than its rows where
+// a wave has two groups.  BFS / CC of RMAT graphs on the device, in ms, with
+// 128 workgroups a CU and by this rule: 4M vertices 0.331 / 0.357 and 0.313 /
+// 0.295, 8M 0.423 / 0.412 and 0.373 / 0.353, 16M 0.565 / 0.531 and 0.525 /
+// 0.518, 33M 0.882 / 0.793 and 0.854 / 0.763; at 67M the two are the same.
+constexpr uint32_t PULL_GROUPS = 8;
 static unsigned pull_grid(uint32_t n) {
-    uint32_t groups = (n + 63) / 64;
-    return grid_for(groups, PULL_THREADS / 64, (unsigned)std::max(1.0, tun().pull_blocks_per_cu * num_cus()));
+    const uint32_t groups = (uint32_t)(((uint64_t)n + 63) / 64), per = PULL_THREADS / 64;
+    const unsigned full = grid_for(groups, per, 8u * (unsigned)num_cus());
+    return std::min(std::max(grid_for(groups, per * PULL_GROUPS), full),
+                    (unsigned)std::max(1.0, tun().pull_blocks_per_cu * num_cus()));
 }
 
 int pr_edgemap(gpr_graph *g, const gpr_emap_desc *desc, gpr_frontier *in, gpr_iter_stats *st);

@@ -500,7 +500,7 @@ int gpr_trace_get(const gpr_graph *g, gpr_iter_stats *out, int cap, int *k);
  *                       and BFS's counts are the same; such a CC run is one
  *                       step in gpr_run_info
  *   pull_serial_max     pull rows up to this in-degree run lane-serially
- *   pull_blocks_per_cu  pull grid size per compute unit
+ *   pull_blocks_per_cu  pull grid size per compute unit, at most
  *   push_blocks_per_cu  push grid cap per compute unit
  *   fusion_spin_limit   fused push: polls of an idle wave without any wave
  *                       claiming work, or of a reserved queue slot, before
