@@ -14,15 +14,17 @@
 //   the pull       the PageRank edgemap (pagerank.hip / pr_cold.hip) sums
 //                  y[d] = sum of decoded contributions over in-edges;
 //   or k_apr_push  for frontiers at or below 1% of the edges (:574,
-//                  frac_threshold(1)): y = 0, then every out-edge of a
-//                  frontier source adds its decoded contribution with a
-//                  hardware FP32 atomic, edges split evenly over workgroups
+//                  frac_threshold(1)): every out-edge of a frontier source
+//                  adds its decoded contribution to y, which the tail left
+//                  zero, with a hardware FP32 atomic, edges split evenly over workgroups
 //                  by the frontier's degree prefix.
 //   k_apr_tail     z = y*factor, delta, x, the active test, the new frontier
-//                  as a bitmap (one ballot per 64 vertices), per-workgroup
-//                  sums of |delta| and |x| and the frontier counts;
-//   k_apr_reduce   the deterministic FP64 totals, read by the host to pick
-//                  the next iteration's branch and to stop.
+//                  as a bitmap (one ballot per 64 vertices), y = 0 for a
+//                  push (zeroing it in the push took a launch: 5 us and a
+//                  gap), and the FP64 sums of |delta| and |x| and the
+//                  frontier counts in a fixed order, which the last
+//                  workgroup writes where the host reads them to pick the
+//                  next iteration's branch and to stop.
 // Vertex arithmetic is FP32 with no contraction, as FloatTy is float in
 // every variant; contraction is switched off so each product and sum
 // rounds separately.
@@ -71,10 +73,6 @@ k_apr_contrib(uint32_t n, const float *__restrict__ delta, const uint32_t *__res
         }
         contrib[v] = c;
     }
-}
-
-__global__ void __launch_bounds__(256) k_apr_zero(float *__restrict__ y, uint32_t n) {
-    for (uint32_t v = blockIdx.x * 256 + threadIdx.x; v < n; v += gridDim.x * 256) y[v] = 0.0f;
 }
 
 // Edge tiles of AP_TILE over the frontier's degree prefix; the sources of a
@@ -149,7 +147,7 @@ k_apr_push(const uint32_t *__restrict__ flist, uint32_t k, const uint64_t *__res
 // fixed order for a given n, so the totals are deterministic.
 template <bool FIRST>
 __global__ void __launch_bounds__(AT_THREADS)
-k_apr_tail(uint32_t n, const float *__restrict__ y, float factor, float dampen, float cst, float ninv, float eps2,
+k_apr_tail(uint32_t n, float *__restrict__ y, float factor, float dampen, float cst, float ninv, float eps2,
            float *__restrict__ x, float *__restrict__ delta, const uint32_t *__restrict__ deg,
            uint64_t *__restrict__ bits, double *part, uint64_t *cpart, unsigned int *ticket, HostScalars *h) {
 #pragma clang fp contract(off)
@@ -195,6 +193,7 @@ k_apr_tail(uint32_t n, const float *__restrict__ y, float factor, float dampen, 
                     }
                 }
                 delta[v] = dl;
+                if (__float_as_uint(yv[u])) y[v] = 0.0f;
                 sl1 += (double)fabsf(dl);
                 sx += (double)fabsf(xv);
                 if (a) ce += deg[v];
@@ -297,10 +296,6 @@ int apr_push(gpr_graph *g, int fmt, gpr_frontier *F, const gpr_prop *dp, float f
     const float *delta = (const float *)dp->d;
     float *y = (float *)yp->d;
     const uint32_t n = g->n;
-    {
-        ProfScope ps(g, "apr_zero");
-        hipLaunchKernelGGL(k_apr_zero, dim3(grid_for(n, 256, 4096)), dim3(256), 0, g->stream, y, n);
-    }
     if (F->kind == GPR_FRONTIER_EMPTY) return GPR_OK;
     GPR_TRY(frontier_to_list(F));
     const uint32_t k = F->nactv;
@@ -328,8 +323,7 @@ int apr_tail(gpr_graph *g, bool first, const gpr_prop *yp, float factor, float e
     GPR_REQUIRE(yp && xp && dp && yp->dtype == GPR_F32 && xp->dtype == GPR_F32 && dp->dtype == GPR_F32 && out &&
                     out->g == g,
                 "apr_tail: y, x and delta must be f32 properties, out a frontier of this graph");
-    const float *y = (const float *)yp->d;
-    float *x = (float *)xp->d, *delta = (float *)dp->d;
+    float *y = (float *)yp->d, *x = (float *)xp->d, *delta = (float *)dp->d;
     const uint32_t n = g->n;
     GPR_TRY(frontier_ensure_bits(out));
     const unsigned grid = grid_for(nwords(n), AT_WAVES, AT_MAX_BLOCKS);

@@ -18,7 +18,8 @@ int apr_check_fmt(int fmt);
 // contrib = enc(delta / (factor*deg)), sources outside `mask` (when given and
 // not all-true) storing 0.
 int apr_contrib(gpr_graph *g, int fmt, const gpr_prop *delta, gpr_prop *contrib, float factor, gpr_frontier *mask);
-// y = 0, then y[d] += the decoded contribution of every out-edge of F.
+// y[d] += the decoded contribution of every out-edge of F; y is zero before
+// (new, or after apr_tail).
 int apr_push(gpr_graph *g, int fmt, gpr_frontier *F, const gpr_prop *delta, float factor, gpr_prop *y);
 // The vertex maps after the edgemap; `out` receives the active bitmap and
 // tot the totals (synchronises).
