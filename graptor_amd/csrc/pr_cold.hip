@@ -31,9 +31,9 @@
 //                   the result does not depend on the order of the atomics.  A bin in one
 //                   chunk updates y directly; the chunks of a heavy bin (the
 //                   hub destinations) write integer partials that
-//   k_cold_combine_groups and k_cold_combine add up per destination in two
-//                   levels (groups of COLD_GROUP partials, then the group
-//                   sums), so a hub bin of hundreds of chunks is summed by
+//   k_cold_combine_groups and k_cold_combine add up per destination, above
+//                   COLD_ONE_LEVEL chunks a bin in two levels (groups of
+//                   COLD_GROUP partials, then the group sums), so a hub bin of hundreds of chunks is summed by
 //                   many workgroups instead of one dependent chain each.
 //
 // After degree relabelling a source's edges fall into few bins relative to
@@ -973,6 +973,11 @@ k_cold_accum(const uint32_t *__restrict__ achunk, uint32_t n, const uint16_t *cd
 }
 
 constexpr int CC_THREADS = 1024;
+// Up to this many chunks in a bin their partials are added in one level: on a
+// directed graph of 1.5M vertices and 23M edges (17 to 64 chunks in its
+// largest bin) a run of 18 iterations takes 2.09 ms instead of 2.18 in two.  A 4M-vertex RMAT graph, whose hub bin has
+// more, takes 20 us longer over a run that way.
+constexpr uint32_t COLD_ONE_LEVEL = 64;
 // workgroups per bin of the two combine kernels
 static uint32_t combine_per_bin(uint32_t n) { return (std::min(n, COLD_BIN) + CC_THREADS - 1) / CC_THREADS; }
 
@@ -996,7 +1001,7 @@ k_cold_combine_groups(const uint32_t *__restrict__ groups, uint32_t n, uint32_t 
 }
 
 // Second level: one workgroup per CC_THREADS destinations of a bin adds its
-// groups' sums (its chunks' sums when no bin has more than COLD_GROUP
+// groups' sums (its chunks' sums when no bin has more than COLD_ONE_LEVEL
 // chunks, direct) and stores y; its y sum and y/deg maximum go to slot
 // nbins + blockIdx.x.  Integer sums: exact in any grouping.
 template <bool F16>
@@ -1107,7 +1112,7 @@ int cold_launch_accum(gpr_graph *g, int fmt, float *y, int add, double *part, fl
     }
 #undef CA
     if (L->nmulti) {
-        const bool direct = L->max_chunks <= COLD_GROUP;
+        const bool direct = L->max_chunks <= COLD_ONE_LEVEL;
         if (!direct)
             hipLaunchKernelGGL(k_cold_combine_groups, dim3(L->ngroups * per_bin), dim3(CC_THREADS), 0, g->stream,
                                L->groups, g->n, per_bin, (const long long *)L->partials, L->partials2);
