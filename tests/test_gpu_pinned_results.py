@@ -83,3 +83,25 @@ def test_batch_labels(shift):
             got = into_pinned(4 * n, shift, lambda d: G._check(G.lib().gpr_batch_cc(b.h, d, C.byref(info))))
             assert np.array_equal(got.view(np.uint32), want)
             assert np.array_equal(b.cc()[0], want)
+
+
+def test_batch_labels_in_link_order():
+    """More than 8 graphs a CU, half of them sparse: pinned labels have a queue order of their own."""
+    count = 2600
+    rng = np.random.default_rng(3)
+    nv = rng.integers(2, 40, count)
+    voff = np.concatenate([[0], np.cumsum(nv)]).astype(np.uint32)
+    src, dst = [], []
+    for g in range(count):
+        m = int(nv[g]) * (1 if g % 2 else 6)
+        src.append(voff[g] + rng.integers(0, nv[g], m))
+        dst.append(voff[g] + rng.integers(0, nv[g], m))
+    n = int(voff[-1])
+    index, nbrs = O.build_csr(n, np.concatenate(src).astype(np.uint32), np.concatenate(dst).astype(np.uint32))
+    want = O.cc_labels(index, nbrs)
+    with G.Batch.from_csr(index, nbrs, voff) as b:
+        info = G.RunInfo()
+        for _ in range(3):
+            got = into_pinned(4 * n, 0, lambda d: G._check(G.lib().gpr_batch_cc(b.h, d, C.byref(info))))
+            assert np.array_equal(got.view(np.uint32), want)
+            assert np.array_equal(b.cc()[0], want)
