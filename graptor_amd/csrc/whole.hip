@@ -54,6 +54,8 @@ constexpr uint32_t WB_LIGHT = 32;    // rows up to this length: a lane each
 constexpr uint32_t WB_SLICE = 256;   // longer rows: a wave per slice of this many edges
 constexpr int WB_U = 4;              // edges per lane in flight
 constexpr uint32_t WB_STAGE = 512;   // staged list entries per wave
+constexpr uint32_t WB_OWN = 64;      // slices of a row that its lane lists alone (with 8: 133 us, not 110, on RMAT of
+                                     // 16384 vertices and 4.5M edges, where most rows have some)
 static_assert(WB_SLICE == 64 * WB_U, "a slice is one pass of the wave");
 // A listed row is its first edge and its length, read with the vertex's
 // degree when it is discovered: the next level then starts at the neighbours,
@@ -149,10 +151,20 @@ __device__ __forceinline__ void wb_relax(const bool (&act)[WB_U], const uint32_t
     uint32_t b = 0;
     if (lane() == 0) b = atomicAdd(&ctl->nheavy[nx], th);
     b = __builtin_amdgcn_readfirstlane(b) + (ih - ch);
+    // A row's lane lists up to WB_OWN slices; more of them the wave lists, 64
+    // at a time (by one lane the slices of a row of 4M edges took 500 us).
 #pragma unroll
-    for (int j = 0; j < WB_U; ++j)
-        if (dg[j] > WB_LIGHT)
-            for (uint32_t k = 0; k < dg[j]; k += WB_SLICE) L.heavy[nb][b++] = wb_slice(first[j], dg[j], k);
+    for (int j = 0; j < WB_U; ++j) {
+        const uint32_t sl = dg[j] > WB_LIGHT ? (dg[j] + WB_SLICE - 1) / WB_SLICE : 0u;
+        if (sl <= WB_OWN)
+            for (uint32_t k = 0; k < sl; ++k) L.heavy[nb][b + k] = wb_slice(first[j], dg[j], k * WB_SLICE);
+        for (uint64_t t = __ballot(sl > WB_OWN); t; t &= t - 1) {
+            const int o = __ffsll((long long)t) - 1;
+            const uint32_t of = __shfl(first[j], o, 64), od = __shfl(dg[j], o, 64), ob = __shfl(b, o, 64);
+            for (uint32_t k = lane(); k * WB_SLICE < od; k += 64) L.heavy[nb][ob + k] = wb_slice(of, od, k * WB_SLICE);
+        }
+        b += sl;
+    }
 }
 
 // The threshold rule (threshold_sparse): integer nactv + nacte <= limit, or

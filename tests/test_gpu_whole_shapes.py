@@ -1,0 +1,85 @@
+"""Whole runs on graphs whose shape works against them: hubs of many slices,
+many vertices that discover the same few, dense rows.  Results against the
+oracle or the graph's own, counts against the host-driven run, and no run
+slower than that by more than the noise of a minimum of eleven (1.4)."""
+import ctypes as C
+import time
+
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+G = pytest.importorskip("graptor_amd")
+
+
+@pytest.fixture(autouse=True)
+def restore_tunables():
+    G.lib()
+    old = G.tune_get("whole_edges")
+    yield
+    G.tune_set("whole_edges", old)
+
+
+def csr(n, src, dst):
+    """Symmetric CSR of distinct edges (src < dst) without loops."""
+    key = np.concatenate((src.astype(np.uint64) * n + dst, dst.astype(np.uint64) * n + src))
+    key.sort()
+    rows = key // n
+    return np.concatenate(([0], np.cumsum(np.bincount(rows.astype(np.int64), minlength=n)))).astype(np.uint64), \
+        (key - rows * n).astype(np.uint32)
+
+
+def bipartite(hubs, n):
+    """Vertices 0..hubs-1 next to all the others."""
+    rest = np.arange(hubs, n, dtype=np.uint64)
+    return csr(n, np.repeat(np.arange(hubs, dtype=np.uint64), len(rest)), np.tile(rest, hubs))
+
+
+def info_call(g, app, out=None):
+    info = G.RunInfo()
+    dst = None if out is None else out.ctypes.data_as(C.c_void_p)
+    if app == "bfs":
+        G._check(G.lib().gpr_bfslvl(g.h, 3, None, dst, C.byref(info)))
+    else:
+        G._check(G.lib().gpr_ccv(g.h, None, dst, C.byref(info)))
+    return info
+
+
+def fastest(g, app, whole):
+    G.tune_set("whole_edges", (1 << 24) if whole else 0)
+    best = 1e9
+    for _ in range(13):
+        t = time.perf_counter()
+        info_call(g, app)
+        best = min(best, time.perf_counter() - t)
+    return best
+
+
+def not_slower(g, app):
+    ratio = min(fastest(g, app, True) / fastest(g, app, False) for _ in range(2))
+    assert ratio <= 1.4, ratio
+
+
+@pytest.mark.parametrize("d", [64 * 256 - 1, 64 * 256, 64 * 256 + 1, 64 * 256 + 257, 130 * 256 + 5])
+def test_bfs_hub_slices(d):
+    """Rows of as many slices as a lane lists alone, and of more."""
+    src = np.concatenate((np.zeros(d, np.uint32), np.ones(d - 1, np.uint32)))
+    dst = np.concatenate((np.arange(1, d + 1, dtype=np.uint32), np.arange(2, d + 1, dtype=np.uint32)))
+    index, nbrs = O.build_csr(d + 3, src, dst)
+    with G.Graph.from_csr(index, nbrs) as g:
+        for s in (0, 1, 3, d):
+            lv, info = g.bfslvl(s)
+            assert np.array_equal(lv, O.bfs_levels(index, nbrs, s))
+            G.tune_set("whole_edges", 0)
+            _, want = g.bfslvl(s)
+            G.tune_set("whole_edges", 1 << 24)
+            assert (info.iters, info.push_iters, info.edges) == (want.iters, want.push_iters, want.edges)
+
+
+def test_bfs_of_a_large_star_is_not_slower():
+    with G.Graph.from_csr(*bipartite(1, 4000000)) as g:
+        lv, _ = g.bfslvl(3)
+        assert lv[3] == 0 and lv[0] == 1 and (np.delete(lv, (0, 3)) == 2).all()
+        not_slower(g, "bfs")
