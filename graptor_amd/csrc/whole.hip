@@ -56,6 +56,8 @@ constexpr int WB_U = 4;              // edges per lane in flight
 constexpr uint32_t WB_STAGE = 512;   // staged list entries per wave
 constexpr uint32_t WB_OWN = 64;      // slices of a row that its lane lists alone (with 8: 133 us, not 110, on RMAT of
                                      // 16384 vertices and 4.5M edges, where most rows have some)
+constexpr uint32_t WB_TAGS = 256;    // destinations that a workgroup remembers to have tried (wb_claim)
+constexpr int WB_CROWD = 16;         // lanes of a wave that gave one up: the rest look past the caches
 static_assert(WB_SLICE == 64 * WB_U, "a slice is one pass of the wave");
 // A listed row is its first edge and its length, read with the vertex's
 // degree when it is discovered: the next level then starts at the neighbours,
@@ -87,10 +89,41 @@ struct WbLists {
 // counts of the level.
 struct WbFound {
     uint32_t *buf;   // WB_STAGE entries of LDS
+    unsigned long long *tag;   // the workgroup's WB_TAGS (wb_claim)
     uint32_t n = 0;  // wave-uniform
     uint32_t act = 0;             // per lane
     unsigned long long edge = 0;  // per lane
 };
+
+// Graphs with hubs (rows of more than LONG_DEG in-edges): of the lanes of a
+// workgroup that see destination d unset, one tries it, as the others' atomics
+// could find nothing any more.  Every wave of a wide level sees a hub unset
+// before the first atomic on it lands, and they would queue on its line: 500K
+// vertices next to the same 16 took 9.8 ms, 0.21 ms like this (host-driven, by
+// a pull: 0.14); 0.43 without the second look of a wave in which many lanes
+// had the same destination (WB_CROWD).  Dense RMAT graphs gain too: 65536
+// vertices with 6M edges 148 -> 130 us.  A slot holds the last destination
+// tried and who tried it; a lane that gives up has read its own destination
+// written by another lane later than by itself, and the last such lane keeps
+// it.  Without hubs the look costs 2-3% and the launch leaves it out.
+__device__ __forceinline__ void wb_claim(bool (&need)[WB_U], const uint32_t (&d)[WB_U], unsigned long long *tag) {
+#pragma unroll
+    for (int j = 0; j < WB_U; ++j) {
+        if (!need[j]) continue;
+        unsigned long long *t = tag + d[j] % WB_TAGS;
+        if ((uint32_t)(__hip_atomic_load(t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) >> 32) == d[j])
+            need[j] = false;
+        else
+            __hip_atomic_store(t, (unsigned long long)d[j] << 32 | (threadIdx.x * WB_U + j), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+#pragma unroll
+    for (int j = 0; j < WB_U; ++j) {
+        if (!need[j]) continue;
+        const unsigned long long t = __hip_atomic_load(tag + d[j] % WB_TAGS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        need[j] = (uint32_t)(t >> 32) != d[j] || (uint32_t)t == threadIdx.x * WB_U + j;
+    }
+}
 
 // The slice of a row's edges from its k-th on.
 __device__ __forceinline__ uint64_t wb_slice(uint32_t first, uint32_t len, uint32_t k) {
@@ -102,6 +135,7 @@ __device__ __forceinline__ void wb_store(uint32_t *list, uint32_t at, const WbFo
 }
 
 // Discover up to WB_U destinations per lane at level nl.  Wave-uniform.
+template <bool HUBS>
 __device__ __forceinline__ void wb_relax(const bool (&act)[WB_U], const uint32_t (&d)[WB_U], uint32_t nl,
                                          uint32_t *level, const uint64_t *__restrict__ index,
                                          const uint32_t *__restrict__ deg, const WbLists &L, int nb, WbCtl *ctl,
@@ -114,6 +148,18 @@ __device__ __forceinline__ void wb_relax(const bool (&act)[WB_U], const uint32_t
 #pragma unroll
     for (int j = 0; j < WB_U; ++j) any |= need[j];
     if (!__ballot(any)) return;
+    if constexpr (HUBS) {
+        const int tried = __popcll(__ballot(any));
+        wb_claim(need, d, f.tag);
+        any = false;
+#pragma unroll
+        for (int j = 0; j < WB_U; ++j) any |= need[j];
+        if (tried - __popcll(__ballot(any)) >= WB_CROWD) {
+#pragma unroll
+            for (int j = 0; j < WB_U; ++j)
+                need[j] = need[j] && __hip_atomic_load(&level[d[j]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) > nl;
+        }
+    }
     uint32_t old[WB_U], dg[WB_U], first[WB_U];
 #pragma unroll
     for (int j = 0; j < WB_U; ++j) {
@@ -208,13 +254,14 @@ k_wb_init(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__rest
     }
 }
 
+template <bool HUBS>
 __global__ void __launch_bounds__(WB_THREADS)
 k_wb_level(uint32_t n, uint32_t lvl, const uint64_t *__restrict__ index, const uint32_t *__restrict__ nbrs,
            const uint32_t *__restrict__ deg, uint32_t *level, WbLists L, WbCtl *ctl, WbRule rule, WbHost *h,
            uint32_t sub_max) {
     __shared__ uint32_t s_stage[WB_WAVES * WB_STAGE];
     __shared__ uint32_t s_n[WB_WAVES], s_act[WB_WAVES], s_base[WB_WAVES];
-    __shared__ unsigned long long s_edge[WB_WAVES];
+    __shared__ unsigned long long s_edge[WB_WAVES], s_tag[WB_TAGS];
     const unsigned ln = lane(), wv = threadIdx.x / 64;
     const uint32_t W = gridDim.x * WB_WAVES;
     // wave rank interleaved over the blocks: a small level lands on many CUs
@@ -253,11 +300,15 @@ k_wb_level(uint32_t n, uint32_t lvl, const uint64_t *__restrict__ index, const u
                 __hip_atomic_store(&h->level, lvl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
     }
+    if constexpr (HUBS) {
+        for (uint32_t i = threadIdx.x; i < WB_TAGS; i += WB_THREADS) s_tag[i] = ~0ull;
+        __syncthreads();
+    }
     // 2^lg lanes a row while there are lanes to spare (up to sub_max)
     uint32_t lg = 0;
     while ((1u << lg) < sub_max && ((uint64_t)nL << (lg + 1)) <= (uint64_t)W * 64) ++lg;
     const uint32_t sub = 1u << lg, rows = 64 >> lg;
-    WbFound f{&s_stage[wv * WB_STAGE]};
+    WbFound f{&s_stage[wv * WB_STAGE], s_tag};
     for (uint32_t base = w * rows; base < nL; base += W * rows) {
         const uint32_t i = base + (ln >> lg);
         if (lg || base != w * 64) row = L.light[cb][min(i, n - 1)];
@@ -276,7 +327,7 @@ k_wb_level(uint32_t n, uint32_t lvl, const uint64_t *__restrict__ index, const u
                 d[j] = act[j] ? nbrs[e + (j << lg)] : 0u;
             }
             e += WB_U << lg;    // < 2^26 + 64: no wrap
-            wb_relax(act, d, lvl + 1, level, index, deg, L, nb, ctl, nx, f);
+            wb_relax<HUBS>(act, d, lvl + 1, level, index, deg, L, nb, ctl, nx, f);
         }
     }
     for (uint32_t j = W - 1 - w; j < nH; j += W) {
@@ -289,7 +340,7 @@ k_wb_level(uint32_t n, uint32_t lvl, const uint64_t *__restrict__ index, const u
             act[k] = ln + 64 * k < len;
             d[k] = act[k] ? nbrs[e0 + ln + 64 * k] : 0u;
         }
-        wb_relax(act, d, lvl + 1, level, index, deg, L, nb, ctl, nx, f);
+        wb_relax<HUBS>(act, d, lvl + 1, level, index, deg, L, nb, ctl, nx, f);
     }
     // the block's stages and counts, with one reservation
     const uint32_t ta = wave_sum(f.act);
@@ -385,16 +436,33 @@ k_uf_init(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__rest
 // been hooked; after two rounds the whole run takes 0.3-0.4 ms.
 constexpr uint64_t UF_FIRST_NBRS = 4;
 constexpr int UF_ROUNDS = 2;
+constexpr uint32_t UF_TAGS = 256;
 __global__ void __launch_bounds__(UF_THREADS)
 k_uf_round(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__restrict__ nbrs, uint32_t *parent) {
     constexpr int WG = __HIP_MEMORY_SCOPE_WORKGROUP;
+    // the pairs that this workgroup tried last, and who did (as wb_claim; a
+    // join given up for nothing is found again): two hubs next to the same 2M
+    // vertices took 1.5 ms of atomics on their lines, 10 us like this
+    __shared__ unsigned long long s_pair[UF_TAGS];
+    __shared__ uint32_t s_who[UF_TAGS];
+    for (uint32_t i = threadIdx.x; i < UF_TAGS; i += UF_THREADS) s_pair[i] = ~0ull;
+    __syncthreads();
     for (uint32_t v = blockIdx.x * UF_THREADS + threadIdx.x; v < n; v += gridDim.x * UF_THREADS) {
         const uint64_t b = index[v], e = min(index[v + 1], b + UF_FIRST_NBRS);
         const uint32_t a = uf_get<WG>(parent, v);
         for (uint64_t j = b; j < e; ++j) {
             const uint32_t c = uf_get<WG>(parent, nbrs[j]);
             const uint32_t hi = a > c ? a : c, lo = a > c ? c : a;
-            if (hi != lo && uf_get<WG>(parent, hi) > lo) atomicMin(&parent[hi], lo);
+            if (hi == lo || uf_get<WG>(parent, hi) <= lo) continue;
+            const unsigned long long pair = (unsigned long long)hi << 32 | lo;
+            unsigned long long *t = s_pair + hi % UF_TAGS;
+            uint32_t *w = s_who + hi % UF_TAGS;
+            if (__hip_atomic_load(t, __ATOMIC_RELAXED, WG) == pair) continue;
+            __hip_atomic_store(t, pair, __ATOMIC_RELAXED, WG);
+            __hip_atomic_store(w, threadIdx.x, __ATOMIC_RELAXED, WG);
+            if (__hip_atomic_load(t, __ATOMIC_RELAXED, WG) == pair && __hip_atomic_load(w, __ATOMIC_RELAXED, WG) != threadIdx.x)
+                continue;
+            atomicMin(&parent[hi], lo);
         }
     }
 }
@@ -579,8 +647,9 @@ int whole_bfs(gpr_graph *g, uint32_t start, float threshold_pct, uint32_t *level
     unsigned launched = 0, polls = 0;
     while (!__atomic_load_n(&((WbHost *)g->whost)->done, __ATOMIC_ACQUIRE)) {
         if (launched - h->level < WB_AHEAD) {
-            hipLaunchKernelGGL(k_wb_level, dim3(grid), dim3(WB_THREADS), 0, g->stream, n, launched, g->index, g->nbrs,
-                               g->deg, level, L, ctl, rule, (WbHost *)g->whost_dev, sub_max);
+            hipLaunchKernelGGL(g->nlong ? k_wb_level<true> : k_wb_level<false>, dim3(grid), dim3(WB_THREADS), 0,
+                               g->stream, n, launched, g->index, g->nbrs, g->deg, level, L, ctl, rule,
+                               (WbHost *)g->whost_dev, sub_max);
             ++launched;
             GPR_HIP(hipGetLastError());
         } else if (++polls % 4096 == 0) {

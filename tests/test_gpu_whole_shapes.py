@@ -83,3 +83,34 @@ def test_bfs_of_a_large_star_is_not_slower():
         lv, _ = g.bfslvl(3)
         assert lv[3] == 0 and lv[0] == 1 and (np.delete(lv, (0, 3)) == 2).all()
         not_slower(g, "bfs")
+
+
+@pytest.mark.parametrize("reorder", [False, True])
+@pytest.mark.parametrize("hubs,n", [(1, 2050), (1, 9000), (5, 40003), (16, 30011), (257, 9001), (300, 5000)])
+def test_many_vertices_reach_the_same_few(hubs, n, reorder):
+    """Levels in which every lane of many workgroups has the same destinations, as many as there are slots to
+    remember them and more."""
+    index, nbrs = bipartite(hubs, n)
+    with G.Graph.from_csr(index, nbrs) as g:
+        if reorder:
+            g.reorder()
+        for s in (0, hubs, n - 1):
+            lv, info = g.bfslvl(s)
+            assert np.array_equal(lv, O.bfs_levels(index, nbrs, s)), s
+            G.tune_set("whole_edges", 0)
+            _, want = g.bfslvl(s)
+            G.tune_set("whole_edges", 1 << 24)
+            assert (info.iters, info.push_iters, info.edges) == (want.iters, want.push_iters, want.edges), s
+        for _ in range(3):
+            assert not g.ccv()[0].any()
+
+
+@pytest.mark.parametrize("hubs,n,app,bar", [(3, 2000003, "bfs", 1.4), (3, 2000003, "cc", 1.4), (16, 500016, "cc", 1.4),
+                                            (16, 500016, "bfs", 2.0)])
+def test_hot_destinations_are_not_queued_on(hubs, n, app, bar):
+    """(The last one's level is cheaper pulled: 211 us and 140.)"""
+    with G.Graph.from_csr(*bipartite(hubs, n)) as g:
+        lv, _ = g.bfslvl(hubs)
+        assert (lv[:hubs] == 1).all() and lv[hubs] == 0 and (lv[hubs + 1:] == 2).all()
+        ratio = min(fastest(g, app, True) / fastest(g, app, False) for _ in range(2))
+        assert ratio <= bar, ratio
