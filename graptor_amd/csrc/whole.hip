@@ -560,9 +560,25 @@ constexpr uint32_t WHOLE_STAGE_V = 1u << 18;   // results up to this many vertic
 // meshes and random graphs, of more levels, gain everywhere (8M edges 1300 /
 // 3200 and 593 / 735).  Whole CC gains to twice that: RMAT 0.1M 47 / 230, 7.6M
 // 131 / 317, 31M 257 / 457, 128M 1055 / 764; random 18M 1150 / 1840.
+// Below these limits too the host-driven run is the better one where its pulls
+// save most of the edges, or where a join's random reads leave the L2:
+//   BFS with 32 edges a vertex or more, from 2^23 edges and 2^15 vertices on
+//   (below, the levels stay in the nearer caches), but for relabelled graphs
+//   with hubs.  Whole / host-driven, results left on the device: random
+//   graphs, 250000 vertices of 60 edges 383 / 215, 500000 of 32 555 / 343,
+//   100000 of 150 198 / 169, 60000 of 250 186 / 159, but 30000 of 500 122 /
+//   184, 250000 of 30 283 / 283, 100000 of 60 208 / 211; RMAT 262144 of 55
+//   234 / 244 in its own order, relabelled 186 / 264;
+//   CC with hubs in their own order, from 2^24 edges on, or 2^23 and more
+//   than 2^20 vertices (a 4 MB L2 of parents): RMAT 33M edges 641 / 386, 31M
+//   378 / 243, 16.6M on 4M vertices 498 / 376, 15.5M on 0.5M 230 / 225.
+static bool host_driven_better(const gpr_graph *g, bool cc) {
+    if (cc) return !g->order && g->nlong && (g->m > (1u << 24) || (g->m > (1u << 23) && g->n > (1u << 20)));
+    return g->m > (1u << 23) && g->n > (1u << 15) && g->m >= 32ull * g->n && !(g->order && g->nlong);
+}
 bool whole_run(const gpr_graph *g, const gpr_run_opts &o, bool cc) {
     const double limit = std::min(tun().whole_edges * (cc ? 2.0 : 1.0), (double)(1u << WB_START_BITS));
-    if ((double)g->m > limit || (double)g->n > limit || g->n == 0) return false;
+    if ((double)g->m > limit || (double)g->n > limit || g->n == 0 || host_driven_better(g, cc)) return false;
     if (o.direction != GPR_DIR_AUTO || o.out_kind != 0 || o.trace || o.deferred_update || g->prof.on) return false;
     return cc ? o.fusion == 0 && g->symmetric && !(o.threshold_pct > 0.f) : o.fusion <= 0;
 }

@@ -496,7 +496,8 @@ int gpr_trace_get(const gpr_graph *g, gpr_iter_stats *out, int cap, int *k);
  *                       direction and output, the benchmark's own fusion
  *                       setting, no trace): graphs of at most this many edges
  *                       (CC: twice, symmetric) run without the host between
- *                       their steps (default 2^24; 0: never).  Levels, labels
+ *                       their steps (default 2^24; 0: never), but for shapes
+ *                       on which the host-driven run's pulls save more.  Levels, labels
  *                       and BFS's counts are the same; such a CC run is one
  *                       step in gpr_run_info
  *   pull_serial_max     pull rows up to this in-degree run lane-serially

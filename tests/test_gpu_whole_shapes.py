@@ -114,3 +114,26 @@ def test_hot_destinations_are_not_queued_on(hubs, n, app, bar):
         assert (lv[:hubs] == 1).all() and lv[hubs] == 0 and (lv[hubs + 1:] == 2).all()
         ratio = min(fastest(g, app, True) / fastest(g, app, False) for _ in range(2))
         assert ratio <= bar, ratio
+
+
+def test_dense_rows_are_pulled():
+    """60 edges a vertex, none above 2048: most of a dense level's edges need no look."""
+    rng = np.random.default_rng(60)
+    n = 250000
+    key = np.unique(rng.integers(0, n, 30 * n, dtype=np.uint64) * n + rng.integers(0, n, 30 * n, dtype=np.uint64))
+    src, dst = key // n, key % n
+    keep = src != dst
+    key = np.unique(np.minimum(src, dst)[keep] * n + np.maximum(src, dst)[keep])
+    index, nbrs = csr(n, key // n, key % n)
+    with G.Graph.from_csr(index, nbrs) as g:
+        assert np.array_equal(g.bfslvl(3)[0], O.bfs_levels(index, nbrs, 3))
+        not_slower(g, "bfs")
+
+
+@pytest.mark.parametrize("scale,edge_factor", [(22, 4), (20, 16)])
+def test_components_of_large_graphs_in_their_own_order(scale, edge_factor):
+    with G.Graph.rmat(scale, edge_factor) as g:
+        lab, _ = g.ccv()
+        G.tune_set("whole_edges", 0)
+        assert np.array_equal(lab, g.ccv()[0])
+        not_slower(g, "cc")
