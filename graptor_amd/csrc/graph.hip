@@ -8,6 +8,7 @@
 #include "device.hpp"
 #include "grid_sync.hpp"
 #include "label_fold.hpp"
+#include "whole.hpp"
 
 #include <stdio.h>
 #include <string.h>
@@ -102,11 +103,14 @@ static int finish_graph(gpr_graph *g, const uint64_t *host_index, const uint64_t
     // the counter read-back target: fine-grained (coherent) pinned host
     // memory that a one-wave kernel writes the sums into, so that a step's
     // counts come back with the stream's completion and no copy
-    GPR_HIP(hipHostMalloc((void **)&g->hctr, sizeof(DevCounters) + sizeof(HostScalars), hipHostMallocMapped | hipHostMallocCoherent));
+    GPR_HIP(hipHostMalloc((void **)&g->hctr, sizeof(DevCounters) + sizeof(HostScalars) + WHOLE_LINE,
+                          hipHostMallocMapped | hipHostMallocCoherent));
     GPR_HIP(hipHostGetDevicePointer((void **)&g->hctr_dev, g->hctr, 0));
     g->hsc = (HostScalars *)(g->hctr + 1);
     g->hsc_dev = (HostScalars *)(g->hctr_dev + 1);
     *g->hsc = HostScalars{};
+    g->wline = g->hsc + 1;
+    g->wline_dev = g->hsc_dev + 1;
     GPR_TRY(dev_alloc((void **)&g->dedup, sizeof(uint64_t) * nwords(n), "dedup bitmap"));
     GPR_HIP(hipMemset(g->dedup, 0, sizeof(uint64_t) * nwords(n)));
     GPR_TRY(dev_alloc((void **)&g->scan, sizeof(uint64_t) * ((size_t)n + 1), "frontier prefix"));
@@ -153,10 +157,7 @@ static void graph_free(gpr_graph *g) {
     dev_free(g->fctl);
     dev_free(g->kbuf);
     dev_free(g->kctl);
-    dev_free(g->wbuf);
-    dev_free(g->wctl);
     if (g->wstage) hipHostFree(g->wstage);
-    if (g->whost) hipHostFree(g->whost);
     if (g->ev0) hipEventDestroy(g->ev0);
     if (g->ev1) hipEventDestroy(g->ev1);
     if (g->rev0) hipEventDestroy(g->rev0);

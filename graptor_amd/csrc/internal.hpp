@@ -309,12 +309,11 @@ struct gpr_graph {
     void *kbuf = nullptr;              // k-core peeling: candidate and frontier lists (built on first use)
     size_t kbuf_bytes = 0;
     void *kctl = nullptr;              // k-core peeling: control block
-    void *wbuf = nullptr;              // whole runs (whole.hip): values, lists, results (built on first use)
-    void *wctl = nullptr;              // whole runs: control block
-    uint32_t *wstage = nullptr;        // whole runs: pinned results of small graphs, and the device's address
+    uint32_t *wstage = nullptr;        // whole runs (whole.hip): pinned results of small graphs, and the device's address
     uint32_t *wstage_dev = nullptr;
-    void *whost = nullptr;             // whole runs: pinned progress line, and the device's address
-    void *whost_dev = nullptr;
+    unsigned wstage_runs = 0;          // whole runs that could have used it before it was there
+    void *wline = nullptr;             // whole runs: the line after hsc, their progress
+    void *wline_dev = nullptr;
 };
 
 struct gpr_prop {

@@ -229,6 +229,7 @@ struct alignas(128) WbHost {
     unsigned int steps, pushes;
     unsigned long long edges;
 };
+static_assert(sizeof(WbHost) == WHOLE_LINE, "the graph keeps one line for it");
 
 // Levels n+1 but for the start's 0, the start's row as the first frontier,
 // the counts.
@@ -583,36 +584,44 @@ bool whole_run(const gpr_graph *g, const gpr_run_opts &o, bool cc) {
     return cc ? o.fusion == 0 && g->symmetric && !(o.threshold_pct > 0.f) : o.fusion <= 0;
 }
 
-struct WholeBuf {
-    uint64_t heavy_cap;
-    size_t light[2], heavy[2], out, bytes;   // byte offsets; values at 0
+// A run's device memory: blocks of the graph's pool, which keeps them for the
+// next run, beside the graph's 8 (n+1) bytes of scan scratch.  Several blocks
+// rather than one, as hipMalloc takes 0.3 ms from 2 MB on and little below:
+// the first BFS of a fresh handle on 200000 vertices and 5.5M edges takes
+// 210 us, 530 with one block, 560 with buffers of its own and staging memory
+// made whatever the destination; host-driven 410.
+struct WholeMem {
+    gpr_graph *g;
+    struct { void *p; size_t bytes; } used[4];
+    int n = 0;
+    explicit WholeMem(gpr_graph *gr) : g(gr) {}
+    WholeMem(const WholeMem &) = delete;
+    ~WholeMem() { while (n) --n, g->pool->give(used[n].p, used[n].bytes); }
+    template <class T> int take(T **p, size_t bytes, const char *what) {
+        void *q = nullptr;
+        GPR_TRY(g->pool->take(&q, bytes, what));
+        used[n++] = {q, bytes};
+        *p = (T *)q;
+        return GPR_OK;
+    }
 };
-static WholeBuf whole_layout(const gpr_graph *g) {
-    WholeBuf b;
-    const uint64_t long_rows = std::min<uint64_t>(g->n, g->m / (WB_LIGHT + 1));
-    b.heavy_cap = g->m / WB_SLICE + long_rows + 64;
-    auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
-    const size_t v = up(4ull * g->n);
-    b.light[0] = v;
-    b.light[1] = 2 * v;
-    b.heavy[0] = 3 * v;
-    b.heavy[1] = b.heavy[0] + up(8 * b.heavy_cap);
-    b.out = b.heavy[1] + up(8 * b.heavy_cap);
-    b.bytes = b.out + v;
-    return b;
-}
-static int whole_ensure(gpr_graph *g, const WholeBuf &b) {
-    if (!g->wbuf) GPR_TRY(dev_alloc(&g->wbuf, b.bytes, "whole-run buffers"));
-    if (!g->wctl) GPR_TRY(dev_alloc(&g->wctl, sizeof(WbCtl), "whole-run control"));
-    if (!g->whost) {
-        GPR_HIP(hipHostMalloc(&g->whost, sizeof(WbHost), hipHostMallocMapped | hipHostMallocCoherent));
-        GPR_HIP(hipHostGetDevicePointer(&g->whost_dev, g->whost, 0));
+
+// Pinned memory for n results that go to a buffer the device cannot write:
+// small graphs', from the second such run on.
+static uint32_t *whole_stage(gpr_graph *g) {
+    if (g->n > WHOLE_STAGE_V || (!g->wstage && g->wstage_runs++ == 0)) return nullptr;
+    if (!g->wstage) {
+        void *p = nullptr, *d = nullptr;
+        if (hipHostMalloc(&p, 4ull * g->n, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
+            hipHostGetDevicePointer(&d, p, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            if (p) hipHostFree(p);
+            return nullptr;
+        }
+        g->wstage = (uint32_t *)p;
+        g->wstage_dev = (uint32_t *)d;
     }
-    if (!g->wstage && g->n <= WHOLE_STAGE_V) {
-        GPR_HIP(hipHostMalloc((void **)&g->wstage, 4ull * g->n, hipHostMallocMapped | hipHostMallocCoherent));
-        GPR_HIP(hipHostGetDevicePointer((void **)&g->wstage_dev, g->wstage, 0));
-    }
-    return GPR_OK;
+    return g->wstage_dev;
 }
 // Waits for the stream; the n results at dev (the staging memory or the
 // device) into host, when asked for.
@@ -636,15 +645,18 @@ constexpr uint64_t WB_BLOCK_EDGES = 4096;
 constexpr uint64_t WB_MIN_BLOCKS = 128;
 
 int whole_bfs(gpr_graph *g, uint32_t start, float threshold_pct, uint32_t *levels, gpr_run_info *info) {
-    const WholeBuf b = whole_layout(g);
-    GPR_TRY(whole_ensure(g, b));
-    char *base = (char *)g->wbuf;
     const uint32_t n = g->n;
-    uint32_t *level = (uint32_t *)base;
     const uint32_t *perm = g->order ? g->perm : nullptr;
-    WbLists L = {{(uint32_t *)(base + b.light[0]), (uint32_t *)(base + b.light[1])},
-                 {(uint64_t *)(base + b.heavy[0]), (uint64_t *)(base + b.heavy[1])}};
-    WbCtl *ctl = (WbCtl *)g->wctl;
+    // a level's slices: each row of more than WB_LIGHT edges has one at least
+    const uint64_t nheavy = g->m / WB_SLICE + std::min<uint64_t>(n, g->m / (WB_LIGHT + 1)) + 64;
+    WholeMem mem(g);
+    uint32_t *level = nullptr;
+    WbCtl *ctl = nullptr;
+    WbLists L = {{(uint32_t *)g->scan, (uint32_t *)g->scan + n}, {nullptr, nullptr}};
+    GPR_TRY(mem.take(&level, 4ull * n, "levels"));
+    GPR_TRY(mem.take(&L.heavy[0], 8 * nheavy, "whole BFS lists"));
+    GPR_TRY(mem.take(&L.heavy[1], 8 * nheavy, "whole BFS lists"));
+    GPR_TRY(mem.take(&ctl, sizeof(WbCtl), "whole BFS control"));
     WbRule rule = {g->m / 20, 0.0, 0};
     if (threshold_pct > 0.f) {
         rule.frac = 1;
@@ -654,18 +666,19 @@ int whole_bfs(gpr_graph *g, uint32_t start, float threshold_pct, uint32_t *level
     // lanes that an average row keeps busy for one step
     uint32_t sub_max = 1;
     while (sub_max * WB_U < WB_LIGHT && (uint64_t)sub_max * WB_U * n < g->m) sub_max *= 2;
-    volatile WbHost *h = (volatile WbHost *)g->whost;
+    WbHost *const hline = (WbHost *)g->wline;
+    volatile WbHost *h = hline;
     h->level = 0;
     h->done = 0;
     stream_time_ms(g, true);
     hipLaunchKernelGGL(k_wb_init, dim3(grid_for(n, WB_THREADS, 1024)), dim3(WB_THREADS), 0, g->stream, n, g->index,
                        g->deg, perm, start, level, L, ctl);
     unsigned launched = 0, polls = 0;
-    while (!__atomic_load_n(&((WbHost *)g->whost)->done, __ATOMIC_ACQUIRE)) {
+    while (!__atomic_load_n(&hline->done, __ATOMIC_ACQUIRE)) {
         if (launched - h->level < WB_AHEAD) {
             hipLaunchKernelGGL(g->nlong ? k_wb_level<true> : k_wb_level<false>, dim3(grid), dim3(WB_THREADS), 0,
                                g->stream, n, launched, g->index, g->nbrs, g->deg, level, L, ctl, rule,
-                               (WbHost *)g->whost_dev, sub_max);
+                               (WbHost *)g->wline_dev, sub_max);
             ++launched;
             GPR_HIP(hipGetLastError());
         } else if (++polls % 4096 == 0) {
@@ -676,7 +689,9 @@ int whole_bfs(gpr_graph *g, uint32_t start, float threshold_pct, uint32_t *level
     }
     stream_time_mark(g);
     uint32_t *const target = (uint32_t *)host_target(levels, 4ull * n);
-    uint32_t *out = target ? target : g->wstage ? g->wstage_dev : (uint32_t *)(base + b.out);
+    uint32_t *out = target;
+    if (levels && !out) out = whole_stage(g);
+    if (!out) out = L.light[0];    // the levels left in flight find no rows
     if (levels)
         hipLaunchKernelGGL(k_wb_out, dim3(grid_for(n, WB_THREADS, 1024)), dim3(WB_THREADS), 0, g->stream, n, level,
                            perm, out);
@@ -690,15 +705,16 @@ int whole_bfs(gpr_graph *g, uint32_t start, float threshold_pct, uint32_t *level
 }
 
 int whole_cc(gpr_graph *g, uint32_t *labels, gpr_run_info *info) {
-    const WholeBuf b = whole_layout(g);
-    GPR_TRY(whole_ensure(g, b));
-    char *base = (char *)g->wbuf;
     const uint32_t n = g->n;
-    uint32_t *parent = (uint32_t *)base;
-    // the recode (labels asked for, vertices relabelled): minima by original ID
-    uint32_t *minorig = labels && g->order ? (uint32_t *)(base + b.light[0]) : nullptr;
     uint32_t *const target = (uint32_t *)host_target(labels, 4ull * n);
-    uint32_t *out = !labels ? nullptr : target ? target : g->wstage ? g->wstage_dev : (uint32_t *)(base + b.out);
+    uint32_t *out = target;
+    if (labels && !out) out = whole_stage(g);
+    // the recode (labels asked for, vertices relabelled): minima by original ID
+    uint32_t *minorig = labels && g->order ? (uint32_t *)g->scan : nullptr;
+    if (labels && !out) out = (uint32_t *)g->scan + n;
+    WholeMem mem(g);
+    uint32_t *parent = nullptr;
+    GPR_TRY(mem.take(&parent, 4ull * n, "parents"));
     const unsigned grid = grid_for(n, UF_THREADS, 4096);
     stream_time_ms(g, true);
     hipLaunchKernelGGL(k_uf_init, dim3(grid), dim3(UF_THREADS), 0, g->stream, n, g->index, g->nbrs, parent, minorig);

@@ -2,8 +2,12 @@
 // their steps (whole.hip).
 #pragma once
 #include "../../include/gpr.h"
+#include <stddef.h>
 
 namespace gpr {
+
+// Bytes of pinned memory that a run reports its progress in (gpr_graph::wline).
+constexpr size_t WHOLE_LINE = 128;
 
 // Whether a run with these options takes that form: the benchmark's default
 // schedule, nothing traced or profiled, a graph of at most whole_edges edges

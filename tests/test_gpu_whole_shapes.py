@@ -12,6 +12,7 @@ import oracle as O
 
 pytestmark = pytest.mark.gpu
 G = pytest.importorskip("graptor_amd")
+torch = pytest.importorskip("torch")
 
 
 @pytest.fixture(autouse=True)
@@ -137,3 +138,44 @@ def test_components_of_large_graphs_in_their_own_order(scale, edge_factor):
         G.tune_set("whole_edges", 0)
         assert np.array_equal(lab, g.ccv()[0])
         not_slower(g, "cc")
+
+
+def first_call(index, nbrs, whole, pinned):
+    """Median time of the first BFS on a handle."""
+    G.tune_set("whole_edges", (1 << 24) if whole else 0)
+    out = torch.empty(len(index) - 1, dtype=torch.int32, pin_memory=pinned).numpy()
+    took = []
+    for _ in range(11):
+        with G.Graph.from_csr(index, nbrs) as g:
+            g.reorder()
+            t = time.perf_counter()
+            info_call(g, "bfs", out)
+            took.append(time.perf_counter() - t)
+    return sorted(took)[5]
+
+
+@pytest.mark.parametrize("pinned", [False, True])
+def test_first_bfs_on_a_handle(pinned):
+    """A program that runs one BFS a graph pays for no more than the host-driven run's buffers."""
+    index, nbrs = O.rmat_graph(17)
+    ratio = min(first_call(index, nbrs, True, pinned) / first_call(index, nbrs, False, pinned) for _ in range(2))
+    assert ratio <= 1.1, ratio
+
+
+@pytest.mark.parametrize("n", [70, 4099, 300007])
+def test_buffers_shared_by_the_runs_of_a_handle(n):
+    """Whole runs keep lists, minima and results in scratch that conversions, scans and downloads use as well."""
+    k = np.arange(3 * n, dtype=np.uint64)
+    index, nbrs = O.build_csr(n, (k * 7919 % n).astype(np.uint32), (k * k * 31 % n).astype(np.uint32))
+    levels, labels = O.bfs_levels(index, nbrs, 1), O.cc_labels(index, nbrs)
+    with G.Graph.from_csr(index, nbrs) as g:
+        g.reorder()
+        p = g.prop()
+        p.upload(np.arange(n, dtype=np.uint32))
+        for _ in range(3):
+            assert np.array_equal(g.bfslvl(1)[0], levels)
+            assert np.array_equal(p.download(), np.arange(n))
+            assert np.array_equal(g.ccv()[0], labels)
+            assert np.array_equal(g.bfslvl(1, direction=G.DIR_PUSH)[0], levels)
+            assert np.array_equal(g.msbfs([1, n - 1])[0][0], levels)
+        p.destroy()
