@@ -64,7 +64,9 @@ void dev_free(void *p);
 
 // Where the device can write a caller's result of `bytes` bytes: the device
 // address of pinned host memory that holds all of it, else nullptr.
-void *host_target(void *host, size_t bytes);
+// *copy_only: the host may not touch the buffer either (device memory, which
+// the runtime's copies take).
+void *host_target(void *host, size_t bytes, bool *copy_only = nullptr);
 
 // Device blocks of one graph's runs (properties, 64-source BFS levels), kept
 // for its next run: a run makes and drops the same sizes every time, and

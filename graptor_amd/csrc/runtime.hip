@@ -19,12 +19,15 @@ void set_error(const char *fmt, ...) {
     va_end(ap);
 }
 
-void *host_target(void *host, size_t bytes) {
+void *host_target(void *host, size_t bytes, bool *copy_only) {
     hipPointerAttribute_t a = {};
     hipDeviceptr_t base = nullptr;
     size_t size = 0;
+    if (copy_only) *copy_only = false;
     if (!host || !bytes) return nullptr;
-    if (hipPointerGetAttributes(&a, host) != hipSuccess || a.type != hipMemoryTypeHost || !a.devicePointer ||
+    const bool known = hipPointerGetAttributes(&a, host) == hipSuccess;
+    if (copy_only) *copy_only = known && a.type != hipMemoryTypeHost && a.type != hipMemoryTypeUnregistered;
+    if (!known || a.type != hipMemoryTypeHost || !a.devicePointer ||
         hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)a.devicePointer) != hipSuccess) {
         (void)hipGetLastError();    // pageable memory is an error to some of these
         return nullptr;

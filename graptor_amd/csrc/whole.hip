@@ -688,9 +688,10 @@ int whole_bfs(gpr_graph *g, uint32_t start, float threshold_pct, uint32_t *level
         }
     }
     stream_time_mark(g);
-    uint32_t *const target = (uint32_t *)host_target(levels, 4ull * n);
+    bool copy_only = false;
+    uint32_t *const target = (uint32_t *)host_target(levels, 4ull * n, &copy_only);
     uint32_t *out = target;
-    if (levels && !out) out = whole_stage(g);
+    if (levels && !out && !copy_only) out = whole_stage(g);
     if (!out) out = L.light[0];    // the levels left in flight find no rows
     if (levels)
         hipLaunchKernelGGL(k_wb_out, dim3(grid_for(n, WB_THREADS, 1024)), dim3(WB_THREADS), 0, g->stream, n, level,
@@ -706,9 +707,10 @@ int whole_bfs(gpr_graph *g, uint32_t start, float threshold_pct, uint32_t *level
 
 int whole_cc(gpr_graph *g, uint32_t *labels, gpr_run_info *info) {
     const uint32_t n = g->n;
-    uint32_t *const target = (uint32_t *)host_target(labels, 4ull * n);
+    bool copy_only = false;
+    uint32_t *const target = (uint32_t *)host_target(labels, 4ull * n, &copy_only);
     uint32_t *out = target;
-    if (labels && !out) out = whole_stage(g);
+    if (labels && !out && !copy_only) out = whole_stage(g);
     // the recode (labels asked for, vertices relabelled): minima by original ID
     uint32_t *minorig = labels && g->order ? (uint32_t *)g->scan : nullptr;
     if (labels && !out) out = (uint32_t *)g->scan + n;
