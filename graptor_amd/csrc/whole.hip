@@ -674,17 +674,27 @@ int whole_bfs(gpr_graph *g, uint32_t start, float threshold_pct, uint32_t *level
     hipLaunchKernelGGL(k_wb_init, dim3(grid_for(n, WB_THREADS, 1024)), dim3(WB_THREADS), 0, g->stream, n, g->index,
                        g->deg, perm, start, level, L, ctl);
     unsigned launched = 0, polls = 0;
+    hipError_t e = hipGetLastError();
     while (!__atomic_load_n(&hline->done, __ATOMIC_ACQUIRE)) {
         if (launched - h->level < WB_AHEAD) {
             hipLaunchKernelGGL(g->nlong ? k_wb_level<true> : k_wb_level<false>, dim3(grid), dim3(WB_THREADS), 0,
                                g->stream, n, launched, g->index, g->nbrs, g->deg, level, L, ctl, rule,
                                (WbHost *)g->wline_dev, sub_max);
             ++launched;
-            GPR_HIP(hipGetLastError());
+            e = hipGetLastError();
         } else if (++polls % 4096 == 0) {
             // a stream that failed would never report a level
-            const hipError_t e = hipStreamQuery(g->stream);
-            if (e != hipSuccess && e != hipErrorNotReady) GPR_HIP(e);
+            e = hipStreamQuery(g->stream);
+            if (e == hipErrorNotReady) {
+                e = hipSuccess;
+                (void)hipGetLastError();
+            }
+        }
+        if (e != hipSuccess) {
+            // the queued levels still write the progress line, which the next
+            // run of the handle resets
+            (void)hipStreamSynchronize(g->stream);
+            GPR_HIP(e);
         }
     }
     stream_time_mark(g);
