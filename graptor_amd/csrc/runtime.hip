@@ -118,6 +118,7 @@ int dev_alloc(void **p, size_t bytes, const char *what) {
         e = hipMalloc(p, bytes);
     }
     if (e != hipSuccess) {
+        (void)hipGetLastError();    // not the next launch's error
         set_error("hipMalloc(%zu) for %s failed: %s", bytes, what, hipGetErrorString(e));
         *p = nullptr;
         return GPR_E_OOM;
