@@ -79,6 +79,14 @@ template <class F> int guarded(F &&f) {
     }
 }
 
+// Whether a whole run came to its end; without memory for its lists the
+// host-driven run, which needs less, is left to try.
+bool whole_done(int rc, const char *what) {
+    if (rc == GPR_E_OOM) return false;
+    check(rc, what);
+    return true;
+}
+
 // ---- BFSLVLv -----------------------------------------------------------------
 struct BFSLVLv {
     Graph GA;
@@ -607,8 +615,8 @@ extern "C" int gpr_bfslvl(gpr_graph *g, uint32_t start, const gpr_run_opts *opts
     if (start >= n) return guarded([&] { check(GPR_E_INVAL, "bfslvl: start vertex out of range"); });
     return guarded([&] {
         gpr_run_info local = {};
-        if (whole_run(g, o, false)) {
-            check(whole_bfs(g, start, o.threshold_pct, levels, &local), "bfslvl");
+        if (whole_run(g, o, false) &&
+            whole_done(whole_bfs(g, start, o.threshold_pct, levels, &local), "bfslvl")) {
             if (info) *info = local;
             return;
         }
@@ -646,8 +654,7 @@ extern "C" int gpr_ccv(gpr_graph *g, const gpr_run_opts *opts, uint32_t *labels,
     gpr_run_opts o = defaults(opts);
     return guarded([&] {
         gpr_run_info local = {};
-        if (whole_run(g, o, true)) {
-            check(whole_cc(g, labels, &local), "ccv");
+        if (whole_run(g, o, true) && whole_done(whole_cc(g, labels, &local), "ccv")) {
             if (info) *info = local;
             return;
         }

@@ -56,8 +56,22 @@ g.destroy()
 print("ok")
 """
 
+HOST_DRIVEN = START + r"""
+slices = 8 * (m // 256 + min(n, m // 33) + 64)
+low.value, high.value = slices, slices + 1         # a whole BFS's slice lists
+lv, info = g.bfslvl(5)
+assert refused.value > 0, "the slice lists were not asked for"
+assert np.array_equal(lv, levels)
+high.value = 0
+lv, again = g.bfslvl(5)
+assert np.array_equal(lv, levels) and (info.iters, info.edges) == (again.iters, again.edges)
+assert np.array_equal(g.ccv()[0], labels)
+g.destroy()
+print("ok")
+"""
 
-@pytest.mark.parametrize("script", [REPORTED_ONCE])
+
+@pytest.mark.parametrize("script", [REPORTED_ONCE, HOST_DRIVEN], ids=["reported_once", "host_driven"])
 def test_refused_allocations(tmp_path, script):
     src, so = tmp_path / "shim.c", tmp_path / "shim.so"
     src.write_text(SHIM)
