@@ -116,6 +116,7 @@ struct Tunables {
 };
 Tunables &tun();
 int num_cus();
+int wall_clock_khz();   // of wall_clock64()
 
 // ---- device-resident counters of one handle ------------------------------
 // The frontier counts are striped: workgroup b adds its totals to stripe

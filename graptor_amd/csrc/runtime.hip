@@ -233,6 +233,17 @@ int num_cus() {
     return cus;
 }
 
+int wall_clock_khz() {
+    static int khz = 0;
+    if (!khz) {
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess || khz <= 0)
+            khz = 100000;
+    }
+    return khz;
+}
+
 std::vector<gpr_iter_stats> &trace_of(gpr_graph *g) { return g->trace; }
 void trace_clear(gpr_graph *g) { g->trace.clear(); }
 

@@ -419,7 +419,8 @@ __device__ __forceinline__ void uf_join(uint32_t *parent, uint32_t a, uint32_t b
 
 __global__ void __launch_bounds__(UF_THREADS)
 k_uf_init(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__restrict__ nbrs, uint32_t *parent,
-          uint32_t *minorig) {
+          uint32_t *minorig, unsigned long long *began) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *began = wall_clock64();
     for (uint32_t v = blockIdx.x * UF_THREADS + threadIdx.x; v < n; v += gridDim.x * UF_THREADS) {
         const uint64_t b = index[v];
         uint32_t p = v;
@@ -520,18 +521,17 @@ k_uf_link(uint32_t nbuckets, const uint32_t *__restrict__ bucket, const uint64_t
 }
 
 // Every vertex under its root; with minorig, the components' smallest
-// original IDs at the roots too, with out the roots as results.  A launch of
-// its own, so no root is hooked meanwhile.  A few parents may still be inner
-// ancestors afterwards: halving stores of other threads that come late.
+// original IDs at the roots too.  A launch of its own, so no root is hooked
+// meanwhile.  A few parents may still be inner ancestors afterwards: halving
+// stores of other threads that come late.
 __global__ void __launch_bounds__(LF_THREADS)
-k_uf_flatten(uint32_t n, uint32_t *parent, const uint32_t *__restrict__ order, uint32_t *minorig, uint32_t *out) {
+k_uf_flatten(uint32_t n, uint32_t *parent, const uint32_t *__restrict__ order, uint32_t *minorig) {
     constexpr int WG = __HIP_MEMORY_SCOPE_WORKGROUP;
     LabelFold f;
     for (uint64_t i = blockIdx.x * (uint64_t)LF_THREADS + threadIdx.x; i < n; i += (uint64_t)gridDim.x * LF_THREADS) {
         const uint32_t r = uf_root<WG>(parent, (uint32_t)i);
         __hip_atomic_store(&parent[i], r, __ATOMIC_RELAXED, WG);
         if (minorig) f.add(minorig, i, r, order[i]);
-        if (out) out[i] = r;
     }
     if (minorig) f.finish(minorig);
 }
@@ -547,9 +547,12 @@ __device__ __forceinline__ uint32_t uf_top(const uint32_t *__restrict__ parent, 
 }
 __global__ void __launch_bounds__(UF_THREADS)
 k_uf_out(uint32_t n, const uint32_t *__restrict__ parent, const uint32_t *__restrict__ perm,
-         const uint32_t *__restrict__ minorig, uint32_t *out) {
-    for (uint32_t o = blockIdx.x * UF_THREADS + threadIdx.x; o < n; o += gridDim.x * UF_THREADS)
-        out[o] = minorig[uf_top(parent, perm[o])];
+         const uint32_t *__restrict__ minorig, uint32_t *out, unsigned long long *ended) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *ended = wall_clock64();
+    for (uint32_t o = blockIdx.x * UF_THREADS + threadIdx.x; o < n; o += gridDim.x * UF_THREADS) {
+        const uint32_t r = uf_top(parent, perm ? perm[o] : o);
+        out[o] = minorig ? minorig[r] : r;
+    }
 }
 
 // ---- host side ------------------------------------------------------------------
@@ -728,8 +731,14 @@ int whole_cc(gpr_graph *g, uint32_t *labels, gpr_run_info *info) {
     uint32_t *parent = nullptr;
     GPR_TRY(mem.take(&parent, 4ull * n, "parents"));
     const unsigned grid = grid_for(n, UF_THREADS, 4096);
-    stream_time_ms(g, true);
-    hipLaunchKernelGGL(k_uf_init, dim3(grid), dim3(UF_THREADS), 0, g->stream, n, g->index, g->nbrs, parent, minorig);
+    // The run's time ends before the labels go out.  Kernels write the clock
+    // (clk) where labels follow: an event between them takes 5 of the 48 us of
+    // 4096 vertices.
+    volatile unsigned long long *const clk = (unsigned long long *)g->wline;
+    unsigned long long *const clk_dev = (unsigned long long *)g->wline_dev;
+    if (!labels) stream_time_ms(g, true);
+    hipLaunchKernelGGL(k_uf_init, dim3(grid), dim3(UF_THREADS), 0, g->stream, n, g->index, g->nbrs, parent, minorig,
+                       clk_dev);
     // a hub next to 1/32 of the vertices, with the smallest ID (relabelled by
     // degree), already holds most of its component: the rounds would cost
     // their launches (10-14 us) and save nothing
@@ -738,21 +747,22 @@ int whole_cc(gpr_graph *g, uint32_t *labels, gpr_run_info *info) {
     for (int k = 0; !hub && k < UF_ROUNDS; ++k) {
         if (k == 0)
             hipLaunchKernelGGL(k_uf_flatten, fgrid, dim3(LF_THREADS), 0, g->stream, n, parent, (const uint32_t *)nullptr,
-                               (uint32_t *)nullptr, (uint32_t *)nullptr);
+                               (uint32_t *)nullptr);
         hipLaunchKernelGGL(k_uf_round, dim3(grid), dim3(UF_THREADS), 0, g->stream, n, g->index, g->nbrs, parent);
         hipLaunchKernelGGL(k_uf_flatten, fgrid, dim3(LF_THREADS), 0, g->stream, n, parent, (const uint32_t *)nullptr,
-                           (uint32_t *)nullptr, (uint32_t *)nullptr);
+                           (uint32_t *)nullptr);
     }
     hipLaunchKernelGGL(k_uf_link, dim3(g->nbuckets + g->nlong_chunks), dim3(UF_THREADS), 0, g->stream, g->nbuckets,
                        g->bucket, g->index, g->nbrs, g->long_rows, g->long_base, g->nlong, parent);
-    hipLaunchKernelGGL(k_uf_flatten, fgrid, dim3(LF_THREADS), 0, g->stream, n, parent, g->order, minorig,
-                       minorig ? nullptr : out);
-    if (minorig)
-        hipLaunchKernelGGL(k_uf_out, dim3(grid), dim3(UF_THREADS), 0, g->stream, n, parent, g->perm, minorig, out);
+    hipLaunchKernelGGL(k_uf_flatten, fgrid, dim3(LF_THREADS), 0, g->stream, n, parent, g->order, minorig);
+    if (labels)
+        hipLaunchKernelGGL(k_uf_out, dim3(grid), dim3(UF_THREADS), 0, g->stream, n, parent,
+                           g->order ? g->perm : nullptr, minorig, out, clk_dev + 1);
+    else
+        stream_time_mark(g);
     GPR_HIP(hipGetLastError());
-    stream_time_mark(g);
     GPR_TRY(whole_results(g, out, labels, target));
-    info->ms = stream_time_read_ms(g);
+    info->ms = labels ? (double)(clk[1] - clk[0]) / wall_clock_khz() : stream_time_read_ms(g);
     // one step, over every edge
     info->iters = 1;
     info->push_iters = 1;

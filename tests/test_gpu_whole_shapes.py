@@ -179,3 +179,20 @@ def test_buffers_shared_by_the_runs_of_a_handle(n):
             assert np.array_equal(g.bfslvl(1, direction=G.DIR_PUSH)[0], levels)
             assert np.array_equal(g.msbfs([1, n - 1])[0][0], levels)
         p.destroy()
+
+
+@pytest.mark.parametrize("reorder", [False, True])
+def test_time_of_a_run_leaves_out_its_results(reorder):
+    """info->ms is run()'s alone, as for a host-driven run: 32 MB of labels take 0.6 ms more over the link than no
+    labels, and the run itself 0.1 to 0.2."""
+    n = 8000000
+    out = torch.empty(n, dtype=torch.int32, pin_memory=True).numpy()
+    with G.Graph.from_csr(*bipartite(1, n)) as g:
+        if reorder:
+            g.reorder()
+        ms = {}
+        for dst in (None, out):
+            for _ in range(7):
+                ms[dst is None] = min(ms.get(dst is None, 1e9), info_call(g, "cc", dst).ms)
+        assert not out.any()
+        assert 0 < ms[False] <= ms[True] + 0.3, ms
