@@ -20,9 +20,11 @@
 //   k_pr_update  x' = (y + w) / s, |x - x'| partials, x = x', contrib =
 //                d*x'/deg encoded in the contribution format; the last
 //                workgroup sums the residual partials into delta.
-// FP32 contributions are accumulated in FP64 registers as PRv does (y_acc
-// is double over FP32 storage, PRv.C:127); 16-bit contributions are
-// accumulated in FP32.
+// Contributions of every format are accumulated in FP64 registers, as PRv
+// does (y_acc is double over FP32 storage, PRv.C:127): a row's sum does not
+// depend on whether it is pulled or binned, but for the last rounding.  With
+// FP32 registers for 16-bit formats it would (20 iterations on RMAT with 60000
+// vertices take 370 us either way, bf16).
 #include "internal.hpp"
 #include "device.hpp"
 #include "pr_codec.hpp"
@@ -66,8 +68,6 @@ k_pr_pull(uint32_t nbuckets, const uint32_t *__restrict__ bucket, const uint64_t
           const uint32_t *__restrict__ long_rows, const uint32_t *__restrict__ long_base, uint32_t nlong,
           double *__restrict__ long_partial, double *part, float *part_max, const PrScalars *prs,
           uint32_t cold_from, PrFold fold, int long_here) {
-    using C = Codec<FMT>;
-    using acc_t = typename C::acc_t;
     __shared__ float vals[PR_LDS_EDGES];
     __shared__ uint32_t rs[STREAM_ITEMS + 1];
     __shared__ uint32_t medq[PR_LDS_EDGES / PR_MED + 1];
@@ -90,7 +90,7 @@ k_pr_pull(uint32_t nbuckets, const uint32_t *__restrict__ bucket, const uint64_t
         const uint64_t rb = cindex[row], re = cindex[row + 1];
         const uint64_t cb = rb + (uint64_t)(c - long_base[li]) * LONG_CHUNK;
         const uint64_t ce = min(re, cb + LONG_CHUNK);
-        acc_t acc = 0;
+        double acc = 0.0;
         // PR_UNROLL independent neighbour loads, then as many gathers, in
         // flight per lane
         for (uint64_t base = cb; base < ce; base += (uint64_t)PR_THREADS * PR_UNROLL) {
@@ -103,9 +103,9 @@ k_pr_pull(uint32_t nbuckets, const uint32_t *__restrict__ bucket, const uint64_t
             float v[PR_UNROLL];
             gather_all<FMT>(contrib, s, cold_from, v);
 #pragma unroll
-            for (int u = 0; u < PR_UNROLL; ++u) acc += (acc_t)v[u];
+            for (int u = 0; u < PR_UNROLL; ++u) acc += (double)v[u];
         }
-        double tot = block_sum((double)acc, dred);
+        double tot = block_sum(acc, dred);
         if (threadIdx.x == 0) {
             st_part(&long_partial[c], tot);
             st_part(&part[b], 0.0);
@@ -164,8 +164,8 @@ k_pr_pull(uint32_t nbuckets, const uint32_t *__restrict__ bucket, const uint64_t
                     medq[atomicAdd(&nmed, 1u)] = i;
                     continue;
                 }
-                acc_t acc = 0;
-                for (uint32_t j = a; j < z; ++j) acc += (acc_t)vals[j];
+                double acc = 0.0;
+                for (uint32_t j = a; j < z; ++j) acc += (double)vals[j];
                 const float yv = (float)acc * dscale;
                 y[r0 + i] = yv;
                 my_sum += (double)yv;
@@ -180,8 +180,8 @@ k_pr_pull(uint32_t nbuckets, const uint32_t *__restrict__ bucket, const uint64_t
             for (uint32_t q = w; q < nm; q += PR_THREADS / 64) {
                 const uint32_t i = medq[q];
                 const uint32_t a = rs[i], z = rs[i + 1];
-                acc_t acc = 0;
-                for (uint32_t j = a + ln; j < z; j += 64) acc += (acc_t)vals[j];
+                double acc = 0.0;
+                for (uint32_t j = a + ln; j < z; j += 64) acc += (double)vals[j];
                 acc = wave_sum(acc);
                 if (ln == 0) {
                     const float yv = (float)acc * dscale;

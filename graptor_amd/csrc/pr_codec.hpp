@@ -1,6 +1,6 @@
 // pr_codec.hpp -- PageRank contribution formats (stored value <-> float).
 //
-// FP32 (PRv, accumulated in FP64 as PRv.C:127 does), bfloat16 with
+// FP32 (PRv), bfloat16 with
 // round-to-nearest-even, bfloat16 by truncation (scustomfp<true,8,7>),
 // IEEE half with a per-iteration power-of-two scale, customfp<6,10>
 // (customfp.h:95-117 encode, :141-169 decode) and the signed
@@ -13,14 +13,12 @@ namespace gpr {
 template <int FMT> struct Codec;
 template <> struct Codec<GPR_CONTRIB_F32> {
     using store_t = float;
-    using acc_t = double;
     __device__ static float dec(float v) { return v; }
     __device__ static float enc(float v) { return v; }
 };
 // bfloat16, round to nearest even
 template <> struct Codec<GPR_CONTRIB_BF16> {
     using store_t = uint16_t;
-    using acc_t = float;
     __device__ static float dec(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
     __device__ static uint16_t enc(float f) {
         uint32_t u = __float_as_uint(f);
@@ -34,7 +32,6 @@ template <> struct Codec<GPR_CONTRIB_BF16> {
 // (customfp.h:95-117 with S=true, E=8, M=7, B=0)
 template <> struct Codec<GPR_CONTRIB_BF16T> {
     using store_t = uint16_t;
-    using acc_t = float;
     __device__ static float dec(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
     __device__ static uint16_t enc(float f) { return (uint16_t)(__float_as_uint(f) >> 16); }
 };
@@ -42,7 +39,6 @@ template <> struct Codec<GPR_CONTRIB_BF16T> {
 // 2^k so that the largest contribution sits near the top of the range
 template <> struct Codec<GPR_CONTRIB_F16> {
     using store_t = uint16_t;
-    using acc_t = float;
     __device__ static float dec(uint16_t h) {
         _Float16 x;
         __builtin_memcpy(&x, &h, 2);
@@ -60,7 +56,6 @@ template <> struct Codec<GPR_CONTRIB_F16> {
 // covers [2^-63, 2) (customfp.h:95-117 encode, :141-169 decode)
 template <> struct Codec<GPR_CONTRIB_CFP16> {
     using store_t = uint16_t;
-    using acc_t = float;
     __device__ static float dec(uint16_t h) { return __uint_as_float(((uint32_t)h | 0x10000u) << 13); }
     __device__ static uint16_t enc(float f) { return (uint16_t)(__float_as_uint(f) >> 13); }
 };
@@ -72,7 +67,6 @@ template <> struct Codec<GPR_CONTRIB_CFP16> {
 // (target/conversion.h:150-189).
 template <> struct Codec<GPR_CONTRIB_SCFP16> {
     using store_t = uint16_t;
-    using acc_t = float;
     __device__ static float dec(uint16_t h) {
         const uint32_t t = ((uint32_t)(h & 0x8000u) << 16) | 0x20000000u | ((uint32_t)(h & 0x7fffu) << 14);
         return h ? __uint_as_float(t) : 0.0f;

@@ -164,9 +164,10 @@ enum {                      /* traversal direction / threshold */
     GPR_DIR_PULL = 2,        /* always_dense */
     GPR_DIR_POLICY = 3       /* learned policy (gpr_policy_*) */
 };
-enum {                      /* contribution storage for GPR_RELAX_PR_SUM */
-    GPR_CONTRIB_F32 = 0,     /* FP32 store, FP64 accumulate (PRv) */
-    GPR_CONTRIB_BF16 = 1,    /* bfloat16 RNE store, FP32 accumulate */
+enum {                      /* contribution storage for GPR_RELAX_PR_SUM;
+                               sums in FP64 or 64-bit fixed point */
+    GPR_CONTRIB_F32 = 0,     /* FP32 store (PRv) */
+    GPR_CONTRIB_BF16 = 1,    /* bfloat16 RNE store */
     GPR_CONTRIB_F16 = 2,     /* IEEE half + per-iteration 2^k scale */
     GPR_CONTRIB_CFP16 = 3,   /* customfp<6,10> truncating (customfp.h) */
     GPR_CONTRIB_BF16T = 4,   /* scustomfp<true,8,7>: bf16 truncating */
