@@ -43,9 +43,9 @@
 // lane per vertex (KC_SUB lanes in small rounds), longer rows one wave per
 // KC_SLICE-edge slice.  Light appends are staged per wave in LDS and reserved
 // in the shared list once per KC_STAGE entries, heavy slices are reserved per
-// wave step.  List counts rotate over three slots per round and level minima over two slots
-// per level, each cleared one phase after its last read and at least one
-// barrier before its next write.
+// wave step.  List counts rotate over three slots (kcore_slots.hpp) and
+// level minima over three per level, each cleared one phase after its last read
+// and at least one barrier before its next write.
 // Memory ordering and the barrier: grid_sync.hpp.  Termination: every block
 // reads the same minimum after a barrier and leaves when no candidate
 // remains; a barrier that makes no progress for the spin limit sets the
@@ -54,6 +54,7 @@
 #include "device.hpp"
 #include "grid_sync.hpp"
 #include "kcore.hpp"
+#include "kcore_slots.hpp"
 
 #include <algorithm>
 #include <cstddef>
@@ -318,6 +319,13 @@ k_kcore(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__restri
     __shared__ uint32_t s_stage[KC_WAVES * KC_STAGE];
     __shared__ uint32_t s_hub[KC_HUBS];
     __shared__ uint32_t s_row[64];   // KC_HUB_ROWS flags, a wave's width for the ballot
+    __shared__ uint32_t s_dmin, s_dflushed, s_smin;
+    // the block's minima of the next iteration, by thread 0 and before a
+    // __syncthreads: other waves lower them without one
+    auto renew_minima = [&]() {
+        if (threadIdx.x == 0) s_dmin = s_dflushed = s_smin = ~0u;
+    };
+    renew_minima();
     for (uint32_t j = threadIdx.x; j < KC_HUBS; j += KC_THREADS) s_hub[j] = 0;
     if (threadIdx.x < 64) s_row[threadIdx.x] = 0;
     __syncthreads();
@@ -327,6 +335,10 @@ k_kcore(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__restri
     const unsigned long long wid = (unsigned long long)(threadIdx.x / 64) * gridDim.x + blockIdx.x;
     const bool leader = blockIdx.x == 0 && threadIdx.x == 0;
     KcStage st = {&s_stage[(threadIdx.x / 64) * KC_STAGE], 0u};
+    auto clear_counts = [&](unsigned slot) {
+        __hip_atomic_store(&ctl->nlight[slot], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&ctl->nheavy[slot], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
     // this wave's segment of the candidates.  The first pass takes, without
     // a list, the 64-vertex chunks wid, wid+W, wid+2W, ... (coalesced, and
     // every wave gets a share of every degree range: after relabelling by
@@ -338,7 +350,7 @@ k_kcore(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__restri
     uint32_t *seg = L.cand + wid * S;
     uint32_t cnt = (uint32_t)(wid < nchunks ? (nchunks - wid + W - 1) / W * 64 : 0ull);
     unsigned ph = 0;          // barriers passed
-    unsigned r = 0;           // rounds run
+    unsigned r = 0;           // the list in turn (kcore_slots.hpp): rounds run and passes but the first
     unsigned levels = 0;      // iterations with a non-empty frontier
     // K, the count of this iteration's frontier, never exceeds the smallest
     // count of a vertex not yet peeled: it is the minimum of the counts the
@@ -348,7 +360,6 @@ k_kcore(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__restri
     // round runs, and the minimum it kept is exact.
     uint32_t K = 0;
     unsigned long long my_edges = 0;
-    __shared__ uint32_t s_dmin, s_dflushed, s_smin;
     __shared__ uint32_t s_wcnt[KC_WAVES];
     __shared__ unsigned long long s_rd[2];
     __shared__ unsigned long long s_wbase[KC_WAVES];
@@ -368,24 +379,21 @@ k_kcore(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__restri
     bool ok = true;
     for (unsigned it = 0; ok; ++it) {
         const int s3 = it % 3;
+        if (it) r = kc_after_empty(r);
         if (leader) {
             // slot (it+1)%3 was last read after iteration it-2's last
             // barrier, so before iteration it-1's first; it is written next
             // in iteration it+1, after this iteration's barriers
             __hip_atomic_store(&ctl->kmin_s[(it + 1) % 3], ~0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(&ctl->kmin_d[(it + 1) % 3], ~0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        if (threadIdx.x == 0) {
-            s_dmin = ~0u;
-            s_dflushed = ~0u;
-            s_smin = ~0u;
+            clear_counts(kc_cleared_by_pass(r));
         }
         // the pass: count K -> this level's frontier; above K -> kept in the
         // segment (written at or below the position read, so in place), and
         // their smallest count; below K -> peeled before, dropped
         uint32_t smin = ~0u;
         {
-            const int c3 = r % 3, cb = r & 1;
+            const int c3 = kc_slot(r), cb = r & 1;
             uint32_t p = 0;
             for (uint32_t base = 0; base < cnt; base += 64 * KC_PU) {
                 uint32_t v[KC_U] = {0u, 0u, 0u, 0u}, c[KC_U];
@@ -438,12 +446,13 @@ k_kcore(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__restri
         mark(1);
         unsigned long long nq[2];   // the frontier's list lengths
         {
-            const int c3 = r % 3;
+            const int c3 = kc_slot(r);
             const unsigned long long *const p[2] = {&ctl->nlight[c3], &ctl->nheavy[c3]};
             block_read(p, s_rd, nq);
             if (nq[0] == 0 && nq[1] == 0) {
                 // no vertex at K: no round runs, the kept counts are exact
-                const uint32_t ks = (uint32_t)block_read_min(ctl->kmin_s[s3], ctl->kmin_s[s3], s_rd);
+                renew_minima();
+                const uint32_t ks = block_read_min(ctl->kmin_s[s3], ctl->kmin_s[s3], s_rd);
                 if (ks == ~0u) break;              // every vertex peeled
                 K = ks;
                 continue;
@@ -452,16 +461,10 @@ k_kcore(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__restri
         // rounds of level K
         uint32_t dmin = ~0u;   // per lane: counts decremented to above K
         for (;;) {
-            const int c3 = r % 3, cb = r & 1;
-            const int n3 = (r + 1) % 3, nb = (r + 1) & 1;
+            const int cb = r & 1, n3 = kc_slot(r + 1), nb = (r + 1) & 1;
             const unsigned long long nL = nq[0], nH = nq[1];
             if (nL == 0 && nH == 0) break;
-            if (leader) {
-                // slot (r+2)%3 was last read in round r-1
-                const int o3 = (r + 2) % 3;
-                __hip_atomic_store(&ctl->nlight[o3], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(&ctl->nheavy[o3], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
+            if (leader) clear_counts(kc_cleared_by_round(r));
             // light rows of a round that leaves most lanes idle otherwise:
             // KC_SUB lanes per vertex, so that a row is one step (a lane per
             // vertex takes up to eight, each a chain of a neighbour, a count
@@ -558,8 +561,9 @@ k_kcore(uint32_t n, const uint64_t *__restrict__ index, const uint32_t *__restri
         if (leader) {
             __hip_atomic_store(&ctl->kmax, K, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(&ctl->levels, levels, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&ctl->rounds, r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&ctl->rounds, r - it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
+        renew_minima();
         const uint32_t kn = block_read_min(ctl->kmin_s[s3], ctl->kmin_d[s3], s_rd);
         if (kn == ~0u) break;                      // nothing left above K
         K = kn;
