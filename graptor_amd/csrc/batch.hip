@@ -71,9 +71,12 @@ constexpr uint32_t BCC_LDS_V = 65536;
 constexpr uint32_t BCC_SPARSE_FIRST = 8;    // graphs a CU from which on pinned labels have an order of their own
 
 template <class P> struct Parents;
-// 16-bit parents packed two per 32-bit LDS word
+// 16-bit parents packed two per 32-bit LDS word, by IDs within the graph
 template <> struct Parents<uint16_t> {
     uint32_t *w;
+    uint32_t base;
+    __device__ uint32_t id(uint32_t v) const { return v; }
+    __device__ uint32_t label(uint32_t x) const { return base + x; }
     __device__ uint32_t get(uint32_t x) const {
         const uint32_t v = __hip_atomic_load(&w[x >> 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         return (x & 1) ? (v >> 16) : (v & 0xffffu);
@@ -103,8 +106,15 @@ template <> struct Parents<uint16_t> {
         return false;
     }
 };
+// Parents in memory, by global IDs: a parent never has a higher ID than its
+// vertex, whichever graph's workgroup wrote it.  (Graphs of a malformed batch
+// can overlap.  IDs within a graph would mean another vertex to each of them,
+// and lead out of the array or in circles.)
 template <> struct Parents<uint32_t> {
     uint32_t *w;
+    uint32_t base;
+    __device__ uint32_t id(uint32_t v) const { return base + v; }
+    __device__ uint32_t label(uint32_t x) const { return x; }
     __device__ uint32_t get(uint32_t x) const {
         return __hip_atomic_load(&w[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
@@ -200,7 +210,7 @@ __device__ bool link_rows(const PT &P, uint32_t base, uint32_t nv, uint32_t v0, 
             }
 #pragma unroll
         for (int k = 0; k < BCC_U; ++k)
-            if (x[k] > v0 + v[k] && x[k] < nv) uf_link(P, v0 + v[k], x[k]);
+            if (x[k] > v0 + v[k] && x[k] < nv) uf_link(P, P.id(v0 + v[k]), P.id(x[k]));
     }
     return true;
 }
@@ -220,7 +230,7 @@ __device__ void solve_graph(const PT &P, BccShare &S, uint32_t base, uint32_t nv
                             const uint64_t *__restrict__ index, const uint32_t *__restrict__ nbrs, uint64_t m,
                             uint32_t *labels) {
     if (threadIdx.x == 0) S.next = S.nheavy = 0;
-    for (uint32_t v = threadIdx.x; v < nv; v += BCC_THREADS) P.set(v, v);
+    for (uint32_t v = threadIdx.x; v < nv; v += BCC_THREADS) P.set(P.id(v), P.id(v));
     __syncthreads();
     // No branch in here is on the lane.  After one, the compiler can know of
     // the other lanes that they do not fetch, give them the fetch's default
@@ -242,7 +252,7 @@ __device__ void solve_graph(const PT &P, BccShare &S, uint32_t base, uint32_t nv
         link_rows(P, base, nv, __builtin_amdgcn_readfirstlane(S.heavy[k]),
                   __builtin_amdgcn_readfirstlane(threadIdx.x / 64), BCC_THREADS / 64, false, index, nbrs, m);
     __syncthreads();
-    for (uint32_t v = threadIdx.x; v < nv; v += BCC_THREADS) labels[base + v] = base + uf_find(P, v);
+    for (uint32_t v = threadIdx.x; v < nv; v += BCC_THREADS) labels[base + v] = P.label(uf_find(P, P.id(v)));
     __syncthreads();
 }
 
@@ -280,11 +290,11 @@ k_batch_cc(uint32_t count, uint32_t n, const uint32_t *__restrict__ work, const 
         if (end < base || end > n) continue;   // malformed offsets: the graph is skipped
         const uint32_t nv = end - base;
         if (nv <= BCC_LDS_V) {
-            Parents<uint16_t> P{words};
+            Parents<uint16_t> P{words, base};
             solve_graph(P, share, base, nv, index, nbrs, m, labels);
         } else {
-            // graphs are vertex-disjoint, so each owns its slice of gparent
-            Parents<uint32_t> P{gparent + base};
+            // each graph of a well-formed batch owns its slice of gparent
+            Parents<uint32_t> P{gparent, base};
             solve_graph(P, share, base, nv, index, nbrs, m, labels);
         }
     }
