@@ -67,6 +67,8 @@ constexpr int BCC_THREADS = 1024;
 constexpr int BCC_U = 2;              // 64-edge blocks of a wave in flight
 constexpr uint32_t BCC_HEAVY = 64;    // runs of 64 vertices left to all waves, at most
 constexpr uint32_t BCC_HEAVY_E = 4096;    // which have more edges than this
+constexpr uint64_t BCC_PIECE = 0xfff00000u;    // edges of a walk in 32-bit positions
+static_assert(BCC_PIECE % (64 * BCC_U * (BCC_THREADS / 64)) == 0, "every wave's steps end with the piece");
 constexpr uint32_t BCC_LDS_V = 65536;
 constexpr uint32_t BCC_SPARSE_FIRST = 8;    // graphs a CU from which on pinned labels have an order of their own
 
@@ -186,31 +188,35 @@ __device__ bool link_rows(const PT &P, uint32_t base, uint32_t nv, uint32_t v0, 
     const uint64_t b = min(index[base + v0 + (ln < rows ? ln : rows)], m);
     const uint64_t b0 = bcast64(b);
     const uint64_t e0 = min(index[base + v0 + rows], m);
-    const uint32_t len = e0 > b0 ? (uint32_t)min(e0 - b0, (uint64_t)0xfff00000u) : 0u;
-    if (defer && len > BCC_HEAVY_E) return false;
-    // row starts from b0 on, in order (a malformed batch's may not be: a
-    // wrong row, no other access)
-    const uint32_t st = b > b0 ? (uint32_t)min(b - b0, (uint64_t)0xffffffffu) : 0u;
-    const uint32_t *nb = nbrs + b0;
-    for (uint32_t i0 = part * (64 * BCC_U); i0 < len; i0 += parts * (64 * BCC_U)) {
-        uint32_t x[BCC_U], v[BCC_U];
-#pragma unroll
-        for (int k = 0; k < BCC_U; ++k) {
-            const uint32_t i = i0 + k * 64 + ln;
-            x[k] = i < len ? nb[i] - base : 0xffffffffu;
-            v[k] = 0;
-        }
-        // the last row that starts at or before the edge
-#pragma unroll
-        for (int h = 32; h > 0; h >>= 1)
+    const uint64_t all = e0 > b0 ? e0 - b0 : 0;
+    if (defer && all > BCC_HEAVY_E) return false;
+    // (32-bit positions within pieces of the walk; one, as a rule)
+    for (uint64_t off = 0; off < all; off += BCC_PIECE) {
+        const uint32_t len = (uint32_t)min(all - off, BCC_PIECE);
+        // row starts from the piece's on, in order (a malformed batch's may
+        // not be: a wrong row, no other access)
+        const uint32_t st = b > b0 + off ? (uint32_t)min(b - b0 - off, (uint64_t)0xffffffffu) : 0u;
+        const uint32_t *nb = nbrs + b0 + off;
+        for (uint32_t i0 = part * (64 * BCC_U); i0 < len; i0 += parts * (64 * BCC_U)) {
+            uint32_t x[BCC_U], v[BCC_U];
 #pragma unroll
             for (int k = 0; k < BCC_U; ++k) {
-                const uint32_t t = v[k] + h;   // <= 63
-                if (__shfl(st, t, 64) <= i0 + k * 64 + ln && t < rows) v[k] = t;
+                const uint32_t i = i0 + k * 64 + ln;
+                x[k] = i < len ? nb[i] - base : 0xffffffffu;
+                v[k] = 0;
             }
+            // the last row that starts at or before the edge
 #pragma unroll
-        for (int k = 0; k < BCC_U; ++k)
-            if (x[k] > v0 + v[k] && x[k] < nv) uf_link(P, P.id(v0 + v[k]), P.id(x[k]));
+            for (int h = 32; h > 0; h >>= 1)
+#pragma unroll
+                for (int k = 0; k < BCC_U; ++k) {
+                    const uint32_t t = v[k] + h;   // <= 63
+                    if (__shfl(st, t, 64) <= i0 + k * 64 + ln && t < rows) v[k] = t;
+                }
+#pragma unroll
+            for (int k = 0; k < BCC_U; ++k)
+                if (x[k] > v0 + v[k] && x[k] < nv) uf_link(P, P.id(v0 + v[k]), P.id(x[k]));
+        }
     }
     return true;
 }

@@ -1,7 +1,7 @@
-"""gpr_batch_cc_noalloc on batches that its host side cannot check: vertex
-ranges that overlap.  The labels of such a batch are not defined; the call
+"""gpr_batch_cc_noalloc at its limits.  Batches that its host side cannot
+check, with vertex ranges that overlap: the labels are not defined; the call
 returns, writes labels that are vertices of the batch, and leaves the next
-batch's labels right."""
+batch's labels right.  And 64 vertices with more edges than 32 bits count."""
 import ctypes as C
 
 import numpy as np
@@ -48,3 +48,25 @@ def test_overlapping_large_graphs(voff):
     src = np.repeat(np.arange(n, dtype=np.uint32), np.diff(index).astype(np.int64))[same]
     ix, nb = O.build_csr(n, src, nbrs[same], symmetrize=False)
     assert np.array_equal(noalloc(ix, nb, two), O.cc_labels(ix, nb))
+
+
+def test_rows_of_more_than_32_bits_of_edges():
+    """All but a few of vertex 0's edges lead to vertex 1; the others lie where positions in 32 bits would end and
+    behind."""
+    G.lib()
+    n, m = 100, (1 << 32) + 1000
+    if torch.cuda.mem_get_info()[0] < 5 * m:
+        pytest.skip("needs 20 GB of device memory")
+    nb = torch.ones(m, dtype=torch.int32, device="cuda")
+    for k, at in enumerate((0xFFF00000 - 1, 0xFFF00000, 0xFFF00000 + 5, (1 << 32) - 1, 1 << 32, m - 1)):
+        nb[at] = 10 + k
+    ix = torch.full((n + 1,), m, dtype=torch.int64, device="cuda")
+    ix[0] = 0
+    vo = torch.tensor([0, n], dtype=torch.int32, device="cuda")
+    lab = torch.full((n,), -1, dtype=torch.int32, device="cuda")
+    G._check(G.lib().gpr_batch_cc_noalloc(ix.data_ptr(), nb.data_ptr(), vo.data_ptr(), 1, n, lab.data_ptr(),
+                                          C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    torch.cuda.synchronize()
+    want = np.arange(n)
+    want[[0, 1, 10, 11, 12, 13, 14, 15]] = 0
+    assert np.array_equal(lab.cpu().numpy(), want)
