@@ -70,7 +70,6 @@ constexpr uint32_t BCC_HEAVY_E = 4096;    // which have more edges than this
 constexpr uint64_t BCC_PIECE = 0xfff00000u;    // edges of a walk in 32-bit positions
 static_assert(BCC_PIECE % (64 * BCC_U * (BCC_THREADS / 64)) == 0, "every wave's steps end with the piece");
 constexpr uint32_t BCC_LDS_V = 65536;
-constexpr uint32_t BCC_SPARSE_FIRST = 8;    // graphs a CU from which on pinned labels have an order of their own
 
 template <class P> struct Parents;
 // 16-bit parents packed two per 32-bit LDS word, by IDs within the graph
@@ -397,23 +396,31 @@ static int batch_finish(gpr_batch *b) {
     // Largest first, so that the queue does not end with a long graph.  Labels
     // that go over the link as graphs end keep it busy from the start if the
     // graphs with few edges a vertex, little work for their labels, come
-    // first, smallest first.  That delays no long graph much where there are
-    // many graphs a CU, all of one workgroup's kind, and the others alone keep
-    // the CUs busy for about as long as their largest takes: 2048 graphs with
-    // pinned labels take 2.83 ms instead of 3.02.  The kernel alone takes 2.19
-    // either way there; it could take a quarter longer where the largest graph
-    // starts late, so a run without pinned labels keeps the first order.
-    const uint32_t cus = (uint32_t)num_cus();
-    if (b->count >= BCC_SPARSE_FIRST * cus && b->max_nv <= BCC_LDS_V) {
+    // first, smallest first.  That delays no graph for long where all are of one
+    // workgroup's kind and the others alone keep the CUs busy for about as long
+    // as the batch's largest graph takes (LINK_BALANCE).  With pinned labels,
+    // largest first / like this, in ms: 1536 graphs of 1024 to 65536
+    // vertices 2.36 / 2.36, 2048 3.01 / 2.75, 3072 4.25 / 4.02; of 16384 to
+    // 65536, 1024 3.59 / 3.56, 2048 6.71 / 6.24; of 1024 to 16384, 1024 0.60 /
+    // 0.60, 4096 2.07 / 1.96.  The kernel alone takes the same either way there,
+    // and could take a quarter longer where the largest graph starts late, so a
+    // run without pinned labels keeps the first order.
+    // LINK_SPARSE, of the batch's mean edges a vertex: with 0.6 none of these is
+    // sparse enough, with 1.2 the dense ones are too few (both 3.02 ms at 2048).
+    // LINK_BALANCE: with 1 the 2048 graphs keep the first order (3.05 ms); with 4
+    // 1400 sparse graphs beside 100 of 60000 vertices and 1.8M edges take 3.50
+    // instead of 2.97.
+    constexpr double LINK_SPARSE = 0.9, LINK_BALANCE = 1.25;
+    if (b->count && b->max_nv <= BCC_LDS_V) {
         auto edges = [&](uint32_t g) { return idx[g + 1] - idx[g]; };
-        const double mean = 0.9 * (double)b->m / (double)std::max<uint32_t>(b->n, 1);
+        const double mean = LINK_SPARSE * (double)b->m / (double)std::max<uint32_t>(b->n, 1);
         std::vector<uint32_t> order(work);
         const auto rest = std::stable_partition(order.begin(), order.end(), [&](uint32_t g) {
             return (double)edges(g) < mean * (double)(b->hvoff[g + 1] - b->hvoff[g]);
         });
         uint64_t sum = 0;
         for (auto g = rest; g != order.end(); ++g) sum += edges(*g);
-        if (rest != order.end() && (double)edges(*rest) <= 1.25 * (double)sum / cus) {
+        if (rest != order.begin() && (double)edges(work[0]) <= LINK_BALANCE * (double)sum / num_cus()) {
             std::reverse(order.begin(), rest);
             GPR_TRY(dev_alloc((void **)&b->work_link, 4ull * b->count, "batch queue order"));
             GPR_HIP(hipMemcpy(b->work_link, order.data(), 4ull * b->count, hipMemcpyHostToDevice));

@@ -70,3 +70,27 @@ def test_rows_of_more_than_32_bits_of_edges():
     want = np.arange(n)
     want[[0, 1, 10, 11, 12, 13, 14, 15]] = 0
     assert np.array_equal(lab.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("sizes", [
+    [(40, 2)] * 700 + [(60, 8)] * 800,                      # others keep the CUs busy: sparse ones first
+    [(40, 2)] * 700 + [(5000, 8)] + [(60, 8)] * 300,        # the largest takes longer than the others
+    [(n, 2 if n % 2 else 9) for n in range(2, 1500)],
+    [(50, 4)] * 3, [(30, 6)],
+])
+def test_pinned_labels_in_either_queue_order(sizes):
+    G.lib()
+    rng = np.random.default_rng(len(sizes))
+    voff = np.concatenate(([0], np.cumsum([n for n, _ in sizes]))).astype(np.uint32)
+    at = np.repeat(voff[:-1], [n * d // 2 for n, d in sizes])
+    size = np.repeat([n for n, _ in sizes], [n * d // 2 for n, d in sizes])
+    src, dst = (at + (rng.random(len(at)) * size).astype(np.uint32) for _ in range(2))
+    index, nbrs = O.build_csr(int(voff[-1]), src.astype(np.uint32), dst.astype(np.uint32))
+    want = O.cc_labels(index, nbrs)
+    lab = torch.empty(len(want), dtype=torch.int32, pin_memory=True).numpy().view(np.uint32)
+    with G.Batch.from_csr(index, nbrs, voff) as b:
+        for _ in range(2):
+            lab[:] = 0xFFFFFFFF
+            G._check(G.lib().gpr_batch_cc(b.h, lab.ctypes.data_as(C.c_void_p), None))
+            assert np.array_equal(lab, want)
+            assert np.array_equal(b.cc()[0], want)
