@@ -973,10 +973,13 @@ k_cold_accum(const uint32_t *__restrict__ achunk, uint32_t n, const uint16_t *cd
 }
 
 constexpr int CC_THREADS = 1024;
-// Up to this many chunks in a bin their partials are added in one level: on a
-// directed graph of 1.5M vertices and 23M edges (17 to 64 chunks in its
-// largest bin) a run of 18 iterations takes 2.09 ms instead of 2.18 in two.  A 4M-vertex RMAT graph, whose hub bin has
-// more, takes 20 us longer over a run that way.
+// Up to this many chunks in a bin, the graph's largest, their partials are
+// added in one level: a launch less, until the hub bin's chain of loads is
+// longer than it.  Runs of 20 iterations in two levels / in one, in us, by the
+// chunks of the largest bin: uniform to skewed destinations 8 2306 / 2174, 27
+// 2188 / 2056, 42 2162 / 2043, 57 2118 / 1987, 82 2072 / 2057; directed RMAT 37
+// 1978 / 1872, 48 1495 / 1441; relabelled RMAT 102 4537 / 4644, 122 2765 / 2908,
+// 149 1696 / 1900.
 constexpr uint32_t COLD_ONE_LEVEL = 64;
 // workgroups per bin of the two combine kernels
 static uint32_t combine_per_bin(uint32_t n) { return (std::min(n, COLD_BIN) + CC_THREADS - 1) / CC_THREADS; }
