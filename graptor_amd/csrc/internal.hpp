@@ -72,12 +72,12 @@ void *host_target(void *host, size_t bytes, bool *copy_only = nullptr);
 // for its next run: a run makes and drops the same sizes every time, and
 // hipFree waits for the whole device (0.1 - 0.3 ms each for tens of MB;
 // hipMalloc 0.02 - 0.1).  A block is given back by size; the oldest go when
-// more than `cap` bytes or POOL_BLOCKS blocks are held, all of them when the
-// graph goes, and when an allocation of any graph fails.  The graph's stream
-// orders a block's next use behind its last one.
+// more than cap() bytes or POOL_BLOCKS blocks are held, all of them when the
+// graph goes, when an allocation of any graph fails, and when tunable
+// pool_vertex_bytes is set to 0.  The graph's stream orders a block's next use
+// behind its last one.
 constexpr size_t POOL_BLOCKS = 32;
-constexpr size_t POOL_BYTES = 256u << 20;    // held by a graph at most, or
-constexpr size_t POOL_VERTEX_BYTES = 64;     // this a vertex where it is more
+constexpr size_t POOL_BYTES = 256u << 20;    // held by a graph at most, or pool_vertex_bytes a vertex where it is more
 struct BufPool {
     BufPool();
     ~BufPool();
@@ -89,15 +89,19 @@ struct BufPool {
         std::lock_guard<std::mutex> lk(mu);
         return !closed;
     }
-    void bound(uint32_t n) { cap = std::max(POOL_BYTES, POOL_VERTEX_BYTES * n); }
+    void bound(uint32_t n) { vertices = n; }
 
   private:
+    size_t cap() const;
     struct Block { size_t bytes; void *p; };
     std::mutex mu;
     std::vector<Block> blocks;    // oldest first
-    size_t held = 0, cap = POOL_BYTES;
+    size_t held = 0;
+    uint32_t vertices = 0;
     bool closed = false;
 };
+
+bool trim_pools();    // every graph's; false if they held nothing
 
 // ---- runtime tunables (set by the autotuner through gpr_tune_set) --------
 struct Tunables {
@@ -106,6 +110,7 @@ struct Tunables {
     double push_blocks_per_cu = 32;           // push grid cap = CUs * this
     double pr_split_bytes = 0;                // FP32 bytes of pulled sources (0: all binned; >= 4n: no split)
     double pr_pull_edges = 1 << 23;           // graphs up to this many edges are pulled when pr_split_bytes is 0
+    double pool_vertex_bytes = 32;            // BufPool: bytes a vertex that a graph's runs keep (delta PageRank's take 24)
     double whole_edges = 1 << 24;             // default BFS and CC of graphs up to this many edges run whole on the device
     double fusion_spin_limit = 1 << 22;       // fused push: polls without progress before it gives up
     double fusion_blocks = 0;                 // fused push: cooperative grid size (0: one per CU)

@@ -45,7 +45,7 @@ static PoolList &pool_list() {
     static PoolList *l = new PoolList();
     return *l;
 }
-static bool trim_pools() {
+bool trim_pools() {
     PoolList &l = pool_list();
     std::lock_guard<std::mutex> lk(l.mu);
     bool any = false;
@@ -83,17 +83,22 @@ int BufPool::take(void **p, size_t bytes, const char *what) {
 void BufPool::give(void *p, size_t bytes) {
     if (!p) return;
     std::lock_guard<std::mutex> lk(mu);
-    if (closed || bytes > cap) {
+    const size_t most = cap();
+    if (closed || bytes > most) {
         dev_free(p);
         return;
     }
-    while (!blocks.empty() && (held + bytes > cap || blocks.size() >= POOL_BLOCKS)) {
+    while (!blocks.empty() && (held + bytes > most || blocks.size() >= POOL_BLOCKS)) {
         held -= blocks.front().bytes;
         dev_free(blocks.front().p);
         blocks.erase(blocks.begin());
     }
     blocks.push_back({bytes, p});
     held += bytes;
+}
+size_t BufPool::cap() const {
+    const double per = tun().pool_vertex_bytes;
+    return per > 0 ? std::max(POOL_BYTES, (size_t)(per * vertices)) : 0;
 }
 bool BufPool::trim() {
     std::lock_guard<std::mutex> lk(mu);
@@ -323,6 +328,7 @@ static double *tunable(const char *name) {
     if (!strcmp(name, "pr_split_bytes")) return &t.pr_split_bytes;
     if (!strcmp(name, "pr_pull_edges")) return &t.pr_pull_edges;
     if (!strcmp(name, "whole_edges")) return &t.whole_edges;
+    if (!strcmp(name, "pool_vertex_bytes")) return &t.pool_vertex_bytes;
     if (!strcmp(name, "fusion_spin_limit")) return &t.fusion_spin_limit;
     if (!strcmp(name, "fusion_blocks")) return &t.fusion_blocks;
     if (!strcmp(name, "pr_write_stage_cells")) return &t.pr_write_stage_cells;
@@ -343,6 +349,7 @@ extern "C" int gpr_tune_set(const char *name, double value) {
         return GPR_E_INVAL;
     }
     *p = value;
+    if (p == &tun().pool_vertex_bytes && value == 0) trim_pools();
     return GPR_OK;
 }
 

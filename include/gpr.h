@@ -501,6 +501,10 @@ int gpr_trace_get(const gpr_graph *g, gpr_iter_stats *out, int cap, int *k);
  *                       on which the host-driven run's pulls save more.  Levels, labels
  *                       and BFS's counts are the same; such a CC run is one
  *                       step in gpr_run_info
+ *   pool_vertex_bytes   device memory that a graph's runs keep for its next
+ *                       one: at most this many bytes a vertex, or 256 MB
+ *                       where that is more (default 32; 0: none, and what
+ *                       all graphs hold is freed)
  *   pull_serial_max     pull rows up to this in-degree run lane-serially
  *   pull_blocks_per_cu  pull grid size per compute unit, at most
  *   push_blocks_per_cu  push grid cap per compute unit
