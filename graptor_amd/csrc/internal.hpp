@@ -110,7 +110,8 @@ struct Tunables {
     double push_blocks_per_cu = 32;           // push grid cap = CUs * this
     double pr_split_bytes = 0;                // FP32 bytes of pulled sources (0: all binned; >= 4n: no split)
     double pr_pull_edges = 1 << 23;           // graphs up to this many edges are pulled when pr_split_bytes is 0
-    double pool_vertex_bytes = 32;            // BufPool: bytes a vertex that a graph's runs keep (delta PageRank's take 24)
+    double pool_vertex_bytes = 64;            // BufPool: bytes a vertex that a graph's runs keep (a 64-source BFS from 4 sources
+                                              // takes them; with 32, one source on 16M vertices took 2.24 ms, not 1.90)
     double whole_edges = 1 << 24;             // default BFS and CC of graphs up to this many edges run whole on the device
     double fusion_spin_limit = 1 << 22;       // fused push: polls without progress before it gives up
     double fusion_blocks = 0;                 // fused push: cooperative grid size (0: one per CU)

@@ -503,7 +503,7 @@ int gpr_trace_get(const gpr_graph *g, gpr_iter_stats *out, int cap, int *k);
  *                       step in gpr_run_info
  *   pool_vertex_bytes   device memory that a graph's runs keep for its next
  *                       one: at most this many bytes a vertex, or 256 MB
- *                       where that is more (default 32; 0: none, and what
+ *                       where that is more (default 64; 0: none, and what
  *                       all graphs hold is freed)
  *   pull_serial_max     pull rows up to this in-degree run lane-serially
  *   pull_blocks_per_cu  pull grid size per compute unit, at most
