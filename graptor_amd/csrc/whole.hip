@@ -573,11 +573,17 @@ constexpr uint32_t WHOLE_STAGE_V = 1u << 18;   // results up to this many vertic
 //   100000 of 150 198 / 169, 60000 of 250 186 / 159, but 30000 of 500 122 /
 //   184, 250000 of 30 283 / 283, 100000 of 60 208 / 211; RMAT 262144 of 55
 //   234 / 244 in its own order, relabelled 186 / 264;
-//   CC with hubs in their own order, from 2^24 edges on, or 2^23 and more
-//   than 2^20 vertices (a 4 MB L2 of parents): RMAT 33M edges 641 / 386, 31M
-//   378 / 243, 16.6M on 4M vertices 498 / 376, 15.5M on 0.5M 230 / 225.
+//   CC with hubs in their own order, from 2^24 edges and 2^16 vertices on, or
+//   3 2^22 edges and 2^20 vertices (a 4 MB L2 of parents).  RMAT, results left
+//   on the device: 33M edges on 4M vertices 641 / 386, 31M on 1M 378 / 243, 23M
+//   on 0.5M 274 / 224, 19M on 131072 240 / 171, but on 65536 175 / 202; 16.6M on
+//   4M 498 / 376, 12.4M on 2M 329 / 314, 15.5M on 0.5M 230 / 225.  Without a hub
+//   next to most of the graph it loses: 1000 hubs, each next to 12000 of 200000
+//   vertices, 303 / 452.
 static bool host_driven_better(const gpr_graph *g, bool cc) {
-    if (cc) return !g->order && g->nlong && (g->m > (1u << 24) || (g->m > (1u << 23) && g->n > (1u << 20)));
+    if (cc)
+        return !g->order && g->nlong && ((g->m > (1u << 24) && g->n > (1u << 16)) ||
+                                         (g->m > 3u << 22 && g->n > (1u << 20)));
     return g->m > (1u << 23) && g->n > (1u << 15) && g->m >= 32ull * g->n && !(g->order && g->nlong);
 }
 bool whole_run(const gpr_graph *g, const gpr_run_opts &o, bool cc) {
