@@ -1,12 +1,21 @@
-// grid_sync.hpp -- the grid-wide barrier of the persistent cooperative
-// launches (the fused push, the k-core peeling).
+// grid_sync.hpp -- workgroups of one launch that need each other's results.
+//
+//   last_workgroup   the ticket by which the last workgroup of a launch knows
+//                    that all others have stored theirs, and then folds their
+//                    partials (st_part, ld_part, part_sum) or scans their
+//                    counts (part_excl_scan): in reductions, frontier scans
+//                    and conversions, PageRank and delta PageRank tails;
+//   grid_barrier     the grid-wide barrier of the persistent cooperative
+//                    launches (the fused push, the k-core peeling), and
+//                    block_read, by which a block reads after it what all of
+//                    its waves need.
 //
 // Every word one block writes and another reads inside such a launch is
 // accessed with agent-scope atomics or coherent loads and stores; before
-// arriving at the barrier each wave waits until its memory operations are
-// acknowledged, so after the barrier every block sees them.  No
-// acquire/release fence is used: on this part each would write back or
-// invalidate an XCD's L2.
+// counting itself or arriving at the barrier each wave (for the ticket thread
+// 0, which stores the workgroup's results) waits until its memory operations
+// are acknowledged, so after it every block sees them.  No acquire/release
+// fence is used: on this part each would write back or invalidate an XCD's L2.
 #pragma once
 #include "device.hpp"
 
