@@ -593,12 +593,13 @@ bool whole_run(const gpr_graph *g, const gpr_run_opts &o, bool cc) {
     return cc ? o.fusion == 0 && g->symmetric && !(o.threshold_pct > 0.f) : o.fusion <= 0;
 }
 
-// A run's device memory: blocks of the graph's pool, which keeps them for the
-// next run, beside the graph's 8 (n+1) bytes of scan scratch.  Several blocks
-// rather than one, as hipMalloc takes 0.3 ms from 2 MB on and little below:
-// the first BFS of a fresh handle on 200000 vertices and 5.5M edges takes
-// 210 us, 530 with one block, 560 with buffers of its own and staging memory
-// made whatever the destination; host-driven 410.
+// A run's device memory: the graph's 8 (n+1) bytes of scan scratch, and blocks
+// of its pool, which keeps them for the next run.  Several blocks rather than
+// one, as hipMalloc takes 0.3 ms from 2 MB on and little below: the first BFS
+// of a fresh handle on 200000 vertices and 5.5M edges takes 210 us, 530 with
+// one block, 560 with buffers of its own and staging memory made whatever the
+// destination; host-driven 410.  A CC needs no block, but for labels in
+// pageable memory: 100 us there, 200 with its own buffers.
 struct WholeMem {
     gpr_graph *g;
     struct { void *p; size_t bytes; } used[4];
@@ -730,12 +731,16 @@ int whole_cc(gpr_graph *g, uint32_t *labels, gpr_run_info *info) {
     uint32_t *const target = (uint32_t *)host_target(labels, 4ull * n, &copy_only);
     uint32_t *out = target;
     if (labels && !out && !copy_only) out = whole_stage(g);
-    // the recode (labels asked for, vertices relabelled): minima by original ID
-    uint32_t *minorig = labels && g->order ? (uint32_t *)g->scan : nullptr;
-    if (labels && !out) out = (uint32_t *)g->scan + n;
+    // the scan scratch holds the parents and, with labels asked for, the
+    // recode's minima by original ID (vertices relabelled) or the labels that
+    // are copied; both, where there are such labels, want a block
+    uint32_t *parent = (uint32_t *)g->scan, *minorig = nullptr;
     WholeMem mem(g);
-    uint32_t *parent = nullptr;
-    GPR_TRY(mem.take(&parent, 4ull * n, "parents"));
+    if (labels && g->order) minorig = parent + n;
+    if (labels && !out) {
+        if (minorig) GPR_TRY(mem.take(&out, 4ull * n, "labels"));
+        else out = parent + n;
+    }
     const unsigned grid = grid_for(n, UF_THREADS, 4096);
     // The run's time ends before the labels go out.  Kernels write the clock
     // (clk) where labels follow: an event between them takes 5 of the 48 us of
